@@ -17,9 +17,9 @@ struct GemmArgs {
     long long sA, sB, sC;              // batch strides in elements
     int accumulate;
     const void* R;                     // optional residual with C's layout: C = R + A*B (accumulate must be 0)
-    int split;                         // > 1: K is cut into this many parts; part p > 0 assigns into partial[p-1]
+    int split;                         // > 1: K is cut into this many parts, see gemm_partial for where each one goes
     int k_part;                        // contraction length of one part (a multiple of the slab)
-    float* partial;                    // [batch][split-1][M][N] f32, summed into C by a second kernel
+    float* partial;                    // [batch][split - kPartsInC][M][N] f32, summed into C by a second kernel
     // SwiGLU-backward epilogue (gate != nullptr): the product is dH, the gradient of h = silu(gate) * up; C receives
     // dgate = dH * up * silu'(gate) and C2 receives dup = dH * silu(gate) (all with C's layout, no accumulation, no split-K)
     const void* gate;
@@ -127,6 +127,17 @@ __device__ __forceinline__ void block_tile(int lin, int m_tiles, int n_tiles, in
 template <int BMT, int BNT>
 __device__ __forceinline__ void xcd_block_tile(int lin, int m_tiles, int n_tiles, int& mt, int& nt) {
     block_tile<BMT, BNT>(xcd_contiguous_id(lin, m_tiles * n_tiles), m_tiles, n_tiles, mt, nt);
+}
+
+// The parts of a split contraction that go straight into C: the first one of an f32 result.  All parts of a bf16 result stay in
+// f32 until their sum (with the old C or the residual) is rounded, once, by the reduction.
+template <typename TC>
+constexpr int kPartsInC = sizeof(TC) == 4 ? 1 : 0;
+// where this part's tile goes instead of C; null: into C
+template <typename TC>
+__device__ __forceinline__ float* gemm_partial(const GemmArgs& g, int bz, int split, int part) {
+    if (split == 1 || part < kPartsInC<TC>) return nullptr;
+    return g.partial + ((long long)bz * (split - kPartsInC<TC>) + (part - kPartsInC<TC>)) * g.M * g.N;
 }
 
 // d(silu(gate) * up) for one element, given dh (src/graph/ops/elementwise.rs:442-455 for silu, :294-331 for mul)
@@ -241,10 +252,10 @@ struct TileEpilogueReads {
     Pack<bf16_t> first[TM][PASSES];
     Pack<bf16_t> second[SECOND ? TM : 1][SECOND ? PASSES : 1];
     bool have_first, have_second;
-    __device__ __forceinline__ void fetch(const GemmArgs& g, const bf16_t* Rsrc, bool add_old, int bz, int part, int m0, int n0, int wm, int wn, int lane) {
+    __device__ __forceinline__ void fetch(const GemmArgs& g, const bf16_t* Rsrc, bool add_old, int bz, int m0, int n0, int wm, int wn, int lane) {
         const bool gate = g.gate != nullptr && SECOND;
         // partial sums of a split contraction read nothing; unaligned C takes the scalar epilogue
-        const bool need = part == 0 && g.vec_c && (gate || (add_old && g.gate == nullptr));
+        const bool need = g.split <= 1 && g.vec_c && (gate || (add_old && g.gate == nullptr));
         have_first = need;
         have_second = need && gate;
         Pack<bf16_t> zero;
@@ -285,7 +296,7 @@ __device__ __forceinline__ void gemm_store_tile(const GemmArgs& g, f32x16 (&acc)
                                                 int wm, int wn, int lane, const PRE& pre = PRE{}) {
     constexpr bool kPre = !std::is_same<PRE, NoEpilogueReads>::value;  // pre.first / pre.second may hold what the staged epilogue reads
     constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
-    float* P = part > 0 ? g.partial + ((long long)bz * (split - 1) + (part - 1)) * g.M * g.N : nullptr;
+    float* P = gemm_partial<TC>(g, bz, split, part);
     constexpr int SP = WN + 4;  // staging pitch in floats
     constexpr bool kCanStage = LDS_BYTES >= (size_t)WGM * WGN * 32 * SP * sizeof(float);
     if (kCanStage && (EDGE || g.vec_c)) {

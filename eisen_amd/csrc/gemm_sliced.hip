@@ -72,7 +72,8 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
     constexpr int PASSES = ST * ST / 8 / (64 * W);               // groups of eight columns per thread
     TC* C = static_cast<TC*>(g.C) + (long long)bz * g.sC;
     const TC* Rsrc = g.R ? static_cast<const TC*>(g.R) + (long long)bz * g.sC : C;
-    const bool add_old = (g.accumulate || g.R != nullptr) && part == 0 && !g.gate;
+    float* P = gemm_partial<TC>(g, bz, split, part);
+    const bool add_old = (g.accumulate || g.R != nullptr) && !P && !g.gate;
     using Eight = LooseEight<TC>;
     Eight first[PASSES], second[PASSES];
 #pragma unroll
@@ -216,7 +217,6 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
                 for (int v = 0; v < 16; v++) mine[(i * 32 + 8 * (v / 4) + 4 * gh + (v % 4)) * ST + (j ^ gh) * 32 + c] = acc[i][j][v];
     }
     __syncthreads();
-    float* P = part > 0 ? g.partial + ((long long)bz * (split - 1) + (part - 1)) * g.M * g.N : nullptr;
 #pragma unroll
     for (int ps = 0; ps < PASSES; ps++) {
         const int idx = ps * 64 * W + tid, r = idx / 8, cg = idx % 8;

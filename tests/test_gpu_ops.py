@@ -773,6 +773,32 @@ def test_gemm_bf16_sliced_tiles_and_packed_rows(ctx, ta, tb, M, N, K):
     _gemm_case(ctx, M, N, K, ta, tb, BF16, F32, False)
 
 
+# Whole-number operands: every product and every f32 sum is exact (below 2^24), so a bf16 result has one right value, the exact
+# sum rounded once.  Split contractions (sliced tiles with whole and cut shapes and packed rows, 128 x 128 tiles), whose parts
+# must not be rounded before they are added, and one product that is not split.
+@pytest.mark.parametrize("batch,M,N,K,ta,tb,epilogue", [(*shape, e) for shape in [
+    (1, 512, 512, 2048, 0, 0), (1, 512, 512, 2048, 0, 1), (1, 264, 100, 4100, 1, 0), (1, 1351, 288, 4099, 0, 0), (1, 2048, 1024, 4096, 0, 1),
+    (3, 128, 256, 3072, 0, 0), (1, 256, 192, 1000, 0, 0)] for e in ("assign", "accumulate", "residual") if e != "residual" or shape[0] == 1])
+def test_gemm_bf16_result_is_rounded_once(ctx, batch, M, N, K, ta, tb, epilogue):
+    rng = np.random.default_rng(M + N + K)
+    a = rng.integers(-4, 5, (batch, K, M) if ta else (batch, M, K)).astype(np.float32)
+    b = rng.integers(-4, 5, (batch, N, K) if tb else (batch, K, N)).astype(np.float32)
+    old = rng.integers(-256, 257, (batch, M, N)).astype(np.float32)
+    exact = np.matmul(a.transpose(0, 2, 1) if ta else a, b.transpose(0, 2, 1) if tb else b)
+    if epilogue != "assign":
+        exact = exact + old
+    assert np.abs(exact).max() < 2 ** 24
+    da, db, do, dc = up(ctx, a, BF16), up(ctx, b, BF16), up(ctx, old, BF16), up(ctx, old if epilogue == "accumulate" else np.zeros_like(old), BF16)
+    if epilogue == "residual":
+        ctx.gemm_residual(da, db, do, dc, BF16, BF16, ta, tb, M, N, K)
+    else:
+        ctx.bmm(da, db, dc, BF16, BF16, ta, tb, batch, M, N, K, int(epilogue == "accumulate"))
+    got = dn(ctx, dc, (batch, M, N), BF16)
+    assert np.array_equal(got, hip.round_bf16(exact)), f"{int((got != hip.round_bf16(exact)).sum())} of {got.size} values differ from the exact sum rounded once"
+    for x in (da, db, do, dc):
+        x.free()
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("M,N,K", [(64, 64, 64), (33, 17, 29), (64, 256, 64)])
 def test_gemm_f32_and_odd_shapes(ctx, ta, tb, M, N, K):
