@@ -39,19 +39,21 @@ __device__ __forceinline__ void load_row(const float* row, int hd, int h, float 
 }
 // Column d = 32 dt + lane % 32 of the 32 rows at first_row, in the order of a score tile's registers.  Rows past the end
 // repeat the last one (their weight is zero).
+template <int K8, bool FULL>
+__device__ __forceinline__ void load_column(const float* base, long long stride, int first_row, int rows, int hd, int c, int h, int dt, float (&f)[16]) {
+    const bool whole = first_row + 32 <= rows;
+    const int d = 32 * dt + c;
+    const bool in = FULL ? (32 * dt + 32 <= 8 * K8 || d < 8 * K8) : d < hd;
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        const int r = first_row + acc_row(v, h);
+        f[v] = in ? base[(long long)(whole ? r : min(r, rows - 1)) * stride + d] : 0.f;
+    }
+}
 template <int K8, int DT, bool FULL>
 __device__ __forceinline__ void load_columns(const float* base, long long stride, int first_row, int rows, int hd, int c, int h, float (&f)[DT][16]) {
-    const bool whole = first_row + 32 <= rows;
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++) {
-        const int d = 32 * dt + c;
-        const bool in = FULL ? (32 * dt + 32 <= 8 * K8 || d < 8 * K8) : d < hd;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = first_row + acc_row(v, h);
-            f[dt][v] = in ? base[(long long)(whole ? r : min(r, rows - 1)) * stride + d] : 0.f;
-        }
-    }
+    for (int dt = 0; dt < DT; dt++) load_column<K8, FULL>(base, stride, first_row, rows, hd, c, h, dt, f[dt]);
 }
 // registers of a transposed result tile -> row `row` (d = 32 dt + 8 vg + 4 h + 0..3)
 template <int K8, bool FULL>
@@ -82,6 +84,46 @@ __device__ __forceinline__ f32x16 row_product(const float (&a)[K8][4], const flo
     return acc;
 }
 
+// Rows that are masked for a lane have weight zero in the second product, and zero times an Inf or NaN would still reach the
+// lane's result: a query must not depend on what stands in later rows of K and V, nor a key on earlier rows of Q and dO.  In
+// the tiles with masked pairs, values that are not finite are therefore taken out of the operand (two instructions each, in one
+// tile of a block's many), and if there were any (wave-uniform result) put_back_nonfinite() gives them to the lanes that do
+// see their row, behind the loop, where the registers are free.
+template <int DT>
+__device__ __forceinline__ bool take_out_nonfinite(float (&col)[DT][16]) {
+    bool found = false;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const bool finite = fabsf(col[dt][v]) < INFINITY;
+            found |= !finite;
+            col[dt][v] = finite ? col[dt][v] : 0.f;
+        }
+    return __builtin_amdgcn_ballot_w64(found) != 0;
+}
+// +-Inf for the weights P of V and dO, which are not negative (POSITIVE), NaN for the others and for NaN.
+template <bool POSITIVE, int K8, int DT, bool FULL, class Visible>
+__device__ __forceinline__ void put_back_nonfinite(const float* base, long long stride, int first_row, int rows, int hd, int c, int h, f32x16 (&acc)[DT],
+                                                   Visible visible) {
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) {
+        float x[16];
+        load_column<K8, FULL>(base, stride, first_row, rows, hd, c, h, dt, x);
+#pragma unroll
+        for (int sign = 0; sign < (POSITIVE ? 2 : 1); sign++) {
+            f32x16 seen = zero16();  // how many such values (of this sign, or NaN) the lane's row sees in each column
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const bool bad = !(fabsf(x[v]) < INFINITY) && !(POSITIVE && (sign == 0 ? x[v] < 0.f : x[v] > 0.f));
+                seen = __builtin_amdgcn_mfma_f32_32x32x2f32(bad ? 1.f : 0.f, visible(v) ? 1.f : 0.f, seen, 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[dt][v] += seen[v] > 0.f ? (!POSITIVE ? NAN : sign == 0 ? INFINITY : -INFINITY) : 0.f;
+        }
+    }
+}
+
 // workgroup -> (query block or key block, head, batch): heads and batches fastest, the longest causal blocks first
 struct RowBlock { int blk, head, b; };
 __device__ __forceinline__ RowBlock decode_block(int heads, int B, int n_blk, bool descending) {
@@ -110,6 +152,7 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_fwd_kernel(AttnArg
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) o[dt] = zero16();
     float m = -INFINITY, l = 0.f;  // m in units of log2
+    int odd_at = -1;               // first row of the tile that take_out_nonfinite() found something in
     const int n_kt = a.causal ? min(rb.blk + 1, (a.S + 31) / 32) : (a.S + 31) / 32;
     if (wave < n_kt) load_row<K8, FULL>(Kp + (long long)min(wave * 32 + c, a.S - 1) * a.k_ss, a.hd, h, kf);
     for (int kt = wave; kt < n_kt; kt += nw) {
@@ -122,6 +165,7 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_fwd_kernel(AttnArg
 #pragma unroll
             for (int v = 0; v < 16; v++)
                 if (acc_row(v, h) > lim) s[v] = -INFINITY;
+            if (take_out_nonfinite(vc)) odd_at = k0;
         }
         float mx = s[0];
 #pragma unroll
@@ -146,6 +190,10 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_fwd_kernel(AttnArg
         for (int v = 0; v < 16; v++)
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vc[dt][v], s[v], o[dt], 0, 0, 0);
+    }
+    if (odd_at >= 0) {
+        const int lim = (a.causal ? q : a.S - 1) - odd_at;
+        put_back_nonfinite<true, K8, DT, FULL>(Vp, a.k_ss, odd_at, a.S, a.hd, c, h, o, [&](int v) { return acc_row(v, h) <= lim; });
     }
     l += __shfl_xor(l, 32, 64);
     if (nw > 1) {  // the waves' keys are disjoint: (m, l, O) of each, added in wave order against the common maximum
@@ -222,6 +270,7 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_bwd_dq_kernel(Attn
     f32x16 dq[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) dq[dt] = zero16();
+    int odd_at = -1;  // see the forward kernel
     const int n_kt = a.causal ? min(rb.blk + 1, (a.S + 31) / 32) : (a.S + 31) / 32;
     auto fetch = [&](int kt) {
         const long long at = (long long)min(kt * 32 + c, a.S - 1) * a.k_ss;
@@ -242,11 +291,16 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_bwd_dq_kernel(Attn
 #pragma unroll
             for (int v = 0; v < 16; v++)
                 if (acc_row(v, h) > lim) s[v] = 0.f;
+            if (take_out_nonfinite(kc)) odd_at = k0;
         }
 #pragma unroll
         for (int v = 0; v < 16; v++)
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) dq[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(kc[dt][v], s[v], dq[dt], 0, 0, 0);
+    }
+    if (odd_at >= 0) {
+        const int lim = (a.causal ? q : a.S - 1) - odd_at;
+        put_back_nonfinite<false, K8, DT, FULL>(Kp, a.k_ss, odd_at, a.S, a.hd, c, h, dq, [&](int v) { return acc_row(v, h) <= lim; });
     }
     if (nw > 1) {
         if (wave > 0) {
@@ -300,6 +354,12 @@ __global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(A
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) dk[dt] = dv[dt] = zero16();
     const int qt_start = a.causal ? rb.blk : 0, per_head = n_t - qt_start, n_items = a.G * per_head;
+    auto masked_tile = [&](int q0) { return (a.causal && q0 < k0 + 31) || q0 + 32 > a.S; };
+    auto visible = [&](int q0, int v) {
+        const int r = q0 + acc_row(v, h);
+        return r < a.S && !(a.causal && k0 + c > r);
+    };
+    bool odd = false;
     for (int item = wave; item < n_items; item += nw) {
         const int hq = rb.head * a.G + item / per_head, q0 = (qt_start + item % per_head) * 32;
         const long long base = rb.b * a.q_sb + hq * a.q_sh;
@@ -322,13 +382,15 @@ __global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(A
         f32x16 dp = row_product<K8>(dor, vf, zero16());
 #pragma unroll
         for (int v = 0; v < 16; v++) s[v] = fast_exp2(fmaf(s[v], a.scale_log2e, -lse2[v] * kLog2e));
-        if (a.causal && q0 < k0 + 31) {
-#pragma unroll
-            for (int v = 0; v < 16; v++)
-                if (k0 + c > q0 + acc_row(v, h)) s[v] = 0.f;
-        }
 #pragma unroll
         for (int v = 0; v < 16; v++) dp[v] = s[v] * (dp[v] - D[v]) * a.scale;
+        if (masked_tile(q0)) {
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                if (!visible(q0, v)) s[v] = dp[v] = 0.f;  // (dp too: D of a masked query may be NaN)
+            const bool odd_do = take_out_nonfinite(doc), odd_q = take_out_nonfinite(qc);
+            odd |= odd_do || odd_q;
+        }
 #pragma unroll
         for (int v = 0; v < 16; v++)
 #pragma unroll
@@ -336,6 +398,15 @@ __global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(A
                 dv[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(doc[dt][v], s[v], dv[dt], 0, 0, 0);
                 dk[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(qc[dt][v], dp[v], dk[dt], 0, 0, 0);
             }
+    }
+    if (odd) {
+        for (int item = wave; item < n_items; item += nw) {
+            const int hq = rb.head * a.G + item / per_head, q0 = (qt_start + item % per_head) * 32;
+            const long long base = rb.b * a.q_sb + hq * a.q_sh;
+            if (!masked_tile(q0)) continue;
+            put_back_nonfinite<true, K8, DT, FULL>(static_cast<const float*>(a.dO) + base, a.q_ss, q0, a.S, a.hd, c, h, dv, [&](int v) { return visible(q0, v); });
+            put_back_nonfinite<false, K8, DT, FULL>(static_cast<const float*>(a.Q) + base, a.q_ss, q0, a.S, a.hd, c, h, dk, [&](int v) { return visible(q0, v); });
+        }
     }
     float* outs[2] = {static_cast<float*>(a.dK) + koff, static_cast<float*>(a.dV) + koff};
 #pragma unroll

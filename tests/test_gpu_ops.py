@@ -1337,6 +1337,55 @@ def test_attention_f32_head_sizes(ctx, B, S, Hq, Hkv, hd, causal, layout):
     _attn_case(ctx, F32, B, S, Hq, Hkv, hd, causal=causal, layout=layout)
 
 
+# A query must not depend on what later rows of K and V hold, nor a key on earlier rows of Q and dO, also where those rows share a
+# 32-row tile of the matrix-core kernels with what is visible and hold Inf or NaN (136: the plain kernels).  What the masked side
+# gets is compared bit by bit with the same input without the planted values.
+@pytest.mark.parametrize("S,Hq,Hkv,hd", [(70, 2, 1, 16), (70, 2, 1, 20), (300, 2, 2, 32), (100, 3, 3, 80), (70, 4, 1, 128), (70, 2, 1, 136)])
+def test_attention_f32_masked_rows_may_hold_anything(ctx, S, Hq, Hkv, hd):
+    sd = 1.0 / np.sqrt(hd)
+    clean = [gen.normal(560 + i, (1, S, h, hd), sd) for i, h in enumerate((Hq, Hkv, Hkv, Hq))]  # q, k, v, dO
+
+    def run(q, k, v, do, causal=True):
+        bufs = [up(ctx, np.ascontiguousarray(t), F32) for t in (q, k, v, do)]
+        out, lse, gq, gk, gv = (ctx.malloc(n * 4) for n in (q.size, Hq * S, q.size, k.size, v.size))
+        shape = (F32, 1, S, Hq, Hkv, hd, float(sd), causal)
+        ctx.attention_forward(*bufs[:3], out, lse, *shape)
+        ctx.attention_backward(*bufs[:3], out, bufs[3], lse, gq, gk, gv, *shape)
+        got = [dn(ctx, b, t.shape, F32) for b, t in ((out, q), (gq, q), (gk, k), (gv, v))]
+        for b in bufs + [out, lse, gq, gk, gv]:
+            b.free()
+        return got
+
+    o, dq, dk, dv = run(*clean)
+    for row in (S // 2 + 3, S - 1):
+        q, k, v, do = (t.copy() for t in clean)
+        v[0, row, 0, 3], v[0, row, 0, 5], v[0, row, 0, 6] = np.inf, -np.inf, np.nan
+        o1 = run(q, k, v, do)[0]
+        seen = o1[0, row:, : Hq // Hkv]
+        assert np.isposinf(seen[..., 3]).all() and np.isneginf(seen[..., 5]).all() and np.isnan(seen[..., 6]).all()
+        seen[..., [3, 5, 6]] = o[0, row:, : Hq // Hkv][..., [3, 5, 6]]
+        assert np.array_equal(o1, o), "a value of V reached a query or a column that does not see it"
+        k[0, row] = np.nan
+        k[0, row, 0, 0] = np.inf
+        o2, dq2, _, _ = run(q, k, v, do)
+        assert np.array_equal(o2[0, :row], o[0, :row]) and np.array_equal(dq2[0, :row], dq[0, :row])
+        assert not np.isfinite(o2[0, row:, : Hq // Hkv]).any() and not np.isfinite(dq2[0, row:, : Hq // Hkv]).any()
+        q, k, v, do = (t.copy() for t in clean)
+        do[0, row, 0, 3], do[0, row, 0, 5] = np.inf, -np.inf
+        dv3 = run(q, k, v, do)[3]
+        assert np.isposinf(dv3[0, : row + 1, 0, 3]).all() and np.isneginf(dv3[0, : row + 1, 0, 5]).all()
+        q[0, row, 0], do[0, row, 0] = np.nan, np.nan
+        _, dq4, dk4, dv4 = run(q, k, v, do)
+        assert np.array_equal(dk4[0, row + 1:], dk[0, row + 1:]) and np.array_equal(dv4[0, row + 1:], dv[0, row + 1:])
+        assert not np.isfinite(dk4[0, : row + 1, 0]).any() and not np.isfinite(dv4[0, : row + 1, 0]).any()
+        others = np.arange(S) != row
+        assert np.array_equal(dq4[0, others], dq[0, others])
+    # no mask: the rows behind the end of the last tile repeat its last row and must not turn its Inf into NaN
+    q, k, v, do = (t.copy() for t in clean)
+    v[0, S - 1, 0, 3] = np.inf
+    assert np.isposinf(run(q, k, v, do, causal=False)[0][0, :, : Hq // Hkv, 3]).all()
+
+
 def test_attention_f32_non_causal_and_reference_vector(ctx):
     _attn_case(ctx, F32, 1, 20, 2, 1, 8, causal=False)
     # tests/gpu_kernels.rs:403-429 and tests/cpu_attention_primitives.rs:70-87: fused == unfused, non-causal
