@@ -104,6 +104,21 @@ struct eisen_function {
 int eisen_set_error(eisen_ctx* ctx, int code, const char* fmt, ...);
 // Returns a device workspace of at least `bytes` (grow-only, stream-ordered reuse).
 int eisen_workspace(eisen_ctx* ctx, size_t bytes, void** out);
+// Scratch of one call, beyond what a context should keep: up to kWorkspaceKeep it is the workspace, a larger block comes from the
+// driver's pool on the active stream and goes back to it, in stream order, when the object goes out of scope.
+constexpr size_t kWorkspaceKeep = size_t(64) << 20;
+struct EisenScratch {
+    void* ptr = nullptr;
+    int get(eisen_ctx* ctx, size_t bytes);
+    ~EisenScratch();
+    EisenScratch() = default;
+    EisenScratch(const EisenScratch&) = delete;
+    EisenScratch& operator=(const EisenScratch&) = delete;
+
+  private:
+    void* own = nullptr;
+    hipStream_t stream = nullptr;
+};
 // Next pinned staging slot, grown to at least `bytes`; waits only if that slot's last copy is still in flight.
 int eisen_staging(eisen_ctx* ctx, size_t bytes, eisen_ctx::StageSlot** out);
 

@@ -225,6 +225,37 @@ extern "C" int eisen_hip_pool_stats(eisen_ctx* ctx, size_t* in_use_bytes, size_t
     return 0;
 }
 
+// A block of the driver's pool on the active stream.  Out of memory: what the free lists hold is given back and the request repeated once.
+static int driver_alloc(eisen_ctx* ctx, size_t bytes, const char* what, void** out) {
+    ctx->driver_allocs++;
+    hipError_t e = hipMallocAsync(out, bytes, ctx->stream);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(ctx->main_stream);  // the lists' blocks may still be in use on either stream
+        (void)hipStreamSynchronize(ctx->side_stream);
+        (void)eisen_hip_pool_trim(ctx);
+        (void)hipStreamSynchronize(ctx->stream);
+        e = hipMallocAsync(out, bytes, ctx->stream);
+    }
+    if (e != hipSuccess) {
+        *out = nullptr;
+        return eisen_set_error(ctx, EISEN_E_NOMEM, "%s of %zu bytes: %s", what, bytes, hipGetErrorString(e));
+    }
+    return 0;
+}
+
+int EisenScratch::get(eisen_ctx* ctx, size_t bytes) {
+    if (bytes <= kWorkspaceKeep) return eisen_workspace(ctx, bytes, &ptr);
+    const int rc = driver_alloc(ctx, bytes, "scratch", &own);
+    if (rc) return rc;
+    stream = ctx->stream;
+    ptr = own;
+    return 0;
+}
+EisenScratch::~EisenScratch() {
+    if (own) (void)hipFreeAsync(own, stream);
+}
+
 int eisen_workspace(eisen_ctx* ctx, size_t bytes, void** out) {
     // one block per stream: each is allocated, used and freed in the order of its own stream
     void*& ws = ctx->side_active ? ctx->ws_side : ctx->ws;
@@ -235,10 +266,8 @@ int eisen_workspace(eisen_ctx* ctx, size_t bytes, void** out) {
         ws = nullptr;
         ws_bytes = 0;
         size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
-        ctx->driver_allocs++;
-        hipError_t e = hipMallocAsync(&ws, want, ctx->stream);
-        if (e != hipSuccess)
-            return eisen_set_error(ctx, EISEN_E_NOMEM, "workspace of %zu bytes: %s", want, hipGetErrorString(e));
+        const int rc = driver_alloc(ctx, want, "workspace", &ws);
+        if (rc) return rc;
         ws_bytes = want;
     }
     *out = ws;

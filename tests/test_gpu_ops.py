@@ -799,6 +799,37 @@ def test_gemm_bf16_result_is_rounded_once(ctx, batch, M, N, K, ta, tb, epilogue)
         x.free()
 
 
+@pytest.mark.parametrize("side", [False, True])
+def test_gemm_large_packed_operand_is_not_kept(ctx, side):
+    # 8200 x 4099 bf16 rows that do not start on 16 bytes: a packed copy of 67 MB, more than a context keeps as its workspace
+    M, N, K = 8200, 64, 4099
+    rng = np.random.default_rng(5)
+    a, b = rng.integers(-4, 5, (M, K)).astype(np.float32), rng.integers(-4, 5, (K, N)).astype(np.float32)
+    da, db, dc = up(ctx, a, BF16), up(ctx, b, BF16), ctx.malloc(M * N * 2)
+    rt = C.CDLL("libamdhip64.so")
+    pool = C.c_void_p()
+    assert rt.hipDeviceGetDefaultMemPool(C.byref(pool), 0) == 0
+
+    def in_use():  # bytes of the driver's pool that are handed out (hipMemPoolAttrUsedMemCurrent)
+        ctx.sync()
+        used = C.c_uint64(0)
+        assert rt.hipMemPoolGetAttribute(pool, 7, C.byref(used)) == 0
+        return used.value
+
+    before = in_use()
+    for _ in range(2):
+        if side:
+            ctx.side_begin()
+        ctx.gemm(da, db, dc, BF16, BF16, 0, 0, M, N, K)
+        if side:
+            ctx.side_end()
+            ctx.side_wait()
+    assert in_use() - before < 32 << 20, "the packed copy stayed allocated"
+    assert np.array_equal(dn(ctx, dc, (M, N), BF16), hip.round_bf16(a @ b))
+    for x in (da, db, dc):
+        x.free()
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("M,N,K", [(64, 64, 64), (33, 17, 29), (64, 256, 64)])
 def test_gemm_f32_and_odd_shapes(ctx, ta, tb, M, N, K):
