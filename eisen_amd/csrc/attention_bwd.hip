@@ -43,7 +43,8 @@ __device__ __forceinline__ void mfma(f32x16& acc, const bf16x8& a, const bf16x8&
 
 // The same with the accumulator in AGPRs.  The compiler does not see an MFMA here, so what it would keep apart is kept apart by
 // hand: two wait states between the vector instruction that wrote an operand and the MFMA, and agpr_settle() between the
-// last MFMA and the first other reader of the accumulators.
+// last MFMA and the first other reader of the accumulators.  No copy and no spill of an accumulator may stand in the loop or
+// before the settling: the build reads the assembly and fails if one does (check_agpr_loops.py).
 __device__ __forceinline__ void mfma_agpr(f32x16& acc, const bf16x8& a, const bf16x8& b) {
     asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
