@@ -799,6 +799,17 @@ def test_gemm_bf16_result_is_rounded_once(ctx, batch, M, N, K, ta, tb, epilogue)
         x.free()
 
 
+# which kernel a weight gradient takes on either side of one 64 x 64 tile per CU, and two parts of unequal length
+@pytest.mark.parametrize("M,N,K,kernel", [(1024, 1024, 3840, "64x64x32_sliced"), (512, 2048, 3136, "64x64x32_sliced"), (768, 1536, 2496, "64x64x32_sliced"),
+                                          (768, 1536, 2624, "128x128x64_splitk"), (1152, 1024, 3136, "128x128x64_splitk"), (2048, 1024, 1088, "128x128x64_splitk")])
+def test_gemm_weight_gradient_route(ctx, M, N, K, kernel):
+    ctx.profile_start()
+    _gemm_case(ctx, M, N, K, 1, 0, BF16, F32, False)
+    _gemm_case(ctx, M, N, K, 1, 0, BF16, F32, True)
+    names = list(ctx.profile_stop())
+    assert names == [f"gemm_tn_bf16_f32out_{kernel}"], names
+
+
 @pytest.mark.parametrize("side", [False, True])
 def test_gemm_large_packed_operand_is_not_kept(ctx, side):
     # 8200 x 4099 bf16 rows that do not start on 16 bytes: a packed copy of 67 MB, more than a context keeps as its workspace
