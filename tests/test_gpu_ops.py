@@ -777,7 +777,7 @@ def test_gemm_bf16_sliced_tiles_and_packed_rows(ctx, ta, tb, M, N, K):
 # sum rounded once.  Split contractions (sliced tiles with whole and cut shapes and packed rows, 128 x 128 tiles), whose parts
 # must not be rounded before they are added, and one product that is not split.
 @pytest.mark.parametrize("batch,M,N,K,ta,tb,epilogue", [(*shape, e) for shape in [
-    (1, 512, 512, 2048, 0, 0), (1, 512, 512, 2048, 0, 1), (1, 264, 100, 4100, 1, 0), (1, 1351, 288, 4099, 0, 0), (1, 2048, 1024, 4096, 0, 1),
+    (1, 512, 512, 3072, 0, 0), (1, 512, 512, 3100, 0, 1), (1, 264, 100, 4100, 1, 0), (1, 1351, 288, 4099, 0, 0), (1, 2048, 1024, 4096, 0, 1),
     (3, 128, 256, 3072, 0, 0), (1, 256, 192, 1000, 0, 0)] for e in ("assign", "accumulate", "residual") if e != "residual" or shape[0] == 1])
 def test_gemm_bf16_result_is_rounded_once(ctx, batch, M, N, K, ta, tb, epilogue):
     rng = np.random.default_rng(M + N + K)
@@ -800,7 +800,8 @@ def test_gemm_bf16_result_is_rounded_once(ctx, batch, M, N, K, ta, tb, epilogue)
 
 
 # which kernel a weight gradient takes on either side of one 64 x 64 tile per CU, and two parts of unequal length
-@pytest.mark.parametrize("M,N,K,kernel", [(1024, 1024, 3840, "64x64x32_sliced"), (512, 2048, 3136, "64x64x32_sliced"), (768, 1536, 2496, "64x64x32_sliced"),
+@pytest.mark.parametrize("M,N,K,kernel", [(1024, 1024, 3840, "64x64x32_sliced"), (512, 2048, 3136, "64x64x32_sliced"), (768, 1536, 2496, "64x64x32_sliced"), (512, 512, 3040, "64x64x32_sliced"),
+                                          (512, 512, 3072, "64x64x32_sliced_splitk"),
                                           (768, 1536, 2624, "128x128x64_splitk"), (1152, 1024, 3136, "128x128x64_splitk"), (2048, 1024, 1088, "128x128x64_splitk")])
 def test_gemm_weight_gradient_route(ctx, M, N, K, kernel):
     ctx.profile_start()
