@@ -44,7 +44,7 @@ template <typename T, int THREADS, int VPT, bool WANT_ARGMAX, bool RAGGED>
 __global__ __launch_bounds__(THREADS) void ce_fused_kernel(const T* __restrict__ logits, const int32_t* __restrict__ targets,
                                                            T* __restrict__ dlogits, float* __restrict__ row_loss,
                                                            int32_t* __restrict__ argmax_out, float* __restrict__ target_logit_out,
-                                                           int classes, float scale) {
+                                                           int rows, int classes, float scale) {
     constexpr int N = Pack<T>::N;
     constexpr int W = THREADS / kWave;
     constexpr float kLog2e = 1.4426950408889634f;
@@ -94,7 +94,9 @@ __global__ __launch_bounds__(THREADS) void ce_fused_kernel(const T* __restrict__
     // keep loads in flight.  Running maximum (and, when asked for, its first index).
     Pack<T> raw[VPT];
     ArgMax am{-INFINITY, 0x7fffffff};
-    const long long left = (long long)(gridDim.x - row) * classes;  // elements from the row's start to the end of the buffer
+    // elements from the row's start to the end of the buffer (rows, not gridDim.x: a kernel that asks for the size of its grid gets
+    // hidden arguments, and filling those in cost 0.5 us of every launch)
+    const long long left = (long long)(rows - (int)row) * classes;
 #pragma unroll
     for (int v = 0; v < VPT; v++) {
         const int c = column(v);
@@ -205,8 +207,8 @@ __global__ __launch_bounds__(THREADS) void ce_fused_kernel(const T* __restrict__
     if (WANT_ARGMAX && threadIdx.x == 0 && argmax_out) argmax_out[row] = am.i;
 }
 
-// Generic row kernel for class counts that do not fit the register-resident variants, and
-// unaligned buffers and a few short rows: three passes over the row (the 2nd and 3rd hit L2).
+// Generic row kernel for class counts that do not fit the register-resident variants and for
+// unaligned buffers: three passes over the row (the 2nd and 3rd hit L2).
 template <typename T, int THREADS>
 __global__ __launch_bounds__(THREADS) void ce_generic_kernel(const T* __restrict__ logits, const int32_t* __restrict__ targets,
                                                              T* __restrict__ dlogits, float* __restrict__ row_loss,
@@ -281,26 +283,23 @@ void launch_fused(eisen_ctx* ctx, const void* logits, const int32_t* targets, vo
                   int32_t* argmax_out, float* target_logit_out, size_t rows, size_t classes, float scale) {
     if (argmax_out)
         ce_fused_kernel<T, THREADS, VPT, true, RAGGED><<<dim3((unsigned)rows), dim3(THREADS), 0, ctx->stream>>>(
-            (const T*)logits, targets, (T*)dlogits, row_loss, argmax_out, target_logit_out, (int)classes, scale);
+            (const T*)logits, targets, (T*)dlogits, row_loss, argmax_out, target_logit_out, (int)rows, (int)classes, scale);
     else
         ce_fused_kernel<T, THREADS, VPT, false, RAGGED><<<dim3((unsigned)rows), dim3(THREADS), 0, ctx->stream>>>(
-            (const T*)logits, targets, (T*)dlogits, row_loss, argmax_out, target_logit_out, (int)classes, scale);
+            (const T*)logits, targets, (T*)dlogits, row_loss, argmax_out, target_logit_out, (int)rows, (int)classes, scale);
 }
 
 template <typename T>
 int ce_dispatch(eisen_ctx* ctx, const void* logits, const int32_t* targets, void* dlogits, float* row_loss,
                 int32_t* argmax_out, float* target_logit_out, size_t rows, size_t classes, float scale) {
     constexpr int N = Pack<T>::N;
-    const bool buffers_aligned = eisen_aligned(logits, 16) && eisen_aligned(dlogits, 16), whole = classes % N == 0;
+    const bool whole = classes % N == 0;
     const size_t packets = whole ? classes / N : (classes + 2 * N - 2) / N;  // that a row may touch
 #define CE_ARGS ctx, logits, targets, dlogits, row_loss, argmax_out, target_logit_out, rows, classes, scale
 #define CE_FUSED(THREADS, VPT) do { if (whole) launch_fused<T, THREADS, VPT, false>(CE_ARGS); else launch_fused<T, THREADS, VPT, true>(CE_ARGS); } while (0)
     // one wave per row up to 256 packets (no barriers, and a row of 38 packets does not hold four waves): 16000 rows of 301 bf16
     // 17.1 us, 25.6 with 256 threads; 16000 x 1000 28.3 -> 19.8
-    // A few short rows that begin inside packets stay with the generic kernel: a grid of two rows per CU is all latency, and at
-    // 432 x 2316 bf16 loss and gradient take 8.4 us with it, 9.0 with the other (433 x 4099: the kernel alone 7.9 and 6.2).
-    const bool few = !whole && rows <= 512 && classes <= 2560;
-    const bool aligned = buffers_aligned && !few;
+    const bool aligned = eisen_aligned(logits, 16) && eisen_aligned(dlogits, 16);
     if (aligned && packets <= 64 * 1) CE_FUSED(64, 1);
     else if (aligned && packets <= 64 * 2) CE_FUSED(64, 2);
     else if (aligned && packets <= 64 * 4) CE_FUSED(64, 4);
