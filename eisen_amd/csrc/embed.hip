@@ -479,9 +479,11 @@ __global__ __launch_bounds__(kThreads) void scatter_runs_kernel(const T* __restr
 }
 
 // How a batch is sorted: chunks of 1024 << k ids, one workgroup each, whose keys (id, position in the chunk) fit 32 bits.  A
-// batch of up to 2048 ids is one chunk.  Beyond that several short chunks beat one long one (16384 ids: one workgroup's 105
-// bitonic steps over 16 registers against 66 steps over 2 and a merge of 8 chunks); from 65536 ids on the merge, whose searches
-// grow with the number of chunks, wants them long.  32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 us, of which sort 10,
+// batch of up to 2048 ids is one chunk, complete with one launch (2048 ids: 11.8 us for the index, 15.6 in two chunks).  Beyond that
+// short chunks and a merge beat one long bitonic network, the shorter ones up to where the merge's searches, which grow with the
+// number of chunks, outweigh the sort (chunks of 1024 / 2048 / 4096 / all in one, us for the index): 2049 ids 15.7 / 19.7 / 19.5,
+// 4096 16.6 / 20.8 / 20.2, 8192 17.7 / 21.9 / 29.8 / 39.6, 16384 20.3 / 24.4 / 32.6 / 85; with the scatter, 24000 ids 62.6 / 62.0, 32768 74.4 / 73.3,
+// 65536 141 / 130.  From 65536 ids on chunks of 16384.  32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 us, of which sort 10,
 // merge 11, list of runs 10, scatter 48; with the host's stable_sort and four rows of a run in flight 2790 us.
 struct ScatterPlan {
     int per_thread, shift;
@@ -490,9 +492,10 @@ struct ScatterPlan {
 constexpr size_t kIndexMax = size_t(1) << 20;
 bool scatter_plan(size_t n_ids, size_t vocab, ScatterPlan* plan) {
     if (n_ids == 0 || n_ids > kIndexMax) return false;
-    const int per_thread = n_ids <= 1024 ? 1 : n_ids <= 65536 ? 2 : 16;
+    const int per_thread = n_ids <= 1024 ? 1 : n_ids <= 2048 ? 2 : n_ids <= kSortMax ? 1 : n_ids <= 65536 ? 2 : 16;
     const int shift = per_thread == 1 ? 10 : per_thread == 2 ? 11 : 14;
-    if ((unsigned long long)vocab << shift >= 0xffffffffull) return false;
+    // (the vocabularies that are taken do not depend on which of the two shorter chunks the batch gets)
+    if ((unsigned long long)vocab << (n_ids <= 1024 ? 10 : std::max(shift, 11)) >= 0xffffffffull) return false;
     const size_t chunk = (size_t)kSortThreads * per_thread;
     *plan = ScatterPlan{per_thread, shift, chunk, eisen_ceil_div(n_ids, chunk)};
     return true;
