@@ -23,6 +23,7 @@
 //     No atomics anywhere: dQ has its own query-stationary pass, so results are reproducible.
 // f32: attention_f32.hip up to head_dim 128; beyond that one wave per query row / key row, plain FMA, for small shapes.
 #include <cmath>
+#include <cstdlib>
 #include <mutex>
 
 #include "attention_common.cuh"
@@ -779,6 +780,9 @@ int fill_args(eisen_ctx* ctx, AttnArgs& a, int dtype, size_t B, size_t S, size_t
     if (dtype == EISEN_BF16)
         EISEN_REQUIRE(ctx, a.q_sb % 8 == 0 && a.q_ss % 8 == 0 && a.q_sh % 8 == 0 && a.k_sb % 8 == 0 && a.k_ss % 8 == 0 && a.k_sh % 8 == 0,
                       EISEN_E_ALIGN, "%s: strides must be multiples of 8 elements for bf16", who);
+    // K / V tiles are addressed by a base and an unsigned 32-bit byte offset per lane, up to row 63
+    if (dtype == EISEN_BF16)
+        EISEN_REQUIRE(ctx, a.k_ss >= 0 && a.k_ss * 64 * 2 <= (1ll << 32), EISEN_E_SHAPE, "%s: sequence stride %lld of K and V outside [0, 2^25]", who, a.k_ss);
     // the key-stationary backward starts its score accumulators at -LSE / scale; a softmax scale is positive anyway
     EISEN_REQUIRE(ctx, std::isfinite(scale) && scale >= 1e-30f && scale <= 1e30f, EISEN_E_ARG, "%s: softmax scale %g is not a positive finite number", who, (double)scale);
     a.scale = scale;
@@ -954,6 +958,9 @@ static int attention_backward_common(eisen_ctx* ctx, const void* q, const void* 
         if (rc) return rc;
     }
     if (dtype == EISEN_BF16) {
+        // the rows of 32 queries: the same in the dQ kernel for head sizes up to 64, a signed element offset in fa_bwd_dkv_kernel
+        EISEN_REQUIRE(ctx, (a.q_ss >= 0 || hd > 64) && std::abs(a.q_ss) <= (1ll << 26), EISEN_E_SHAPE,
+                      "attention_backward: sequence stride %lld of Q is out of range (up to 2^26, not negative for head_dim up to 64)", a.q_ss);
         EISEN_REQUIRE(ctx, eisen_aligned(q, 16) && eisen_aligned(k, 16) && eisen_aligned(v, 16) && eisen_aligned(out, 16) &&
                                eisen_aligned(dout, 16) && eisen_aligned(dq, 16) && eisen_aligned(dk, 16) && eisen_aligned(dv, 16),
                       EISEN_E_ALIGN, "attention_backward: bf16 buffers must be 16-byte aligned");

@@ -1478,6 +1478,23 @@ def test_attention_bf16_layout_bhsd_and_non_causal(ctx):
     _attn_case(ctx, BF16, 1, 70, 2, 1, 128, causal=False)
 
 
+def test_attention_bf16_refuses_strides_it_cannot_address(ctx):
+    # refused before anything is launched: the small buffer is never touched
+    d = ctx.malloc(1 << 16)
+    def forward(q_ss, k_ss, hd=64):
+        ctx.attention_forward(d, d, d, d, d, BF16, 1, 128, 1, 1, hd, 0.125, True, (0, q_ss, hd), (0, k_ss, hd))
+    def backward(q_ss, k_ss, hd=64):
+        ctx.attention_backward(d, d, d, d, d, d, d, d, d, BF16, 1, 128, 1, 1, hd, 0.125, True, (0, q_ss, hd), (0, k_ss, hd))
+    for call in (forward, backward):
+        for k_ss in (-64, (1 << 25) + 8):
+            with pytest.raises(hip.EisenHipError, match="sequence stride"):
+                call(64, k_ss)
+    for q_ss, hd in ((-64, 64), ((1 << 26) + 8, 64), (-(1 << 26) - 8, 128), ((1 << 26) + 8, 128)):
+        with pytest.raises(hip.EisenHipError, match="sequence stride"):
+            backward(q_ss, 128, hd)
+    d.free()
+
+
 @pytest.mark.parametrize("dtype,B,S,Hq,Hkv,hd", [(BF16, 2, 70, 4, 2, 48), (BF16, 1, 70, 3, 3, 80), (F32, 1, 70, 4, 2, 48), (BF16, 2, 96, 4, 2, 64), (BF16, 1, 100, 8, 2, 64), (BF16, 2, 160, 8, 2, 32), (BF16, 1, 130, 2, 1, 128),
                                                  (F32, 2, 37, 4, 2, 16)])
 def test_attention_rope_backward(ctx, dtype, B, S, Hq, Hkv, hd):
