@@ -320,7 +320,7 @@ def test_rope_pair(ctx, dtype):
     (BF16, 2, 1, 1024, 512, 128, 256, 64),     # a K|V pair of 128 x 128 tiles: K rotated, V plain
     (BF16, 2, 2, 512, 256, 64, 128, 32),       # a Q|K pair, both rotated
     (BF16, 2, 1, 512, 64, 256, 256, 32),       # a narrow K|V pair on 64 x 64 tiles
-    (BF16, 2, 1, 96, 64, 40, 32, 16),          # ragged: the product, then the rotation in place
+    (BF16, 2, 1, 96, 64, 40, 32, 16),          # ragged: the rotation in the epilogue of cut tiles
     (BF16, 1, 0, 256, 128, 64, 64, 32),        # nothing to rotate
     (F32, 2, 1, 64, 32, 24, 16, 8),
 ], ids=["256x128", "kv_pair", "qk_pair", "kv_pair_64", "ragged", "plain", "f32"])
@@ -336,9 +336,9 @@ def test_gemm_rope_is_the_product_followed_by_the_rotation(ctx, case):
     ctx.profile_start()
     ctx.gemm_rope(dx, dw, got, dtype, batch, M, N, K, K * N, M * N, members, seq, hd)
     names = list(ctx.profile_stop())
-    # whole tiles of a kernel that stages C: one launch, no separate rotation
-    one_kernel = dtype == BF16 and members > 0 and M % 64 == 0 and N % 64 == 0 and K % 32 == 0
-    assert any(n.endswith("_rope") for n in names) == one_kernel and (not one_kernel or len(names) == 1), names
+    # bf16: the rotation runs in the product's epilogue, in cut tiles too: one launch, no separate rotation
+    one_kernel = dtype == BF16 and members > 0
+    assert any("_rope" in n for n in names) == one_kernel and (not one_kernel or len(names) == 1), names
     ctx.gemm_strided_batched(dx, dw, ref, dtype, dtype, 0, 0, batch, M, N, K, 0, K * N, M * N, 0)
     plain = dn(ctx, ref, (batch, M, N), dtype)
     for b in range(members):
@@ -811,6 +811,48 @@ def test_gemm_weight_gradient_route(ctx, M, N, K, kernel):
     assert names == [f"gemm_tn_bf16_f32out_{kernel}"], names
 
 
+# Operands whose rows do not start on 16 bytes, in the entry points beyond the plain product: sums of whole numbers are exact in
+# f32, so a result has one right value.
+@pytest.mark.parametrize("M,N,K", [(67, 35, 51), (130, 257, 1025), (40, 36, 3100), (2050, 1029, 37)])
+def test_gemm_bf16_residual_packed_rows(ctx, M, N, K):
+    rng = np.random.default_rng(M)
+    a, b, r = (rng.integers(-4, 5, shape).astype(np.float32) for shape in ((M, K), (K, N), (M, N)))
+    da, db, dr, dc = up(ctx, a, BF16), up(ctx, b, BF16), up(ctx, r, BF16), ctx.malloc(M * N * 2)
+    ctx.gemm_residual(da, db, dr, dc, BF16, BF16, 0, 0, M, N, K)
+    assert np.array_equal(dn(ctx, dc, (M, N), BF16), hip.round_bf16(a @ b + r))
+    ctx.gemm_residual(da, db, dr, dr, BF16, BF16, 0, 0, M, N, K)  # in place
+    assert np.array_equal(dn(ctx, dr, (M, N), BF16), hip.round_bf16(a @ b + r))
+    for x in (da, db, dr, dc):
+        x.free()
+
+
+@pytest.mark.parametrize("M,N,K", [(67, 35, 51), (130, 257, 129), (1030, 3003, 20)])
+def test_gemm_swiglu_backward_packed_rows(ctx, M, N, K):
+    test_gemm_swiglu_backward(ctx, M, N, K, BF16)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(33, 27, 45), (130, 65, 31), (64, 64, 3073)])
+@pytest.mark.parametrize("shared", ["none", "a", "b"])
+def test_bmm_bf16_packed_rows(ctx, ta, tb, M, N, K, shared):
+    batch = 3
+    rng = np.random.default_rng(M + K)
+    a = rng.integers(-4, 5, (1 if shared == "a" else batch,) + ((K, M) if ta else (M, K))).astype(np.float32)
+    b = rng.integers(-4, 5, (1 if shared == "b" else batch,) + ((N, K) if tb else (K, N))).astype(np.float32)
+    old = rng.integers(-64, 65, (batch, M, N)).astype(np.float32)
+    exact = np.matmul(a.transpose(0, 2, 1) if ta else a, b.transpose(0, 2, 1) if tb else b)
+    da, db = up(ctx, a, BF16), up(ctx, b, BF16)
+    for dtype in (F32, BF16):
+        dc = up(ctx, old, dtype)
+        for accumulate in (1, 0):
+            ctx.gemm_strided_batched(da, db, dc, BF16, dtype, ta, tb, batch, M, N, K, 0 if shared == "a" else M * K, 0 if shared == "b" else K * N, M * N, accumulate)
+            want = exact + old if accumulate else exact
+            assert np.array_equal(dn(ctx, dc, (batch, M, N), dtype), want if dtype == F32 else hip.round_bf16(want)), (dtype, accumulate)
+        dc.free()
+    for x in (da, db):
+        x.free()
+
+
 @pytest.mark.parametrize("side", [False, True])
 def test_gemm_large_packed_operand_is_not_kept(ctx, side):
     # 8200 x 4099 bf16 rows that do not start on 16 bytes: a packed copy of 67 MB, more than a context keeps as its workspace
@@ -847,7 +889,7 @@ def test_gemm_large_packed_operand_is_not_kept(ctx, side):
 def test_gemm_f32_and_odd_shapes(ctx, ta, tb, M, N, K):
     _gemm_case(ctx, M, N, K, ta, tb, F32, F32, False)
     _gemm_case(ctx, M, N, K, ta, tb, F32, F32, True)
-    _gemm_case(ctx, M, N, K, ta, tb, BF16, BF16, False)        # odd shapes fall back to the FMA kernel
+    _gemm_case(ctx, M, N, K, ta, tb, BF16, BF16, False)        # odd shapes: rows packed, cut tiles
 
 
 # f32 tiles: 64x64 (256 of them, last ones cut), 32x32, a split contraction whose last part is short, the same with rows
@@ -1077,9 +1119,9 @@ def test_side_stream_orders_after_fork_and_before_join(ctx):
                                     (2048, 256, (2048, 512, 3072)), (256, 2048, (256, 64, 64, 256, 1024, 1024)), (128, 1024, (64, 192))])
 @pytest.mark.parametrize("accumulate", [0, 1])
 def test_gemm_grouped_weight_gradients(ctx, M, K, Ns, accumulate):
-    # dW_p (+)= X_p^T dY_p with X_p [K, M] and dY_p [K, N_p] (here K is the token count): the first two shapes run as one
-    # grid of 128x128 tiles, the third falls back to one launch per product, the fourth is one grid of 176 tiles of 256x256, the last
-    # two (few 64x64 tiles, long contraction) one grid over products and parts of the contraction plus one reduction
+    # dW_p (+)= X_p^T dY_p with X_p [K, M] and dY_p [K, N_p] (here K is the token count).  (2048, 128, ...) and (2048, 192, ...) run as one
+    # grid of larger tiles, (2048, 256, ...) as one of 176 tiles of 256x256, the others (few 64x64 tiles) as one grid of sliced tiles
+    # over all products, (64, 3100, ...) over the parts of the contraction as well, with one reduction behind it
     xs = [prep(gen.normal(550 + i, (K, M)), BF16) for i in range(len(Ns))]
     dys = [prep(gen.normal(560 + i, (K, n)), BF16) for i, n in enumerate(Ns)]
     c0 = [gen.normal(570 + i, (M, n)).astype(np.float32) for i, n in enumerate(Ns)]
@@ -1154,6 +1196,64 @@ def test_gemm_leading_dimension_beyond_32_bit_lane_offsets(ctx, trans_b):
     exp = np.float32(K) * np.outer(np.array(a_row, np.float32), np.array(b_row, np.float32))
     assert np.array_equal(got, exp), f"trans_b={trans_b}: {int((got != exp).sum())} of {M * N} elements differ, first at {np.argwhere(got != exp)[:1]}"
     for x in (A, B, C):
+        x.free()
+
+
+# the same for few tiles, and batches whose products have 4 tiles of 64 x 64 but one of 128 x 128: gemm_mfma_kernel's 64 x 64 tiles
+@pytest.mark.parametrize("M,N", [(64, 64), (40, 72)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1)])
+def test_gemm_leading_dimension_beyond_32_bit_lane_offsets_few_tiles(ctx, M, N, ta, tb):
+    K = (1 << 22) + 64
+    a_row = np.array([2.0 ** ((i % 5) - 2) for i in range(M)], np.float32)
+    b_row = np.array([2.0 ** ((j % 3) - 1) for j in range(N)], np.float32)
+
+    def operand(row, along_k):  # [rows, K] with one value to a row, or K copies of one row
+        n = len(row)
+        buf = ctx.malloc(n * K * 2)
+        if along_k:
+            for i in range(n):
+                ctx.fill(buf.ptr + i * K * 2, BF16, float(row[i]), K)
+        else:
+            bits = hip.f32_to_bf16_bits(row)
+            ctx._call("eisen_hip_htod", C.c_void_p(buf.ptr), bits.ctypes.data_as(C.c_void_p), C.c_size_t(bits.nbytes))
+            done = 1
+            while done < K:
+                m = min(done, K - done)
+                ctx.dtod(buf.ptr + done * n * 2, buf, m * n * 2)
+                done += m
+        return buf
+
+    A, B = operand(a_row, not ta), operand(b_row, bool(tb))
+    exp = np.float32(K) * np.outer(a_row, b_row)
+    for dtype in (F32, BF16):
+        out = ctx.malloc(M * N * 4)
+        ctx.profile_start()
+        ctx.gemm(A, B, out, BF16, dtype, ta, tb, M, N, K)
+        names = list(ctx.profile_stop())
+        assert len(names) == 1 and names[0].endswith("64x64x32"), names
+        assert np.array_equal(dn(ctx, out, (M, N), dtype), exp if dtype == F32 else hip.round_bf16(exp))
+        out.free()
+    for x in (A, B):
+        x.free()
+    ctx.pool_trim()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_bmm_bf16_many_products_of_64x64_tiles(ctx, ta, tb):
+    batch, M, N, K = 160, 72, 88, 40
+    rng = np.random.default_rng(3)
+    a, b = (rng.integers(-4, 5, (batch, r, c)).astype(np.float32) for r, c in ((K, M) if ta else (M, K), (N, K) if tb else (K, N)))
+    exact = np.matmul(a.transpose(0, 2, 1) if ta else a, b.transpose(0, 2, 1) if tb else b)
+    da, db = up(ctx, a, BF16), up(ctx, b, BF16)
+    for dtype in (F32, BF16):
+        out = ctx.malloc(batch * M * N * 4)
+        ctx.profile_start()
+        ctx.bmm(da, db, out, BF16, dtype, ta, tb, batch, M, N, K)
+        names = list(ctx.profile_stop())
+        assert len(names) == 1 and names[0].endswith("64x64x32"), names
+        assert np.array_equal(dn(ctx, out, exact.shape, dtype), exact if dtype == F32 else hip.round_bf16(exact))
+        out.free()
+    for x in (da, db):
         x.free()
 
 
@@ -1476,6 +1576,41 @@ def test_attention_bf16_layout_bhsd_and_non_causal(ctx):
     # keys past the end of a ragged last tile, for the other two head sizes' LDS tile layouts
     _attn_case(ctx, BF16, 1, 200, 4, 2, 32, causal=False)
     _attn_case(ctx, BF16, 1, 70, 2, 1, 128, causal=False)
+
+
+# Rows of Q, dO, O and dQ 2^25 elements apart: the dK/dV kernel with 32-bit tile offsets does not take them, the other one does.
+# Same inputs in contiguous rows as the reference (the two kernels add the same products in another order).
+@pytest.mark.parametrize("hd", [16, 32, 48, 64, 80, 96, 112, 128])
+def test_attention_bf16_backward_with_rows_far_apart(ctx, hd):
+    S, Hq, Hkv, far, sd = 40, 2, 1, 1 << 25, 1.0 / np.sqrt(hd)
+    q, do = prep(gen.normal(570, (S, Hq, hd), sd), BF16), prep(gen.normal(571, (S, Hq, hd), sd), BF16)
+    k, v = prep(gen.normal(572, (S, Hkv, hd), sd), BF16), prep(gen.normal(573, (S, Hkv, hd), sd), BF16)
+    dk_, dv_ = up(ctx, k, BF16), up(ctx, v, BF16)
+    results = {}
+    for stride in (Hq * hd, far):
+        big = [ctx.malloc(((S - 1) * stride + Hq * hd) * 2 if stride < far else S * far * 2) for _ in range(4)]  # q, dO, O, dQ
+        for buf, x in zip(big, (q, do)):
+            bits = hip.f32_to_bf16_bits(x)
+            for s in range(S):
+                ctx._call("eisen_hip_htod", C.c_void_p(buf.ptr + s * stride * 2), bits[s].ctypes.data_as(C.c_void_p), C.c_size_t(bits[s].nbytes))
+        lse, gk, gv = ctx.malloc(Hq * S * 4), ctx.malloc(k.size * 2), ctx.malloc(v.size * 2)
+        strides = (0, stride, hd), (0, Hkv * hd, hd)
+        ctx.attention_forward(big[0], dk_, dv_, big[2], lse, BF16, 1, S, Hq, Hkv, hd, float(sd), True, *strides)
+        ctx.attention_backward(big[0], dk_, dv_, big[2], big[1], lse, big[3], gk, gv, BF16, 1, S, Hq, Hkv, hd, float(sd), True, *strides)
+        rows = [np.stack([dn(ctx, buf.ptr + s * stride * 2, (Hq, hd), BF16) for s in range(S)]) for buf in (big[2], big[3])]
+        results[stride] = rows + [dn(ctx, gk, k.shape, BF16), dn(ctx, gv, v.shape, BF16)]
+        for b in big + [lse, gk, gv]:
+            b.free()
+    near, apart = results.values()
+    assert np.array_equal(near[0], apart[0]) and np.array_equal(near[1], apart[1])
+    assert_close(apart[2], near[2], 2e-2, "dK")
+    assert_close(apart[3], near[3], 2e-2, "dV")
+    eo, edq, edk, edv = oracle_attention(q[None], k[None], v[None], do[None], np.float32(sd), True)
+    for name, got, want in zip(("O", "dQ", "dK", "dV"), apart, (eo, edq, edk, edv)):
+        assert_close(got, want[0], 2e-2, name)
+    for b in (dk_, dv_):
+        b.free()
+    ctx.pool_trim()
 
 
 def test_attention_bf16_refuses_strides_it_cannot_address(ctx):
