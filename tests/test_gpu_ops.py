@@ -799,9 +799,9 @@ def test_gemm_bf16_result_is_rounded_once(ctx, batch, M, N, K, ta, tb, epilogue)
         x.free()
 
 
-# which kernel a weight gradient takes on either side of one 64 x 64 tile per CU, and two parts of unequal length
-@pytest.mark.parametrize("M,N,K,kernel", [(1024, 1024, 3840, "64x64x32_sliced"), (512, 2048, 3136, "64x64x32_sliced"), (768, 1536, 2496, "64x64x32_sliced"), (512, 512, 3040, "64x64x32_sliced"),
-                                          (512, 512, 3072, "64x64x32_sliced_splitk"),
+# which kernel a weight gradient takes on either side of its lines (contraction length, tiles per CU), and two parts of unequal length
+@pytest.mark.parametrize("M,N,K,kernel", [(1024, 1024, 3008, "64x64x32_sliced"), (1024, 1024, 3072, "128x128x64_splitk"), (512, 2048, 3136, "128x128x64_splitk"), (768, 1536, 2496, "64x64x32_sliced"), (512, 512, 2016, "64x64x32_sliced"),
+                                          (512, 512, 2048, "64x64x32_sliced_splitk"),
                                           (768, 1536, 2624, "128x128x64_splitk"), (1152, 1024, 3136, "128x128x64_splitk"), (2048, 1024, 1088, "128x128x64_splitk")])
 def test_gemm_weight_gradient_route(ctx, M, N, K, kernel):
     ctx.profile_start()
