@@ -1,8 +1,8 @@
 // Fused softmax-cross-entropy forward+backward: one read of the logits, one write of dLogits.
 //
 // One workgroup owns one row.  The row is loaded once with 16-byte packets and stays in
-// registers (VPT packets per lane, widened to f32) across the three phases: row max (+ first
-// argmax when asked for), exponentials (computed once, kept) and their sum, gradient write.  Reductions are wave64 shuffles plus one LDS exchange
+// registers in its storage type (VPT packets per lane) across the three phases: row max (+ first
+// argmax when asked for), exponentials and their sum, gradient write (exponentials formed again).  Reductions are wave64 shuffles plus one LDS exchange
 // between the block's waves.  The row is read and its gradient written with streaming (non-temporal) accesses: each byte
 // is touched once, and keeping it out of the caches' way is worth 4-5 % at 8192 x 32000.  Per-row losses go to a buffer; a second one-block kernel sums
 // them in a fixed order, so the loss carries no float atomics and is reproducible.

@@ -16,7 +16,7 @@ struct FileCloser {
 void write_all(FILE* f, const void* p, size_t n, const std::string& path) {
     if (n && fwrite(p, 1, n, f) != n) throw Error("write to " + path + " failed: " + strerror(errno));
 }
-// host is little-endian (x86-64 / the GPU boxes); f32 and u64 go out as they lie in memory
+// host is little-endian (x86-64); f32 and u64 go out as they lie in memory
 static_assert(sizeof(float) == 4, "f32");
 }  // namespace
 

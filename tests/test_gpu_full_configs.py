@@ -1,4 +1,4 @@
-"""The BASELINE configurations at their real sizes on the GPU.
+"""The benchmark configurations at their real sizes on the GPU.
 
   config 5 (~1.1B: vocab 32000, d 2048, 16 layers, 32 q / 8 kv heads, ffn 5632, untied, 4 x 1024 tokens per micro-batch):
       the whole model, one micro-step: loss against an f64 host recomputation from the downloaded logits, the gradient
@@ -161,7 +161,7 @@ def test_config5_one_layer_full_width_against_the_oracle(ctx):
 
 
 def test_config4_real_micro_batch_against_the_oracle(ctx):
-    """Config 4 exactly as BASELINE states it: 6 layers, tied embeddings, Zipf ids, micro-batch 32 x seq 256 (8192 tokens, so
+    """Config 4 as it is benchmarked: 6 layers, tied embeddings, Zipf ids, micro-batch 32 x seq 256 (8192 tokens, so
     the tile and split-K choices of M = 8192 are the ones checked), bf16 mixed step against the f32 oracle at rtol 2e-2.
     Of the 2,097,152 elements of the tied embedding's gradient, a handful sit at the per-element bound 2e-2 (|e| + max |row|)
     (observed: one element at 1.03 x, which of them depends on the rounding order of the bf16 GEMMs): 2e-6 of a tensor's

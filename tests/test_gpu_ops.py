@@ -1,7 +1,7 @@
 """GPU parity tests: every C-ABI op against the CPU oracle on the same seeded inputs.
 
 Run on an MI355X with `pytest -m gpu`.  All calls go through libeisen_hip.so's C-ABI
-(eisen_amd.hip is a ctypes mirror of include/eisen_hip.h); the oracle is only the checker.
+(eisen_amd.hip is a ctypes mirror of include/eisen_hip.h); the oracle only checks.
 """
 import ctypes as C
 import os
@@ -640,7 +640,7 @@ def test_cross_entropy_reference_vector_and_ties(ctx):
 
 def test_cross_entropy_config2_full_size_against_the_oracle(ctx):
     """[8192 x 32000] bf16 (config 2), every row against the oracle (src/graph/ops/reduction.rs:668-716): the mean loss to
-    1e-3 relative (BASELINE config 2's bar), every row's loss, the gradient of all 8192 rows to 2e-2, argmax and target
+    1e-3 relative (config 2's bar), every row's loss, the gradient of all 8192 rows to 2e-2, argmax and target
     logit bit-exact on every row, and gradient rows summing to ~0."""
     rows, classes = 8192, 32000
     rng = np.random.default_rng(7)
