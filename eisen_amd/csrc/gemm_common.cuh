@@ -43,7 +43,7 @@ struct GemmArgs {
     const void* B_seg[2];
     int lda_seg[2], ldb_seg[2];
     int seg_end[2];
-    // Rotary-embedding epilogue (rope != nullptr; bf16 C, whole tiles, no accumulation, residual or split): the batch members
+    // Rotary-embedding epilogue (rope != nullptr; bf16 C, no accumulation or residual; of a split product in the reduction): the batch members
     // below rope_members leave as rope(A*B), row m at position m % rope_seq, heads of rope_head_dim columns (a multiple of 8)
     const float2* rope;                // cos/sin table [>= rope_seq][rope_head_dim / 2]
     int rope_seq, rope_head_dim, rope_members;

@@ -356,6 +356,23 @@ def test_gemm_rope_is_the_product_followed_by_the_rotation(ctx, case):
         t.free()
 
 
+@pytest.mark.parametrize("batch,members,M,N,K,seq,hd", [(1, 1, 128, 64, 4096, 64, 32), (2, 1, 256, 96, 2048, 64, 32), (1, 1, 2048, 1024, 4096, 256, 64)])
+def test_gemm_rope_has_the_bits_of_a_split_product_too(ctx, batch, members, M, N, K, seq, hd):
+    # products whose contraction eisen_hip_gemm cuts into parts: the order of its sums must not depend on the rotation behind it
+    x, w = _rand_bf16(660, (M, K), 0.5), _rand_bf16(661, (batch, K, N), 0.2)
+    dx, dw = up(ctx, x, BF16), up(ctx, w, BF16)
+    got, ref = ctx.malloc(batch * M * N * 2), ctx.malloc(batch * M * N * 2)
+    ctx.gemm_rope(dx, dw, got, BF16, batch, M, N, K, K * N, M * N, members, seq, hd)
+    ctx.gemm_strided_batched(dx, dw, ref, BF16, BF16, 0, 0, batch, M, N, K, 0, K * N, M * N, 0)
+    for b in range(members):
+        part = ref.ptr + b * M * N * 2
+        ctx.rope(part, part, BF16, M // seq, seq, N, hd)
+    a, e = dn(ctx, got, (batch, M, N), BF16), dn(ctx, ref, (batch, M, N), BF16)
+    assert np.array_equal(a, e), f"{int((a != e).sum())} of {a.size} values differ"
+    for t in (dx, dw, got, ref):
+        t.free()
+
+
 def test_rope_reference_vector(ctx):
     # tests/gpu_kernels.rs:485-513
     x = np.ones((1, 2, 4), np.float32)
