@@ -262,7 +262,7 @@ int eisen_hip_softmax_backward(eisen_ctx* ctx, const void* out, const void* go, 
  *   dW += X^T * dY (matmul_backward_b_f32, ops_f32.cu:225; linear.rs:278-287): trans_a=1, accumulate=1
  *   tied lm_head (matmul_trans_b_f32 / matmul_trans_a_f32, ops_f32.cu:842-882; linear.rs:301-517).
  * dtype_ab: element type of A and B; dtype_c: element type of C (f32 operands need f32 C).
- * bf16 operands run on MFMA with f32 accumulation; f32 operands on an FMA kernel. */
+ * bf16 and f32 operands run on the matrix cores with f32 accumulation; a bf16 result is the f32 sum (with the old C) rounded once. */
 int eisen_hip_gemm(eisen_ctx* ctx, const void* A, const void* B, void* C, int dtype_ab, int dtype_c, int trans_a,
                    int trans_b, size_t M, size_t N, size_t K, int accumulate);
 /* Batched form with contiguous batches (bmm_f32 and its four backward kernels,
@@ -327,7 +327,8 @@ int eisen_hip_gemm_swiglu_backward(eisen_ctx* ctx, const void* A, const void* B,
  * contraction length K_s (A_s is [M,K_s] or, transposed, [K_s,M]; B_s is [K_s,N] or [N,K_s]).  This is the
  * input gradient of several linear layers that read the same tensor (dX = dQ Wq^T + dK Wk^T + dV Wv^T, which
  * the reference accumulates with three matmul backward calls, src/graph/ops/linear.rs:266-277) as one launch
- * and one write of dX.  Segments that are not multiples of 64 run as consecutive accumulating GEMMs. */
+ * and one write of dX.  bf16 segments that are no multiples of 8 (of 64, from 512 tiles of 64 x 64 on) and f32 segments shorter
+ * than 4 or long enough to be split run as consecutive accumulating GEMMs. */
 int eisen_hip_gemm_ksegments(eisen_ctx* ctx, size_t n_segments, const void* const* A, const void* const* B, const size_t* K, void* C,
                              int dtype_ab, int dtype_c, int trans_a, int trans_b, size_t M, size_t N, int accumulate);
 
