@@ -483,7 +483,7 @@ __global__ __launch_bounds__(kThreads) void scatter_runs_kernel(const T* __restr
 // short chunks and a merge beat one long bitonic network, the shorter ones up to where the merge's searches, which grow with the
 // number of chunks, outweigh the sort (chunks of 1024 / 2048 / 4096 / all in one, us for the index): 2049 ids 15.7 / 19.7 / 19.5,
 // 4096 16.6 / 20.8 / 20.2, 8192 17.7 / 21.9 / 29.8 / 39.6, 16384 20.3 / 24.4 / 32.6 / 85; with the scatter, 24000 ids 62.6 / 62.0, 32768 74.4 / 73.3,
-// 65536 141 / 130.  From 65536 ids on chunks of 16384.  32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 us, of which sort 10,
+// 65536 141 / 130.  Beyond 65536 ids chunks of 16384.  32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 us, of which sort 10,
 // merge 11, list of runs 10, scatter 48; with the host's stable_sort and four rows of a run in flight 2790 us.
 struct ScatterPlan {
     int per_thread, shift;
