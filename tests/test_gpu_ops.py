@@ -1546,6 +1546,39 @@ def test_attention_f32_masked_rows_may_hold_anything(ctx, S, Hq, Hkv, hd):
     assert np.isposinf(run(q, k, v, do, causal=False)[0][0, :, : Hq // Hkv, 3]).all()
 
 
+# Beyond 8192 keys, where head sizes up to 128 have no limit: many key tiles per query block and offsets past 2^20, against float64
+# (row blocks, so that the host never holds a whole score matrix).
+@pytest.mark.parametrize("S,Hq,Hkv,hd", [(8230, 2, 1, 16), (8225, 1, 1, 128)])
+def test_attention_f32_long_sequence(ctx, S, Hq, Hkv, hd):
+    sd = 1.0 / np.sqrt(hd)
+    q, k, v, do = (gen.normal(590 + i, (1, S, h, hd), 1.0) for i, h in enumerate((Hq, Hkv, Hkv, Hq)))
+    bufs = [up(ctx, t, F32) for t in (q, k, v, do)]
+    out, lse, gq, gk, gv = (ctx.malloc(n * 4) for n in (q.size, Hq * S, q.size, k.size, v.size))
+    shape = (F32, 1, S, Hq, Hkv, hd, float(sd), True)
+    ctx.attention_forward(*bufs[:3], out, lse, *shape)
+    ctx.attention_backward(*bufs[:3], out, bufs[3], lse, gq, gk, gv, *shape)
+    got = [dn(ctx, b, t.shape, F32) for b, t in ((out, q), (gq, q), (gk, k), (gv, v))]
+    for b in bufs + [out, lse, gq, gk, gv]:
+        b.free()
+    want = [np.zeros(t.shape) for t in (q, q, k, v)]
+    for h in range(Hq):
+        g = h * Hkv // Hq
+        Q, K, V, dO = (t[0, :, i].astype(np.float64) for t, i in ((q, h), (k, g), (v, g), (do, h)))
+        for r in range(0, S, 1024):
+            e = min(S, r + 1024)
+            s = Q[r:e] @ K[:e].T * sd
+            s[np.arange(e)[None, :] > np.arange(r, e)[:, None]] = -np.inf
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            p /= p.sum(axis=1, keepdims=True)
+            o = p @ V[:e]
+            ds = p * (dO[r:e] @ V[:e].T - (dO[r:e] * o).sum(axis=1, keepdims=True)) * sd
+            want[0][0, r:e, h], want[1][0, r:e, h] = o, ds @ K[:e]
+            want[2][0, :e, g] += ds.T @ Q[r:e]
+            want[3][0, :e, g] += p.T @ dO[r:e]
+    for what, x, y in zip(("O", "dQ", "dK", "dV"), got, want):
+        assert_close(x, y.astype(np.float32), tol_for(F32), f"{what} S={S} hd={hd}")
+
+
 def test_attention_f32_non_causal_and_reference_vector(ctx):
     _attn_case(ctx, F32, 1, 20, 2, 1, 8, causal=False)
     # tests/gpu_kernels.rs:403-429 and tests/cpu_attention_primitives.rs:70-87: fused == unfused, non-causal
