@@ -17,6 +17,7 @@ struct GemmArgs {
     long long sA, sB, sC;              // batch strides in elements
     int accumulate;
     const void* R;                     // optional residual with C's layout: C = R + A*B (accumulate must be 0)
+    int blocks;                        // sliced kernel: workgroups of the launch
     int split;                         // > 1: K is cut into this many parts, see gemm_partial for where each one goes
     int k_part;                        // contraction length of one part (a multiple of the slab)
     float* partial;                    // [batch][split - kPartsInC][M][N] f32, summed into C by a second kernel
@@ -83,7 +84,7 @@ bool eisen_gemm_wide_window_supports(const WideWindow& w, const WideWindowRow* h
 void eisen_gemm_launch_wide_window(eisen_ctx* ctx, const WideWindow& w, unsigned tiles);
 
 // gemm_sliced.hip: bf16 operands, any shape, the contraction dealt to 4 or 8 waves (see there for what the operands must allow)
-void eisen_gemm_launch_sliced(eisen_ctx* ctx, const GemmArgs& g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c, unsigned group_tiles = 0);
+void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c);
 
 // gemm_f32.hip: f32 operands and result, any shape
 struct F32GemmPlan {
@@ -158,29 +159,37 @@ __device__ __forceinline__ bf16x8 zero_from(bf16x8 f, int k, int k_limit) {
     return f;
 }
 
-// Eight consecutive columns of a row of C at any alignment (one or two 16-byte accesses).
-template <typename TC>
-struct __attribute__((packed, aligned(sizeof(TC)))) LooseEight {
-    Pack<TC> p[8 / Pack<TC>::N];
-    __device__ __forceinline__ float get(int e) const { return p[e / Pack<TC>::N].get(e % Pack<TC>::N); }
-    __device__ __forceinline__ void set(int e, float v) { p[e / Pack<TC>::N].set(e % Pack<TC>::N, v); }
+// Eight consecutive columns of a row of C, at any alignment in memory (one or two 16-byte accesses) and in registers.  (A vector and
+// not a struct with an array: those end up in scratch memory where two paths read one element from the struct and from C.)
+template <typename TC> struct Eight;
+template <> struct Eight<bf16_t> {
+    typedef bf16x8 V;
+    typedef bf16x8 Loose __attribute__((aligned(2)));
 };
+template <> struct Eight<float> {
+    typedef float V __attribute__((ext_vector_type(8)));
+    typedef V Loose __attribute__((aligned(4)));
+};
+template <typename TC>
+__device__ __forceinline__ typename Eight<TC>::V load_eight(const TC* p) { return *reinterpret_cast<const typename Eight<TC>::Loose*>(p); }
+template <typename TC>
+__device__ __forceinline__ void store_eight(TC* p, typename Eight<TC>::V v) { *reinterpret_cast<typename Eight<TC>::Loose*>(p) = v; }
 
 // Row m, columns n..n+7 of the product, stored with whatever epilogue the launch asks for; columns from g.N on are left out.
 // P: the partial result goes there instead.  first: the old C or the residual (add_old), or gate, and second: up, for the
 // columns of a whole packet (a cut one reads its own).
 template <typename TC>
 __device__ __forceinline__ void gemm_store_eight(const GemmArgs& g, float (&val)[8], int m, int n, int bz, TC* C, const TC* Rsrc, bool add_old, float* P,
-                                                 const LooseEight<TC>& first, const LooseEight<TC>& second) {
+                                                 typename Eight<TC>::V first, typename Eight<TC>::V second) {
     const long long at = (long long)m * g.ldc + n;
     const bool whole = n + 8 <= g.N;
     if (P) {
         float* dst = P + (long long)m * g.N + n;
         if (whole) {
-            LooseEight<float> o;
+            Eight<float>::V o;
 #pragma unroll
-            for (int e = 0; e < 8; e++) o.set(e, val[e]);
-            *reinterpret_cast<LooseEight<float>*>(dst) = o;
+            for (int e = 0; e < 8; e++) o[e] = val[e];
+            store_eight(dst, o);
         } else {
 #pragma unroll
             for (int e = 0; e < 8; e++)
@@ -193,24 +202,31 @@ __device__ __forceinline__ void gemm_store_eight(const GemmArgs& g, float (&val)
         TC* d2 = static_cast<TC*>(g.C2) + in_batch;
         const TC* gs = static_cast<const TC*>(g.gate) + in_batch;
         const TC* us = static_cast<const TC*>(g.up) + in_batch;
-        LooseEight<TC> og, ou;
+        if (!whole) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (n + e < g.N) {
+                    first[e] = gs[e];
+                    second[e] = us[e];
+                }
+        }
+        typename Eight<TC>::V og, ou;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            float dgate = 0.f, dup = 0.f;
-            if (whole) swiglu_backward_elem(first.get(e), second.get(e), val[e], dgate, dup);
-            else if (n + e < g.N) swiglu_backward_elem(to_f32(gs[e]), to_f32(us[e]), val[e], dgate, dup);
-            og.set(e, dgate);
-            ou.set(e, dup);
+            float dgate, dup;
+            swiglu_backward_elem(to_f32(first[e]), to_f32(second[e]), val[e], dgate, dup);
+            og[e] = from_f32<TC>(dgate);
+            ou[e] = from_f32<TC>(dup);
         }
         if (whole) {
-            *reinterpret_cast<LooseEight<TC>*>(C + at) = og;
-            *reinterpret_cast<LooseEight<TC>*>(d2) = ou;
+            store_eight(C + at, og);
+            store_eight(d2, ou);
         } else {
 #pragma unroll
             for (int e = 0; e < 8; e++)
                 if (n + e < g.N) {
-                    C[at + e] = from_f32<TC>(og.get(e));
-                    d2[e] = from_f32<TC>(ou.get(e));
+                    C[at + e] = og[e];
+                    d2[e] = ou[e];
                 }
         }
         return;
@@ -229,10 +245,10 @@ __device__ __forceinline__ void gemm_store_eight(const GemmArgs& g, float (&val)
         }
     }
     if (whole) {
-        LooseEight<TC> o;
+        typename Eight<TC>::V o;
 #pragma unroll
-        for (int e = 0; e < 8; e++) o.set(e, add_old ? first.get(e) + val[e] : val[e]);
-        *reinterpret_cast<LooseEight<TC>*>(C + at) = o;
+        for (int e = 0; e < 8; e++) o[e] = from_f32<TC>(add_old ? to_f32(first[e]) + val[e] : val[e]);
+        store_eight(C + at, o);
     } else {
 #pragma unroll
         for (int e = 0; e < 8; e++)
@@ -344,13 +360,13 @@ __device__ __forceinline__ void gemm_store_tile(const GemmArgs& g, f32x16 (&acc)
                 const int m = m0 + wm * WM + i * 32 + r, n = n0 + wn * WN + cg * 8;
                 if constexpr (EDGE) {
                     if (m < g.M && n < g.N) {
-                        LooseEight<TC> first, second;
+                        typename Eight<TC>::V first = {}, second = {};
                         const long long at = (long long)m * g.ldc + n;
                         const bool whole = n + 8 <= g.N;
-                        if (whole && add_old && !P && !g.gate) first = *reinterpret_cast<const LooseEight<TC>*>(Rsrc + at);
+                        if (whole && add_old && !P && !g.gate) first = load_eight(Rsrc + at);
                         if (whole && g.gate) {
-                            first = *reinterpret_cast<const LooseEight<TC>*>(static_cast<const TC*>(g.gate) + (long long)bz * g.sC + at);
-                            second = *reinterpret_cast<const LooseEight<TC>*>(static_cast<const TC*>(g.up) + (long long)bz * g.sC + at);
+                            first = load_eight(static_cast<const TC*>(g.gate) + (long long)bz * g.sC + at);
+                            second = load_eight(static_cast<const TC*>(g.up) + (long long)bz * g.sC + at);
                         }
                         gemm_store_eight<TC>(g, val, m, n, bz, C, Rsrc, add_old, P, first, second);
                     }
@@ -518,6 +534,11 @@ __device__ __forceinline__ void load_to_lds_16(const void* src, bf16_t* lds_dst)
 __device__ __forceinline__ void load_to_lds_16(const void* base, unsigned lane_offset, bf16_t* lds_dst) {
     const unsigned lds_addr = (unsigned)(size_t)(lds_void_ptr)lds_dst;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(lane_offset), "s"(base) : "m0");
+}
+// the same, to OFFSET bytes behind an LDS address held as a (wave-uniform) number
+template <int OFFSET>
+__device__ __forceinline__ void load_to_lds_16_at(const void* base, unsigned lane_offset, unsigned lds_addr) {
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(lane_offset), "s"(base), "n"(OFFSET) : "m0", "scc");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads_but() {  // until at most N of this wave's vector memory loads are outstanding

@@ -3,11 +3,16 @@
 // The kernels of gemm.hip and gemm_wide.hip want whole tiles of 128 or 256 and enough of them to fill 256 CUs.  This one takes the
 // rest: odd batch and sequence lengths, head and vocabulary sizes that are no multiple of anything, and products with few
 // output tiles, whose time is latency (a wave of a shared tile waits for memory, then for a barrier, once per slab, with one
-// workgroup on the CU).  Here a wave owns the whole 64 x 64 tile for every W-th 32-deep slice of the contraction and a private
-// two-stage LDS ring filled by direct-to-LDS loads: no barrier in the loop, W independent chains per CU that cover each other's
-// waits, and even K = 256 keeps all of them busy.  The W partial tiles meet in LDS once, where a thread ends up with eight
-// consecutive columns of a row, so every epilogue works on 16-byte packets.  The price is LDS traffic (every operand byte is
-// written and read once per 64 x 64 tile and slice), which caps it near half of the matrix rate.
+// workgroup on the CU).  Here a wave owns the whole 64 x 64 tile for every W-th 64-deep slice of the contraction and a private
+// 16 KB of LDS filled by direct-to-LDS loads: no barrier in the loop, W independent chains per CU that cover each other's waits.  A
+// slice is read into registers as a whole, the loads of the wave's next one go out, and its 16 MFMAs run under them.  The W partial
+// tiles meet in LDS once, where a thread ends up with eight consecutive columns of a row, so every epilogue works on 16-byte packets.
+//
+// What bounds it: a CU fetches 256 bytes per contraction index for its tile, from an L2 that gives it about 40 bytes per clock; the
+// matrix cores would need 4 clocks for what that takes 6.  Long contractions of one tile per CU run at 0.6 PFLOP/s for that
+// reason, short ones at their latency (launch, first slice, meeting).  us with operands from memory, slices 32 deep in a two-stage
+// ring / now: 1024 x 1024 x 1024 NT 8.4 / 7.3, NN 9.0 / 7.9, x 4096 NT in two segments 22.5 / 18.2; 2048 x 768 x 4096 38.4 / 29.0;
+// 8192 x 256 x 256 7.6 / 6.5; 512 x 768 x 768 7.3 / 6.3; 201 x 256 x 1024 7.7 / 6.6; weight gradients 768 x 768 x 2048 12.6 / 12.0.
 //
 // Edges.  Rows (m, n) past the end re-read the last row or chunk: they only reach outputs that are not stored.  Contraction
 // indices past the end of a segment re-read the last one, and both fragments are zeroed there.  Operand rows must start on
@@ -16,147 +21,147 @@
 
 namespace {
 
-constexpr int ST = 64, SK = 32;  // tile rows and columns, depth of a slice
+constexpr int ST = 64, SK = 64;  // tile rows and columns, depth of a slice
 
-template <int W, bool A_KC, bool B_KC, typename TC>
+// One operand of a slice, 64 x 64 elements, into the LDS: eight loads of eight rows of 128 bytes, whole cache lines.  (Slices 32 deep read
+// half a line at a time of an operand stored along the contraction; the other half belonged to the next wave, and the L1 had
+// dropped the line by then more often than not: 1.5 times the L2 reads, which is what bounds this kernel for long contractions.)
+// The rows are operand rows or contraction indices, whichever way the operand is stored; row_last, chunk_last: the last ones that exist.
+__device__ __forceinline__ void load_slice(const bf16_t* base, int ld, unsigned tile, int row_last, int chunk_last, int lane) {
+    const int row = lane >> 3;  // of load 0; its chunk is permuted by the row, whose bit 3 is the load's parity
+    if (row_last >= 63 && chunk_last >= 7) {
+        unsigned off[2];
+#pragma unroll
+        for (int odd = 0; odd < 2; odd++) off[odd] = (unsigned)(row * ld + ((lane & 7) ^ lds_swz<128>(row + 8 * odd)) * 8) * 2u;
+        static_for<8>([&](auto i_c) {
+            constexpr int i = decltype(i_c)::value;
+            load_to_lds_16_at<i * 1024>(base + (long long)i * 8 * ld, off[i & 1], tile);
+        });
+    } else {
+        static_for<8>([&](auto i_c) {
+            constexpr int i = decltype(i_c)::value;
+            const int chunk = (lane & 7) ^ lds_swz<128>(row + 8 * i);
+            load_to_lds_16_at<i * 1024>(base, (unsigned)(min(row + 8 * i, row_last) * ld + min(chunk, chunk_last) * 8) * 2u, tile);
+        });
+    }
+}
+
+// What a launch is: one product (or a batch), a product whose contraction runs over several operand pairs, or several products.
+// A kernel per kind: the tables of the other kinds would be loaded into, and spilled from, scalar registers.
+// integer divisions leave values that are the same in every lane in vector registers
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+enum class Kind { kPlain, kSegments, kGroup };
+
+template <int W, bool A_KC, bool B_KC, typename TC, Kind KIND>
 __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
     using TA = DirectOperandTile<ST, A_KC, SK, 1>;
     using TB = DirectOperandTile<ST, B_KC, SK, 1>;
-    constexpr int NLOADS = TA::LOADS + TB::LOADS, STAGE = TA::ELEMS + TB::ELEMS;
-    static_assert(2 * STAGE * sizeof(bf16_t) == ST * ST * sizeof(float), "a wave's partial tile takes the place of its ring");
-    __shared__ __attribute__((aligned(1024))) bf16_t lds[W][2 * STAGE];
+    constexpr int STAGE = TA::ELEMS + TB::ELEMS, STEPS = SK / 16;
+    static_assert(STAGE * sizeof(bf16_t) == ST * ST * sizeof(float), "a wave's partial tile takes the place of its slice");
+    __shared__ __attribute__((aligned(1024))) bf16_t lds[W][STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blocks of 4 x 8 tiles, which share 12 operand panels, on one XCD
-    const int gx = gridDim.x, gy = gridDim.y;
-    const int lin = xcd_contiguous_id(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * gy * gridDim.z);
-    const int zz = lin / (gx * gy);
-    int nt = lin % (gx * gy), mt = 0;
-    if (g.ngroup == 0) block_tile<4, 8>(nt, gy, gx, mt, nt);
-    if (g.ngroup > 0) {  // which product this tile belongs to (uniform); static indices keep the tables in scalar registers
-        const int t = nt;
+    const int split = g.split > 1 ? g.split : 1;
+    int nt, mt = 0, zz;
+    if constexpr (KIND == Kind::kGroup) {  // which product this tile belongs to (uniform); static indices keep the tables in scalar registers
+        const int tiles = g.grp_tile_end[kMaxGroup - 1];
+        const int lin = xcd_contiguous_id(blockIdx.x, tiles * split);
+        zz = uniform(lin / tiles);
+        const int t = lin - zz * tiles;
         int first = 0;
         long long partial_off = g.grp_partial_off[0];
         g.A = g.grp_A[0]; g.B = g.grp_B[0]; g.C = g.grp_C[0]; g.N = g.grp_N[0];
 #pragma unroll
         for (int q = 1; q < kMaxGroup; q++)
-            if (q < g.ngroup && t >= g.grp_tile_end[q - 1]) {
+            if (t >= g.grp_tile_end[q - 1]) {
                 first = g.grp_tile_end[q - 1];
                 partial_off = g.grp_partial_off[q];
                 g.A = g.grp_A[q]; g.B = g.grp_B[q]; g.C = g.grp_C[q]; g.N = g.grp_N[q];
             }
-        if (g.split > 1) g.partial += partial_off;
+        if (split > 1) g.partial += partial_off;
         const int n_tiles = (g.N + ST - 1) / ST;
         mt = (t - first) / n_tiles;
         nt = (t - first) % n_tiles;
         g.ldc = g.N;
         if (!B_KC) g.ldb = g.N;
+    } else {
+        const int gx = (g.N + ST - 1) / ST, gy = (g.M + ST - 1) / ST;
+        const int lin = xcd_contiguous_id(blockIdx.x, g.blocks);
+        zz = uniform(lin / (gx * gy));
+        block_tile<4, 8>(lin - zz * (gx * gy), gy, gx, mt, nt);
     }
-    const int m0 = mt * ST, n0 = nt * ST;
-    const int split = g.split > 1 ? g.split : 1;
-    const int bz = zz / split, part = zz % split;
+    const int m0 = uniform(mt * ST), n0 = uniform(nt * ST);
+    const int bz = uniform(zz / split), part = uniform(zz % split);
     const bf16_t* A = static_cast<const bf16_t*>(g.A) + (long long)bz * g.sA;
     const bf16_t* B = static_cast<const bf16_t*>(g.B) + (long long)bz * g.sB;
 
     // Slices of the contraction: segment by segment, each with a last slice of its own.  This workgroup's are [s_lo, s_hi).
-    const int len0 = g.nseg > 1 ? g.seg_end[0] : g.K;
+    constexpr bool SEG = KIND == Kind::kSegments;
+    const int len0 = SEG ? g.seg_end[0] : g.K;
     const int sl0 = (len0 + SK - 1) / SK;
-    const int len1 = g.nseg > 2 ? g.seg_end[1] - g.seg_end[0] : g.nseg > 1 ? g.K - g.seg_end[0] : 0, sl1 = (len1 + SK - 1) / SK;
-    const int len2 = g.nseg > 2 ? g.K - g.seg_end[1] : 0, sl2 = (len2 + SK - 1) / SK;
+    const int len1 = !SEG ? 0 : g.nseg > 2 ? g.seg_end[1] - g.seg_end[0] : g.K - g.seg_end[0], sl1 = (len1 + SK - 1) / SK;
+    const int len2 = SEG && g.nseg > 2 ? g.K - g.seg_end[1] : 0, sl2 = (len2 + SK - 1) / SK;
+    const bf16_t *A1 = nullptr, *A2 = nullptr, *B1 = nullptr, *B2 = nullptr;
+    int lda1 = 0, lda2 = 0, ldb1 = 0, ldb2 = 0;
+    const int lda0 = g.lda, ldb0 = g.ldb;
+    if constexpr (SEG) {
+        A1 = static_cast<const bf16_t*>(g.A_seg[0]); A2 = static_cast<const bf16_t*>(g.A_seg[1]);
+        B1 = static_cast<const bf16_t*>(g.B_seg[0]); B2 = static_cast<const bf16_t*>(g.B_seg[1]);
+        lda1 = g.lda_seg[0]; lda2 = g.lda_seg[1];
+        ldb1 = g.ldb_seg[0]; ldb2 = g.ldb_seg[1];
+    }
     const int s_lo = part * (g.k_part / SK), s_hi = split > 1 ? min(sl0, s_lo + g.k_part / SK) : sl0 + sl1 + sl2;
     const int n_mine = s_hi - s_lo > wave ? (s_hi - s_lo - wave + W - 1) / W : 0;
     const int n_parts = min(W, s_hi - s_lo);  // waves with something to add
 
-    // What the epilogue reads (the old C or the residual; gate and up) is requested first.
+    bf16_t* As = lds[wave];
+    bf16_t* Bs = As + TA::ELEMS;
+    const int m_last = g.M - 1 - m0, n_last = g.N - 1 - n0;  // last row of the tile that exists
+    const unsigned lds_a = uniform((int)(size_t)(lds_void_ptr)As), lds_b = lds_a + TA::ELEMS * 2;  // their LDS addresses
+    // the loads of this wave's i-th slice; returns how many of its contraction indices exist
+    auto issue = [&](int i) __attribute__((always_inline)) -> int {
+        int s = s_lo + wave + i * W, lda = lda0, ldb = ldb0, len = len0;
+        const bf16_t* Ap = A;
+        const bf16_t* Bp = B;
+        if (SEG && s >= sl0) {
+            s -= sl0;
+            Ap = A1; Bp = B1; lda = lda1; ldb = ldb1; len = len1;
+            if (s >= sl1) {
+                s -= sl1;
+                Ap = A2; Bp = B2; lda = lda2; ldb = ldb2; len = len2;
+            }
+        }
+        const int k0 = s * SK, left = len - k0;
+        load_slice(A_KC ? Ap + (long long)m0 * lda + k0 : Ap + (long long)k0 * lda + m0, lda, lds_a, A_KC ? m_last : left - 1, (A_KC ? left - 1 : m_last) / 8, lane);
+        load_slice(B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0, ldb, lds_b, B_KC ? n_last : left - 1, (B_KC ? left - 1 : n_last) / 8, lane);
+        return min(left, SK);
+    };
+
+    int left = 0;
+    if (n_mine > 0) left = issue(0);
+
+    // What the epilogue reads (the old C or the residual; gate and up) is requested behind the first slice (in front of it, the branches
+    // around these loads would make every wave wait for them before it asks for an operand).
     constexpr int PASSES = ST * ST / 8 / (64 * W);               // groups of eight columns per thread
     TC* C = static_cast<TC*>(g.C) + (long long)bz * g.sC;
     const TC* Rsrc = g.R ? static_cast<const TC*>(g.R) + (long long)bz * g.sC : C;
     float* P = gemm_partial<TC>(g, bz, split, part);
     const bool add_old = (g.accumulate || g.R != nullptr) && !P && !g.gate;
-    using Eight = LooseEight<TC>;
-    Eight first[PASSES], second[PASSES];
-#pragma unroll
-    for (int ps = 0; ps < PASSES; ps++) {
+    typename Eight<TC>::V first[PASSES] = {}, second[PASSES] = {};
+    static_for<PASSES>([&](auto ps_c) {
+        constexpr int ps = decltype(ps_c)::value;
         const int idx = ps * 64 * W + tid, m = m0 + idx / 8, n = n0 + (idx % 8) * 8;
         const bool whole = m < g.M && n + 8 <= g.N;
         const long long at = (long long)m * g.ldc + n;
-        if (whole && add_old) first[ps] = *reinterpret_cast<const Eight*>(Rsrc + at);
+        if (whole && add_old) first[ps] = load_eight(Rsrc + at);
         if (whole && g.gate) {
-            first[ps] = *reinterpret_cast<const Eight*>(static_cast<const TC*>(g.gate) + (long long)bz * g.sC + at);
-            second[ps] = *reinterpret_cast<const Eight*>(static_cast<const TC*>(g.up) + (long long)bz * g.sC + at);
+            first[ps] = load_eight(static_cast<const TC*>(g.gate) + (long long)bz * g.sC + at);
+            second[ps] = load_eight(static_cast<const TC*>(g.up) + (long long)bz * g.sC + at);
         }
-    }
-
-    int a_row[TA::LOADS], a_chunk[TA::LOADS], b_row[TB::LOADS], b_chunk[TB::LOADS];
-    unsigned a_off[TA::LOADS], b_off[TB::LOADS];
-    const int m_last = g.M - 1 - m0, n_last = g.N - 1 - n0;  // last row of the tile that exists
-#pragma unroll
-    for (int i = 0; i < TA::LOADS; i++) {
-        TA::lane_chunk(i, 0, lane, a_row[i], a_chunk[i]);
-        if (A_KC) a_row[i] = min(a_row[i], m_last);
-        else a_chunk[i] = min(a_chunk[i], m_last / 8);
-    }
-#pragma unroll
-    for (int i = 0; i < TB::LOADS; i++) {
-        TB::lane_chunk(i, 0, lane, b_row[i], b_chunk[i]);
-        if (B_KC) b_row[i] = min(b_row[i], n_last);
-        else b_chunk[i] = min(b_chunk[i], n_last / 8);
-    }
-    int off_lda = -1, off_ldb = -1;
-    auto set_offsets = [&](int lda, int ldb) {
-        if (lda != off_lda) {
-#pragma unroll
-            for (int i = 0; i < TA::LOADS; i++) a_off[i] = (unsigned)(a_row[i] * lda + a_chunk[i] * 8) * 2u;
-            off_lda = lda;
-        }
-        if (ldb != off_ldb) {
-#pragma unroll
-            for (int i = 0; i < TB::LOADS; i++) b_off[i] = (unsigned)(b_row[i] * ldb + b_chunk[i] * 8) * 2u;
-            off_ldb = ldb;
-        }
-    };
-    bf16_t* ring = lds[wave];
-    // the loads of this wave's i-th slice into ring stage i % 2; returns how many of its contraction indices exist
-    auto issue = [&](int i) -> int {
-        int s = s_lo + wave + i * W, lda = g.lda, ldb = g.ldb, len = len0;
-        const bf16_t* Ap = A;
-        const bf16_t* Bp = B;
-        if (g.nseg > 1) {
-            const bool s1 = s >= sl0, s2 = g.nseg > 2 && s >= sl0 + sl1;
-            Ap = s2 ? static_cast<const bf16_t*>(g.A_seg[1]) : s1 ? static_cast<const bf16_t*>(g.A_seg[0]) : A;
-            Bp = s2 ? static_cast<const bf16_t*>(g.B_seg[1]) : s1 ? static_cast<const bf16_t*>(g.B_seg[0]) : B;
-            lda = s2 ? g.lda_seg[1] : s1 ? g.lda_seg[0] : lda;
-            ldb = s2 ? g.ldb_seg[1] : s1 ? g.ldb_seg[0] : ldb;
-            len = s2 ? len2 : s1 ? len1 : len0;
-            s -= s2 ? sl0 + sl1 : s1 ? sl0 : 0;
-        }
-        const int k0 = s * SK, left = len - k0;
-        const bf16_t* a0 = A_KC ? Ap + (long long)m0 * lda + k0 : Ap + (long long)k0 * lda + m0;
-        const bf16_t* b0 = B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0;
-        bf16_t* As = ring + (i & 1) * STAGE;
-        bf16_t* Bs = As + TA::ELEMS;
-        set_offsets(lda, ldb);
-        if (left >= SK) {
-#pragma unroll
-            for (int h = 0; h < TA::LOADS; h++) load_to_lds_16(a0, a_off[h], As + TA::lds_block(h, 0));
-#pragma unroll
-            for (int h = 0; h < TB::LOADS; h++) load_to_lds_16(b0, b_off[h], Bs + TB::lds_block(h, 0));
-            return SK;
-        }
-        const int last = left - 1;
-#pragma unroll
-        for (int h = 0; h < TA::LOADS; h++) {
-            const int row = A_KC ? a_row[h] : min(a_row[h], last), chunk = A_KC ? min(a_chunk[h], last / 8) : a_chunk[h];
-            load_to_lds_16(a0, (unsigned)(row * lda + chunk * 8) * 2u, As + TA::lds_block(h, 0));
-        }
-#pragma unroll
-        for (int h = 0; h < TB::LOADS; h++) {
-            const int row = B_KC ? b_row[h] : min(b_row[h], last), chunk = B_KC ? min(b_chunk[h], last / 8) : b_chunk[h];
-            load_to_lds_16(b0, (unsigned)(row * ldb + chunk * 8) * 2u, Bs + TB::lds_block(h, 0));
-        }
-        return left;
-    };
+    });
 
     f32x16 acc[2][2];
 #pragma unroll
@@ -166,29 +171,22 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
 
-    int left[2] = {0, 0};
-    if (n_mine > 0) left[0] = issue(0);
-    if (n_mine > 1) left[1] = issue(1);
     for (int i = 0; i < n_mine; i++) {
-        if (i + 1 < n_mine) wait_loads_but<NLOADS>();
-        else wait_loads_but<0>();
-        const bf16_t* As = ring + (i & 1) * STAGE;
-        const bf16_t* Bs = As + TA::ELEMS;
-        bf16x8 a[2][2], b[2][2];
+        wait_loads_but<0>();
+        bf16x8 a[STEPS][2], b[STEPS][2];
 #pragma unroll
-        for (int st = 0; st < 2; st++)
+        for (int st = 0; st < STEPS; st++)
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 a[st][h] = TA::fragment(As, h * 32, st * 16, lane);
                 b[st][h] = TB::fragment(Bs, h * 32, st * 16, lane);
             }
-        const int now = left[0];
-        left[0] = left[1];
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read: the slice after next may overwrite it
-        if (i + 2 < n_mine) left[1] = issue(i + 2);
+        const int now = left;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is in registers: the next one may overwrite it
+        if (i + 1 < n_mine) left = issue(i + 1);
         if (now < SK) {
 #pragma unroll
-            for (int st = 0; st < 2; st++)
+            for (int st = 0; st < STEPS; st++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const int k = st * 16 + 8 * (lane >> 5);
@@ -197,7 +195,7 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
                 }
         }
 #pragma unroll
-        for (int st = 0; st < 2; st++)
+        for (int st = 0; st < STEPS; st++)
 #pragma unroll
             for (int p = 0; p < 2; p++)
 #pragma unroll
@@ -206,7 +204,7 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
 
     // The waves' tiles, each in the place of its (now idle) ring: row r, column n at r * 64 + ((n / 32) ^ (r / 4 % 2)) * 32 + n % 32,
     // so that the two halves of a wave (rows 4 apart) write to different banks.
-    float* mine = reinterpret_cast<float*>(ring);
+    float* mine = reinterpret_cast<float*>(As);
     if (n_mine > 0) {
         const int c = lane & 31, gh = lane >> 5;
 #pragma unroll
@@ -217,11 +215,11 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
                 for (int v = 0; v < 16; v++) mine[(i * 32 + 8 * (v / 4) + 4 * gh + (v % 4)) * ST + (j ^ gh) * 32 + c] = acc[i][j][v];
     }
     __syncthreads();
-#pragma unroll
-    for (int ps = 0; ps < PASSES; ps++) {
+    static_for<PASSES>([&](auto ps_c) {
+        constexpr int ps = decltype(ps_c)::value;
         const int idx = ps * 64 * W + tid, r = idx / 8, cg = idx % 8;
         const int m = m0 + r, n = n0 + cg * 8;
-        if (m >= g.M || n >= g.N) continue;
+        if (m >= g.M || n >= g.N) return;
         const float* src = reinterpret_cast<const float*>(lds[0]) + r * ST + ((cg >> 2) ^ ((r >> 2) & 1)) * 32 + (cg & 3) * 8;
         float val[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         for (int w = 0; w < n_parts; w++) {  // in wave order
@@ -230,27 +228,41 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
             val[4] += hi.x; val[5] += hi.y; val[6] += hi.z; val[7] += hi.w;
         }
         gemm_store_eight<TC>(g, val, m, n, bz, C, Rsrc, add_old, P, first[ps], second[ps]);
-    }
+    });
 }
 
-template <int W, typename TC>
-void launch_sliced(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc, dim3 grid) {
-    if (a_kc && b_kc) gemm_sliced_kernel<W, true, true, TC><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else if (a_kc) gemm_sliced_kernel<W, true, false, TC><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else if (b_kc) gemm_sliced_kernel<W, false, true, TC><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else gemm_sliced_kernel<W, false, false, TC><<<grid, 64 * W, 0, ctx->stream>>>(g);
+template <int W, typename TC, Kind KIND>
+void launch_sliced(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc) {
+    const unsigned grid = (unsigned)g.blocks;
+    if constexpr (KIND == Kind::kGroup) {
+        gemm_sliced_kernel<W, false, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    } else {
+        if (a_kc && b_kc) gemm_sliced_kernel<W, true, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+        else if (a_kc) gemm_sliced_kernel<W, true, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+        else if (b_kc) gemm_sliced_kernel<W, false, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+        else gemm_sliced_kernel<W, false, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    }
+}
+template <int W>
+void launch_sliced_w(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc, int dtype_c) {
+    if (g.ngroup > 0) launch_sliced<W, float, Kind::kGroup>(ctx, g, false, false);
+    else if (g.nseg > 1 && dtype_c == EISEN_BF16) launch_sliced<W, bf16_t, Kind::kSegments>(ctx, g, a_kc, b_kc);
+    else if (g.nseg > 1) launch_sliced<W, float, Kind::kSegments>(ctx, g, a_kc, b_kc);
+    else if (dtype_c == EISEN_BF16) launch_sliced<W, bf16_t, Kind::kPlain>(ctx, g, a_kc, b_kc);
+    else launch_sliced<W, float, Kind::kPlain>(ctx, g, a_kc, b_kc);
 }
 
 }  // namespace
 
-void eisen_gemm_launch_sliced(eisen_ctx* ctx, const GemmArgs& g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c, unsigned group_tiles) {
-    const dim3 grid(g.ngroup > 0 ? group_tiles : (unsigned)eisen_ceil_div(g.N, ST), g.ngroup > 0 ? 1u : (unsigned)eisen_ceil_div(g.M, ST),
-                    (unsigned)(batch * (g.split > 1 ? g.split : 1)));
-    if (waves == 8) {
-        if (dtype_c == EISEN_BF16) launch_sliced<8, bf16_t>(ctx, g, a_kc, b_kc, grid);
-        else launch_sliced<8, float>(ctx, g, a_kc, b_kc, grid);
+// Grouped launches (g.ngroup > 0) are weight gradients: operands stored along their rows, f32 results.
+void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c) {
+    const int split = g.split > 1 ? g.split : 1;
+    if (g.ngroup > 0) {
+        for (int p = g.ngroup; p < kMaxGroup; p++) g.grp_tile_end[p] = g.grp_tile_end[g.ngroup - 1];  // no tile belongs to the missing ones
+        g.blocks = g.grp_tile_end[kMaxGroup - 1] * split;
     } else {
-        if (dtype_c == EISEN_BF16) launch_sliced<4, bf16_t>(ctx, g, a_kc, b_kc, grid);
-        else launch_sliced<4, float>(ctx, g, a_kc, b_kc, grid);
+        g.blocks = eisen_ceil_div(g.M, ST) * eisen_ceil_div(g.N, ST) * batch * split;
     }
+    if (waves == 8) launch_sliced_w<8>(ctx, g, a_kc, b_kc, dtype_c);
+    else launch_sliced_w<4>(ctx, g, a_kc, b_kc, dtype_c);
 }

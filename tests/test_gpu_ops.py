@@ -790,6 +790,36 @@ def test_gemm_bf16_sliced_tiles_and_packed_rows(ctx, ta, tb, M, N, K):
     _gemm_case(ctx, M, N, K, ta, tb, BF16, F32, False)
 
 
+# Slices of 64: a contraction that ends at, before and behind a slice, with fewer, as many and more slices than four and eight waves
+# take in one go, in whole and cut tiles, one segment and several, one product and a group.  Whole-number operands: f32 results are exact.
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,Ks", [(64, 64, (56,)), (64, 128, (64,)), (72, 136, (72,)), (128, 64, (256,)), (136, 72, (264,)), (64, 64, (512,)), (200, 64, (520,)),
+                                    (1024, 2048, (320,)), (72, 64, (56, 64, 72)), (128, 200, (8, 128)), (64, 72, (264, 8, 320))])
+def test_gemm_bf16_sliced_ends_of_slices(ctx, ta, tb, M, N, Ks):
+    rng = np.random.default_rng(M + N + sum(Ks))
+    a = [rng.integers(-4, 5, (k, M) if ta else (M, k)).astype(np.float32) for k in Ks]
+    b = [rng.integers(-4, 5, (N, k) if tb else (k, N)).astype(np.float32) for k in Ks]
+    old = rng.integers(-256, 257, (M, N)).astype(np.float32)
+    exact = [(x.T if ta else x) @ (y.T if tb else y) for x, y in zip(a, b)]
+    da, db, dc = [up(ctx, x, BF16) for x in a], [up(ctx, y, BF16) for y in b], ctx.upload(old)
+    ctx.profile_start()
+    ctx.gemm_ksegments(da, db, list(Ks), dc, BF16, F32, ta, tb, M, N, 1)
+    names = list(ctx.profile_stop())
+    assert len(names) == 1 and "_sliced" in names[0], names
+    assert np.array_equal(dn(ctx, dc, (M, N), F32), old + sum(exact))
+    if len(Ks) == 1 and ta and not tb:  # and as a group of two weight gradients, the second one narrower
+        N2, d1, d2 = 64, ctx.malloc(M * N * 4), ctx.malloc(M * 64 * 4)
+        b2 = rng.integers(-4, 5, (Ks[0], N2)).astype(np.float32)
+        db2 = up(ctx, b2, BF16)
+        ctx.gemm_grouped([da[0], da[0]], [db[0], db2], [d1, d2], [N, N2], BF16, F32, 1, 0, M, Ks[0], 0)
+        assert np.array_equal(dn(ctx, d1, (M, N), F32), exact[0])
+        assert np.array_equal(dn(ctx, d2, (M, N2), F32), a[0].T @ b2)
+        for x in (d1, d2, db2):
+            x.free()
+    for x in da + db + [dc]:
+        x.free()
+
+
 # Whole-number operands: every product and every f32 sum is exact (below 2^24), so a bf16 result has one right value, the exact
 # sum rounded once.  Split contractions (sliced tiles with whole and cut shapes and packed rows, 128 x 128 tiles), whose parts
 # must not be rounded before they are added, and one product that is not split.
