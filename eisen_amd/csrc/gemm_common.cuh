@@ -86,6 +86,9 @@ void eisen_gemm_launch_wide_window(eisen_ctx* ctx, const WideWindow& w, unsigned
 // gemm_sliced.hip: bf16 operands, any shape, the contraction dealt to 4 or 8 waves (see there for what the operands must allow)
 void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c);
 
+// gemm_f32_sliced.hip: f32 operands and result, operand rows that start on 16-byte boundaries
+void eisen_gemm_launch_f32_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int tile, bool a_kc, bool b_kc, int batch);
+
 // gemm_f32.hip: f32 operands and result, any shape
 struct F32GemmPlan {
     int tile;    // 64 or 32

@@ -1022,6 +1022,52 @@ def test_gemm_f32_ksegments(ctx, M, N, Ks, accumulate):
         x.free()
 
 
+# f32 operands split into bf16 parts: slices that end at, before and behind 32 indices, cut tiles of 32 and 64, four and eight waves, parts
+# of the contraction.  Whole numbers of 17 bits times small ones: every product needs the middle parts, and every sum is exact.
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(32, 32, 4), (36, 40, 28), (64, 64, 32), (100, 68, 36), (32, 64, 128), (72, 36, 260), (4, 4, 1024), (68, 100, 1100), (1024, 1024, 40),
+                                   (1028, 900, 160), (256, 1024, 4096)])
+def test_gemm_f32_split_operands(ctx, ta, tb, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    a = rng.integers(-(2 ** 16), 2 ** 16, (K, M) if ta else (M, K)).astype(np.float32)
+    a[rng.random(a.shape) > min(1.0, 64 / K)] = 0  # sums stay below 2^24
+    b = rng.integers(-1, 2, (N, K) if tb else (K, N)).astype(np.float32)
+    old = rng.integers(-256, 257, (M, N)).astype(np.float32)
+    exact = old + (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)
+    assert np.abs(exact).max() < 2 ** 24
+    da, db, dc = ctx.upload(a), ctx.upload(b), ctx.upload(old)
+    ctx.profile_start()
+    ctx.gemm(da, db, dc, F32, F32, ta, tb, M, N, K, 1)
+    names = list(ctx.profile_stop())
+    assert "x32_sliced" in names[0], names
+    assert np.array_equal(dn(ctx, dc, (M, N), F32), exact)
+    for x in (da, db, dc):
+        x.free()
+
+
+# What is not finite stays what f32 arithmetic makes of it, in every tile it reaches and in no other: infinities (times zero, times both
+# signs, of both signs in one sum), NaN, and the largest f32, which rounds to infinity in bf16.
+@pytest.mark.parametrize("M,N,K", [(64, 96, 40), (1024, 1024, 64), (40, 36, 1100)])
+def test_gemm_f32_split_operands_not_finite(ctx, M, N, K):
+    rng = np.random.default_rng(K)
+    a, b = rng.integers(-8, 9, (M, K)).astype(np.float32), rng.integers(-8, 9, (K, N)).astype(np.float32)
+    a[1, 3], a[33, 5], a[34, 5], a[34, 6], a[2, K - 1] = np.inf, -np.inf, np.inf, -np.inf, np.finfo(np.float32).max
+    b[7, 35], b[8, 4] = np.nan, np.inf
+    b[3, 0], b[K - 1] = 0.0, rng.integers(0, 2, N) * 0.5
+    with np.errstate(invalid="ignore"):
+        exact = a.astype(np.float64) @ b.astype(np.float64)
+    da, db, dc = ctx.upload(a), ctx.upload(b), ctx.malloc(M * N * 4)
+    ctx.gemm(da, db, dc, F32, F32, 0, 0, M, N, K)
+    got = dn(ctx, dc, (M, N), F32)
+    assert np.array_equal(np.isnan(got), np.isnan(exact)) and np.array_equal(np.isinf(got), np.isinf(exact))
+    finite = np.isfinite(exact)
+    assert np.array_equal(got[~finite & ~np.isnan(exact)], exact[~finite & ~np.isnan(exact)].astype(np.float32))
+    # sums of at most 1100 products below 64, exact, except in the row of the largest f32: there within an ulp of its half
+    assert np.all(np.abs(got - exact)[finite] <= np.abs(exact)[finite] * 2.0 ** -23)
+    for x in (da, db, dc):
+        x.free()
+
+
 @pytest.mark.parametrize("accumulate", [0, 1])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
 @pytest.mark.parametrize("M,K,Ns", [(64, 64, (64, 16, 16)), (33, 70, (65, 1, 31)), (200, 1500, (96, 32, 100)), (40, 2048, (33, 8)), (1000, 40, (520, 1032)), (2, 3, (5, 2))])
