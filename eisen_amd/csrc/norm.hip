@@ -1,6 +1,5 @@
 // RMSNorm forward/backward and row softmax forward/backward.
-// One 64-lane wave owns one row; lanes stride the row in 16-byte packets so every global
-// access is a fully coalesced 1 KiB wave transaction.  Reductions are wave shuffles.
+// A wave owns a row, or 8, 16 or 32 of its lanes own one each where that many hold it in 16-byte packets; lanes stride the row in packets.
 #include "device_utils.cuh"
 #include "runtime.h"
 
@@ -55,22 +54,71 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_fwd_kernel(const T* __re
     }
 }
 
+// The same for rows of whole packets that fit LPR lanes x MAXP packets: the row and its gains are requested together and stay in
+// registers, so a row is one memory latency, not three.  These kernels last 2 to 5 us, of which the launch is about 2: 8192 x 256 in bf16 4.7 ->
+// 4.1 us, 1024 x 1024 4.0 -> 3.2, 4096 x 256 in f32 5.1 -> 4.5, 64 x 64 3.0 -> 2.4.
+template <typename T, int LPR, int MAXP>
+__global__ __launch_bounds__(kRowThreads) void rms_norm_fwd_rows_kernel(const T* __restrict__ x, const float* __restrict__ w, T* __restrict__ out,
+                                                                        float* __restrict__ rrms_out, size_t rows, int dim, float eps) {
+    constexpr int N = Pack<T>::N, RPB = kRowThreads / LPR;
+    const int lane = threadIdx.x % LPR;
+    const size_t row = (size_t)blockIdx.x * RPB + threadIdx.x / LPR;
+    if (row >= rows) return;
+    Pack<T> p[MAXP];
+    float4 g[MAXP][N / 4];
+#pragma unroll
+    for (int k = 0; k < MAXP; k++) {
+        const int c = min((k * LPR + lane) * N, dim - N);  // lanes past the end re-read the last packet and leave it out below
+        p[k] = load_pack(x + row * dim + c);
+#pragma unroll
+        for (int j = 0; j < N / 4; j++) g[k][j] = *reinterpret_cast<const float4*>(w + c + 4 * j);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < MAXP; k++) {
+        float q = 0.f;
+#pragma unroll
+        for (int j = 0; j < N; j++) q += p[k].get(j) * p[k].get(j);
+        ss += (k * LPR + lane) * N < dim ? q : 0.f;
+    }
+    ss = lanes_sum<LPR>(ss);
+    const float rrms = 1.0f / sqrtf(ss / (float)dim + eps);
+    if (lane == 0) rrms_out[row] = rrms;
+#pragma unroll
+    for (int k = 0; k < MAXP; k++) {
+        const int c = (k * LPR + lane) * N;
+        if (c >= dim) continue;
+        Pack<T> o;
+#pragma unroll
+        for (int j = 0; j < N; j += 4) {
+            const float4 g4 = g[k][j / 4];
+            o.set(j, p[k].get(j) * rrms * g4.x);
+            o.set(j + 1, p[k].get(j + 1) * rrms * g4.y);
+            o.set(j + 2, p[k].get(j + 2) * rrms * g4.z);
+            o.set(j + 3, p[k].get(j + 3) * rrms * g4.w);
+        }
+        store_pack(out + row * dim + c, o);
+    }
+}
+
 // dx = rrms*(go*w) - x*(rrms^3/D)*sum_d(go*x*w);  dw_partial[d] += go*x*rrms
 // (src/graph/ops/normalization.rs:157-171).  Each wave walks rows wave_id, wave_id+W, ...
 // and keeps its dw partial in registers; partials meet in LDS and leave as one row of
-// `partial` per block.  A second kernel sums the block rows in fixed order.
-template <typename T, int MAXP>
+// `partial` per block.  A second kernel sums the block rows in fixed order.  LPR lanes have a row (64 for every row: 8192 x 256 in bf16,
+// half of the lanes idle, 8.2 us; 32: 6.0).
+template <typename T, int LPR, int MAXP>
 __global__ __launch_bounds__(kBwdThreads) void rms_norm_bwd_kernel(const T* __restrict__ x, const float* __restrict__ w,
                                                                    const float* __restrict__ rrms_in,
                                                                    const T* __restrict__ go, const T* gx_old, T* gx,
-                                                                   float* __restrict__ partial, size_t rows, int dim) {
+                                                                   float* __restrict__ partial, size_t rows, int dim, unsigned n_blocks) {
     // gx_old: what dx is added to (gx itself for an in-place accumulation, another buffer of the same layout, or null to assign)
     const bool accumulate_x = gx_old != nullptr;
     constexpr int N = Pack<T>::N;
-    extern __shared__ float lds[];  // [kBwdWaves][dim]
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const size_t wave_global = (size_t)blockIdx.x * kBwdWaves + wid;
-    const size_t wave_stride = (size_t)gridDim.x * kBwdWaves;
+    constexpr int kGroups = kBwdThreads / LPR;  // rows the workgroup has at a time
+    extern __shared__ float lds[];              // [kGroups][dim]
+    const int lane = threadIdx.x % LPR, wid = threadIdx.x / LPR;
+    const size_t wave_global = (size_t)blockIdx.x * kGroups + wid;
+    const size_t wave_stride = (size_t)n_blocks * kGroups;
     float dw[MAXP][N];
 #pragma unroll
     for (int p = 0; p < MAXP; p++)
@@ -81,7 +129,7 @@ __global__ __launch_bounds__(kBwdThreads) void rms_norm_bwd_kernel(const T* __re
     float wv[MAXP][N];
 #pragma unroll
     for (int p = 0; p < MAXP; p++) {
-        const int c = (p * kWave + lane) * N;
+        const int c = (p * LPR + lane) * N;
 #pragma unroll
         for (int j = 0; j < N; j += 4) {
             const float4 t = c < dim ? *reinterpret_cast<const float4*>(w + c + j) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -96,7 +144,7 @@ __global__ __launch_bounds__(kBwdThreads) void rms_norm_bwd_kernel(const T* __re
     auto fetch = [&](size_t row, Pack<T>* xd, Pack<T>* gd, Pack<T>* od) {
 #pragma unroll
         for (int p = 0; p < MAXP; p++) {
-            const int c = (p * kWave + lane) * N;
+            const int c = (p * LPR + lane) * N;
             if (c < dim) {
                 xd[p] = load_pack(x + row * dim + c);
                 gd[p] = load_pack(go + row * dim + c);
@@ -104,26 +152,33 @@ __global__ __launch_bounds__(kBwdThreads) void rms_norm_bwd_kernel(const T* __re
             }
         }
     };
-    if (wave_global < rows) fetch(wave_global, xp, gp, op);
+    float rrms_next = 0.f;
+    if (wave_global < rows) {
+        rrms_next = rrms_in[wave_global];
+        fetch(wave_global, xp, gp, op);
+    }
     for (size_t row = wave_global; row < rows; row += wave_stride) {
         T* gxr = gx + row * dim;
-        const float rrms = rrms_in[row];
+        const float rrms = rrms_next;
         const size_t next = row + wave_stride;
-        if (next < rows) fetch(next, xn, gn, on);
+        if (next < rows) {
+            rrms_next = rrms_in[next];
+            fetch(next, xn, gn, on);
+        }
         float gdxw = 0.f;
 #pragma unroll
         for (int p = 0; p < MAXP; p++) {
-            const int c = (p * kWave + lane) * N;
+            const int c = (p * LPR + lane) * N;
             if (c < dim) {
 #pragma unroll
                 for (int j = 0; j < N; j++) gdxw += gp[p].get(j) * xp[p].get(j) * wv[p][j];
             }
         }
-        gdxw = wave_sum(gdxw);
+        gdxw = lanes_sum<LPR>(gdxw);
         const float rrc_d = rrms * rrms * rrms / (float)dim;
 #pragma unroll
         for (int p = 0; p < MAXP; p++) {
-            const int c = (p * kWave + lane) * N;
+            const int c = (p * LPR + lane) * N;
             if (c < dim) {
                 Pack<T> o = op[p];
 #pragma unroll
@@ -143,10 +198,10 @@ __global__ __launch_bounds__(kBwdThreads) void rms_norm_bwd_kernel(const T* __re
             op[p] = on[p];
         }
     }
-    // combine the block's waves in a fixed order
+    // combine the block's rows in a fixed order
 #pragma unroll
     for (int p = 0; p < MAXP; p++) {
-        const int c = (p * kWave + lane) * N;
+        const int c = (p * LPR + lane) * N;
         if (c < dim)
 #pragma unroll
             for (int j = 0; j < N; j++) lds[wid * dim + c + j] = dw[p][j];
@@ -155,7 +210,7 @@ __global__ __launch_bounds__(kBwdThreads) void rms_norm_bwd_kernel(const T* __re
     for (int c = threadIdx.x; c < dim; c += kBwdThreads) {
         float s = 0.f;
 #pragma unroll
-        for (int k = 0; k < kBwdWaves; k++) s += lds[k * dim + c];
+        for (int k = 0; k < kGroups; k++) s += lds[k * dim + c];
         partial[(size_t)blockIdx.x * dim + c] = s;
     }
 }
@@ -267,7 +322,16 @@ int rms_norm_fwd(eisen_ctx* ctx, const void* x, const float* w, void* out, float
     const bool vec = dim % Pack<T>::N == 0 && eisen_aligned(x, 16) && eisen_aligned(out, 16) && eisen_aligned(w, 16);
     // algorithmic bytes: x read, y written, one rrms per row
     EisenProfScope prof(ctx, sizeof(T) == 2 ? "rms_norm_fwd_bf16" : "rms_norm_fwd_f32", 2.0 * (double)rows * (double)dim * sizeof(T) + 4.0 * (double)rows);
-    if (vec)
+    const size_t packs = vec ? dim / Pack<T>::N : 0;
+#define EISEN_FWD(LPR, MAXP) rms_norm_fwd_rows_kernel<T, LPR, MAXP><<<(unsigned)eisen_ceil_div(rows, kRowThreads / LPR), kRowThreads, 0, ctx->stream>>>((const T*)x, w, (T*)out, rrms, rows, (int)dim, eps)
+    if (packs > 0 && packs <= 8) EISEN_FWD(8, 1);
+    else if (packs > 0 && packs <= 16) EISEN_FWD(16, 1);
+    else if (packs > 0 && packs <= 32) EISEN_FWD(32, 1);
+    else if (packs > 0 && packs <= 64) EISEN_FWD(64, 1);
+    else if (packs > 0 && packs <= 128) EISEN_FWD(64, 2);
+    else if (packs > 0 && packs <= 256) EISEN_FWD(64, 4);
+#undef EISEN_FWD
+    else if (vec)  // rows beyond 256 packets: the second pass reads them from the caches
         rms_norm_fwd_kernel<T, true><<<blocks, kRowThreads, 0, ctx->stream>>>((const T*)x, w, (T*)out, rrms, rows, (int)dim, eps);
     else
         rms_norm_fwd_kernel<T, false><<<blocks, kRowThreads, 0, ctx->stream>>>((const T*)x, w, (T*)out, rrms, rows, (int)dim, eps);
@@ -277,12 +341,12 @@ int rms_norm_fwd(eisen_ctx* ctx, const void* x, const float* w, void* out, float
 
 constexpr unsigned kMaxPartialRows = EISEN_RMS_NORM_PARTIAL_ROWS;
 
-template <typename T, int MAXP>
+template <typename T, int LPR, int MAXP>
 int rms_norm_bwd_vec(eisen_ctx* ctx, const void* x, const float* w, const float* rrms, const void* go, const void* gx_old, void* gx, float* partial,
                      unsigned blocks, size_t rows, size_t dim) {
-    const size_t lds = (size_t)kBwdWaves * dim * sizeof(float);
-    rms_norm_bwd_kernel<T, MAXP><<<blocks, kBwdThreads, lds, ctx->stream>>>((const T*)x, w, rrms, (const T*)go, (const T*)gx_old, (T*)gx, partial, rows,
-                                                                            (int)dim);
+    const size_t lds = (size_t)(kBwdThreads / LPR) * dim * sizeof(float);
+    rms_norm_bwd_kernel<T, LPR, MAXP><<<blocks, kBwdThreads, lds, ctx->stream>>>((const T*)x, w, rrms, (const T*)go, (const T*)gx_old, (T*)gx, partial, rows,
+                                                                            (int)dim, blocks);
     EISEN_LAUNCH_CHECK(ctx, "rms_norm_bwd_kernel");
     return 0;
 }
@@ -300,13 +364,16 @@ int rms_norm_bwd_partial(eisen_ctx* ctx, const void* x, const float* w, const fl
                         (accumulate_x ? 4.0 : 3.0) * (double)rows * (double)dim * sizeof(T) + 4.0 * (double)rows);
     if (vec) {
         // enough waves to cover the chip a few times over, few enough that the partial rows stay small
-        const unsigned blocks = (unsigned)std::min<size_t>(eisen_ceil_div(rows, kBwdWaves), kMaxPartialRows);
+        const size_t packs = dim / N, lpr = packs <= 8 ? 8 : packs <= 16 ? 16 : packs <= 32 ? 32 : 64;
+        const unsigned blocks = (unsigned)std::min<size_t>(eisen_ceil_div(rows, kBwdThreads / lpr), kMaxPartialRows);
         *nrows = blocks;
-        const size_t packs = eisen_ceil_div(dim, (size_t)kWave * N);
-        if (packs <= 1) return rms_norm_bwd_vec<T, 1>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
-        if (packs <= 2) return rms_norm_bwd_vec<T, 2>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
-        if (packs <= 4) return rms_norm_bwd_vec<T, 4>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
-        return rms_norm_bwd_vec<T, 8>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
+        if (packs <= 8) return rms_norm_bwd_vec<T, 8, 1>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
+        if (packs <= 16) return rms_norm_bwd_vec<T, 16, 1>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
+        if (packs <= 32) return rms_norm_bwd_vec<T, 32, 1>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
+        if (packs <= 64) return rms_norm_bwd_vec<T, 64, 1>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
+        if (packs <= 128) return rms_norm_bwd_vec<T, 64, 2>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
+        if (packs <= 256) return rms_norm_bwd_vec<T, 64, 4>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
+        return rms_norm_bwd_vec<T, 64, 8>(ctx, x, w, rrms, go, gx_old, gx, partial, blocks, rows, dim);
     }
     rms_norm_bwd_scalar_kernel<T><<<(unsigned)eisen_ceil_div(rows, kRowWaves), kRowThreads, 0, ctx->stream>>>(
         (const T*)x, w, rrms, (const T*)go, (const T*)gx_old, (T*)gx, rows, (int)dim);

@@ -239,6 +239,35 @@ def test_rms_norm(ctx, dtype, rows, dim):
     assert np.array_equal(dn(ctx, gw2, (dim,), F32), dn(ctx, gw3, (dim,), F32))
 
 
+# 8, 16, 32 and 64 lanes per row, one to eight packets per lane and rows beyond them: the last width of each and the first of the next;
+# rows that do not fill a wave, a workgroup, the grid.  Every row by itself: a row's lanes read nobody else's.
+@pytest.mark.parametrize("dtype", DTYPES, ids=_ids.get)
+@pytest.mark.parametrize("packs", [1, 7, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257])
+@pytest.mark.parametrize("rows", [1, 5, 67])
+def test_rms_norm_lanes_per_row(ctx, dtype, packs, rows):
+    dim = packs * (8 if dtype == BF16 else 4)
+    x, go = prep(gen.normal(700 + packs, (rows, dim), 1.5), dtype), prep(gen.normal(701 + packs, (rows, dim)), dtype)
+    x *= (4.0 ** (np.arange(rows) % 5 - 2)).astype(np.float32)[:, None]  # a neighbour's row would show
+    w = (1.0 + gen.normal(702, (dim,), 0.2)).astype(np.float32)
+    dx, dw, dgo = up(ctx, x, dtype), up(ctx, w, F32), up(ctx, go, dtype)
+    out, rr, gx, gw = ctx.malloc(x.nbytes), ctx.malloc(rows * 4), ctx.malloc(x.nbytes), ctx.upload(np.zeros(dim, np.float32))
+    ctx.rms_norm(dx, dw, out, rr, dtype, rows, dim, 1e-5)
+    ctx.rms_norm_backward(dx, dw, rr, dgo, gx, gw, dtype, rows, dim, 0)
+    x64, go64 = x.astype(np.float64), go.astype(np.float64)
+    er = 1.0 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-5)
+    egx = er * go64 * w - x64 * er ** 3 / dim * (go64 * x64 * w).sum(1, keepdims=True)
+    assert_close(dn(ctx, rr, (rows,), F32), er[:, 0], 1e-5, "rrms")
+    got = dn(ctx, out, x.shape, dtype)
+    for r in range(rows):
+        assert_close(got[r], x64[r] * er[r] * w, tol_for(dtype), f"row {r}")
+    got = dn(ctx, gx, x.shape, dtype)
+    for r in range(rows):
+        assert_close(got[r], egx[r], tol_for(dtype), f"dx row {r}")
+    assert_close(dn(ctx, gw, (dim,), F32), (go64 * x64 * er).sum(0), tol_for(dtype) if dtype == BF16 else 2e-4, "dw")
+    for b in (dx, dw, dgo, out, rr, gx, gw):
+        b.free()
+
+
 @pytest.mark.parametrize("dtype,dim", [(BF16, 2048), (F32, 256), (BF16, 100)], ids=["bf16-2048", "f32-256", "bf16-scalar-path"])
 def test_rms_norm_backward_in_two_parts(ctx, dtype, dim):
     # three norms of different row counts leave their gain gradients as partial rows; one launch finishes them all
