@@ -85,6 +85,7 @@ void eisen_gemm_launch_wide_window(eisen_ctx* ctx, const WideWindow& w, unsigned
 
 // gemm_sliced.hip: bf16 operands, any shape, the contraction dealt to 4 or 8 waves (see there for what the operands must allow)
 void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c);
+void eisen_gemm_launch_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves);
 
 // gemm_f32_sliced.hip: f32 operands and result, operand rows that start on 16-byte boundaries
 void eisen_gemm_launch_f32_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int tile, bool a_kc, bool b_kc, int batch);
@@ -538,7 +539,11 @@ __device__ __forceinline__ void load_to_lds_16(const void* base, unsigned lane_o
     const unsigned lds_addr = (unsigned)(size_t)(lds_void_ptr)lds_dst;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(lane_offset), "s"(base) : "m0");
 }
-// the same, to OFFSET bytes behind an LDS address held as a (wave-uniform) number
+// the same two, to OFFSET bytes behind an LDS address held as a (wave-uniform) number
+template <int OFFSET>
+__device__ __forceinline__ void load_to_lds_16_at(const void* src, unsigned lds_addr) {
+    asm volatile("s_add_u32 m0, %0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(src), "n"(OFFSET) : "m0", "scc");
+}
 template <int OFFSET>
 __device__ __forceinline__ void load_to_lds_16_at(const void* base, unsigned lane_offset, unsigned lds_addr) {
     asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(lane_offset), "s"(base), "n"(OFFSET) : "m0", "scc");

@@ -46,12 +46,22 @@ __device__ __forceinline__ void load_slice(const bf16_t* base, int ld, unsigned 
     }
 }
 
-// What a launch is: one product (or a batch), a product whose contraction runs over several operand pairs, or several products.
-// A kernel per kind: the tables of the other kinds would be loaded into, and spilled from, scalar registers.
+// What a launch is: one product (or a batch), a product whose contraction runs over several operand pairs, several products, or the gate
+// and up projections with their SwiGLU.  A kernel per kind: the tables of the other kinds would be loaded into, and spilled from, scalar
+// registers.
+// The same for 32 columns each of two operands [K][N] side by side: the first four chunks of a row are the first one's.
+__device__ __forceinline__ void load_slice_of_two(const bf16_t* first, const bf16_t* second, int ld, unsigned tile, int row_last, int chunk_last, int lane) {
+    static_for<8>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        const int row = (lane >> 3) + 8 * i, chunk = (lane & 7) ^ lds_swz<128>(row);
+        load_to_lds_16_at<i * 1024>((chunk < 4 ? first : second) + (long long)(min(row, row_last) * ld + min(chunk & 3, chunk_last) * 8), tile);
+    });
+}
+
 // integer divisions leave values that are the same in every lane in vector registers
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-enum class Kind { kPlain, kSegments, kGroup };
+enum class Kind { kPlain, kSegments, kGroup, kSwiglu };
 
 template <int W, bool A_KC, bool B_KC, typename TC, Kind KIND>
 __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
@@ -65,7 +75,7 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blocks of 4 x 8 tiles, which share 12 operand panels, on one XCD
     const int split = g.split > 1 ? g.split : 1;
-    int nt, mt = 0, zz;
+    int nt, mt = 0, zz, member = 0;
     if constexpr (KIND == Kind::kGroup) {  // which product this tile belongs to (uniform); static indices keep the tables in scalar registers
         const int tiles = g.grp_tile_end[kMaxGroup - 1];
         const int lin = xcd_contiguous_id(blockIdx.x, tiles * split);
@@ -77,6 +87,7 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
 #pragma unroll
         for (int q = 1; q < kMaxGroup; q++)
             if (t >= g.grp_tile_end[q - 1]) {
+                member = q;
                 first = g.grp_tile_end[q - 1];
                 partial_off = g.grp_partial_off[q];
                 g.A = g.grp_A[q]; g.B = g.grp_B[q]; g.C = g.grp_C[q]; g.N = g.grp_N[q];
@@ -88,13 +99,15 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
         g.ldc = g.N;
         if (!B_KC) g.ldb = g.N;
     } else {
-        const int gx = (g.N + ST - 1) / ST, gy = (g.M + ST - 1) / ST;
+        constexpr int COLS = KIND == Kind::kSwiglu ? ST / 2 : ST;  // columns of each product
+        const int gx = (g.N + COLS - 1) / COLS, gy = (g.M + ST - 1) / ST;
         const int lin = xcd_contiguous_id(blockIdx.x, g.blocks);
         zz = uniform(lin / (gx * gy));
         block_tile<4, 8>(lin - zz * (gx * gy), gy, gx, mt, nt);
     }
-    const int m0 = uniform(mt * ST), n0 = uniform(nt * ST);
+    const int m0 = uniform(mt * ST), n0 = uniform(nt * (KIND == Kind::kSwiglu ? ST / 2 : ST));
     const int bz = uniform(zz / split), part = uniform(zz % split);
+    if constexpr (KIND != Kind::kGroup) member = bz;
     const bf16_t* A = static_cast<const bf16_t*>(g.A) + (long long)bz * g.sA;
     const bf16_t* B = static_cast<const bf16_t*>(g.B) + (long long)bz * g.sB;
 
@@ -136,7 +149,10 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
         }
         const int k0 = s * SK, left = len - k0;
         load_slice(A_KC ? Ap + (long long)m0 * lda + k0 : Ap + (long long)k0 * lda + m0, lda, lds_a, A_KC ? m_last : left - 1, (A_KC ? left - 1 : m_last) / 8, lane);
-        load_slice(B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0, ldb, lds_b, B_KC ? n_last : left - 1, (B_KC ? left - 1 : n_last) / 8, lane);
+        if constexpr (KIND == Kind::kSwiglu)
+            load_slice_of_two(Bp + (long long)k0 * ldb + n0, static_cast<const bf16_t*>(g.B_seg[0]) + (long long)k0 * ldb + n0, ldb, lds_b, left - 1, n_last / 8, lane);
+        else
+            load_slice(B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0, ldb, lds_b, B_KC ? n_last : left - 1, (B_KC ? left - 1 : n_last) / 8, lane);
         return min(left, SK);
     };
 
@@ -149,12 +165,12 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
     TC* C = static_cast<TC*>(g.C) + (long long)bz * g.sC;
     const TC* Rsrc = g.R ? static_cast<const TC*>(g.R) + (long long)bz * g.sC : C;
     float* P = gemm_partial<TC>(g, bz, split, part);
-    const bool add_old = (g.accumulate || g.R != nullptr) && !P && !g.gate;
+    const bool add_old = KIND != Kind::kSwiglu && (g.accumulate || g.R != nullptr) && !P && !g.gate;
     typename Eight<TC>::V first[PASSES] = {}, second[PASSES] = {};
     static_for<PASSES>([&](auto ps_c) {
         constexpr int ps = decltype(ps_c)::value;
         const int idx = ps * 64 * W + tid, m = m0 + idx / 8, n = n0 + (idx % 8) * 8;
-        const bool whole = m < g.M && n + 8 <= g.N;
+        const bool whole = KIND != Kind::kSwiglu && m < g.M && n + 8 <= g.N;
         const long long at = (long long)m * g.ldc + n;
         if (whole && add_old) first[ps] = load_eight(Rsrc + at);
         if (whole && g.gate) {
@@ -202,7 +218,7 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
                 for (int q = 0; q < 2; q++) acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st][p], b[st][q], acc[p][q], 0, 0, 0);
     }
 
-    // The waves' tiles, each in the place of its (now idle) ring: row r, column n at r * 64 + ((n / 32) ^ (r / 4 % 2)) * 32 + n % 32,
+    // The waves' tiles, each in the place of its (now idle) slice: row r, column n at r * 64 + ((n / 32) ^ (r / 4 % 2)) * 32 + n % 32,
     // so that the two halves of a wave (rows 4 apart) write to different banks.
     float* mine = reinterpret_cast<float*>(As);
     if (n_mine > 0) {
@@ -215,37 +231,60 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
                 for (int v = 0; v < 16; v++) mine[(i * 32 + 8 * (v / 4) + 4 * gh + (v % 4)) * ST + (j ^ gh) * 32 + c] = acc[i][j][v];
     }
     __syncthreads();
-    static_for<PASSES>([&](auto ps_c) {
-        constexpr int ps = decltype(ps_c)::value;
-        const int idx = ps * 64 * W + tid, r = idx / 8, cg = idx % 8;
-        const int m = m0 + r, n = n0 + cg * 8;
-        if (m >= g.M || n >= g.N) return;
+    auto sum_of_waves = [&](int r, int cg, float (&val)[8]) __attribute__((always_inline)) {
         const float* src = reinterpret_cast<const float*>(lds[0]) + r * ST + ((cg >> 2) ^ ((r >> 2) & 1)) * 32 + (cg & 3) * 8;
-        float val[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 8; e++) val[e] = 0.f;
         for (int w = 0; w < n_parts; w++) {  // in wave order
             const float4 lo = *reinterpret_cast<const float4*>(src + w * ST * ST), hi = *reinterpret_cast<const float4*>(src + w * ST * ST + 4);
             val[0] += lo.x; val[1] += lo.y; val[2] += lo.z; val[3] += lo.w;
             val[4] += hi.x; val[5] += hi.y; val[6] += hi.z; val[7] += hi.w;
         }
-        gemm_store_eight<TC>(g, val, m, n, bz, C, Rsrc, add_old, P, first[ps], second[ps]);
-    });
+    };
+    if constexpr (KIND == Kind::kSwiglu) {
+        // G = X Wg and U = X Wu leave rounded, and H = silu(G) * U is formed from what was rounded, as a separate kernel would
+        const int idx = tid, r = idx / 4, cg = idx % 4, m = m0 + r, n = n0 + cg * 8;
+        if (idx >= ST * 4 || m >= g.M || n >= g.N) return;
+        float gv[8], uv[8];
+        sum_of_waves(r, cg, gv);
+        sum_of_waves(r, cg + 4, uv);
+        bf16x8 og, ou, oh;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            og[e] = (bf16_t)gv[e];
+            ou[e] = (bf16_t)uv[e];
+            const float x = (float)og[e];
+            oh[e] = (bf16_t)(x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)) * (float)ou[e]);  // 1-ulp reciprocal: the result is rounded to bf16
+        }
+        const long long at = (long long)m * g.N + n;  // (N is a multiple of 8 and the results start on 16-byte boundaries)
+        *reinterpret_cast<bf16x8*>(static_cast<bf16_t*>(g.C) + at) = og;
+        *reinterpret_cast<bf16x8*>(static_cast<bf16_t*>(g.C2) + at) = ou;
+        *reinterpret_cast<bf16x8*>(static_cast<bf16_t*>(g.grp_C[0]) + at) = oh;
+    } else {
+        static_for<PASSES>([&](auto ps_c) {
+            constexpr int ps = decltype(ps_c)::value;
+            const int idx = ps * 64 * W + tid, r = idx / 8, cg = idx % 8;
+            const int m = m0 + r, n = n0 + cg * 8;
+            if (m >= g.M || n >= g.N) return;
+            float val[8];
+            sum_of_waves(r, cg, val);
+            gemm_store_eight<TC>(g, val, m, n, member, C, Rsrc, add_old, P, first[ps], second[ps]);
+        });
+    }
 }
 
 template <int W, typename TC, Kind KIND>
 void launch_sliced(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc) {
     const unsigned grid = (unsigned)g.blocks;
-    if constexpr (KIND == Kind::kGroup) {
-        gemm_sliced_kernel<W, false, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    } else {
-        if (a_kc && b_kc) gemm_sliced_kernel<W, true, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-        else if (a_kc) gemm_sliced_kernel<W, true, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-        else if (b_kc) gemm_sliced_kernel<W, false, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-        else gemm_sliced_kernel<W, false, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    }
+    if (a_kc && b_kc) gemm_sliced_kernel<W, true, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    else if (a_kc) gemm_sliced_kernel<W, true, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    else if (b_kc) gemm_sliced_kernel<W, false, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    else gemm_sliced_kernel<W, false, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
 }
 template <int W>
 void launch_sliced_w(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc, int dtype_c) {
-    if (g.ngroup > 0) launch_sliced<W, float, Kind::kGroup>(ctx, g, false, false);
+    if (g.ngroup > 0 && dtype_c == EISEN_BF16) gemm_sliced_kernel<W, true, false, bf16_t, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+    else if (g.ngroup > 0) gemm_sliced_kernel<W, false, false, float, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
     else if (g.nseg > 1 && dtype_c == EISEN_BF16) launch_sliced<W, bf16_t, Kind::kSegments>(ctx, g, a_kc, b_kc);
     else if (g.nseg > 1) launch_sliced<W, float, Kind::kSegments>(ctx, g, a_kc, b_kc);
     else if (dtype_c == EISEN_BF16) launch_sliced<W, bf16_t, Kind::kPlain>(ctx, g, a_kc, b_kc);
@@ -254,15 +293,23 @@ void launch_sliced_w(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc, in
 
 }  // namespace
 
-// Grouped launches (g.ngroup > 0) are weight gradients: operands stored along their rows, f32 results.
+// Grouped launches (g.ngroup > 0) are weight gradients (both operands stored along their rows, f32 results) or forward products (A
+// stored along the contraction, B along its rows, bf16 results).
 void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c) {
     const int split = g.split > 1 ? g.split : 1;
     if (g.ngroup > 0) {
         for (int p = g.ngroup; p < kMaxGroup; p++) g.grp_tile_end[p] = g.grp_tile_end[g.ngroup - 1];  // no tile belongs to the missing ones
         g.blocks = g.grp_tile_end[kMaxGroup - 1] * split;
     } else {
-        g.blocks = eisen_ceil_div(g.M, ST) * eisen_ceil_div(g.N, ST) * batch * split;
+        g.blocks = (int)eisen_ceil_div(g.M, ST) * (int)eisen_ceil_div(g.N, ST) * batch * split;
     }
     if (waves == 8) launch_sliced_w<8>(ctx, g, a_kc, b_kc, dtype_c);
     else launch_sliced_w<4>(ctx, g, a_kc, b_kc, dtype_c);
+}
+
+// G = X Wg, U = X Wu, H = silu(G) * U: A = X [M][K], B = Wg and B_seg[0] = Wu [K][N], C = G, C2 = U, grp_C[0] = H.
+void eisen_gemm_launch_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves) {
+    g.blocks = (int)eisen_ceil_div(g.M, ST) * (int)eisen_ceil_div(g.N, ST / 2);
+    if (waves == 8) gemm_sliced_kernel<8, true, false, bf16_t, Kind::kSwiglu><<<(unsigned)g.blocks, 512, 0, ctx->stream>>>(g);
+    else gemm_sliced_kernel<4, true, false, bf16_t, Kind::kSwiglu><<<(unsigned)g.blocks, 256, 0, ctx->stream>>>(g);
 }

@@ -858,43 +858,32 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
         for (size_t i = 0; i < n; i++) record(std::vector<size_t>(ws.begin(), ws.end()), outs[i], fn);
         return outs;
     }
-    // pair[i]: member i runs batched with member i+1
+    // pair[i]: member i runs batched with member i+1 in the weight gradients
     std::vector<char> pair(n, 0);
     auto congruent = [](const void* p, const void* q, size_t elem) { return ((const char*)q - (const char*)p) % (ptrdiff_t)(8 * elem) == 0; };
     for (size_t i = 0; i + 1 < n; i++)
         if (!(i > 0 && pair[i - 1]) && at(ws[i]).shape == at(ws[i + 1]).shape &&
             congruent(compute_data(ws[i]).ptr, compute_data(ws[i + 1]).ptr, 2) && congruent(at(outs[i]).data.ptr, at(outs[i + 1]).data.ptr, 2))
             pair[i] = 1;
-    // shapes whose gate|up + SwiGLU kernel exists (eisen_hip_gemm_swiglu_forward would otherwise run three launches
-    // where the batched pair below and the SwiGLU kernel are two)
-    const bool with_h = swiglu_h && n == 2 && N[0] == N[1] && M % 256 == 0 && N[0] % 128 == 0 && K % 32 == 0 && (M / 256) * (N[0] / 128) >= 256;
+    const bool with_h = swiglu_h && n == 2 && N[0] == N[1];
     if (swiglu_h) *swiglu_h = with_h ? push_tensor({M, N[0]}, da.dtype, true) : (size_t)-1;
-    if (with_h)
+    if (with_h) {
         check(eisen_hip_gemm_swiglu_forward(ctx_, da.ptr, compute_data(ws[0]).ptr, compute_data(ws[1]).ptr, at(outs[0]).data.ptr, at(outs[1]).data.ptr,
                                             at(*swiglu_h).data.ptr, da.dtype, M, N[0], K),
               "matmul_group");
-    // rotary embedding of the first outputs by the kernel that forms them ([batch, seq, hidden] inputs, whole heads)
-    size_t rope_n = (rotated && !swiglu_h && sa.size() == 3 && sa[1] > 0 && rope_head_dim >= 8 && rope_head_dim % 8 == 0) ? std::min(rope_members, n) : 0;
-    for (size_t i = 0; i < rope_n; i++)
-        if (N[i] % rope_head_dim) rope_n = 0;
-    if (rope_n > 0) *rotated = true;
-    const size_t seq = sa.size() == 3 ? sa[1] : 0;
-    for (size_t i = 0; i < n && !with_h; i++) {
-        const Storage w = compute_data(ws[i]);
-        if (pair[i]) {
-            const ptrdiff_t wd = ((const char*)compute_data(ws[i + 1]).ptr - (const char*)w.ptr) / 2;
-            const ptrdiff_t od = ((const char*)at(outs[i + 1]).data.ptr - (const char*)at(outs[i]).data.ptr) / 2;
-            const size_t members = (i < rope_n ? 1 : 0) + (i + 1 < rope_n ? 1 : 0);
-            if (members > 0)
-                check(eisen_hip_gemm_rope(ctx_, da.ptr, w.ptr, at(outs[i]).data.ptr, da.dtype, 2, M, N[i], K, wd, od, members, seq, rope_head_dim), "matmul_group");
-            else
-                check(eisen_hip_gemm_strided_batched(ctx_, da.ptr, w.ptr, at(outs[i]).data.ptr, da.dtype, da.dtype, 0, 0, 2, M, N[i], K, 0, wd, od, 0), "matmul_group");
-            i++;
-        } else if (i < rope_n) {
-            check(eisen_hip_gemm_rope(ctx_, da.ptr, w.ptr, at(outs[i]).data.ptr, da.dtype, 1, M, N[i], K, 0, 0, 1, seq, rope_head_dim), "matmul_group");
-        } else {
-            check(eisen_hip_gemm(ctx_, da.ptr, w.ptr, at(outs[i]).data.ptr, da.dtype, da.dtype, 0, 0, M, N[i], K, 0), "matmul_group");
+    } else {
+        // rotary embedding of the first outputs by the kernel that forms them ([batch, seq, hidden] inputs, whole heads)
+        size_t rope_n = (rotated && !swiglu_h && sa.size() == 3 && sa[1] > 0 && rope_head_dim >= 8 && rope_head_dim % 8 == 0) ? std::min(rope_members, n) : 0;
+        for (size_t i = 0; i < rope_n; i++)
+            if (N[i] % rope_head_dim) rope_n = 0;
+        if (rope_n > 0) *rotated = true;
+        const void* Bs[3];
+        void* Cs[3];
+        for (size_t i = 0; i < n; i++) {
+            Bs[i] = compute_data(ws[i]).ptr;
+            Cs[i] = at(outs[i]).data.ptr;
         }
+        check(eisen_hip_gemm_forward_group(ctx_, n, da.ptr, Bs, Cs, N.data(), da.dtype, M, K, rope_n, sa.size() == 3 ? sa[1] : 0, rope_head_dim), "matmul_group");
     }
     auto epoch = std::make_shared<size_t>((size_t)-1);
     auto fn = [=](Graph& g) {

@@ -295,6 +295,11 @@ class Context:
         self._call("eisen_hip_gemm_rope", _ptr(A), _ptr(B), _ptr(Cm), _i(dtype), _sz(batch), _sz(M), _sz(N), _sz(K), C.c_longlong(stride_b),
                    C.c_longlong(stride_c), _sz(rope_members), _sz(seq), _sz(head_dim))
 
+    def gemm_forward_group(self, A, Bs, Cs, Ns, dtype, M, K, rope_members=0, seq=0, head_dim=0):
+        n = len(Bs)
+        self._call("eisen_hip_gemm_forward_group", _sz(n), _ptr(A), (_vp * n)(*[_ptr(b) for b in Bs]), (_vp * n)(*[_ptr(c) for c in Cs]), (_sz * n)(*Ns),
+                   _i(dtype), _sz(M), _sz(K), _sz(rope_members), _sz(seq), _sz(head_dim))
+
     def rope_backward(self, go, gx, dtype, batch, seq, hidden, head_dim, accumulate=0):
         self._call("eisen_hip_rope_backward", _ptr(go), _ptr(gx), _i(dtype), _sz(batch), _sz(seq), _sz(hidden), _sz(head_dim), _i(accumulate))
 

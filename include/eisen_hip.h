@@ -233,6 +233,13 @@ int eisen_hip_rope_backward(eisen_ctx* ctx, const void* go, void* gx, int dtype,
 int eisen_hip_gemm_rope(eisen_ctx* ctx, const void* A, const void* B, void* C, int dtype, size_t batch, size_t M, size_t N, size_t K,
                         long long stride_b, long long stride_c, size_t rope_members, size_t seq, size_t head_dim);
 
+/* The forward products of up to 8 Linear layers that read the same input, the first `rope_members` of them rotated as in
+ * eisen_hip_gemm_rope (Q, K and V: src/nn/attention.rs:300-305; gate and up: src/nn/transformer.rs:41-44): C_p = A B_p with A [M, K],
+ * B_p [K, N_p], C_p [M, N_p] of `dtype`.  One launch where the products are few tiles; otherwise equally shaped neighbours run
+ * as a batch of two and the others by themselves.  rope_members = 0: seq and head_dim are not looked at. */
+int eisen_hip_gemm_forward_group(eisen_ctx* ctx, size_t n, const void* A, const void* const* B, void* const* C, const size_t* N, int dtype, size_t M,
+                                 size_t K, size_t rope_members, size_t seq, size_t head_dim);
+
 /* eisen_hip_rope of two tensors that share batch, seq and head_dim in one launch: the q and k projections of
  * GroupedQueryAttention::forward_with_mask (src/nn/attention.rs:304-305, two `g.rope` calls). */
 int eisen_hip_rope_pair(eisen_ctx* ctx, const void* q, void* q_out, size_t hidden_q, const void* k, void* k_out, size_t hidden_k, int dtype,

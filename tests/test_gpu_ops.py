@@ -849,6 +849,49 @@ def test_gemm_bf16_sliced_ends_of_slices(ctx, ta, tb, M, N, Ks):
         x.free()
 
 
+# Forward products of one input as one launch of sliced tiles (few tiles; four and eight waves; cut tiles) and by themselves (a width that is no
+# multiple of 8; many tiles; f32): the bits of each product by itself, rotated where asked for.  Whole numbers: f32 sums are exact.
+@pytest.mark.parametrize("dtype,M,K,Ns,members,seq,hd,one", [
+    (BF16, 201, 256, (256, 64, 64), 2, 201, 32, True), (BF16, 66, 72, (96, 48), 1, 33, 48, True), (BF16, 128, 520, (64, 128, 8), 0, 0, 0, True),
+    (BF16, 1300, 640, (640, 640, 640), 2, 650, 64, True), (BF16, 64, 40, (36, 36), 0, 0, 0, False), (BF16, 2048, 256, (2048, 512, 512), 2, 512, 64, False), (F32, 96, 64, (64, 32, 32), 2, 48, 16, False)])
+def test_gemm_forward_group(ctx, dtype, M, K, Ns, members, seq, hd, one):
+    rng = np.random.default_rng(M + K)
+    a = rng.integers(-2, 3, (M, K)).astype(np.float32)
+    ws = [rng.integers(-2, 3, (K, n)).astype(np.float32) for n in Ns]
+    da, dws, outs, refs = up(ctx, a, dtype), [up(ctx, w, dtype) for w in ws], [], []
+    outs = [ctx.malloc(M * n * 4, zero=True) for n in Ns]
+    ctx.profile_start()
+    ctx.gemm_forward_group(da, dws, outs, list(Ns), dtype, M, K, members, seq, hd)
+    names = list(ctx.profile_stop())
+    assert (len(names) == 1 and "_sliced_grouped" in names[0]) == one, names
+    for i, n in enumerate(Ns):
+        ref = up(ctx, a @ ws[i], dtype)
+        if i < members:
+            ctx.rope(ref, ref, dtype, M // seq, seq, n, hd)
+        assert np.array_equal(dn(ctx, outs[i], (M, n), dtype), dn(ctx, ref, (M, n), dtype)), i
+        ref.free()
+    for x in [da] + dws + outs:
+        x.free()
+
+
+# gate, up and their SwiGLU in sliced tiles of 32 + 32 columns: cut on every side, contractions that end inside a slice, four and eight waves
+@pytest.mark.parametrize("M,N,K", [(64, 32, 64), (67, 40, 72), (1, 8, 8), (130, 200, 264), (201, 1024, 256), (300, 72, 520), (2000, 776, 136)])
+def test_gemm_swiglu_forward_sliced(ctx, M, N, K):
+    x, wg, wu = prep(gen.normal(760, (M, K)), BF16), prep(gen.normal(761, (K, N), 0.3), BF16), prep(gen.normal(762, (K, N), 0.3), BF16)
+    dx, dg, du = up(ctx, x, BF16), up(ctx, wg, BF16), up(ctx, wu, BF16)
+    outs = [ctx.malloc(M * N * 2) for _ in range(3)]
+    ctx.profile_start()
+    ctx.gemm_swiglu_forward(dx, dg, du, *outs, BF16, M, N, K)
+    assert list(ctx.profile_stop()) == ["gemm_nn_bf16_swiglu_64x64x32_sliced"]
+    g, u, h = (dn(ctx, o, (M, N), BF16) for o in outs)
+    assert_close(g, x.astype(np.float64) @ wg.astype(np.float64), 2e-2, "gate")
+    assert_close(u, x.astype(np.float64) @ wu.astype(np.float64), 2e-2, "up")
+    g64 = g.astype(np.float64)  # h is formed from the rounded gate and up: one rounding (2^-9) and an approximate reciprocal and exponential
+    assert_close(h, g64 / (1.0 + np.exp(-g64)) * u, 2.0 ** -8, "h of what was written")
+    for b in [dx, dg, du] + outs:
+        b.free()
+
+
 # Whole-number operands: every product and every f32 sum is exact (below 2^24), so a bf16 result has one right value, the exact
 # sum rounded once.  Split contractions (sliced tiles with whole and cut shapes and packed rows, 128 x 128 tiles), whose parts
 # must not be rounded before they are added, and one product that is not split.
