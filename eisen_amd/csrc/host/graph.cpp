@@ -440,8 +440,9 @@ void Graph::run_beside(bool beside, const std::vector<const void*>& reads, const
         check(launch(), what);
         return;
     }
-    check(eisen_hip_side_begin(ctx_), "side stream");
-    in_beside_ = true;
+    int forked = 0;
+    check(eisen_hip_side_begin_if_behind(ctx_, &forked), "side stream");
+    in_beside_ = forked != 0;  // (on the main stream: a write to what the side stream still writes waits for it)
     int rc = 0;
     try {
         rc = launch();
@@ -452,9 +453,10 @@ void Graph::run_beside(bool beside, const std::vector<const void*>& reads, const
     }
     in_beside_ = false;
     const int rc_end = eisen_hip_side_end(ctx_);  // back on the main stream whatever the launch returned
-    for (const void* p : reads) retained_.emplace(p, false);
+    if (forked)
+        for (const void* p : reads) retained_.emplace(p, false);
     for (size_t w : weights)
-        if (std::find(side_written_.begin(), side_written_.end(), w) == side_written_.end()) side_written_.push_back(w);
+        if (forked && std::find(side_written_.begin(), side_written_.end(), w) == side_written_.end()) side_written_.push_back(w);
     check(rc, what);
     check(rc_end, "side stream");
 }

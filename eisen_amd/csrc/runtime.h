@@ -37,8 +37,9 @@ struct eisen_ctx {
     int device = 0;
     hipStream_t stream = nullptr;       // the stream every entry point launches on (the side stream between side_begin and side_end)
     hipStream_t main_stream = nullptr, side_stream = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_side = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_side = nullptr, ev_mark = nullptr;
     bool side_active = false, side_pending = false;
+    bool mark_set = false, side_inline = false;  // see eisen_hip_side_begin_if_behind
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     bool timer_running = false;
     // size-keyed free lists in front of hipMallocAsync (exact-size buckets, like the

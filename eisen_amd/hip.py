@@ -330,6 +330,12 @@ class Context:
                    _sz(M), _sz(N), _sz(K), C.c_longlong(stride_a), C.c_longlong(stride_b), C.c_longlong(stride_c), _i(accumulate))
 
     def side_begin(self): self._call("eisen_hip_side_begin")
+    def side_begin_if_behind(self):
+        """Begin side work; False: the device has caught up and the work stays on the main stream."""
+        forked = _i(0)
+        self._call("eisen_hip_side_begin_if_behind", C.byref(forked))
+        return bool(forked.value)
+
     def side_end(self): self._call("eisen_hip_side_end")
     def side_wait(self): self._call("eisen_hip_side_wait")
 

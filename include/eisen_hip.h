@@ -61,6 +61,10 @@ int eisen_hip_stream_sync(eisen_ctx* ctx);
  * (eisen_hip_stream_sync waits for both).  Buffers the side work reads must not be written or freed before side_wait.
  * No counterpart in the reference, which runs one stream (src/graph/mod.rs:776-788). */
 int eisen_hip_side_begin(eisen_ctx* ctx);
+/* side_begin when the device is behind the host.  When it has caught up (what the main stream was given before the last such call is
+ * done), *forked is 0 and the calls up to side_end stay on the main stream, in order with the others: a fork costs the host
+ * more than several launches.  Same kernels and same results either way; a captured stream always forks. */
+int eisen_hip_side_begin_if_behind(eisen_ctx* ctx, int* forked);
 int eisen_hip_side_end(eisen_ctx* ctx);
 int eisen_hip_side_wait(eisen_ctx* ctx);
 /* The hipStream_t of the context, as void*, for callers that enqueue their own work. */

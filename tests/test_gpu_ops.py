@@ -1280,6 +1280,38 @@ def test_side_stream_orders_after_fork_and_before_join(ctx):
         t.free()
 
 
+def test_side_begin_stays_on_the_main_stream_when_the_device_has_caught_up(ctx):
+    # a chain of products, each begun as side work and waited for: the same result whether it forked (a long queue ahead) or not
+    n = 256
+    rng = np.random.default_rng(3)
+    perm = np.eye(n, dtype=np.float32)[rng.permutation(n)]
+    big, out = ctx.malloc(4096 * 4096 * 2, zero=True), ctx.malloc(4096 * 4096 * 2)
+    dp, a, b = up(ctx, perm, BF16), up(ctx, np.eye(n, dtype=np.float32), BF16), ctx.malloc(n * n * 2)
+    exp, forked = np.eye(n, dtype=np.float32), []
+    for long_queue in (False, True, False):
+        for _ in range(3):
+            if long_queue:
+                for _ in range(10):
+                    ctx.gemm(big, big, out, BF16, BF16, 0, 0, 4096, 4096, 4096)
+            else:
+                ctx.sync()
+            forked.append(ctx.side_begin_if_behind())
+            ctx.gemm(a, dp, b, BF16, BF16, 0, 0, n, n, n)
+            ctx.side_end()
+            ctx.side_wait()
+            a, b, exp = b, a, exp @ perm
+    assert np.array_equal(dn(ctx, a, (n, n), BF16), exp)
+    # the mark of the last call is done after a synchronisation; a queue of milliseconds was put in front of the later marks of the middle part
+    assert forked[1:3] == [False, False] and forked[4:6] == [True, True] and forked[7:] == [False, False], forked
+    ctx.side_begin_if_behind()
+    for call in (ctx.side_begin, ctx.side_begin_if_behind, ctx.side_wait):
+        with pytest.raises(hip.EisenHipError):
+            call()              # already begun, wherever the work went
+    ctx.side_end()
+    for x in (big, out, dp, a, b):
+        x.free()
+
+
 @pytest.mark.parametrize("M,K,Ns", [(72, 203, (72, 24, 40)), (64, 3100, (64, 200)), (2048, 128, (2048, 512, 512, 2048)), (2048, 192, (1024, 3072)), (256, 64, (128, 256, 128)),
                                     (2048, 256, (2048, 512, 3072)), (256, 2048, (256, 64, 64, 256, 1024, 1024)), (128, 1024, (64, 192))])
 @pytest.mark.parametrize("accumulate", [0, 1])
