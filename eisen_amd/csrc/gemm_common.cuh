@@ -87,6 +87,9 @@ void eisen_gemm_launch_wide_window(eisen_ctx* ctx, const WideWindow& w, unsigned
 void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c);
 void eisen_gemm_launch_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves);
 
+// gemm_edge.hip: bf16 operands, any shape, tiles of 256 or 128 rows and 128 columns (see there for what the operands must allow)
+void eisen_gemm_launch_edge(eisen_ctx* ctx, GemmArgs g, int tile_rows, bool a_kc, bool b_kc, int batch, int dtype_c);
+
 // gemm_f32_sliced.hip: f32 operands and result, operand rows that start on 16-byte boundaries
 void eisen_gemm_launch_f32_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int tile, bool a_kc, bool b_kc, int batch);
 

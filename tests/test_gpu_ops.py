@@ -849,11 +849,76 @@ def test_gemm_bf16_sliced_ends_of_slices(ctx, ta, tb, M, N, Ks):
         x.free()
 
 
+# Tiles with bounds: 256 and 128 rows, cut on every side and whole in some, contractions of one to many slabs that end inside one (also at the first
+# indices of a step, where the rest of the slab is left out), rows that are packed first.  Whole numbers: f32 sums are exact.
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(1352, 1544, 8), (1290, 1664, 72), (2048, 1096, 136), (1351, 1600, 193), (3000, 1032, 320), (4104, 640, 264), (5000, 520, 64), (65, 33000, 40)])
+def test_gemm_bf16_tiles_with_bounds(ctx, ta, tb, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    a = rng.integers(-4, 5, (K, M) if ta else (M, K)).astype(np.float32)
+    b = rng.integers(-4, 5, (N, K) if tb else (K, N)).astype(np.float32)
+    old = rng.integers(-256, 257, (M, N)).astype(np.float32)
+    exact = (a.T if ta else a) @ (b.T if tb else b)
+    da, db, dc, do = up(ctx, a, BF16), up(ctx, b, BF16), ctx.upload(old), up(ctx, old, BF16)
+    ctx.profile_start()
+    ctx.gemm(da, db, dc, BF16, F32, ta, tb, M, N, K, 1)
+    assert "x128x64_edge" in list(ctx.profile_stop())[0]
+    assert np.array_equal(dn(ctx, dc, (M, N), F32), old + exact)
+    ctx.gemm_residual(da, db, do, dc, BF16, BF16, ta, tb, M, N, K)
+    assert np.array_equal(dn(ctx, dc, (M, N), BF16), hip.round_bf16(old + exact))
+    for x in (da, db, dc, do):
+        x.free()
+
+
+# ... segments of the contraction that are no whole slabs, a batch with the rotary epilogue, the SwiGLU backward
+@pytest.mark.parametrize("M,N,Ks", [(1352, 1544, (72, 8, 200)), (3000, 1032, (40, 64)), (2000, 2176, (128, 136, 24))])
+def test_gemm_bf16_tiles_with_bounds_segments(ctx, M, N, Ks):
+    rng = np.random.default_rng(M)
+    a = [rng.integers(-4, 5, (M, k)).astype(np.float32) for k in Ks]
+    b = [rng.integers(-4, 5, (N, k)).astype(np.float32) for k in Ks]
+    da, db, dc = [up(ctx, x, BF16) for x in a], [up(ctx, x, BF16) for x in b], ctx.malloc(M * N * 2)
+    ctx.profile_start()
+    ctx.gemm_ksegments(da, db, list(Ks), dc, BF16, BF16, 0, 1, M, N, 0)
+    names = list(ctx.profile_stop())
+    assert len(names) == 1 and "_edge" in names[0], names
+    assert np.array_equal(dn(ctx, dc, (M, N), BF16), hip.round_bf16(sum(x @ y.T for x, y in zip(a, b))))
+    for x in da + db + [dc]:
+        x.free()
+
+
+def test_gemm_bf16_tiles_with_bounds_rope_and_swiglu_backward(ctx):
+    M, N, K, seq, hd = 1350, 864, 72, 675, 48
+    rng = np.random.default_rng(9)
+    a, b = rng.integers(-2, 3, (M, K)).astype(np.float32), rng.integers(-2, 3, (2, K, N)).astype(np.float32)
+    da, db, dc = up(ctx, a, BF16), up(ctx, b, BF16), ctx.malloc(2 * M * N * 2)
+    ctx.profile_start()
+    ctx.gemm_rope(da, db, dc, BF16, 2, M, N, K, K * N, M * N, 1, seq, hd)
+    assert list(ctx.profile_stop()) == ["gemm_nn_bf16_bf16out_128x128x64_edge_rope"]
+    ref = up(ctx, np.stack([a @ b[0], a @ b[1]]), BF16)
+    ctx.rope(ref, ref, BF16, M // seq, seq, N, hd)
+    assert np.array_equal(dn(ctx, dc, (2, M, N), BF16), dn(ctx, ref, (2, M, N), BF16))
+    for x in (da, db, dc, ref):
+        x.free()
+    M, N, K = 1700, 1288, 136
+    dy, w = prep(gen.normal(770, (M, K)), BF16), prep(gen.normal(771, (N, K), 0.3), BF16)
+    gate, up_ = prep(gen.normal(772, (M, N)), BF16), prep(gen.normal(773, (M, N)), BF16)
+    bufs = [up(ctx, x, BF16) for x in (dy, w, gate, up_)] + [ctx.malloc(M * N * 2), ctx.malloc(M * N * 2)]
+    ctx.profile_start()
+    ctx.gemm_swiglu_backward(*bufs, BF16, 0, 1, M, N, K)
+    assert "_edge_swiglu_bwd" in list(ctx.profile_stop())[0]
+    dh, g64 = dy.astype(np.float64) @ w.astype(np.float64).T, gate.astype(np.float64)
+    sig = 1.0 / (1.0 + np.exp(-g64))
+    assert_close(dn(ctx, bufs[4], (M, N), BF16), dh * up_ * (g64 * sig + sig * (1.0 - g64 * sig)), 2e-2, "dgate")
+    assert_close(dn(ctx, bufs[5], (M, N), BF16), dh * g64 * sig, 2e-2, "dup")
+    for x in bufs:
+        x.free()
+
+
 # Forward products of one input as one launch of sliced tiles (few tiles; four and eight waves; cut tiles) and by themselves (a width that is no
 # multiple of 8; many tiles; f32): the bits of each product by itself, rotated where asked for.  Whole numbers: f32 sums are exact.
 @pytest.mark.parametrize("dtype,M,K,Ns,members,seq,hd,one", [
     (BF16, 201, 256, (256, 64, 64), 2, 201, 32, True), (BF16, 66, 72, (96, 48), 1, 33, 48, True), (BF16, 128, 520, (64, 128, 8), 0, 0, 0, True),
-    (BF16, 1300, 640, (640, 640, 640), 2, 650, 64, True), (BF16, 64, 40, (36, 36), 0, 0, 0, False), (BF16, 2048, 256, (2048, 512, 512), 2, 512, 64, False), (F32, 96, 64, (64, 32, 32), 2, 48, 16, False)])
+    (BF16, 1300, 448, (448, 448, 448), 2, 650, 64, True), (BF16, 64, 40, (36, 36), 0, 0, 0, False), (BF16, 2048, 256, (2048, 512, 512), 2, 512, 64, False), (F32, 96, 64, (64, 32, 32), 2, 48, 16, False)])
 def test_gemm_forward_group(ctx, dtype, M, K, Ns, members, seq, hd, one):
     rng = np.random.default_rng(M + K)
     a = rng.integers(-2, 3, (M, K)).astype(np.float32)
