@@ -39,7 +39,8 @@ struct eisen_ctx {
     hipStream_t main_stream = nullptr, side_stream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_side = nullptr, ev_mark = nullptr;
     bool side_active = false, side_pending = false;
-    bool mark_set = false, side_inline = false;  // see eisen_hip_side_begin_if_behind
+    hipEvent_t mark = nullptr;  // the last of ev_fork and ev_mark that was recorded, see eisen_hip_side_begin_if_behind
+    bool side_inline = false;
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     bool timer_running = false;
     // size-keyed free lists in front of hipMallocAsync (exact-size buckets, like the
