@@ -84,7 +84,7 @@ bool eisen_gemm_wide_window_supports(const WideWindow& w, const WideWindowRow* h
 void eisen_gemm_launch_wide_window(eisen_ctx* ctx, const WideWindow& w, unsigned tiles);
 
 // gemm_sliced.hip: bf16 operands, any shape, the contraction dealt to 4 or 8 waves (see there for what the operands must allow)
-void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c);
+void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int tile, bool a_kc, bool b_kc, int batch, int dtype_c);
 void eisen_gemm_launch_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves);
 
 // gemm_edge.hip: bf16 operands, any shape, tiles of 256 or 128 rows and 128 columns (see there for what the operands must allow)

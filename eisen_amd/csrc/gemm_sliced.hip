@@ -1,18 +1,20 @@
-// bf16 GEMM for any shape, 64 x 64 tiles whose contraction is dealt to the waves of the workgroup (f32 accumulate).
+// bf16 GEMM for any shape, 64 x 64 or 32 x 32 tiles whose contraction is dealt to the waves of the workgroup (f32 accumulate).
 //
 // The kernels of gemm.hip and gemm_wide.hip want whole tiles of 128 or 256 and enough of them to fill 256 CUs.  This one takes the
 // rest: odd batch and sequence lengths, head and vocabulary sizes that are no multiple of anything, and products with few
 // output tiles, whose time is latency (a wave of a shared tile waits for memory, then for a barrier, once per slab, with one
-// workgroup on the CU).  Here a wave owns the whole 64 x 64 tile for every W-th 64-deep slice of the contraction and a private
-// 16 KB of LDS filled by direct-to-LDS loads: no barrier in the loop, W independent chains per CU that cover each other's waits.  A
-// slice is read into registers as a whole, the loads of the wave's next one go out, and its 16 MFMAs run under them.  The W partial
+// workgroup on the CU).  Here a wave owns the whole tile for every W-th 64-deep slice of the contraction and a private
+// 16 KB (8 KB) of LDS filled by direct-to-LDS loads: no barrier in the loop, W independent chains per CU that cover each other's waits.  A
+// slice is read into registers as a whole, the loads of the wave's next one go out, and its 16 (4) MFMAs run under them.  The W partial
 // tiles meet in LDS once, where a thread ends up with eight consecutive columns of a row, so every epilogue works on 16-byte packets.
 //
 // What bounds it: a CU fetches 256 bytes per contraction index for its tile, from an L2 that gives it about 40 bytes per clock; the
 // matrix cores would need 4 clocks for what that takes 6.  Long contractions of one tile per CU run at 0.6 PFLOP/s for that
 // reason, short ones at their latency (launch, first slice, meeting).  us with operands from memory, slices 32 deep in a two-stage
 // ring / now: 1024 x 1024 x 1024 NT 8.4 / 7.3, NN 9.0 / 7.9, x 4096 NT in two segments 22.5 / 18.2; 2048 x 768 x 4096 38.4 / 29.0;
-// 8192 x 256 x 256 7.6 / 6.5; 512 x 768 x 768 7.3 / 6.3; 201 x 256 x 1024 7.7 / 6.6; weight gradients 768 x 768 x 2048 12.6 / 12.0.
+// 8192 x 256 x 256 7.6 / 6.5; 512 x 768 x 768 7.3 / 6.3; 201 x 256 x 1024 7.7 / 6.6; weight gradients 768 x 768 x 2048 12.6 / 12.0.  Tiles of 32
+// where there are few of 64: the same latency over four times the workgroups with a quarter of the work each (201 x 256 x 1024 6.6 -> 5.2; figures at the rule in
+// gemm.hip).
 //
 // Edges.  Rows (m, n) past the end re-read the last row or chunk: they only reach outputs that are not stored.  Contraction
 // indices past the end of a segment re-read the last one, and both fragments are zeroed there.  Operand rows must start on
@@ -21,34 +23,34 @@
 
 namespace {
 
-constexpr int ST = 64, SK = 64;  // tile rows and columns, depth of a slice
+constexpr int SK = 64;  // depth of a slice
 
-// One operand of a slice, 64 x 64 elements, into the LDS: eight loads of eight rows of 128 bytes, whole cache lines.  (Slices 32 deep read
-// half a line at a time of an operand stored along the contraction; the other half belonged to the next wave, and the L1 had
-// dropped the line by then more often than not: 1.5 times the L2 reads, which is what bounds this kernel for long contractions.)
+// One operand of a slice, ST x 64 elements, into the LDS, in loads of 1 KB: rows of 128 bytes, whole cache lines, except for tiles of 32 of an operand
+// that is stored along its rows.  (Slices 32 deep read half a line at a time of an operand stored along the contraction; the other half
+// belonged to the next wave, and the L1 had dropped the line by then more often than not: 1.5 times the L2 reads, which is what bounds this
+// kernel for long contractions.)
 // The rows are operand rows or contraction indices, whichever way the operand is stored; row_last, chunk_last: the last ones that exist.
+template <int ST, bool KC>
 __device__ __forceinline__ void load_slice(const bf16_t* base, int ld, unsigned tile, int row_last, int chunk_last, int lane) {
-    const int row = lane >> 3;  // of load 0; its chunk is permuted by the row, whose bit 3 is the load's parity
-    if (row_last >= 63 && chunk_last >= 7) {
-        unsigned off[2];
+    constexpr int CPR = KC ? 8 : ST / 8, RPL = 64 / CPR, LOADS = ST / 8;  // 16-byte chunks per row, rows per load, loads
+    const int row = lane / CPR;  // of load 0
+    if (row_last >= RPL * LOADS - 1 && chunk_last >= CPR - 1) {
+        unsigned off[2];  // (the permutation of the chunks repeats after 16 rows)
 #pragma unroll
-        for (int odd = 0; odd < 2; odd++) off[odd] = (unsigned)(row * ld + ((lane & 7) ^ lds_swz<128>(row + 8 * odd)) * 8) * 2u;
-        static_for<8>([&](auto i_c) {
+        for (int odd = 0; odd < 2; odd++) off[odd] = (unsigned)(row * ld + ((lane % CPR) ^ lds_swz<CPR * 16>(row + 8 * odd)) * 8) * 2u;
+        static_for<LOADS>([&](auto i_c) {
             constexpr int i = decltype(i_c)::value;
-            load_to_lds_16_at<i * 1024>(base + (long long)i * 8 * ld, off[i & 1], tile);
+            load_to_lds_16_at<i * 1024>(base + (long long)i * RPL * ld, off[RPL == 8 ? i & 1 : 0], tile);
         });
     } else {
-        static_for<8>([&](auto i_c) {
+        static_for<LOADS>([&](auto i_c) {
             constexpr int i = decltype(i_c)::value;
-            const int chunk = (lane & 7) ^ lds_swz<128>(row + 8 * i);
-            load_to_lds_16_at<i * 1024>(base, (unsigned)(min(row + 8 * i, row_last) * ld + min(chunk, chunk_last) * 8) * 2u, tile);
+            const int r = row + RPL * i, chunk = (lane % CPR) ^ lds_swz<CPR * 16>(r);
+            load_to_lds_16_at<i * 1024>(base, (unsigned)(min(r, row_last) * ld + min(chunk, chunk_last) * 8) * 2u, tile);
         });
     }
 }
 
-// What a launch is: one product (or a batch), a product whose contraction runs over several operand pairs, several products, or the gate
-// and up projections with their SwiGLU.  A kernel per kind: the tables of the other kinds would be loaded into, and spilled from, scalar
-// registers.
 // The same for 32 columns each of two operands [K][N] side by side: the first four chunks of a row are the first one's.
 __device__ __forceinline__ void load_slice_of_two(const bf16_t* first, const bf16_t* second, int ld, unsigned tile, int row_last, int chunk_last, int lane) {
     static_for<8>([&](auto i_c) {
@@ -63,12 +65,13 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 
 enum class Kind { kPlain, kSegments, kGroup, kSwiglu };
 
-template <int W, bool A_KC, bool B_KC, typename TC, Kind KIND>
+template <int W, int ST, bool A_KC, bool B_KC, typename TC, Kind KIND>
 __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
     using TA = DirectOperandTile<ST, A_KC, SK, 1>;
     using TB = DirectOperandTile<ST, B_KC, SK, 1>;
-    constexpr int STAGE = TA::ELEMS + TB::ELEMS, STEPS = SK / 16;
-    static_assert(STAGE * sizeof(bf16_t) == ST * ST * sizeof(float), "a wave's partial tile takes the place of its slice");
+    constexpr int STAGE = TA::ELEMS + TB::ELEMS, STEPS = SK / 16, TM = ST / 32;
+    static_assert(KIND != Kind::kSwiglu || ST == 64, "32 columns of each product");
+    static_assert(STAGE * sizeof(bf16_t) >= ST * ST * sizeof(float), "a wave's partial tile takes the place of its slice");
     __shared__ __attribute__((aligned(1024))) bf16_t lds[W][STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -148,11 +151,11 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
             }
         }
         const int k0 = s * SK, left = len - k0;
-        load_slice(A_KC ? Ap + (long long)m0 * lda + k0 : Ap + (long long)k0 * lda + m0, lda, lds_a, A_KC ? m_last : left - 1, (A_KC ? left - 1 : m_last) / 8, lane);
+        load_slice<ST, A_KC>(A_KC ? Ap + (long long)m0 * lda + k0 : Ap + (long long)k0 * lda + m0, lda, lds_a, A_KC ? m_last : left - 1, (A_KC ? left - 1 : m_last) / 8, lane);
         if constexpr (KIND == Kind::kSwiglu)
             load_slice_of_two(Bp + (long long)k0 * ldb + n0, static_cast<const bf16_t*>(g.B_seg[0]) + (long long)k0 * ldb + n0, ldb, lds_b, left - 1, n_last / 8, lane);
         else
-            load_slice(B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0, ldb, lds_b, B_KC ? n_last : left - 1, (B_KC ? left - 1 : n_last) / 8, lane);
+            load_slice<ST, B_KC>(B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0, ldb, lds_b, B_KC ? n_last : left - 1, (B_KC ? left - 1 : n_last) / 8, lane);
         return min(left, SK);
     };
 
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
 
     // What the epilogue reads (the old C or the residual; gate and up) is requested behind the first slice (in front of it, the branches
     // around these loads would make every wave wait for them before it asks for an operand).
-    constexpr int PASSES = ST * ST / 8 / (64 * W);               // groups of eight columns per thread
+    constexpr int GROUPS = ST * ST / 8, PASSES = (GROUPS + 64 * W - 1) / (64 * W);  // groups of eight columns: of the tile, per thread
     TC* C = static_cast<TC*>(g.C) + (long long)bz * g.sC;
     const TC* Rsrc = g.R ? static_cast<const TC*>(g.R) + (long long)bz * g.sC : C;
     float* P = gemm_partial<TC>(g, bz, split, part);
@@ -169,8 +172,8 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
     typename Eight<TC>::V first[PASSES] = {}, second[PASSES] = {};
     static_for<PASSES>([&](auto ps_c) {
         constexpr int ps = decltype(ps_c)::value;
-        const int idx = ps * 64 * W + tid, m = m0 + idx / 8, n = n0 + (idx % 8) * 8;
-        const bool whole = KIND != Kind::kSwiglu && m < g.M && n + 8 <= g.N;
+        const int idx = ps * 64 * W + tid, m = m0 + idx / (ST / 8), n = n0 + (idx % (ST / 8)) * 8;
+        const bool whole = KIND != Kind::kSwiglu && idx < GROUPS && m < g.M && n + 8 <= g.N;
         const long long at = (long long)m * g.ldc + n;
         if (whole && add_old) first[ps] = load_eight(Rsrc + at);
         if (whole && g.gate) {
@@ -179,21 +182,21 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
         }
     });
 
-    f32x16 acc[2][2];
+    f32x16 acc[TM][TM];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < TM; j++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
 
     for (int i = 0; i < n_mine; i++) {
         wait_loads_but<0>();
-        bf16x8 a[STEPS][2], b[STEPS][2];
+        bf16x8 a[STEPS][TM], b[STEPS][TM];
 #pragma unroll
         for (int st = 0; st < STEPS; st++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
+            for (int h = 0; h < TM; h++) {
                 a[st][h] = TA::fragment(As, h * 32, st * 16, lane);
                 b[st][h] = TB::fragment(Bs, h * 32, st * 16, lane);
             }
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
 #pragma unroll
             for (int st = 0; st < STEPS; st++)
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < TM; h++) {
                     const int k = st * 16 + 8 * (lane >> 5);
                     a[st][h] = zero_from(a[st][h], k, now);
                     b[st][h] = zero_from(b[st][h], k, now);
@@ -213,30 +216,30 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
 #pragma unroll
         for (int st = 0; st < STEPS; st++)
 #pragma unroll
-            for (int p = 0; p < 2; p++)
+            for (int p = 0; p < TM; p++)
 #pragma unroll
-                for (int q = 0; q < 2; q++) acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st][p], b[st][q], acc[p][q], 0, 0, 0);
+                for (int q = 0; q < TM; q++) acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st][p], b[st][q], acc[p][q], 0, 0, 0);
     }
 
-    // The waves' tiles, each in the place of its (now idle) slice: row r, column n at r * 64 + ((n / 32) ^ (r / 4 % 2)) * 32 + n % 32,
-    // so that the two halves of a wave (rows 4 apart) write to different banks.
+    // The waves' tiles, each in the place of its (now idle) slice, rows 4 apart (the two halves of a wave) in different halves of the banks.
+    auto place = [](int r, int n) { return ST == 64 ? r * 64 + (n ^ ((r >> 2 & 1) * 32)) : (r ^ (r >> 2 & 1)) * 32 + n; };
     float* mine = reinterpret_cast<float*>(As);
     if (n_mine > 0) {
         const int c = lane & 31, gh = lane >> 5;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < TM; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) mine[(i * 32 + 8 * (v / 4) + 4 * gh + (v % 4)) * ST + (j ^ gh) * 32 + c] = acc[i][j][v];
+                for (int v = 0; v < 16; v++) mine[place(i * 32 + 8 * (v / 4) + 4 * gh + (v % 4), j * 32 + c)] = acc[i][j][v];
     }
     __syncthreads();
     auto sum_of_waves = [&](int r, int cg, float (&val)[8]) __attribute__((always_inline)) {
-        const float* src = reinterpret_cast<const float*>(lds[0]) + r * ST + ((cg >> 2) ^ ((r >> 2) & 1)) * 32 + (cg & 3) * 8;
+        const float* src = reinterpret_cast<const float*>(lds[0]) + place(r, cg * 8);
 #pragma unroll
         for (int e = 0; e < 8; e++) val[e] = 0.f;
         for (int w = 0; w < n_parts; w++) {  // in wave order
-            const float4 lo = *reinterpret_cast<const float4*>(src + w * ST * ST), hi = *reinterpret_cast<const float4*>(src + w * ST * ST + 4);
+            const float4 lo = *reinterpret_cast<const float4*>(src + w * (STAGE / 2)), hi = *reinterpret_cast<const float4*>(src + w * (STAGE / 2) + 4);
             val[0] += lo.x; val[1] += lo.y; val[2] += lo.z; val[3] += lo.w;
             val[4] += hi.x; val[5] += hi.y; val[6] += hi.z; val[7] += hi.w;
         }
@@ -263,9 +266,9 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
     } else {
         static_for<PASSES>([&](auto ps_c) {
             constexpr int ps = decltype(ps_c)::value;
-            const int idx = ps * 64 * W + tid, r = idx / 8, cg = idx % 8;
+            const int idx = ps * 64 * W + tid, r = idx / (ST / 8), cg = idx % (ST / 8);
             const int m = m0 + r, n = n0 + cg * 8;
-            if (m >= g.M || n >= g.N) return;
+            if (idx >= GROUPS || m >= g.M || n >= g.N) return;
             float val[8];
             sum_of_waves(r, cg, val);
             gemm_store_eight<TC>(g, val, m, n, member, C, Rsrc, add_old, P, first[ps], second[ps]);
@@ -276,15 +279,31 @@ __global__ __launch_bounds__(64 * W) void gemm_sliced_kernel(GemmArgs g) {
 template <int W, typename TC, Kind KIND>
 void launch_sliced(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc) {
     const unsigned grid = (unsigned)g.blocks;
-    if (a_kc && b_kc) gemm_sliced_kernel<W, true, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else if (a_kc) gemm_sliced_kernel<W, true, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else if (b_kc) gemm_sliced_kernel<W, false, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else gemm_sliced_kernel<W, false, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    if (a_kc && b_kc) gemm_sliced_kernel<W, 64, true, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    else if (a_kc) gemm_sliced_kernel<W, 64, true, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    else if (b_kc) gemm_sliced_kernel<W, 64, false, true, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    else gemm_sliced_kernel<W, 64, false, false, TC, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+}
+// 32 x 32 tiles: products with A stored along the contraction, and weight gradients
+template <int W, typename TC, Kind KIND>
+void launch_sliced_32(eisen_ctx* ctx, const GemmArgs& g, bool b_kc) {
+    if (b_kc) gemm_sliced_kernel<W, 32, true, true, TC, KIND><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+    else gemm_sliced_kernel<W, 32, true, false, TC, KIND><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+}
+template <int W>
+void launch_sliced_32_w(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc, int dtype_c) {
+    if (!a_kc && g.ngroup > 0) gemm_sliced_kernel<W, 32, false, false, float, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+    else if (!a_kc) gemm_sliced_kernel<W, 32, false, false, float, Kind::kPlain><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+    else if (g.ngroup > 0) gemm_sliced_kernel<W, 32, true, false, bf16_t, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+    else if (g.nseg > 1 && dtype_c == EISEN_BF16) launch_sliced_32<W, bf16_t, Kind::kSegments>(ctx, g, b_kc);
+    else if (g.nseg > 1) launch_sliced_32<W, float, Kind::kSegments>(ctx, g, b_kc);
+    else if (dtype_c == EISEN_BF16) launch_sliced_32<W, bf16_t, Kind::kPlain>(ctx, g, b_kc);
+    else launch_sliced_32<W, float, Kind::kPlain>(ctx, g, b_kc);
 }
 template <int W>
 void launch_sliced_w(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc, int dtype_c) {
-    if (g.ngroup > 0 && dtype_c == EISEN_BF16) gemm_sliced_kernel<W, true, false, bf16_t, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
-    else if (g.ngroup > 0) gemm_sliced_kernel<W, false, false, float, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+    if (g.ngroup > 0 && dtype_c == EISEN_BF16) gemm_sliced_kernel<W, 64, true, false, bf16_t, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
+    else if (g.ngroup > 0) gemm_sliced_kernel<W, 64, false, false, float, Kind::kGroup><<<(unsigned)g.blocks, 64 * W, 0, ctx->stream>>>(g);
     else if (g.nseg > 1 && dtype_c == EISEN_BF16) launch_sliced<W, bf16_t, Kind::kSegments>(ctx, g, a_kc, b_kc);
     else if (g.nseg > 1) launch_sliced<W, float, Kind::kSegments>(ctx, g, a_kc, b_kc);
     else if (dtype_c == EISEN_BF16) launch_sliced<W, bf16_t, Kind::kPlain>(ctx, g, a_kc, b_kc);
@@ -295,21 +314,23 @@ void launch_sliced_w(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc, in
 
 // Grouped launches (g.ngroup > 0) are weight gradients (both operands stored along their rows, f32 results) or forward products (A
 // stored along the contraction, B along its rows, bf16 results).
-void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, bool a_kc, bool b_kc, int batch, int dtype_c) {
+void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int tile, bool a_kc, bool b_kc, int batch, int dtype_c) {
     const int split = g.split > 1 ? g.split : 1;
     if (g.ngroup > 0) {
         for (int p = g.ngroup; p < kMaxGroup; p++) g.grp_tile_end[p] = g.grp_tile_end[g.ngroup - 1];  // no tile belongs to the missing ones
         g.blocks = g.grp_tile_end[kMaxGroup - 1] * split;
     } else {
-        g.blocks = (int)eisen_ceil_div(g.M, ST) * (int)eisen_ceil_div(g.N, ST) * batch * split;
+        g.blocks = (int)eisen_ceil_div(g.M, tile) * (int)eisen_ceil_div(g.N, tile) * batch * split;
     }
-    if (waves == 8) launch_sliced_w<8>(ctx, g, a_kc, b_kc, dtype_c);
-    else launch_sliced_w<4>(ctx, g, a_kc, b_kc, dtype_c);
+    if (tile == 64 && waves == 8) launch_sliced_w<8>(ctx, g, a_kc, b_kc, dtype_c);
+    else if (tile == 64) launch_sliced_w<4>(ctx, g, a_kc, b_kc, dtype_c);
+    else if (waves == 8) launch_sliced_32_w<8>(ctx, g, a_kc, b_kc, dtype_c);
+    else launch_sliced_32_w<4>(ctx, g, a_kc, b_kc, dtype_c);
 }
 
 // G = X Wg, U = X Wu, H = silu(G) * U: A = X [M][K], B = Wg and B_seg[0] = Wu [K][N], C = G, C2 = U, grp_C[0] = H.
 void eisen_gemm_launch_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves) {
-    g.blocks = (int)eisen_ceil_div(g.M, ST) * (int)eisen_ceil_div(g.N, ST / 2);
-    if (waves == 8) gemm_sliced_kernel<8, true, false, bf16_t, Kind::kSwiglu><<<(unsigned)g.blocks, 512, 0, ctx->stream>>>(g);
-    else gemm_sliced_kernel<4, true, false, bf16_t, Kind::kSwiglu><<<(unsigned)g.blocks, 256, 0, ctx->stream>>>(g);
+    g.blocks = (int)eisen_ceil_div(g.M, 64) * (int)eisen_ceil_div(g.N, 32);
+    if (waves == 8) gemm_sliced_kernel<8, 64, true, false, bf16_t, Kind::kSwiglu><<<(unsigned)g.blocks, 512, 0, ctx->stream>>>(g);
+    else gemm_sliced_kernel<4, 64, true, false, bf16_t, Kind::kSwiglu><<<(unsigned)g.blocks, 256, 0, ctx->stream>>>(g);
 }

@@ -823,7 +823,8 @@ def test_gemm_bf16_sliced_tiles_and_packed_rows(ctx, ta, tb, M, N, K):
 # take in one go, in whole and cut tiles, one segment and several, one product and a group.  Whole-number operands: f32 results are exact.
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,Ks", [(64, 64, (56,)), (64, 128, (64,)), (72, 136, (72,)), (128, 64, (256,)), (136, 72, (264,)), (64, 64, (512,)), (200, 64, (520,)),
-                                    (1024, 2048, (320,)), (72, 64, (56, 64, 72)), (128, 200, (8, 128)), (64, 72, (264, 8, 320))])
+                                    (1024, 2048, (320,)), (72, 64, (56, 64, 72)), (128, 200, (8, 128)), (64, 72, (264, 8, 320)),
+                                    (32, 32, (64,)), (33, 40, (72,)), (8, 264, (520,)), (300, 1000, (72,)), (1024, 800, (64, 128)), (520, 520, (1100,))])
 def test_gemm_bf16_sliced_ends_of_slices(ctx, ta, tb, M, N, Ks):
     rng = np.random.default_rng(M + N + sum(Ks))
     a = [rng.integers(-4, 5, (k, M) if ta else (M, k)).astype(np.float32) for k in Ks]
