@@ -92,6 +92,7 @@ void eisen_gemm_launch_edge(eisen_ctx* ctx, GemmArgs g, int tile_rows, bool a_kc
 
 // gemm_f32_sliced.hip: f32 operands and result, operand rows that start on 16-byte boundaries
 void eisen_gemm_launch_f32_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int tile, bool a_kc, bool b_kc, int batch);
+void eisen_gemm_launch_f32_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves, int tile);
 
 // gemm_f32.hip: f32 operands and result, any shape
 struct F32GemmPlan {

@@ -23,7 +23,7 @@ namespace {
 
 constexpr int FK = 32;  // depth of a slice
 
-enum class Kind { kPlain, kSegments, kGroup };
+enum class Kind { kPlain, kSegments, kGroup, kSwiglu };
 
 // integer divisions leave values that are the same in every lane in vector registers
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -54,6 +54,29 @@ struct F32SliceTile {
                 constexpr int i = decltype(i_c)::value;
                 const int r = row + i * ROWS;
                 load_to_lds_16_at<i * 1024>(base, (unsigned)(min(row_at(r), row_last) * ld + min(chunk_at(r, lane % CPR), chunk_last) * 4) * 4u, tile);
+            });
+        }
+    }
+    // The same for T/2 columns each of two operands [K][N] side by side: the first half of a row's chunks is the first one's.  The operands start `first` and
+    // `second` bytes behind base (32-bit offsets: a 64-bit address per lane and load would cost the vector unit, which bounds the kernel).
+    static __device__ __forceinline__ void load_two(const float* base, unsigned first, unsigned second, int ld, unsigned tile, int row_last, int chunk_last, int lane) {
+        static_assert(!KC, "columns side by side");
+        constexpr int HALF = CPR / 2;
+        const int row = lane / CPR;
+        auto at = [&](int chunk, int last) __attribute__((always_inline)) { return (unsigned)min(chunk % HALF, last) * 16u + (chunk < HALF ? first : second); };
+        if (row_last >= ROWS * LOADS - 1 && chunk_last >= HALF - 1) {
+            unsigned off[2];
+#pragma unroll
+            for (int odd = 0; odd < 2; odd++) off[odd] = (unsigned)((row_at(row + 8 * odd) - 8 * odd) * ld) * 4u + at(chunk_at(row + 8 * odd, lane % CPR), HALF - 1);
+            static_for<LOADS>([&](auto i_c) {
+                constexpr int i = decltype(i_c)::value;
+                load_to_lds_16_at<i * 1024>(base + (long long)i * ROWS * ld, off[(i * ROWS >> 3) & 1], tile);
+            });
+        } else {
+            static_for<LOADS>([&](auto i_c) {
+                constexpr int i = decltype(i_c)::value;
+                const int r = row + i * ROWS;
+                load_to_lds_16_at<i * 1024>(base, (unsigned)(min(row_at(r), row_last) * ld) * 4u + at(chunk_at(r, lane % CPR), chunk_last), tile);
             });
         }
     }
@@ -107,6 +130,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
     using TA = F32SliceTile<FT, A_KC>;
     using TB = F32SliceTile<FT, B_KC>;
     constexpr int TM = FT / 32, kOperandBytes = FT * FK * 4;
+    constexpr int COLS = KIND == Kind::kSwiglu ? FT / 2 : FT;  // columns of each product
     static_assert(2 * kOperandBytes >= FT * FT * (int)sizeof(float), "a wave's partial tile takes the place of its slice");
     __shared__ __attribute__((aligned(1024))) char lds[W][2 * kOperandBytes];
 
@@ -136,15 +160,15 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
         g.ldc = g.N;
         if (!B_KC) g.ldb = g.N;
     } else {
-        const int gx = (g.N + FT - 1) / FT, gy = (g.M + FT - 1) / FT;
+        const int gx = (g.N + COLS - 1) / COLS, gy = (g.M + FT - 1) / FT;
         const int lin = xcd_contiguous_id(blockIdx.x, g.blocks);
         zz = uniform(lin / (gx * gy));
         block_tile<4, 8>(lin - zz * (gx * gy), gy, gx, mt, nt);
     }
-    const int m0 = uniform(mt * FT), n0 = uniform(nt * FT);
+    const int m0 = uniform(mt * FT), n0 = uniform(nt * COLS);
     const int bz = uniform(zz / split), part = uniform(zz % split);
-    const float* A = static_cast<const float*>(g.A) + (long long)bz * g.sA;
-    const float* B = static_cast<const float*>(g.B) + (long long)bz * g.sB;
+    const float* A = static_cast<const float*>(g.A) + (KIND == Kind::kSwiglu ? 0 : (long long)bz * g.sA);
+    const float* B = static_cast<const float*>(g.B) + (KIND == Kind::kSwiglu ? 0 : (long long)bz * g.sB);
 
     // Slices of the contraction: segment by segment, each with a last slice of its own.  This workgroup's are [s_lo, s_hi).
     constexpr bool SEG = KIND == Kind::kSegments;
@@ -184,11 +208,18 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
         }
         const int k0 = s * FK, left = len - k0;
         TA::load(A_KC ? Ap + (long long)m0 * lda + k0 : Ap + (long long)k0 * lda + m0, lda, lds_a, A_KC ? m_last : left - 1, (A_KC ? left - 1 : m_last) / 4, lane);
-        TB::load(B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0, ldb, lds_b, B_KC ? n_last : left - 1, (B_KC ? left - 1 : n_last) / 4, lane);
+        if constexpr (KIND == Kind::kSwiglu)
+            TB::load_two(Bp + (long long)k0 * ldb + n0, (unsigned)g.sA, (unsigned)g.sB, ldb, lds_b, left - 1, n_last / 4, lane);
+        else
+            TB::load(B_KC ? Bp + (long long)n0 * ldb + k0 : Bp + (long long)k0 * ldb + n0, ldb, lds_b, B_KC ? n_last : left - 1, (B_KC ? left - 1 : n_last) / 4, lane);
         return min(left, FK);
     };
 
-    constexpr int GROUPS = FT * FT / 8, PASSES = (GROUPS + 64 * W - 1) / (64 * W);  // groups of eight columns: of the tile, per thread
+    // groups of eight columns: of the tile, per thread; with the SwiGLU a thread has a group of the gate and the same one of up
+    constexpr int GROUPS = FT * FT / 8, HALF = FT / 16, PASSES = KIND == Kind::kSwiglu ? 2 : (GROUPS + 64 * W - 1) / (64 * W);
+    auto has_group = [&](int ps) { return KIND == Kind::kSwiglu ? tid < GROUPS / 2 : GROUPS % (64 * W) == 0 || ps * 64 * W + tid < GROUPS; };
+    auto group_row = [&](int ps) { return KIND == Kind::kSwiglu ? tid / HALF : (ps * 64 * W + tid) / (FT / 8); };
+    auto group_of = [&](int ps) { return KIND == Kind::kSwiglu ? tid % HALF + ps * HALF : (ps * 64 * W + tid) % (FT / 8); };
     float* C = static_cast<float*>(g.C) + (long long)bz * g.sC;
     const float* Rsrc = g.R ? static_cast<const float*>(g.R) + (long long)bz * g.sC : C;
     float* P = gemm_partial<float>(g, bz, split, part);
@@ -238,10 +269,10 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
         int bad = 0;
         static_for<PASSES>([&](auto ps_c) {
             constexpr int ps = decltype(ps_c)::value;
-            const int idx = ps * 64 * W + tid, r = idx / (FT / 8), cg = idx % (FT / 8);
+            const int r = group_row(ps), cg = group_of(ps);
 #pragma unroll
             for (int e = 0; e < 8; e++) val[ps][e] = 0.f;
-            if (GROUPS % (64 * W) != 0 && idx >= GROUPS) return;
+            if (!has_group(ps)) return;
             const float* src = reinterpret_cast<const float*>(lds[0]) + place(r, cg * 8);
             for (int w = 0; w < n_parts; w++) {  // in wave order
                 const float4 lo = *reinterpret_cast<const float4*>(src + w * (kOperandBytes / 2)), hi = *reinterpret_cast<const float4*>(src + w * (kOperandBytes / 2) + 4);
@@ -251,7 +282,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
             }
             if (m0 + r < g.M)
 #pragma unroll
-                for (int e = 0; e < 8; e++) bad |= n0 + cg * 8 + e < g.N && !(fabsf(val[ps][e]) < INFINITY);
+                for (int e = 0; e < 8; e++) bad |= n0 + cg * 8 % COLS + e < g.N && !(fabsf(val[ps][e]) < INFINITY);
         });
         return bad;
     };
@@ -343,6 +374,23 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
         }
         (void)meet(1.f);
     }
+    if constexpr (KIND == Kind::kSwiglu) {  // N is a multiple of 8 and the results start on 16-byte boundaries
+        const int m = m0 + group_row(0), n = n0 + group_of(0) * 8;
+        if (!has_group(0) || m >= g.M || n >= g.N) return;
+        float h[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) h[e] = val[0][e] * (1.0f / (1.0f + __expf(-val[0][e]))) * val[1][e];
+        const long long at = (long long)m * g.N + n;
+        auto store = [&](void* to, const float (&x)[8]) {
+            float4* p = reinterpret_cast<float4*>(static_cast<float*>(to) + at);
+            p[0] = make_float4(x[0], x[1], x[2], x[3]);
+            p[1] = make_float4(x[4], x[5], x[6], x[7]);
+        };
+        store(g.C, val[0]);
+        store(g.C2, val[1]);
+        store(g.grp_C[0], h);
+        return;
+    }
     static_for<PASSES>([&](auto ps_c) {
         constexpr int ps = decltype(ps_c)::value;
         const int idx = ps * 64 * W + tid, m = m0 + idx / (FT / 8), n = n0 + (idx % (FT / 8)) * 8;
@@ -389,4 +437,14 @@ void eisen_gemm_launch_f32_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int til
     else if (tile == 64) launch_f32_sliced_w<4, 64>(ctx, g, a_kc, b_kc);
     else if (waves == 8) launch_f32_sliced_w<8, 32>(ctx, g, a_kc, b_kc);
     else launch_f32_sliced_w<4, 32>(ctx, g, a_kc, b_kc);
+}
+
+// G = X Wg, U = X Wu, H = silu(G) * U: A = X [M][K], C = G, C2 = U, grp_C[0] = H; Wg and Wu [K][N] start sA and sB bytes (below 2^31) behind B.
+void eisen_gemm_launch_f32_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves, int tile) {
+    g.blocks = (int)eisen_ceil_div(g.M, tile) * (int)eisen_ceil_div(g.N, tile / 2);
+    const unsigned grid = (unsigned)g.blocks;
+    if (tile == 64 && waves == 8) gemm_f32_sliced_kernel<8, 64, true, false, Kind::kSwiglu><<<grid, 512, 0, ctx->stream>>>(g);
+    else if (tile == 64) gemm_f32_sliced_kernel<4, 64, true, false, Kind::kSwiglu><<<grid, 256, 0, ctx->stream>>>(g);
+    else if (waves == 8) gemm_f32_sliced_kernel<8, 32, true, false, Kind::kSwiglu><<<grid, 512, 0, ctx->stream>>>(g);
+    else gemm_f32_sliced_kernel<4, 32, true, false, Kind::kSwiglu><<<grid, 256, 0, ctx->stream>>>(g);
 }

@@ -815,8 +815,10 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
             Bs[i] = compute_data(ws[i]).ptr;
             Cs[i] = at(outs[i]).data.ptr;
         }
-        if (swiglu_h) *swiglu_h = (size_t)-1;
-        check(eisen_hip_gemm_grouped(ctx_, n, As, Bs, Cs, N.data(), EISEN_F32, EISEN_F32, 0, 0, M, K, 0), "matmul_group");
+        const bool with_h = swiglu_h && n == 2 && N[0] == N[1];
+        if (swiglu_h) *swiglu_h = with_h ? push_tensor({M, N[0]}, da.dtype, true) : (size_t)-1;
+        if (with_h) check(eisen_hip_gemm_swiglu_forward(ctx_, da.ptr, Bs[0], Bs[1], Cs[0], Cs[1], at(*swiglu_h).data.ptr, EISEN_F32, M, N[0], K), "matmul_group");
+        else check(eisen_hip_gemm_grouped(ctx_, n, As, Bs, Cs, N.data(), EISEN_F32, EISEN_F32, 0, 0, M, K, 0), "matmul_group");
         auto epoch = std::make_shared<size_t>((size_t)-1);
         auto fn = [=](Graph& g) {
             if (*epoch == g.backward_epoch()) return;  // the node is on the tape once per output; it runs once per backward

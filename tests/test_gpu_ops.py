@@ -940,6 +940,41 @@ def test_gemm_forward_group(ctx, dtype, M, K, Ns, members, seq, hd, one):
         x.free()
 
 
+# The same in f32: tiles of 64 with 32 + 32 columns and of 32 with 16 + 16, cut on every side, four and eight waves, either weight first in memory, a value that is
+# not finite in one product (its tile is formed again).  The sums are those of the grouped launch, in its order.
+@pytest.mark.parametrize("M,N,K,up_first,inf", [(32, 16, 32, 0, 0), (64, 256, 64, 1, 0), (1, 8, 4, 0, 0), (67, 40, 100, 1, 1), (200, 72, 260, 0, 1), (700, 1000, 36, 1, 0),
+                                                (1024, 392, 136, 0, 1), (513, 776, 64, 1, 1)])
+def test_gemm_swiglu_forward_f32_sliced(ctx, M, N, K, up_first, inf):
+    x, wg, wu = gen.normal(770, (M, K)), gen.normal(771, (K, N), 0.3), gen.normal(772, (K, N), 0.3)
+    if inf:
+        wu[K // 2, N - 1], x[M - 1, 0] = np.inf, np.finfo(np.float32).max
+    pair = ctx.upload(np.concatenate([wu, wg] if up_first else [wg, wu]))
+    lo, hi = pair.ptr, pair.ptr + K * N * 4
+    dg, du, dx = (hi, lo, ctx.upload(x)) if up_first else (lo, hi, ctx.upload(x))
+    outs, ref = [ctx.malloc(M * N * 4) for _ in range(3)], [ctx.malloc(M * N * 4) for _ in range(2)]
+    ctx.profile_start()
+    ctx.gemm_swiglu_forward(dx, dg, du, *outs, F32, M, N, K)
+    names = list(ctx.profile_stop())
+    assert len(names) == 1 and names[0].startswith("gemm_nn_f32_swiglu_"), names
+    ctx.gemm_grouped([dx, dx], [dg, du], ref, [N, N], F32, F32, 0, 0, M, K, 0)
+    g, u, h = (dn(ctx, o, (M, N), F32) for o in outs)
+    for got, r, w in zip((g, u), ref, (wg, wu)):
+        r = dn(ctx, r, (M, N), F32)
+        if not inf:
+            assert np.array_equal(got, r)
+            continue
+        # a tile that is formed again takes its other product's columns along, whose sums are then those of the f32 MFMAs: K + 6 roundings of 2^-24
+        assert np.array_equal(np.isnan(got), np.isnan(r)) and np.array_equal(np.isinf(got), np.isinf(r))
+        ok = np.isfinite(r)
+        bound = (np.abs(x).astype(np.float64) @ np.abs(np.where(np.isfinite(w), w, 0)).astype(np.float64)) * (K + 6) * 2.0 ** -24
+        assert np.all(np.abs(got[ok].astype(np.float64) - r[ok]) <= bound[ok])
+    finite = np.isfinite(g) & np.isfinite(u) & (np.abs(g) < 80)
+    g64 = np.where(finite, g, 0).astype(np.float64)  # the exponential's argument is rounded: 80 * 2^-24 relative
+    assert finite.sum() > 0 and np.all(np.abs(h - g64 / (1.0 + np.exp(-g64)) * np.where(finite, u, 0))[finite] <= 1e-5 * np.abs(g64 * np.where(finite, u, 0))[finite] + 1e-30)
+    for b in [pair, dx] + outs + ref:
+        b.free()
+
+
 # gate, up and their SwiGLU in sliced tiles of 32 + 32 columns: cut on every side, contractions that end inside a slice, four and eight waves
 @pytest.mark.parametrize("M,N,K", [(64, 32, 64), (67, 40, 72), (1, 8, 8), (130, 200, 264), (201, 1024, 256), (300, 72, 520), (2000, 776, 136)])
 def test_gemm_swiglu_forward_sliced(ctx, M, N, K):
