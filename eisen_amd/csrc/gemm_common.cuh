@@ -88,6 +88,22 @@ void eisen_gemm_launch_wide_window(eisen_ctx* ctx, const WideWindow& w, unsigned
 void eisen_gemm_launch_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int tile, bool a_kc, bool b_kc, int batch, int dtype_c);
 void eisen_gemm_launch_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves);
 
+// gemm_dw.hip: up to kMaxDw products A^T B over one contraction, f32 results (see there for what the operands must allow)
+constexpr int kMaxDw = 64;  // (the table travels with the launch, whose arguments may take 4 KB)
+struct DwProduct {
+    const void* A;  // [K][M]
+    const void* B;  // [K][N]
+    void* C;        // [M][N]
+    int M, N;
+    int accumulate;
+};
+struct DwArgs {
+    int K, tiles, n;
+    int tile_end[kMaxDw];  // tiles of products 0..p
+    DwProduct p[kMaxDw];
+};
+void eisen_gemm_launch_dw(eisen_ctx* ctx, const DwArgs& g, int tile);
+
 // gemm_edge.hip: bf16 operands, any shape, tiles of 256 or 128 rows and 128 columns (see there for what the operands must allow)
 void eisen_gemm_launch_edge(eisen_ctx* ctx, GemmArgs g, int tile_rows, bool a_kc, bool b_kc, int batch, int dtype_c);
 
@@ -515,7 +531,7 @@ struct DirectOperandTile {
     // MFMA operand of the 32 operand rows starting at `row0` for contraction offsets ks..ks+15 (same register
     // contents as OperandTile::fragment)
     static __device__ __forceinline__ bf16x8 fragment(const bf16_t* tile, int row0, int ks, int lane) {
-        if (KC) {
+        if constexpr (KC) {
             const int r = row0 + (lane & 31);
             return *reinterpret_cast<const bf16x8*>(tile + r * BK + ((((ks >> 3) + (lane >> 5)) ^ lds_swz<BK * 2>(r)) << 3));
         }

@@ -214,6 +214,7 @@ void Graph::reinterpret_shape(size_t id, const std::vector<size_t>& shape) {
 // Graph::restore_save_point / clear_activations (src/graph/mod.rs:336-365, :432-435): buffers go
 // back to the size-keyed pool inside the runtime.
 void Graph::restore_save_point(size_t save_point) {
+    flush_left_dw();                        // (only a backward pass that threw, or one that is still running, has left any)
     if (!side_guards.empty()) side_join();  // a backward pass that threw may have left side-stream work reading these buffers
     // buffers kept for side-stream GEMMs (no window): given back now, so that a block-by-block recompute keeps its low
     // high-water mark (the main stream waits for the side stream here; after a whole backward pass it already has)
@@ -246,6 +247,7 @@ void Graph::record(std::vector<size_t> inputs, size_t output, std::function<void
 Storage& Graph::grad_for_write(size_t id, int* accumulate, const void** add_from) {
     Tensor& t = at(id);
     if (t.is_param) {
+        settle_dw(id);
         if (!in_beside_ && !side_written_.empty() && std::find(side_written_.begin(), side_written_.end(), id) != side_written_.end()) side_join();
         *accumulate = t.grad_zero_pending ? 0 : 1;
         t.grad_zero_pending = false;
@@ -414,6 +416,66 @@ void Graph::flush_weight_gradients(size_t only_weight) {
     check(rc, "weight gradients of the window");
 }
 
+// ---- weight gradients of a pass as one launch (see graph.hpp) -----------------------------------------------------
+
+// Products the one launch takes and serves better than a launch each: at least 32 x 32, fewer 128 x 128 tiles than the chip has CUs, or than twice
+// that where the 256 x 256 tiles of the large products do not fit; contractions that need no parts.  Layers of one pass, a launch each / one launch, us: 12 of
+// 1024 x 1024 over 4096 tokens 317 / 116, 6 of 1024 x 3096 x 1024 113 / 83, 6 of 1024 x 4096 (256 tiles) x 4096 275 / 257, 4 of 1280 x 5000 (400) x 4096 298 / 267;
+// 2 of 8192 x 1024 (512) x 1024 54 / 67.
+bool Graph::left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out) {
+    if (backward_root_ == (size_t)-1 || dtype != EISEN_BF16 || rows == 0 || rows > 16384 || in % 8 || out % 8 || in < 32 || out < 32) return false;
+    if (((in + 127) / 128) * ((out + 127) / 128) >= (in % 256 || out % 256 ? 512u : 256u)) return false;
+    if ((uintptr_t)x % 16 || (uintptr_t)dy % 16) return false;
+    const Tensor& tw = at(weight);
+    return tw.is_param && tw.grad.dtype == EISEN_F32 && tw.size() == in * out;
+}
+
+bool Graph::leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out) {
+    if (!left_fits(weight, x, dy, dtype, rows, in, out)) return false;
+    settle_dw(weight);  // a weight used twice: its products one after the other
+    left_dw_.push_back(LeftDW{weight, x, dy, rows, in, out, dtype});
+    retained_.emplace(x, false);
+    retained_.emplace(dy, false);
+    return true;
+}
+
+void Graph::settle_dw(size_t weight) {
+    for (const LeftDW& e : left_dw_)
+        if (e.weight == weight) {
+            flush_left_dw();
+            return;
+        }
+}
+
+void Graph::flush_left_dw() {
+    std::vector<LeftDW> list;
+    list.swap(left_dw_);
+    while (!list.empty()) {  // one launch per contraction length and element type: one for a pass
+        const LeftDW first = list.front();
+        std::vector<const void*> As, Bs;
+        std::vector<void*> Cs;
+        std::vector<size_t> Ms, Ns;
+        std::vector<int> accs;
+        std::vector<LeftDW> rest;
+        for (const LeftDW& e : list) {
+            if (e.rows != first.rows || e.dtype != first.dtype) {
+                rest.push_back(e);
+                continue;
+            }
+            int acc = 0;
+            Cs.push_back(grad_for_write(e.weight, &acc).ptr);
+            As.push_back(e.x);
+            Bs.push_back(e.dy);
+            Ms.push_back(e.in);
+            Ns.push_back(e.out);
+            accs.push_back(acc);
+        }
+        list.swap(rest);
+        check(eisen_hip_gemm_weight_gradients(ctx_, Cs.size(), As.data(), Bs.data(), Cs.data(), Ms.data(), Ns.data(), accs.data(), first.dtype, first.rows),
+              "weight gradients of the pass");
+    }
+}
+
 void Graph::side_join() {
     check(eisen_hip_side_wait(ctx_), "side stream join");
     side_guards.clear();
@@ -422,7 +484,7 @@ void Graph::side_join() {
 }
 
 void Graph::release_retained() {
-    if (retained_.empty()) return;
+    if (retained_.empty() || !left_dw_.empty()) return;  // (what is left for the pass's launch still has to be read)
     std::unordered_map<const void*, bool> held;
     held.swap(retained_);
     for (auto& kv : held)
@@ -473,6 +535,7 @@ const Storage& Graph::grad_for_read(size_t id) {
 }
 
 void Graph::request_zero_grad(size_t id) {
+    settle_dw(id);
     if (!window_dw.empty() && at(id).is_param) flush_weight_gradients();  // what the window holds is added first, then cleared with the rest
     Tensor& t = at(id);
     if (t.is_param) t.grad_zero_pending = true;
@@ -485,6 +548,7 @@ void Graph::materialize_grad(size_t id) {
 }
 
 void Graph::apply_pending_zero(size_t id) {
+    settle_dw(id);
     if (!side_written_.empty() && std::find(side_written_.begin(), side_written_.end(), id) != side_written_.end()) side_join();
     Tensor& t = at(id);
     if (t.grad_zero_pending) {
@@ -505,6 +569,7 @@ void Graph::backward(size_t loss_id) {
     check(eisen_hip_fill(ctx_, lg.ptr, lg.dtype, 1.0f, lg.numel), "backward seed");
     backward_nodes_from(0);
     backward_root_ = (size_t)-1;
+    flush_left_dw();
     flush_norm_dw(true);
     side_join();
     if (!pending_dw.empty()) {
@@ -646,6 +711,7 @@ size_t Graph::matmul(size_t a, size_t b) {
         Storage& ga = g.grad_for_write(a, &acc);
         g.check(eisen_hip_gemm(g.ctx(), go.ptr, g.compute_data(b).ptr, ga.ptr, go.dtype, ga.dtype, 0, 1, M, K, N, acc), "matmul backward dA");
         if (g.window_take(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N)) return;
+        if (g.leave_dw(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N)) return;
         const void* xa = g.compute_data(a).ptr;
         g.run_beside(g.at(b).is_param && g.beside_fits(K, N), {xa, go.ptr}, {b}, [&]() {
             int accb = 0;
@@ -688,8 +754,8 @@ size_t Graph::matmul_residual(size_t a, size_t b, size_t r, bool defer_dw) {
         }
         Storage& ga = g.grad_for_write(a, &acc);
         g.check(eisen_hip_gemm(g.ctx(), go.ptr, g.compute_data(b).ptr, ga.ptr, go.dtype, ga.dtype, 0, 1, M, K, N, acc), "matmul_residual backward dA");
-        if (g.window_take(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N)) {
-            // left for the window's launch; whoever adds to dOut's buffer (now dR's) next gets a fresh one
+        if (g.window_take(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N) || g.leave_dw(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N)) {
+            // left for the window's or the pass's launch; whoever adds to dOut's buffer (now dR's) next gets a fresh one
         } else if (defer_dw && go.dtype == EISEN_BF16 && g.at(b).is_param) {
             // dOut's buffer (now also dR's) is only added to by nodes that run after the collecting group
             g.pending_dw.push_back(PendingDW{b, g.compute_data(a).ptr, go.ptr, M, K, N});
@@ -741,7 +807,7 @@ size_t Graph::swiglu_matmul_residual(size_t gate, size_t up, size_t b, size_t r,
             g.check(eisen_hip_accumulate(g.ctx(), gr.ptr, go.ptr, go.dtype, M * N, acc), "swiglu_matmul_residual backward dR");
         }
         // large products only: a small one gains nothing from running beside the chain
-        const bool windowed = g.window_take(b, g.at(h).data.ptr, go.ptr, go.dtype, M, K, N);
+        const bool windowed = g.window_take(b, g.at(h).data.ptr, go.ptr, go.dtype, M, K, N) || g.leave_dw(b, g.at(h).data.ptr, go.ptr, go.dtype, M, K, N);
         const bool side = !windowed && go.dtype == EISEN_BF16 && g.at(b).is_param && K % 256 == 0 && N % 128 == 0 && M % 64 == 0 && (K / 256) * (N / 128) >= 128;
         if (side) {
             // dB beside the input-gradient chain: it reads h and dOut; dOut's buffer (now dR's) is next written by whoever
@@ -925,11 +991,19 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
         // launch (same rows, same input width, same accumulate state, f32 gradients).
         const Storage xa = g.compute_data(a);
         if (all) {
-            // every member joins the window or none: a group split between the window and this pass gains nothing
-            bool fits = true;
-            for (size_t i = 0; i < n; i++) fits = fits && g.window_fits(ws[i], EISEN_BF16, M, K, N[i]);
-            if (fits) {
-                for (size_t i = 0; i < n; i++) g.window_take(ws[i], xa.ptr, g.grad_for_read(outs[i]).ptr, EISEN_BF16, M, K, N[i]);
+            // every member joins the window (or is left for the pass's launch) or none: a group split between them and this node gains nothing
+            bool fits = true, left = true;
+            for (const PendingDW& p : g.pending_dw) left = left && std::find(collect_dw.begin(), collect_dw.end(), p.weight) == collect_dw.end();  // these wait for this node's launch
+            for (size_t i = 0; i < n; i++) {
+                fits = fits && g.window_fits(ws[i], EISEN_BF16, M, K, N[i]);
+                left = left && g.left_fits(ws[i], xa.ptr, g.grad_for_read(outs[i]).ptr, EISEN_BF16, M, K, N[i]);
+            }
+            if (fits || left) {
+                for (size_t i = 0; i < n; i++) {
+                    const void* dy = g.grad_for_read(outs[i]).ptr;
+                    if (fits) g.window_take(ws[i], xa.ptr, dy, EISEN_BF16, M, K, N[i]);
+                    else g.leave_dw(ws[i], xa.ptr, dy, EISEN_BF16, M, K, N[i]);
+                }
                 for (size_t e = 0; e < g.pending_dw.size();) {  // gradients this group was to collect (none in a model whose layers all join the window)
                     const PendingDW p = g.pending_dw[e];
                     if (std::find(collect_dw.begin(), collect_dw.end(), p.weight) == collect_dw.end()) {
@@ -1073,6 +1147,7 @@ size_t Graph::matmul_trans_b(size_t a, size_t b) {
         Storage& ga = g.grad_for_write(a, &acc);
         g.check(eisen_hip_gemm(g.ctx(), go.ptr, g.compute_data(b).ptr, ga.ptr, go.dtype, ga.dtype, 0, 0, M, K, N, acc), "matmul_trans_b backward dA");
         const void* xa = g.compute_data(a).ptr;
+        if (g.leave_dw(b, go.ptr, xa, go.dtype, M, N, K)) return;
         g.run_beside(g.at(b).is_param && g.beside_fits(N, K), {go.ptr, xa}, {b}, [&]() {
             int accb = 0;
             Storage& gb = g.grad_for_write(b, &accb);

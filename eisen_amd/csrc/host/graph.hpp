@@ -226,7 +226,26 @@ class Graph {
     };
     std::vector<WindowDW> window_dw;
 
+    // ---- weight gradients of a pass as one launch ------------------------------------------------------------------
+    // The products of a narrow model's layers are each too small for the chip, and nothing in the pass reads them: they are left until
+    // the pass ends, or until something else writes, reads or clears the gradient of one of the weights, and then run together
+    // (eisen_hip_gemm_weight_gradients).  Operands are kept as for the window.  The bits of a product do not depend on when its turn comes or on what
+    // runs with it.  The step of the ~14 M model: see leave_dw.
+    void flush_left_dw();
+
    private:
+    struct LeftDW {
+        size_t weight;
+        const void *x, *dy;
+        size_t rows, in, out;
+        int dtype;
+    };
+    std::vector<LeftDW> left_dw_;
+    bool left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out);
+    // left until later when left_fits; false: the caller forms the product now
+    bool leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out);
+    // before anything else touches the gradient of a weight
+    void settle_dw(size_t weight);
     eisen_ctx* ctx_;
     size_t backward_root_ = (size_t)-1;
     size_t backward_epoch_ = 0;

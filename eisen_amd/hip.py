@@ -362,6 +362,12 @@ class Context:
         pn = (C.c_size_t * n)(*Ns)
         self._call("eisen_hip_gemm_grouped_ksegments", _sz(n), _sz(ns), pa, pb, pc, pm, pn, _sz(seg_k), _i(accumulate))
 
+    def gemm_weight_gradients(self, As, Bs, Cs, Ms, Ns, accumulate, dtype, K):
+        """C_p (+)= As[p]^T Bs[p] over one contraction, f32 results."""
+        n = len(Cs)
+        self._call("eisen_hip_gemm_weight_gradients", _sz(n), (_vp * n)(*[_ptr(a) for a in As]), (_vp * n)(*[_ptr(b) for b in Bs]), (_vp * n)(*[_ptr(c) for c in Cs]),
+                   (C.c_size_t * n)(*Ms), (C.c_size_t * n)(*Ns), (C.c_int * n)(*accumulate), _i(dtype), _sz(K))
+
     def gemm_swiglu_forward(self, X, Wg, Wu, G, U, H, dtype, M, N, K):
         """G = X Wg, U = X Wu, H = silu(G) * U."""
         self._call("eisen_hip_gemm_swiglu_forward", _ptr(X), _ptr(Wg), _ptr(Wu), _ptr(G), _ptr(U), _ptr(H), _i(dtype), _sz(M), _sz(N), _sz(K))

@@ -315,6 +315,13 @@ int eisen_hip_gemm_grouped(eisen_ctx* ctx, size_t n, const void* const* A, const
 int eisen_hip_gemm_grouped_ksegments(eisen_ctx* ctx, size_t n_products, size_t n_segments, const void* const* A, const void* const* B,
                                      void* const* C, const size_t* M, const size_t* N, size_t seg_k, int accumulate);
 
+/* C_p (+)= A_p^T B_p for any number of products over one contraction: the dB += A^T dC of the matmul backward
+ * (src/graph/ops/linear.rs:279-287) for the layers of a backward pass at once, whose products are each too small to fill the
+ * chip.  A[p] is [K, M_p], B[p] [K, N_p] (both `dtype`), C[p] f32 [M_p, N_p], added to where accumulate[p].  The bits of a
+ * product do not depend on the others of the call. */
+int eisen_hip_gemm_weight_gradients(eisen_ctx* ctx, size_t n, const void* const* A, const void* const* B, void* const* C, const size_t* M, const size_t* N,
+                                    const int* accumulate, int dtype, size_t K);
+
 /* Tuning of the one-launch form of eisen_hip_gemm_grouped_ksegments (no counterpart in the reference).  An XCD of the GPU
  * runs 32 tiles at a time, which share twelve operand panels in its L2 as long as they walk their contraction close
  * together; left alone they drift apart over the launch and fetch the panels several times.  So a workgroup counts itself
