@@ -103,6 +103,7 @@ struct DwArgs {
     DwProduct p[kMaxDw];
 };
 void eisen_gemm_launch_dw(eisen_ctx* ctx, const DwArgs& g, int tile);
+void eisen_gemm_launch_f32_dw(eisen_ctx* ctx, const DwArgs& g, int tile);  // gemm_f32_sliced.hip
 
 // gemm_edge.hip: bf16 operands, any shape, tiles of 256 or 128 rows and 128 columns (see there for what the operands must allow)
 void eisen_gemm_launch_edge(eisen_ctx* ctx, GemmArgs g, int tile_rows, bool a_kc, bool b_kc, int batch, int dtype_c);

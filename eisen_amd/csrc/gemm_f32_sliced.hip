@@ -27,7 +27,8 @@ namespace {
 
 constexpr int FK = 32;  // depth of a slice
 
-enum class Kind { kPlain, kSegments, kGroup, kSwiglu };
+enum class Kind { kPlain, kSegments, kGroup, kSwiglu, kLayers };
+struct NoLayers {};
 
 // integer divisions leave values that are the same in every lane in vector registers
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -135,7 +136,7 @@ __device__ __forceinline__ void split_bf16(const float (&x)[8], float scale, bf1
 }
 
 template <int W, int FT, bool A_KC, bool B_KC, Kind KIND>
-__global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) {
+__global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g, std::conditional_t<KIND == Kind::kLayers, DwArgs, NoLayers> layers) {
     using TA = F32SliceTile<FT, A_KC>;
     using TB = F32SliceTile<FT, B_KC>;
     constexpr int TM = FT / 32, kOperandBytes = FT * FK * 4;
@@ -168,6 +169,16 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
         nt = (t - first) % n_tiles;
         g.ldc = g.N;
         if (!B_KC) g.ldb = g.N;
+    } else if constexpr (KIND == Kind::kLayers) {  // every lane looks at one product
+        int t = xcd_contiguous_id(blockIdx.x, layers.tiles);
+        const int p = __popcll(__ballot(lane < layers.n && t >= layers.tile_end[lane]));
+        const DwProduct& pr = layers.p[p];
+        if (p > 0) t -= layers.tile_end[p - 1];
+        g.A = pr.A; g.B = pr.B; g.C = pr.C; g.M = pr.M; g.N = pr.N;
+        g.lda = g.M; g.ldb = g.ldc = g.N;
+        g.accumulate = pr.accumulate;
+        zz = 0;
+        block_tile<4, 8>(t, (g.M + FT - 1) / FT, (g.N + FT - 1) / FT, mt, nt);
     } else {
         const int gx = (g.N + COLS - 1) / COLS, gy = (g.M + FT - 1) / FT;
         const int lin = xcd_contiguous_id(blockIdx.x, g.blocks);
@@ -305,7 +316,27 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
     int left = 0;
     if (n_mine > 0) left = issue(0);
     clear();
+    // kLayers: four waves take whole contractions, where other launches give eight waves a part each.  The sums of two slices are added up apart, so that no
+    // accumulator rounds a longer one: error against float64, two slices / all of a wave's / eight waves and parts, 256 x 1024 x 448 1.0e-7 / 1.5e-7 / 1.05e-7,
+    // x 4096 1.3e-7 / 4.9e-7 / 1.7e-7, positive 5.0e-8 / 1.7e-7 / 5.0e-8, x 16384 1.8e-7 / 9.8e-7 / 3.4e-7, 96 x 256 x 1351 1.1e-7 / 2.7e-7 / 0.9e-7; us, the products of
+    // the ~14 M model's layers over 4096 tokens 535 / 498 / 832 in launches of their own.
+    constexpr int kRun = 2;
+    f32x16 total[KIND == Kind::kLayers ? TM : 1][KIND == Kind::kLayers ? TM : 1];
+    auto add_to_total = [&](bool first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < TM; p++)
+#pragma unroll
+            for (int q = 0; q < TM; q++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) total[p][q][v] = first ? acc[p][q][v] : total[p][q][v] + acc[p][q][v];
+    };
+    if constexpr (KIND == Kind::kLayers) add_to_total(true);
     for (int i = 0; i < n_mine; i++) {
+        if constexpr (KIND == Kind::kLayers)
+            if (i > 0 && i % kRun == 0) {
+                add_to_total(false);
+                clear();
+            }
         wait_loads_but<0>();
         float a[2][TM][8], b[2][TM][8];
         read(0, a[0], b[0]);
@@ -367,6 +398,13 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
             block(I1{}, I0{}, I0{}, No{});
         }
     }
+    if constexpr (KIND == Kind::kLayers) {
+        add_to_total(false);
+#pragma unroll
+        for (int p = 0; p < TM; p++)
+#pragma unroll
+            for (int q = 0; q < TM; q++) acc[p][q] = total[p][q];
+    }
     const int bad = meet(-1.f, kUnscale);
     if (__syncthreads_or(bad)) {  // something that is not finite: once more in f32
         clear();
@@ -426,10 +464,10 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g) 
 template <int W, int FT, Kind KIND>
 void launch_f32_sliced(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc) {
     const unsigned grid = (unsigned)g.blocks;
-    if (a_kc && b_kc) gemm_f32_sliced_kernel<W, FT, true, true, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else if (a_kc) gemm_f32_sliced_kernel<W, FT, true, false, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else if (b_kc) gemm_f32_sliced_kernel<W, FT, false, true, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
-    else gemm_f32_sliced_kernel<W, FT, false, false, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g);
+    if (a_kc && b_kc) gemm_f32_sliced_kernel<W, FT, true, true, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g, NoLayers{});
+    else if (a_kc) gemm_f32_sliced_kernel<W, FT, true, false, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g, NoLayers{});
+    else if (b_kc) gemm_f32_sliced_kernel<W, FT, false, true, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g, NoLayers{});
+    else gemm_f32_sliced_kernel<W, FT, false, false, KIND><<<grid, 64 * W, 0, ctx->stream>>>(g, NoLayers{});
 }
 template <int W, int FT>
 void launch_f32_sliced_w(eisen_ctx* ctx, const GemmArgs& g, bool a_kc, bool b_kc) {
@@ -454,12 +492,20 @@ void eisen_gemm_launch_f32_sliced(eisen_ctx* ctx, GemmArgs g, int waves, int til
     else launch_f32_sliced_w<4, 32>(ctx, g, a_kc, b_kc);
 }
 
+// Weight gradients of many layers (see gemm_dw.hip); rows start on 16-byte boundaries.  Four waves whatever the tile, so that the bits are the same.
+void eisen_gemm_launch_f32_dw(eisen_ctx* ctx, const DwArgs& layers, int tile) {
+    GemmArgs g{};
+    g.K = layers.K;
+    if (tile == 64) gemm_f32_sliced_kernel<4, 64, false, false, Kind::kLayers><<<(unsigned)layers.tiles, 256, 0, ctx->stream>>>(g, layers);
+    else gemm_f32_sliced_kernel<4, 32, false, false, Kind::kLayers><<<(unsigned)layers.tiles, 256, 0, ctx->stream>>>(g, layers);
+}
+
 // G = X Wg, U = X Wu, H = silu(G) * U: A = X [M][K], C = G, C2 = U, grp_C[0] = H; Wg and Wu [K][N] start sA and sB bytes (below 2^31) behind B.
 void eisen_gemm_launch_f32_sliced_swiglu(eisen_ctx* ctx, GemmArgs g, int waves, int tile) {
     g.blocks = (int)eisen_ceil_div(g.M, tile) * (int)eisen_ceil_div(g.N, tile / 2);
     const unsigned grid = (unsigned)g.blocks;
-    if (tile == 64 && waves == 8) gemm_f32_sliced_kernel<8, 64, true, false, Kind::kSwiglu><<<grid, 512, 0, ctx->stream>>>(g);
-    else if (tile == 64) gemm_f32_sliced_kernel<4, 64, true, false, Kind::kSwiglu><<<grid, 256, 0, ctx->stream>>>(g);
-    else if (waves == 8) gemm_f32_sliced_kernel<8, 32, true, false, Kind::kSwiglu><<<grid, 512, 0, ctx->stream>>>(g);
-    else gemm_f32_sliced_kernel<4, 32, true, false, Kind::kSwiglu><<<grid, 256, 0, ctx->stream>>>(g);
+    if (tile == 64 && waves == 8) gemm_f32_sliced_kernel<8, 64, true, false, Kind::kSwiglu><<<grid, 512, 0, ctx->stream>>>(g, NoLayers{});
+    else if (tile == 64) gemm_f32_sliced_kernel<4, 64, true, false, Kind::kSwiglu><<<grid, 256, 0, ctx->stream>>>(g, NoLayers{});
+    else if (waves == 8) gemm_f32_sliced_kernel<8, 32, true, false, Kind::kSwiglu><<<grid, 512, 0, ctx->stream>>>(g, NoLayers{});
+    else gemm_f32_sliced_kernel<4, 32, true, false, Kind::kSwiglu><<<grid, 256, 0, ctx->stream>>>(g, NoLayers{});
 }

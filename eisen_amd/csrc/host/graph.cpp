@@ -418,12 +418,13 @@ void Graph::flush_weight_gradients(size_t only_weight) {
 
 // ---- weight gradients of a pass as one launch (see graph.hpp) -----------------------------------------------------
 
-// Products the one launch takes and serves better than a launch each: at least 32 x 32, fewer 128 x 128 tiles than the chip has CUs, or than twice
+// Products the one launch takes and serves better than a launch each: at least 32 x 32 (bf16), fewer 128 x 128 tiles than the chip has CUs, or than twice
 // that where the 256 x 256 tiles of the large products do not fit; contractions that need no parts.  Layers of one pass, a launch each / one launch, us: 12 of
 // 1024 x 1024 over 4096 tokens 317 / 116, 6 of 1024 x 3096 x 1024 113 / 83, 6 of 1024 x 4096 (256 tiles) x 4096 275 / 257, 4 of 1280 x 5000 (400) x 4096 298 / 267;
 // 2 of 8192 x 1024 (512) x 1024 54 / 67.
 bool Graph::left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out) {
-    if (backward_root_ == (size_t)-1 || dtype != EISEN_BF16 || rows == 0 || rows > 16384 || in % 8 || out % 8 || in < 32 || out < 32) return false;
+    if (backward_root_ == (size_t)-1 || rows == 0 || rows > 16384) return false;
+    if (dtype == EISEN_BF16 ? in % 8 || out % 8 || in < 32 || out < 32 : in % 4 || out % 4) return false;
     if (((in + 127) / 128) * ((out + 127) / 128) >= (in % 256 || out % 256 ? 512u : 256u)) return false;
     if ((uintptr_t)x % 16 || (uintptr_t)dy % 16) return false;
     const Tensor& tw = at(weight);
@@ -909,6 +910,14 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
             Storage& ga = g.grad_for_write(a, &acc);
             g.check(eisen_hip_gemm_ksegments(g.ctx(), m, As, Bs, Ks, ga.ptr, EISEN_F32, ga.dtype, 0, 1, M, K, acc), "matmul_group backward dA");
             const void* xa = g.compute_data(a).ptr;
+            bool left = true;
+            for (size_t i = 0; i < n; i++)
+                if (g.has_grad(outs[i])) left = left && g.left_fits(ws[i], xa, g.grad_for_read(outs[i]).ptr, EISEN_F32, M, K, N[i]);
+            if (left) {
+                for (size_t i = 0; i < n; i++)
+                    if (g.has_grad(outs[i])) g.leave_dw(ws[i], xa, g.grad_for_read(outs[i]).ptr, EISEN_F32, M, K, N[i]);
+                return;
+            }
             int accs[3];
             size_t Ns[3];
             m = 0;
