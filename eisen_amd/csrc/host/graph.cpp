@@ -1156,7 +1156,7 @@ size_t Graph::matmul_trans_b(size_t a, size_t b) {
         Storage& ga = g.grad_for_write(a, &acc);
         g.check(eisen_hip_gemm(g.ctx(), go.ptr, g.compute_data(b).ptr, ga.ptr, go.dtype, ga.dtype, 0, 0, M, K, N, acc), "matmul_trans_b backward dA");
         const void* xa = g.compute_data(a).ptr;
-        if (g.leave_dw(b, go.ptr, xa, go.dtype, M, N, K)) return;
+        if (g.window_take(b, go.ptr, xa, go.dtype, M, N, K) || g.leave_dw(b, go.ptr, xa, go.dtype, M, N, K)) return;
         g.run_beside(g.at(b).is_param && g.beside_fits(N, K), {go.ptr, xa}, {b}, [&]() {
             int accb = 0;
             Storage& gb = g.grad_for_write(b, &accb);

@@ -50,7 +50,7 @@ int eisen_graph_restore_save_point(eisen_graph* g, size_t save_point);
  * needs it to stay on the device. */
 /* Weight gradients over a window of backward passes (no counterpart in the reference, whose Linear backward adds
  * A^T dC to the gradient in every pass, src/graph/ops/linear.rs:279-287).  With backward_passes = n in 2..8 the weight
- * gradients of bf16 Linear layers of at least 16 tiles of 256 x 256 are not formed by the pass that produces their
+ * gradients of bf16 Linear layers (a head that is the transposed embedding among them) of at least 16 tiles of 256 x 256 are not formed by the pass that produces their
  * operands: the operands stay allocated (they outlive clear_activations) and one launch per group of equally shaped
  * weights contracts over all passes of the window (eisen_hip_gemm_grouped_ksegments) when the n-th pass ends, or as
  * soon as a parameter's gradient is read, cleared or handed to the optimizer.  The sums are the reference's in another

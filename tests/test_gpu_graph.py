@@ -245,6 +245,36 @@ def test_weight_gradient_window_sums_over_micro_batches(ctx, fused, checkpointin
     assert windowed == 7 * cfg["layers"] + 1
 
 
+def test_weight_gradient_window_holds_the_head_of_a_tied_embedding(ctx):
+    # The head's product C = A E^T leaves dC^T A for the window; the lookup's scatter adds its rows to the same gradient in every pass.
+    # A full window of two passes, then one that a gradient read ends: losses the same, gradients equal up to the order of an f32 sum.
+    cfg = dict(vocab=4096, hidden=256, heads=4, kv_heads=2, ffn=512, layers=1, tie=True)
+    batches = [gen.lm_batch(960 + i, 2, 128, cfg["vocab"], "zipf") for i in range(3)]
+    results = []
+    for window in (0, 2):
+        gg = G.Graph(ctx, G.BF16_MIXED)
+        lm = G.TransformerLM(gg, **cfg)
+        for pid, (_, w) in enumerate(gen.lm_weights(36, **cfg)):
+            gg.load_tensor_data(pid, w)
+        gg.mark_params()
+        gg.set_weight_gradient_window(window)
+        opt = G.AdamW(gg, lm.params(), 1e-3)
+        opt.zero_grad()
+        ctx.sync()
+        base = ctx.pool_stats()[0]
+        losses = [lm.micro_step(x, y) for x, y in batches]
+        grads = [gg.sync_grad_to_cpu(p) for p in lm.params()]
+        ctx.sync()
+        assert ctx.pool_stats()[0] == base, "buffers kept for the window were not given back"
+        results.append((losses, grads))
+        gg.close()
+    (l0, g0), (l1, g1) = results
+    assert l0 == l1
+    for i, (a, b) in enumerate(zip(g0, g1)):
+        assert a.any()
+        assert_close(b, a, 1e-4, f"gradient {i}")
+
+
 def test_weight_gradient_window_flushes_when_a_gradient_is_read_cleared_or_outgrows_it(ctx):
     # The corners of Graph::set_weight_gradient_window on a two-matmul graph whose weight is used twice per pass: a
     # gradient read in the middle of a window sees every pass so far; zero_grad in the middle of a window discards what
