@@ -63,7 +63,7 @@ constexpr int kMaxWindowSegments = 8;
 struct WideWindowRow {
     int M, N;
     int tile_end;  // number of 256 x 256 tiles of products 0..p
-    int pad;
+    int accumulate;
     void* C;
     const void* A[kMaxWindowSegments];  // entries from nseg on repeat the last piece
     const void* B[kMaxWindowSegments];
@@ -71,7 +71,6 @@ struct WideWindowRow {
 struct WideWindow {
     int nprod, nseg;
     int seg_slabs;  // 32-deep slabs per piece, a multiple of 4
-    int accumulate;
     const WideWindowRow* rows;  // device memory, nprod entries
     // Optional meeting point for the workgroups an XCD runs at one time (null: none).  One counter per XCD and group of 32
     // consecutive tiles of its range, zero at launch.  A workgroup counts itself in and waits until its group is complete or

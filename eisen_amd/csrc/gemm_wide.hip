@@ -66,6 +66,7 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(GemmArgs g, std::conditi
         if (prod > 0) t -= __builtin_amdgcn_readfirstlane(w.rows[prod - 1].tile_end);
         const WideWindowRow& row = w.rows[prod];
         g.M = __builtin_amdgcn_readfirstlane(row.M); g.N = __builtin_amdgcn_readfirstlane(row.N);
+        g.accumulate = __builtin_amdgcn_readfirstlane(row.accumulate);
         g.C = uniform_pointer(row.C);
         g.A = uniform_pointer(row.A[0]); g.B = uniform_pointer(row.B[0]);
         g.lda = g.M; g.ldb = g.N; g.ldc = g.N;
@@ -336,7 +337,6 @@ bool eisen_gemm_wide_window_supports(const WideWindow& w, const WideWindowRow* h
 
 void eisen_gemm_launch_wide_window(eisen_ctx* ctx, const WideWindow& w, unsigned tiles) {
     GemmArgs g{};
-    g.accumulate = w.accumulate;
     g.vec_c = 1;
     gemm_wide_kernel<false, false, float, true><<<dim3(tiles, 1, 1), 256, 0, ctx->stream>>>(g, w);
 }

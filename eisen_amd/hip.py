@@ -362,6 +362,13 @@ class Context:
         pn = (C.c_size_t * n)(*Ns)
         self._call("eisen_hip_gemm_grouped_ksegments", _sz(n), _sz(ns), pa, pb, pc, pm, pn, _sz(seg_k), _i(accumulate))
 
+    def gemm_weight_gradients_window(self, As, Bs, Cs, Ms, Ns, seg_k, accumulate):
+        """gemm_grouped_ksegments with an accumulate state per product."""
+        n, ns = len(Cs), len(As[0])
+        self._call("eisen_hip_gemm_weight_gradients_window", _sz(n), _sz(ns), (_vp * (n * ns))(*[_ptr(a) for row in As for a in row]),
+                   (_vp * (n * ns))(*[_ptr(b) for row in Bs for b in row]), (_vp * n)(*[_ptr(c) for c in Cs]), (C.c_size_t * n)(*Ms), (C.c_size_t * n)(*Ns), _sz(seg_k),
+                   (C.c_int * n)(*accumulate))
+
     def gemm_weight_gradients(self, As, Bs, Cs, Ms, Ns, accumulate, dtype, K):
         """C_p (+)= As[p]^T Bs[p] over one contraction, f32 results."""
         n = len(Cs)

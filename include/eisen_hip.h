@@ -310,10 +310,15 @@ int eisen_hip_gemm_grouped(eisen_ctx* ctx, size_t n, const void* const* A, const
  * micro-batch at a time, in f32; here the pieces of a product are summed in the MFMA accumulators of one launch (any
  * number of products of up to 8 pieces, every M_p and N_p a multiple of 256, seg_k of 128, at least 176 tiles of
  * 256 x 256 in all), which reads and writes each gradient once per window instead of once per micro-batch.  Other
- * shapes run one accumulating GEMM per product and piece, in piece order. */
+ * shapes are added piece by piece, in piece order. */
 #define EISEN_GEMM_MAX_KSEGMENTS 8
 int eisen_hip_gemm_grouped_ksegments(eisen_ctx* ctx, size_t n_products, size_t n_segments, const void* const* A, const void* const* B,
                                      void* const* C, const size_t* M, const size_t* N, size_t seg_k, int accumulate);
+
+/* The same with an accumulate state per product.  What the one launch does not take and has fewer 128 x 128 tiles than twice the chip's CUs runs as one launch per
+ * piece (eisen_hip_gemm_weight_gradients). */
+int eisen_hip_gemm_weight_gradients_window(eisen_ctx* ctx, size_t n_products, size_t n_segments, const void* const* A, const void* const* B,
+                                           void* const* C, const size_t* M, const size_t* N, size_t seg_k, const int* accumulate);
 
 /* C_p (+)= A_p^T B_p for any number of products over one contraction: the dB += A^T dC of the matmul backward
  * (src/graph/ops/linear.rs:279-287) for the layers of a backward pass at once, whose products are each too small to fill the
