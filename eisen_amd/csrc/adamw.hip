@@ -1,6 +1,6 @@
 // Fused multi-tensor AdamW over f32 master weights, global gradient norm, zero_grad.
-// One launch covers every parameter tensor: a device table of slots plus a prefix table of
-// 16-byte-packet chunks maps each workgroup to its tensor.  HBM-bound: 16 B read each of
+// One launch covers every parameter tensor: a table of slots with each tensor's first workgroup maps a workgroup to its tensor; up to 64 of them
+// travel with the launch, more stand in device memory.  HBM-bound: 16 B read each of
 // w, g, m, v and 16 B written each of w, m, v per packet (+ 8 B for the bf16 copy).
 #include "device_utils.cuh"
 #include "runtime.h"
@@ -17,14 +17,29 @@ struct SlotDev {
     float* v;
     bf16_t* wb;
     unsigned long long n;
-    unsigned long long first_block;  // index of this tensor's first workgroup
 };
-
-__device__ __forceinline__ int find_slot(const SlotDev* __restrict__ slots, int n_slots, unsigned block) {
-    int lo = 0, hi = n_slots - 1;  // last slot with first_block <= block
+// The table of a launch.  Up to kInline slots are part of its arguments: a copy to the device is a launch of its own in front of a kernel that takes a few
+// microseconds for a small model (gradient norm and update, two copies: the step of the smallest model 303 -> 280 us, 150 M parameters in 40 tensors 937 -> 918).
+constexpr int kInline = 64;
+struct SlotsInline {
+    int n_slots;
+    unsigned first_block[kInline];  // index of a tensor's first workgroup
+    SlotDev slot[kInline];
+};
+struct SlotsDevice {
+    int n_slots;
+    const unsigned* first_block;
+    const SlotDev* slot;
+};
+__device__ __forceinline__ int find_slot(const SlotsInline& t, unsigned block) {  // every lane looks at one
+    const int lane = threadIdx.x & 63;
+    return __popcll(__ballot(lane < t.n_slots && t.first_block[lane] <= block)) - 1;
+}
+__device__ __forceinline__ int find_slot(const SlotsDevice& t, unsigned block) {
+    int lo = 0, hi = t.n_slots - 1;  // last slot with first_block <= block
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (slots[mid].first_block <= block) lo = mid;
+        if (t.first_block[mid] <= block) lo = mid;
         else hi = mid - 1;
     }
     return lo;
@@ -56,11 +71,11 @@ __device__ __forceinline__ void adam_elem(float& w, float g, float& m, float& v,
     w = decayed - p.lr * m_hat / (sqrtf(v_hat) + p.eps);
 }
 
-__global__ __launch_bounds__(kThreads) void adamw_kernel(const SlotDev* __restrict__ slots, int n_slots, AdamParams p,
-                                                         const float* __restrict__ grad_scale) {
-    const int si = find_slot(slots, n_slots, blockIdx.x);
-    const SlotDev s = slots[si];
-    const size_t base = (size_t)(blockIdx.x - s.first_block) * kChunk;
+template <class Slots>
+__global__ __launch_bounds__(kThreads) void adamw_kernel(Slots table, AdamParams p, const float* __restrict__ grad_scale) {
+    const int si = __builtin_amdgcn_readfirstlane(find_slot(table, blockIdx.x));
+    const SlotDev s = table.slot[si];
+    const size_t base = (size_t)(blockIdx.x - table.first_block[si]) * kChunk;
     const float gs = grad_scale ? grad_scale[0] : 1.0f;
     // All 16 loads of the thread are issued before the first use: 16 KB per stream and workgroup in flight.  The last
     // s.n % 4 elements of a tensor (bases are 16-byte aligned, so only they are no whole packet) are taken by one thread each.
@@ -106,10 +121,11 @@ __global__ __launch_bounds__(kThreads) void adamw_kernel(const SlotDev* __restri
     }
 }
 
-__global__ __launch_bounds__(kThreads) void zero_grads_kernel(const SlotDev* __restrict__ slots, int n_slots) {
-    const int si = find_slot(slots, n_slots, blockIdx.x);
-    const SlotDev s = slots[si];
-    const size_t base = (size_t)(blockIdx.x - s.first_block) * kChunk;
+template <class Slots>
+__global__ __launch_bounds__(kThreads) void zero_grads_kernel(Slots table) {
+    const int si = __builtin_amdgcn_readfirstlane(find_slot(table, blockIdx.x));
+    const SlotDev s = table.slot[si];
+    const size_t base = (size_t)(blockIdx.x - table.first_block[si]) * kChunk;
     float* g = const_cast<float*>(s.g);
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -122,11 +138,12 @@ __global__ __launch_bounds__(kThreads) void zero_grads_kernel(const SlotDev* __r
 }
 
 // stage 1: one f64 partial per workgroup (src/nn/optim.rs:258-262 accumulates x*x in f64)
-__global__ __launch_bounds__(kThreads) void sumsq_kernel(const SlotDev* __restrict__ slots, int n_slots, double* __restrict__ partial) {
+template <class Slots>
+__global__ __launch_bounds__(kThreads) void sumsq_kernel(Slots table, double* __restrict__ partial) {
     __shared__ double sh[kThreads / kWave];
-    const int si = find_slot(slots, n_slots, blockIdx.x);
-    const SlotDev s = slots[si];
-    const size_t base = (size_t)(blockIdx.x - s.first_block) * kChunk;
+    const int si = __builtin_amdgcn_readfirstlane(find_slot(table, blockIdx.x));
+    const SlotDev s = table.slot[si];
+    const size_t base = (size_t)(blockIdx.x - table.first_block[si]) * kChunk;
     double acc = 0.0;
     float4 g[4];
 #pragma unroll
@@ -157,6 +174,7 @@ __global__ __launch_bounds__(kThreads) void sumsq_kernel(const SlotDev* __restri
         partial[blockIdx.x] = t;
     }
 }
+// (The workgroup that arrives last adding the partials up itself costs 23 ns per workgroup, more than a launch from 200 on.)
 // stage 2: one workgroup, fixed order; writes norm and clip coefficient (src/nn/optim.rs:282-287)
 __global__ __launch_bounds__(1024) void norm_finish_kernel(const double* __restrict__ partial, size_t n, float max_norm, float* __restrict__ out) {
     __shared__ double sh[1024 / kWave];
@@ -176,11 +194,15 @@ __global__ __launch_bounds__(1024) void norm_finish_kernel(const double* __restr
     }
 }
 
-// Uploads the slot table; returns the device copy and the total workgroup count.
-int upload_slots(eisen_ctx* ctx, const eisen_param_slot* slots, size_t n_slots, bool need_moments, SlotDev** dev_out,
-                 size_t* blocks_out, const char* who) {
+// Checks the slots, forms the launch's table and calls launch(table, workgroups).
+template <class F>
+int with_slots(eisen_ctx* ctx, const eisen_param_slot* slots, size_t n_slots, bool need_moments, const char* who, F&& launch) {
     EISEN_REQUIRE(ctx, slots && n_slots > 0 && n_slots < (size_t(1) << 20), EISEN_E_ARG, "%s: bad slot table", who);
-    std::vector<SlotDev> host(n_slots);
+    SlotsInline small;
+    std::vector<char> large;  // [slots | first workgroups]
+    if (n_slots > (size_t)kInline) large.resize(n_slots * (sizeof(SlotDev) + sizeof(unsigned)));
+    SlotDev* slot = large.empty() ? small.slot : reinterpret_cast<SlotDev*>(large.data());
+    unsigned* first = large.empty() ? small.first_block : reinterpret_cast<unsigned*>(large.data() + n_slots * sizeof(SlotDev));
     size_t blocks = 0;
     for (size_t i = 0; i < n_slots; i++) {
         const eisen_param_slot& s = slots[i];
@@ -188,21 +210,23 @@ int upload_slots(eisen_ctx* ctx, const eisen_param_slot* slots, size_t n_slots, 
         EISEN_REQUIRE(ctx, !need_moments || (s.w && s.m && s.v), EISEN_E_ARG, "%s: slot %zu lacks w/m/v", who, i);
         EISEN_REQUIRE(ctx, eisen_aligned(s.g, 16) && eisen_aligned(s.w, 16) && eisen_aligned(s.m, 16) && eisen_aligned(s.v, 16) && eisen_aligned(s.w_bf16, 8),
                       EISEN_E_ALIGN, "%s: slot %zu buffers must be 16-byte aligned", who, i);
-        host[i] = SlotDev{s.w, s.g, s.m, s.v, (bf16_t*)s.w_bf16, (unsigned long long)s.n, (unsigned long long)blocks};
+        EISEN_REQUIRE(ctx, blocks < (size_t(1) << 31), EISEN_E_SHAPE, "%s: too many elements for one launch", who);
+        slot[i] = SlotDev{s.w, s.g, s.m, s.v, (bf16_t*)s.w_bf16, (unsigned long long)s.n};
+        first[i] = (unsigned)blocks;
         blocks += eisen_ceil_div(s.n, kChunk);
     }
     EISEN_REQUIRE(ctx, blocks < (size_t(1) << 31), EISEN_E_SHAPE, "%s: too many elements for one launch", who);
-    void* dev = nullptr;
-    int rc = eisen_hip_malloc(ctx, n_slots * sizeof(SlotDev), &dev);
-    if (rc) return rc;
-    rc = eisen_hip_htod(ctx, dev, host.data(), n_slots * sizeof(SlotDev));
-    if (rc) {
-        (void)eisen_hip_free(ctx, dev);
-        return rc;
+    if (large.empty()) {
+        small.n_slots = (int)n_slots;
+        return launch(small, (unsigned)blocks);
     }
-    *dev_out = (SlotDev*)dev;
-    *blocks_out = blocks;
-    return 0;
+    void* dev = nullptr;
+    int rc = eisen_hip_malloc(ctx, large.size(), &dev);
+    if (rc) return rc;
+    rc = eisen_hip_htod(ctx, dev, large.data(), large.size());
+    if (!rc) rc = launch(SlotsDevice{(int)n_slots, reinterpret_cast<const unsigned*>(static_cast<char*>(dev) + n_slots * sizeof(SlotDev)), static_cast<const SlotDev*>(dev)}, (unsigned)blocks);
+    const int rc_free = eisen_hip_free(ctx, dev);
+    return rc ? rc : rc_free;
 }
 
 }  // namespace
@@ -211,50 +235,41 @@ extern "C" int eisen_hip_adamw_step(eisen_ctx* ctx, const eisen_param_slot* slot
                                     float beta2, float eps, float weight_decay, float bc1, float bc2,
                                     const float* grad_scale_device) {
     EISEN_CHECK_CTX(ctx);
-    SlotDev* dev = nullptr;
-    size_t blocks = 0;
-    int rc = upload_slots(ctx, slots, n_slots, true, &dev, &blocks, "adamw_step");
-    if (rc) return rc;
-    AdamParams p{lr, beta1, beta2, eps, weight_decay, bc1, bc2};
-    double bytes = 0.0;  // per parameter: w, g, m, v read, w, m, v written (28 B) and the bf16 copy written where there is one
-    for (size_t i = 0; i < n_slots; i++) bytes += (double)slots[i].n * (slots[i].w_bf16 ? 30.0 : 28.0);
-    EisenProfScope prof(ctx, "adamw", bytes);
-    adamw_kernel<<<(unsigned)blocks, kThreads, 0, ctx->stream>>>(dev, (int)n_slots, p, grad_scale_device);
-    EISEN_LAUNCH_CHECK(ctx, "adamw_kernel");
-    return eisen_hip_free(ctx, dev);
+    return with_slots(ctx, slots, n_slots, true, "adamw_step", [&](const auto& table, unsigned blocks) -> int {
+        AdamParams p{lr, beta1, beta2, eps, weight_decay, bc1, bc2};
+        double bytes = 0.0;  // per parameter: w, g, m, v read, w, m, v written (28 B) and the bf16 copy written where there is one
+        for (size_t i = 0; i < n_slots; i++) bytes += (double)slots[i].n * (slots[i].w_bf16 ? 30.0 : 28.0);
+        EisenProfScope prof(ctx, "adamw", bytes);
+        adamw_kernel<<<blocks, kThreads, 0, ctx->stream>>>(table, p, grad_scale_device);
+        EISEN_LAUNCH_CHECK(ctx, "adamw_kernel");
+        return 0;
+    });
 }
 
 extern "C" int eisen_hip_zero_grads(eisen_ctx* ctx, const eisen_param_slot* slots, size_t n_slots) {
     EISEN_CHECK_CTX(ctx);
-    SlotDev* dev = nullptr;
-    size_t blocks = 0;
-    int rc = upload_slots(ctx, slots, n_slots, false, &dev, &blocks, "zero_grads");
-    if (rc) return rc;
-    zero_grads_kernel<<<(unsigned)blocks, kThreads, 0, ctx->stream>>>(dev, (int)n_slots);
-    EISEN_LAUNCH_CHECK(ctx, "zero_grads_kernel");
-    return eisen_hip_free(ctx, dev);
+    return with_slots(ctx, slots, n_slots, false, "zero_grads", [&](const auto& table, unsigned blocks) -> int {
+        zero_grads_kernel<<<blocks, kThreads, 0, ctx->stream>>>(table);
+        EISEN_LAUNCH_CHECK(ctx, "zero_grads_kernel");
+        return 0;
+    });
 }
 
 extern "C" int eisen_hip_grad_norm(eisen_ctx* ctx, const eisen_param_slot* slots, size_t n_slots, float max_norm,
                                    float* out_device) {
     EISEN_CHECK_CTX(ctx);
     EISEN_REQUIRE(ctx, out_device != nullptr, EISEN_E_ARG, "grad_norm: null output");
-    SlotDev* dev = nullptr;
-    size_t blocks = 0;
-    int rc = upload_slots(ctx, slots, n_slots, false, &dev, &blocks, "grad_norm");
-    if (rc) return rc;
-    void* ws = nullptr;
-    rc = eisen_workspace(ctx, blocks * sizeof(double), &ws);
-    if (rc) {
-        (void)eisen_hip_free(ctx, dev);
-        return rc;
-    }
-    double bytes = 0.0;
-    for (size_t i = 0; i < n_slots; i++) bytes += (double)slots[i].n * 4.0;
-    EisenProfScope prof(ctx, "grad_sumsq", bytes);
-    sumsq_kernel<<<(unsigned)blocks, kThreads, 0, ctx->stream>>>(dev, (int)n_slots, (double*)ws);
-    EISEN_LAUNCH_CHECK(ctx, "sumsq_kernel");
-    norm_finish_kernel<<<1, 1024, 0, ctx->stream>>>((const double*)ws, blocks, max_norm, out_device);
-    EISEN_LAUNCH_CHECK(ctx, "norm_finish_kernel");
-    return eisen_hip_free(ctx, dev);
+    return with_slots(ctx, slots, n_slots, false, "grad_norm", [&](const auto& table, unsigned blocks) -> int {
+        void* ws = nullptr;
+        int rc = eisen_workspace(ctx, blocks * sizeof(double), &ws);
+        if (rc) return rc;
+        double bytes = 0.0;
+        for (size_t i = 0; i < n_slots; i++) bytes += (double)slots[i].n * 4.0;
+        EisenProfScope prof(ctx, "grad_sumsq", bytes);
+        sumsq_kernel<<<blocks, kThreads, 0, ctx->stream>>>(table, (double*)ws);
+        EISEN_LAUNCH_CHECK(ctx, "sumsq_kernel");
+        norm_finish_kernel<<<1, 1024, 0, ctx->stream>>>((const double*)ws, blocks, max_norm, out_device);
+        EISEN_LAUNCH_CHECK(ctx, "norm_finish_kernel");
+        return 0;
+    });
 }
