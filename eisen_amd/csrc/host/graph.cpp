@@ -164,27 +164,11 @@ void Graph::load_tensor_data(size_t id, const float* host, size_t n) {
     }
 }
 
-// bf16 -> f32, exact.  (optimize: the loop is a quarter of a large read-back when it is not vectorised)
-__attribute__((optimize("O3"))) static void widen(const uint16_t* __restrict__ raw, uint32_t* __restrict__ out, size_t n) {
-    for (size_t i = 0; i < n; i++) out[i] = (uint32_t)raw[i] << 16;
-}
-// A storage's values as f32, straight into the caller's memory; bf16 goes through one buffer of limited size that is not
-// cleared first.  What a large read-back costs beside the copy is fresh host memory touched for the first time: 201 x 8192
-// logits passed through three such buffers of together 16 MB, and a forward pass that took 1071 us takes 679 without.
+// A storage's values as f32, straight into the caller's memory (of what a large read-back costs, fresh host memory touched for the first time is a good part).
 void Graph::download(const Storage& s, float* out) {
     if (!s.numel) return;
-    if (s.dtype == EISEN_F32) {
-        check(eisen_hip_dtoh(ctx_, out, s.ptr, s.numel * sizeof(float)), "sync_to_cpu");
-        return;
-    }
-    static_assert(sizeof(float) == sizeof(uint32_t), "");
-    const size_t block = std::min<size_t>(s.numel, size_t(1) << 21);
-    const std::unique_ptr<uint16_t[]> raw(new uint16_t[block]);
-    for (size_t at = 0; at < s.numel; at += block) {
-        const size_t n = std::min(block, s.numel - at);
-        check(eisen_hip_dtoh(ctx_, raw.get(), static_cast<const uint16_t*>(s.ptr) + at, n * 2), "sync_to_cpu");
-        widen(raw.get(), reinterpret_cast<uint32_t*>(out + at), n);
-    }
+    if (s.dtype == EISEN_F32) check(eisen_hip_dtoh(ctx_, out, s.ptr, s.numel * sizeof(float)), "sync_to_cpu");
+    else check(eisen_hip_dtoh_widen(ctx_, out, s.ptr, s.numel), "sync_to_cpu");
 }
 
 // Tensor::sync_to_cpu / Graph::sync_grad_to_cpu (src/tensor.rs:177-223, src/graph/mod.rs:629-668).

@@ -50,17 +50,26 @@ struct eisen_ctx {
     size_t in_use_bytes = 0, cached_bytes = 0;
     size_t peak_in_use_bytes = 0;  // high-water mark of in_use_bytes since the last reset
     size_t driver_allocs = 0;      // requests for memory that reached the driver (device pool misses, workspace growth, tables, pinned staging)
-    // pinned staging ring for asynchronous uploads: a slot is reused only after its copy's event fired
+    // pinned staging ring for asynchronous uploads: a slot is reused only after its copy is done, which an event tells or, behind an upload by a kernel,
+    // a word in pinned memory that the kernel sets to the number it was given
     struct StageSlot {
         void* ptr = nullptr;
         size_t bytes = 0;
         hipEvent_t done = nullptr;
+        unsigned* word = nullptr;
+        unsigned number = 0;
+        hipStream_t stream = nullptr;  // of that kernel
+        bool by_word = false;
         bool in_flight = false;
         bool reserved = false;  // holds the result of a device-to-host copy that eisen_hip_dtoh_finish has not collected yet
     };
     static constexpr int kStageSlots = 16;
     StageSlot stage[kStageSlots];
     int stage_next = 0;
+    unsigned* words = nullptr;  // pinned: one per slot, then those of a read-back in flight (eisen_hip_dtoh)
+    void* back = nullptr;       // pinned ring of a read-back
+    size_t back_bytes = 0;
+    unsigned back_number = 0;
     // grow-only device workspace for two-stage reductions and tables
     void* ws = nullptr;
     size_t ws_bytes = 0;

@@ -3,6 +3,10 @@
 // (src/graph/mod.rs:152-307, src/graph/memory.rs:189-266, src/tensor.rs:145-223).
 #include "runtime.h"
 
+#include <algorithm>
+#include <atomic>
+#include <thread>
+
 int eisen_set_error(eisen_ctx* ctx, int code, const char* fmt, ...) {
     if (ctx) {
         va_list ap;
@@ -12,6 +16,97 @@ int eisen_set_error(eisen_ctx* ctx, int code, const char* fmt, ...) {
     }
     return code;
 }
+
+namespace {
+
+// ---- copies between device memory and pinned host memory as kernels --------------------------------------------
+// The runtime's own copies of 32 KB and more go through a copy engine, which a chain of kernels waits for: a kernel, such a copy and a kernel take 19.5 us where the
+// copy as a kernel of one workgroup makes it 9; and an event behind a copy, recorded to know when its staging memory is free, is 3 us of
+// the stream.  So an upload of up to kCopyKernelBytes is one workgroup here, and says itself that it is done.  (Not the tickets of eisen_hip_dtoh_begin: a
+// few bytes, where making them visible to the host writes the caches back: 1 us more than the event.)
+constexpr int kCopyThreads = 1024;
+constexpr size_t kCopyKernelBytes = size_t(256) << 10;
+
+template <typename T>
+__device__ __forceinline__ void copy_by_workgroup(const T* __restrict__ src, T* __restrict__ dst, unsigned n) {
+    constexpr int U = 4;
+    for (unsigned i = threadIdx.x; i < n; i += U * kCopyThreads) {
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i + u * kCopyThreads < n) v[u] = src[i + u * kCopyThreads];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i + u * kCopyThreads < n) dst[i + u * kCopyThreads] = v[u];
+    }
+}
+// The word says that the staging memory has been read (a thread that stores has what it read).
+template <typename T>
+__global__ __launch_bounds__(kCopyThreads) void copy_in_kernel(const T* __restrict__ src, T* __restrict__ dst, unsigned n, unsigned* word, unsigned number) {
+    copy_by_workgroup(src, dst, n);
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// A read-back in pieces: kBackGroup workgroups bring each piece, two groups in turn, and every workgroup has a word per piece, so that the host takes a piece while the
+// next ones travel.
+constexpr size_t kBackPiece = size_t(256) << 10, kBackRing = size_t(8) << 20;
+constexpr int kBackGroup = 8, kBackPieces = (int)(kBackRing / kBackPiece), kBackWords = kBackPieces * kBackGroup;
+__global__ __launch_bounds__(kCopyThreads) void read_back_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, unsigned n, unsigned* words, unsigned number) {
+    constexpr unsigned PIECE = (unsigned)(kBackPiece / 16), SHARE = PIECE / kBackGroup;
+    const unsigned member = blockIdx.x % kBackGroup;
+    for (unsigned piece = blockIdx.x / kBackGroup; piece * PIECE < n; piece += 2) {
+        const unsigned at = piece * PIECE + member * SHARE;
+        if (at < n) copy_by_workgroup(src + at, dst + at, min(SHARE, n - at));
+        __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(words + piece * kBackGroup + member, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// Waits until a kernel of `stream` has set the word; a stream that has run dry or failed ends the wait as well.
+int wait_word(eisen_ctx* ctx, const unsigned* word, unsigned number, hipStream_t stream) {
+    for (unsigned spin = 0; __atomic_load_n(word, __ATOMIC_ACQUIRE) != number; spin++) {
+        if (spin < 20000) {
+            __builtin_ia32_pause();
+            continue;
+        }
+        if (spin % 4096 != 0) {
+            std::this_thread::yield();
+            continue;
+        }
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (asking a stream ends a capture in another mode)
+        EISEN_HIP_TRY(ctx, hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t q = hipStreamQuery(stream);
+        EISEN_HIP_TRY(ctx, hipThreadExchangeStreamCaptureMode(&mode));
+        if (q == hipSuccess) break;
+        (void)hipGetLastError();
+        if (q != hipErrorNotReady) EISEN_HIP_TRY(ctx, q);
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return 0;
+}
+// Until the slot's copy is done.
+int wait_slot(eisen_ctx* ctx, eisen_ctx::StageSlot& s) {
+    if (s.by_word) return wait_word(ctx, s.word, s.number, s.stream);
+    EISEN_HIP_TRY(ctx, hipEventSynchronize(s.done));
+    return 0;
+}
+// The slot's memory to the device by a kernel, where size and alignment let it and nothing is being captured (a replay would set the word again); false: not.
+bool upload_by_kernel(eisen_ctx* ctx, eisen_ctx::StageSlot& s, void* dst, size_t bytes) {
+    if (bytes > kCopyKernelBytes || bytes % 4 != 0 || !eisen_aligned(dst, 4)) return false;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+    s.number++;
+    if (bytes % 16 == 0 && eisen_aligned(dst, 16))
+        copy_in_kernel<<<1, kCopyThreads, 0, ctx->stream>>>(static_cast<const uint4*>(s.ptr), static_cast<uint4*>(dst), (unsigned)(bytes / 16), s.word, s.number);
+    else
+        copy_in_kernel<<<1, kCopyThreads, 0, ctx->stream>>>(static_cast<const unsigned*>(s.ptr), static_cast<unsigned*>(dst), (unsigned)(bytes / 4), s.word, s.number);
+    s.stream = ctx->stream;
+    s.by_word = true;
+    return true;
+}
+
+}  // namespace
 
 extern "C" const char* eisen_hip_last_error(eisen_ctx* ctx) { return ctx ? ctx->last_error : "null context"; }
 
@@ -97,6 +192,8 @@ extern "C" int eisen_hip_destroy(eisen_ctx* ctx) {
         if (sl.ptr) (void)hipHostFree(sl.ptr);
         if (sl.done) (void)hipEventDestroy(sl.done);
     }
+    if (ctx->back) (void)hipHostFree(ctx->back);
+    if (ctx->words) (void)hipHostFree(ctx->words);
     for (hipEvent_t e : ctx->prof.pool) (void)hipEventDestroy(e);
     (void)hipEventDestroy(ctx->ev_start);
     (void)hipEventDestroy(ctx->ev_stop);
@@ -316,6 +413,16 @@ int eisen_workspace(eisen_ctx* ctx, size_t bytes, void** out) {
     return 0;
 }
 
+// the pinned words: 64 bytes per slot, then a read-back's
+static int eisen_words(eisen_ctx* ctx) {
+    if (ctx->words) return 0;
+    ctx->driver_allocs++;
+    const size_t bytes = 64 * (size_t)eisen_ctx::kStageSlots + sizeof(unsigned) * (size_t)kBackWords;
+    EISEN_HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->words), bytes, hipHostMallocDefault));
+    memset(ctx->words, 0, bytes);
+    return 0;
+}
+
 int eisen_staging(eisen_ctx* ctx, size_t bytes, eisen_ctx::StageSlot** out) {
     int tries = 0;
     while (ctx->stage[ctx->stage_next].reserved && tries < eisen_ctx::kStageSlots) {
@@ -325,11 +432,18 @@ int eisen_staging(eisen_ctx* ctx, size_t bytes, eisen_ctx::StageSlot** out) {
     EISEN_REQUIRE(ctx, tries < eisen_ctx::kStageSlots, EISEN_E_STATE, "every staging slot holds an uncollected eisen_hip_dtoh_begin result");
     eisen_ctx::StageSlot& s = ctx->stage[ctx->stage_next];
     ctx->stage_next = (ctx->stage_next + 1) % eisen_ctx::kStageSlots;
-    if (!s.done) EISEN_HIP_TRY(ctx, hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+    if (!s.done) {
+        EISEN_HIP_TRY(ctx, hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+        const int rc = eisen_words(ctx);
+        if (rc) return rc;
+        s.word = ctx->words + 16 * (&s - ctx->stage);
+    }
     if (s.in_flight) {
-        EISEN_HIP_TRY(ctx, hipEventSynchronize(s.done));
+        const int rc = wait_slot(ctx, s);
+        if (rc) return rc;
         s.in_flight = false;
     }
+    s.by_word = false;
     if (bytes > s.bytes) {
         if (s.ptr) EISEN_HIP_TRY(ctx, hipHostFree(s.ptr));
         s.ptr = nullptr;
@@ -355,8 +469,12 @@ extern "C" int eisen_hip_htod(eisen_ctx* ctx, void* dst, const void* src, size_t
         int rc = eisen_staging(ctx, bytes, &st);
         if (rc) return rc;
         memcpy(st->ptr, src, bytes);
-        EISEN_HIP_TRY(ctx, hipMemcpyAsync(dst, st->ptr, bytes, hipMemcpyHostToDevice, ctx->stream));
-        EISEN_HIP_TRY(ctx, hipEventRecord(st->done, ctx->stream));
+        if (upload_by_kernel(ctx, *st, dst, bytes)) {
+            EISEN_LAUNCH_CHECK(ctx, "eisen_hip_htod");
+        } else {
+            EISEN_HIP_TRY(ctx, hipMemcpyAsync(dst, st->ptr, bytes, hipMemcpyHostToDevice, ctx->stream));
+            EISEN_HIP_TRY(ctx, hipEventRecord(st->done, ctx->stream));
+        }
         st->in_flight = true;
         return 0;
     }
@@ -365,13 +483,80 @@ extern "C" int eisen_hip_htod(eisen_ctx* ctx, void* dst, const void* src, size_t
     return 0;
 }
 
+// Device memory into the caller's, as it is or (widen) bf16 as f32.  Through pinned memory in pieces (read_back_kernel); what is small, not aligned or under capture
+// goes by the runtime's copy.  That copy and this, in us: 4 KB 24 and 25 (the line is at 16 KB, where they part), 64 KB 37 and 19, 256 KB 118 and 25, 1 MB 67 and
+// 50, 8 MB 512 and 240, 512 MB 32100 and 24900.  A forward pass with its 201 x 8192 bf16 logits read back 579 and 369.
+static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, bool widen) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    EISEN_HIP_TRY(ctx, hipStreamIsCapturing(ctx->stream, &capture));
+    const size_t whole = bytes / 16 * 16;
+    char* out = static_cast<char*>(dst);
+    auto take = [&](const void* from, size_t n) {
+        if (widen) {
+            const uint16_t* __restrict__ f = static_cast<const uint16_t*>(from);
+            uint32_t* __restrict__ t = reinterpret_cast<uint32_t*>(out);
+            for (size_t i = 0; i < n / 2; i++) t[i] = (uint32_t)f[i] << 16;
+        } else {
+            memcpy(out, from, n);
+        }
+        out += widen ? 2 * n : n;
+    };
+    size_t done = 0;
+    if (whole >= (size_t(16) << 10) && eisen_aligned(src, 16) && capture == hipStreamCaptureStatusNone) {
+        const int rc = eisen_words(ctx);
+        if (rc) return rc;
+        const size_t want = (std::min(whole, kBackRing) + kBackPiece - 1) / kBackPiece * kBackPiece;
+        if (ctx->back_bytes < want) {
+            if (ctx->back) EISEN_HIP_TRY(ctx, hipHostFree(ctx->back));
+            ctx->back = nullptr;
+            ctx->back_bytes = 0;
+            ctx->driver_allocs++;
+            EISEN_HIP_TRY(ctx, hipHostMalloc(&ctx->back, want, hipHostMallocDefault));
+            ctx->back_bytes = want;
+        }
+        unsigned* words = ctx->words + 16 * eisen_ctx::kStageSlots;
+        while (done < whole) {
+            const size_t n = std::min(whole - done, ctx->back_bytes);
+            const unsigned number = ++ctx->back_number;
+            read_back_kernel<<<2 * kBackGroup, kCopyThreads, 0, ctx->stream>>>(reinterpret_cast<const uint4*>(static_cast<const char*>(src) + done), static_cast<uint4*>(ctx->back),
+                                                                              (unsigned)(n / 16), words, number);
+            EISEN_LAUNCH_CHECK(ctx, "eisen_hip_dtoh");
+            for (size_t at = 0, piece = 0; at < n; at += kBackPiece, piece++) {
+                for (int w = 0; w < kBackGroup; w++) {
+                    const int rw = wait_word(ctx, words + piece * kBackGroup + w, number, ctx->stream);
+                    if (rw) return rw;
+                }
+                take(static_cast<char*>(ctx->back) + at, std::min(kBackPiece, n - at));
+            }
+            done += n;
+        }
+    }
+    if (done == bytes) return 0;
+    const size_t left = bytes - done;
+    char* raw = widen ? out + left : out;  // (in the upper half of what is to hold it as f32: element i is read before any write reaches it)
+    EISEN_HIP_TRY(ctx, hipMemcpyAsync(raw, static_cast<const char*>(src) + done, left, hipMemcpyDeviceToHost, ctx->stream));
+    EISEN_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    for (size_t i = 0; widen && i < left / 2; i++) {
+        uint16_t half;
+        memcpy(&half, raw + 2 * i, 2);
+        const uint32_t value = (uint32_t)half << 16;
+        memcpy(out + 4 * i, &value, 4);
+    }
+    return 0;
+}
+
 extern "C" int eisen_hip_dtoh(eisen_ctx* ctx, void* dst, const void* src, size_t bytes) {
     EISEN_CHECK_CTX(ctx);
     EISEN_REQUIRE(ctx, dst && src, EISEN_E_ARG, "eisen_hip_dtoh: null pointer");
     if (bytes == 0) return 0;
-    EISEN_HIP_TRY(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    EISEN_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    return 0;
+    return read_back(ctx, dst, src, bytes, false);
+}
+
+extern "C" int eisen_hip_dtoh_widen(eisen_ctx* ctx, float* dst, const void* src_bf16, size_t n) {
+    EISEN_CHECK_CTX(ctx);
+    EISEN_REQUIRE(ctx, dst && src_bf16, EISEN_E_ARG, "eisen_hip_dtoh_widen: null pointer");
+    if (n == 0) return 0;
+    return read_back(ctx, dst, src_bf16, 2 * n, true);
 }
 
 extern "C" int eisen_hip_dtoh_begin(eisen_ctx* ctx, const void* src, size_t bytes, int* ticket_out) {
@@ -400,7 +585,8 @@ extern "C" int eisen_hip_dtoh_finish(eisen_ctx* ctx, int ticket, void* dst, size
     eisen_ctx::StageSlot& s = ctx->stage[ticket];
     EISEN_REQUIRE(ctx, bytes <= s.bytes, EISEN_E_ARG, "eisen_hip_dtoh_finish: %zu bytes asked of a %zu-byte slot", bytes, s.bytes);
     s.reserved = false;
-    EISEN_HIP_TRY(ctx, hipEventSynchronize(s.done));  // waits for this copy only: later work stays queued
+    const int rc = wait_slot(ctx, s);  // for this copy only: later work stays queued
+    if (rc) return rc;
     s.in_flight = false;
     memcpy(dst, s.ptr, bytes);
     return 0;

@@ -94,6 +94,8 @@ int eisen_hip_pool_peak(eisen_ctx* ctx, size_t* peak_in_use_bytes, int reset);
 int eisen_hip_htod(eisen_ctx* ctx, void* dst_device, const void* src_host, size_t bytes);
 /* stream.clone_dtoh (src/tensor.rs:177-223): synchronises the stream before returning. */
 int eisen_hip_dtoh(eisen_ctx* ctx, void* dst_host, const void* src_device, size_t bytes);
+/* n bf16 values as f32. */
+int eisen_hip_dtoh_widen(eisen_ctx* ctx, float* dst_host, const void* src_device_bf16, size_t n);
 /* clone_dtoh in two halves, for a value the host wants without draining the stream (the loss of a micro-batch,
  * examples/train_llm.rs:450, read while the backward pass is already queued): `begin` enqueues the copy into pinned
  * memory of the library and returns a ticket, `finish` waits for that copy alone and fills dst_host.  At most 8 tickets
