@@ -28,7 +28,7 @@
 //     between the halves, 250 moves in the loop), and a workgroup takes one key block where there is more than one pair for
 //     every CU, the longest first: two pairs on one CU and one on the next cost a third of the time.
 //     1 x 6001 x 16 heads of 128 on 4 KV heads, causal: 445 us; the register-staged kernel this replaced took 708.
-#include "attention_common.cuh"
+#include "attention_dq.cuh"
 
 namespace {
 
@@ -51,16 +51,42 @@ __device__ __forceinline__ void mfma_agpr(f32x16& acc, const bf16x8& a, const bf
 __device__ __forceinline__ void agpr_settle(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 7" : "+a"(acc)); }
 
 // ABL: a part of the tile loop left out for a measurement (AttnAblation; kAblNone is the kernel)
-template <int HD, int ABL>
+// GW > 0: short sequences, both passes side by side in one launch, the first dq_blocks workgroups on dQ (with GW query heads to a workgroup).  One after the other they are
+// two latencies and a launch, with much of the chip idle: 4 x 256 tokens, 16 heads of 64, dQ 12.3 us and dK / dV 8.3.  The workgroups of this pass compute the
+// statistics that the dQ pass would have left them (the results are the same to the bit), which takes them 1 to 2 us where they see 8 to 16
+// query tiles.  Where it is used, and what it takes: eisen_attention_bwd_short_supports.
+constexpr int kOwnTiles = 64;  // places for the statistics of a tile, behind the rings
+template <int HD>
+struct DqLds {
+    __attribute__((aligned(1024))) bf16_t k[kDqTiles<HD>];
+    __attribute__((aligned(1024))) bf16_t v[kDqTiles<HD>];
+    __attribute__((aligned(1024))) bf16_t rows[kDqRows<HD, kAblNone>];
+};
+template <int HD, int ABL, int GW = 0>
 __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(AttnArgs a) {
+    constexpr bool OWN = GW > 0;
     constexpr int KSTEPS = HD / 16, DT = (HD + 31) / 32, NST = 2;
-    constexpr int TILE = 32 * kTileRow<HD>;              // elements of a Q or dO tile
-    constexpr int STAGE_BYTES = 2 * TILE * 2 + 256;      // Q tile, dO tile, 32 x (-LSE / scale | D)
+    constexpr int TILE = 32 * kTileRow<HD>;                          // elements of a Q or dO tile
+    constexpr int STAGE_BYTES = 2 * TILE * 2 + (OWN ? 0 : 256);      // Q tile, dO tile, 32 x (-LSE / scale | D)
+    // dK and dV in AGPRs (not beside the dQ role, where the compiler reads the accumulators before the wait states; in short loops its moves matter less)
+    constexpr bool AGPR = HD > 64 && !OWN;
     using Loader = DirectTile<HD, 32, 1>;
     constexpr int LOADS = 2 * Loader::PER_WAVE + 1;      // load instructions per tile
     static_assert(LOADS <= 63, "the tile in flight must fit the vmcnt counter");
     static_assert(2 * 4 * 32 * HD * sizeof(float) <= 4 * NST * STAGE_BYTES, "the reduction of dK and dV reuses the rings");
-    __shared__ __attribute__((aligned(1024))) char lds[4 * NST * STAGE_BYTES];
+    constexpr int RINGS = 4 * NST * STAGE_BYTES, BYTES = !OWN ? RINGS : RINGS + kOwnTiles * 256 > (int)sizeof(DqLds<HD>) ? RINGS + kOwnTiles * 256 : (int)sizeof(DqLds<HD>);
+    static_assert(!OWN || BYTES <= (HD <= 64 ? 80 : 160) * 1024, "two workgroups per CU, one for the head sizes above 64");
+    __shared__ __attribute__((aligned(1024))) char lds[BYTES];
+    int block = blockIdx.x, blocks = gridDim.x;
+    if constexpr (OWN) {
+        if (block < a.dq_blocks) {
+            DqLds<HD>& dq = *reinterpret_cast<DqLds<HD>*>(lds);
+            bwd_dq<HD, GW, kAblNone, false>(a, dq.k, dq.v, dq.rows, block, a.dq_blocks);
+            return;
+        }
+        block -= a.dq_blocks;
+        blocks -= a.dq_blocks;
+    }
 
     const int lane = threadIdx.x & 63, g = lane >> 5, c = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -68,8 +94,8 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
     // grid: x = key-block pair, fastest; then KV head, then batch.  Blocks of one (batch, KV head) read the same
     // Q / dO tiles, so they are kept on one XCD.
     // Without pairs: the key block slowest, longest (causal) first.
-    const bool paired = HD <= 64 || a.paired;
-    const int bid = paired ? xcd_contiguous_id(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+    const bool paired = HD <= 64 || OWN || a.paired;
+    const int bid = paired ? xcd_contiguous_id(block, blocks) : block;
     const int pair = paired ? bid % n_pairs : bid / (a.Hkv * a.B), of = paired ? bid / n_pairs : bid % (a.Hkv * a.B);
     const int kvh = of % a.Hkv, b = of / a.Hkv;
     char* ring = lds + wave * (NST * STAGE_BYTES);
@@ -77,6 +103,8 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
     // lanes 0-31 fetch the tile's -LSE / scale, lanes 32-63 its D: byte offset of the lane's value from D's entry for the
     // tile's first query (the launcher has checked that the statistics are less than 2 GiB apart)
     const unsigned stat_off = (unsigned)(g == 0 ? (a.L2 - a.D) * 4 : 0) + 4 * (unsigned)c;
+    float* const own = reinterpret_cast<float*>(lds + (OWN ? RINGS : 0));  // OWN: [query head of the group][query tile from own_first]
+    const int own_first = a.causal ? pair : 0, own_per_head = n_qt - own_first;
     Loader loader;
     loader.init(a.q_ss, 0, lane);
     constexpr bool TL = ABL == kAblTimeline;
@@ -94,6 +122,44 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
             vraw[st] = key_ < a.S ? *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(a.V) + koff + d) : zero8;
         }
     };
+
+    if constexpr (OWN) {
+        // The statistics of every tile that these keys see (of the second pass's as well: a part of them), as the dQ pass computes them, the loads
+        // of U tiles at a time in flight.
+        constexpr int U = HD <= 32 ? 8 : HD <= 64 ? 4 : 2;
+        const int tiles = a.G * own_per_head;
+        for (int t0 = wave; t0 < tiles; t0 += 4 * U) {
+            bf16x8 x[U][KSTEPS], y[U][KSTEPS];
+            float lse[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int t = t0 + 4 * u;
+                if (t >= tiles) break;
+                const int head = t / own_per_head, row = min((own_first + t - head * own_per_head) * 32 + c, a.S - 1);
+                const long long at = b * a.q_sb + (kvh * a.G + head) * a.q_sh + (long long)row * a.q_ss + 8 * g;
+#pragma unroll
+                for (int st = 0; st < KSTEPS; st++) {
+                    x[u][st] = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(a.dO) + at + st * 16);
+                    y[u][st] = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(a.O) + at + st * 16);
+                }
+                lse[u] = a.LSE[((long long)b * a.Hq + kvh * a.G + head) * a.S + row];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int t = t0 + 4 * u;
+                if (t >= tiles) break;
+                float part = 0.f;
+#pragma unroll
+                for (int st = 0; st < KSTEPS; st++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) part += (float)x[u][st][e] * (float)y[u][st][e];
+                const float sum = part + __shfl_xor(part, 32, 64);
+                const bool past = (own_first + t % own_per_head) * 32 + c >= a.S;  // a query past the end: probabilities exactly zero
+                own[t * 64 + lane] = g ? sum : past ? -INFINITY : -lse[u] / a.scale;
+            }
+        }
+        __syncthreads();
+    }
 
     for (int pass = 0; pass < 2; pass++) {
         const int kb = pass == 0 ? pair : n_qt - 1 - pair;
@@ -123,6 +189,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
             ntile = b * a.q_sb + hq * a.q_sh + (long long)nq0 * a.q_ss;
             nstat = ((long long)b * a.Hq + hq) * a.S + nq0;
         }
+        int nown = wave / per_head * own_per_head + qt_start - own_first + nrel;  // OWN: its place
         const long long tile_wrap = a.q_sh - (long long)per_head * 32 * a.q_ss, stat_wrap = (long long)a.S - per_head * 32;
         auto issue = [&](int i) -> int {  // the loads of this wave's i-th tile into ring stage i % NST; returns the tile's first query
             const int q0 = nq0;
@@ -130,15 +197,15 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
             const char* qbase = reinterpret_cast<const char*>(static_cast<const bf16_t*>(a.Q) + ntile);
             const char* dobase = reinterpret_cast<const char*>(static_cast<const bf16_t*>(a.dO) + ntile);
             const char* sbase = reinterpret_cast<const char*>(a.D + nstat);
-            nrel += 4; nq0 += 128; ntile += 128 * a.q_ss; nstat += 128;
-            while (nrel >= per_head) { nrel -= per_head; nq0 -= per_head * 32; ntile += tile_wrap; nstat += stat_wrap; }
+            nrel += 4; nq0 += 128; ntile += 128 * a.q_ss; nstat += 128; nown += 4;
+            while (nrel >= per_head) { nrel -= per_head; nq0 -= per_head * 32; ntile += tile_wrap; nstat += stat_wrap; nown += own_per_head - per_head; }
             if (q0 + 32 <= a.S) {
 #pragma unroll
                 for (int r = 0; r < Loader::PER_WAVE; r++) {
                     load_lds_16(qbase, loader.off[r], stage + r * 1024);
                     load_lds_16(dobase, loader.off[r], stage + TILE * 2 + r * 1024);
                 }
-                load_lds_4(sbase, stat_off, stage + 2 * TILE * 2);
+                if (!OWN) load_lds_4(sbase, stat_off, stage + 2 * TILE * 2);
             } else {  // ragged last tile: rows past the end re-read the last row (they are given zero weight)
 #pragma unroll
                 for (int r = 0; r < Loader::PER_WAVE; r++) {
@@ -147,11 +214,12 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
                     load_lds_16(qbase, off, stage + r * 1024);
                     load_lds_16(dobase, off, stage + TILE * 2 + r * 1024);
                 }
-                load_lds_4(sbase, stat_off - 4 * (unsigned)(c - min(c, a.S - 1 - q0)), stage + 2 * TILE * 2);
+                if (!OWN) load_lds_4(sbase, stat_off - 4 * (unsigned)(c - min(c, a.S - 1 - q0)), stage + 2 * TILE * 2);
             }
             return q0;
         };
 
+        int own_next = nown;
         int q0_next = n_mine > 0 ? issue(0) : 0;
         bf16x8 kf[KSTEPS], vn[KSTEPS];  // K and -V of the 32 keys, MFMA B operands (requested before the first tile, used after it is)
 #pragma unroll
@@ -171,8 +239,8 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
             const int q0 = q0_next;
             const bf16_t* Qs = reinterpret_cast<const bf16_t*>(stage_of(i));
             const bf16_t* dOs = Qs + TILE;
-            float* st = reinterpret_cast<float*>(stage_of(i) + 2 * TILE * 2);
-            if (q0 + 32 > a.S) {  // a query past the end gets LSE = +inf (stored negated): its probabilities are exactly zero
+            float* st = OWN ? own + own_next * 64 : reinterpret_cast<float*>(stage_of(i) + 2 * TILE * 2);
+            if (!OWN && q0 + 32 > a.S) {  // a query past the end gets LSE = +inf (stored negated): its probabilities are exactly zero
                 if (g == 0 && q0 + c >= a.S) st[c] = -INFINITY;
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
@@ -211,6 +279,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
                 }
             // the next tile's loads go out while the score MFMAs run (the other stage was read by tile i - 1, whose operand reads
             // have all returned)
+            own_next = nown;
             if (ABL != kAblTileLoads && i + 1 < n_mine) q0_next = issue(i + 1);
             float p[16];
 #pragma unroll
@@ -234,7 +303,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
                 for (int t = 0; t < 2; t++) {
                     if (ABL == kAblSecondMfmas) { dv[dt][0] += (float)pf[t][0] * (float)dotr[dt][t][0]; dk[dt][0] += (float)dsf[t][0] * (float)qtr[dt][t][0]; }
                     else {
-                    if (HD > 64) {
+                    if (AGPR) {
                         mfma_agpr(dv[dt], pf[t], dotr[dt][t]);
                         mfma_agpr(dk[dt], dsf[t], qtr[dt][t]);
                     } else {
@@ -244,7 +313,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
                     }
                 }
         }
-        if (HD > 64) {
+        if (AGPR) {
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) { agpr_settle(dv[dt]); agpr_settle(dk[dt]); }
         }
@@ -298,6 +367,41 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
 // stride) and between the two statistics arrays fit 32 bits.
 bool eisen_attention_dkv32_supports(const AttnArgs& a) {
     return a.hd <= 128 && a.hd % 16 == 0 && a.q_ss > 0 && a.q_ss * 32 * 2 < (1ll << 31) && a.L2 > a.D && (a.L2 - a.D) * 4 < (1ll << 31);
+}
+
+// Where one launch (fa_bwd_dkv32_kernel with GW > 0) takes less time than two: where every workgroup is on the chip at once, two to a CU (head sizes above 64: one), and a
+// workgroup of the dK / dV role has few enough statistics to compute before it starts.  With larger query groups there are fewer of these
+// workgroups, each with more tiles, and the statistics come on top of what was the longer pass already.  Two launches / one, us, causal, batch x sequence,
+// query heads on KV heads, head size: 4 x 256 16 on 16 64 16.1 / 12.9; 7 x 193 6 on 6 48 14.7 / 8.7; 1 x 2048 8 on 8 64 49.6 / 39.7; 4 x 512 8 on 4 128 45.1 /
+// 38.3; 4 x 256 8 on 8 128 30.6 / 19.4.  Beyond the lines: 8 x 256 16 on 16 64 (768 workgroups) 20.2 / 20.6, 16 x 256 33.0 / 37.9; 4 x 256 24 on 8 64 19.3 / 19.8;
+// 1 x 512 32 on 8 64 28.6 / 33.4; 1 x 512 16 on 4 128 53.5 / 61.2; 2 x 256 32 on 4 64 26.2 / 34.2.  At them: 8 x 128 8 on 2 64 15.3 / 13.9; 21 x 256 8 on 2 32 17.6 / 16.2;
+// 8 x 256 8 on 2 48 19.0 / 18.1; 4 x 64 16 on 2 64 15.2 / 14.6; 1 x 1024 16 on 8 64 35.3 / 34.1.
+bool eisen_attention_bwd_short_supports(const AttnArgs& a, int dq_blocks) {
+    const int n_qt = (a.S + 31) / 32;
+    const int most = a.G <= 2 ? kOwnTiles : a.G <= 4 && a.hd != 64 ? 32 : 16;
+    const long long blocks = dq_blocks + (long long)(n_qt + 1) / 2 * a.Hkv * a.B;
+    return a.G * n_qt <= most && blocks <= (a.hd <= 64 ? 512 : 256) && a.ablation == kAblNone && eisen_attention_dkv32_supports(a);
+}
+
+void eisen_attention_launch_bwd_short(eisen_ctx* ctx, AttnArgs a, int gw, int dq_blocks) {
+    a.dq_blocks = dq_blocks;
+    const int blocks = dq_blocks + ((a.S + 31) / 32 + 1) / 2 * a.Hkv * a.B;
+    auto launch = [&](auto hd) {
+        constexpr int HD = decltype(hd)::value;
+        if (gw == 4) fa_bwd_dkv32_kernel<HD, kAblNone, 4><<<blocks, 256, 0, ctx->stream>>>(a);
+        else if (gw == 2) fa_bwd_dkv32_kernel<HD, kAblNone, 2><<<blocks, 256, 0, ctx->stream>>>(a);
+        else fa_bwd_dkv32_kernel<HD, kAblNone, 1><<<blocks, 256, 0, ctx->stream>>>(a);
+    };
+    switch (a.hd) {
+        case 16: return launch(std::integral_constant<int, 16>{});
+        case 32: return launch(std::integral_constant<int, 32>{});
+        case 48: return launch(std::integral_constant<int, 48>{});
+        case 64: return launch(std::integral_constant<int, 64>{});
+        case 80: return launch(std::integral_constant<int, 80>{});
+        case 96: return launch(std::integral_constant<int, 96>{});
+        case 112: return launch(std::integral_constant<int, 112>{});
+        default: return launch(std::integral_constant<int, 128>{});
+    }
 }
 
 // a.L2 (-LSE / scale) and a.D must have been written (by the dQ kernel).

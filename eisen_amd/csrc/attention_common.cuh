@@ -17,6 +17,7 @@ struct AttnArgs {
     float scale, scale_log2e;
     int causal;
     int paired;  // a block runs a long query (dK / dV kernel: key) block and its short mirror image
+    int dq_blocks;  // both passes of the backward in one launch: the workgroups of the dQ pass
     // backward only: when set ([S][hd/2] cos/sin), Q and K are rotary-embedded projections and dQ, dK are the
     // gradients of the projections before the rotation (the inverse rotation is applied as the gradients are stored)
     const float2* rope;
@@ -49,6 +50,10 @@ enum AttnStamp { kStampStart = 0, kStampLoop = 1, kStampLoopEnd = 2, kStampStore
 // the key-stationary dK / dV kernel (attention_bwd.hip); a.D and a.L2 must have been written
 bool eisen_attention_dkv32_supports(const AttnArgs& a);
 void eisen_attention_launch_dkv32(eisen_ctx* ctx, AttnArgs a);
+
+// both passes of the backward in one launch (attention_bwd.hip)
+bool eisen_attention_bwd_short_supports(const AttnArgs& a, int dq_blocks);
+void eisen_attention_launch_bwd_short(eisen_ctx* ctx, AttnArgs a, int gw, int dq_blocks);
 
 // attention_f32.hip: f32 operands, head_dim up to 128
 bool eisen_attention_f32_mfma_supports(const AttnArgs& a);
