@@ -432,8 +432,8 @@ int eisen_staging(eisen_ctx* ctx, size_t bytes, eisen_ctx::StageSlot** out) {
     EISEN_REQUIRE(ctx, tries < eisen_ctx::kStageSlots, EISEN_E_STATE, "every staging slot holds an uncollected eisen_hip_dtoh_begin result");
     eisen_ctx::StageSlot& s = ctx->stage[ctx->stage_next];
     ctx->stage_next = (ctx->stage_next + 1) % eisen_ctx::kStageSlots;
-    if (!s.done) {
-        EISEN_HIP_TRY(ctx, hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+    if (!s.done) EISEN_HIP_TRY(ctx, hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+    if (!s.word) {
         const int rc = eisen_words(ctx);
         if (rc) return rc;
         s.word = ctx->words + 16 * (&s - ctx->stage);
