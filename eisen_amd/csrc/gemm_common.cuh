@@ -101,7 +101,7 @@ struct DwArgs {
     int tile_end[kMaxDw];  // tiles of products 0..p
     DwProduct p[kMaxDw];
 };
-void eisen_gemm_launch_dw(eisen_ctx* ctx, const DwArgs& g, int tile);
+void eisen_gemm_launch_dw(eisen_ctx* ctx, const DwArgs& g, int rows);  // tiles of rows x 64
 void eisen_gemm_launch_f32_dw(eisen_ctx* ctx, const DwArgs& g, int tile);  // gemm_f32_sliced.hip
 
 // gemm_edge.hip: bf16 operands, any shape, tiles of 256 or 128 rows and 128 columns (see there for what the operands must allow)

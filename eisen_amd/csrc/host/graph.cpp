@@ -415,14 +415,14 @@ void Graph::flush_weight_gradients(size_t only_weight) {
 
 // ---- weight gradients of a pass as one launch (see graph.hpp) -----------------------------------------------------
 
-// Products the one launch takes and serves better than a launch each: at least 32 x 32 (bf16), fewer 128 x 128 tiles than the chip has CUs, or than twice
-// that where the 256 x 256 tiles of the large products do not fit; contractions that need no parts.  Layers of one pass, a launch each / one launch, us: 12 of
-// 1024 x 1024 over 4096 tokens 317 / 116, 6 of 1024 x 3096 x 1024 113 / 83, 6 of 1024 x 4096 (256 tiles) x 4096 275 / 257, 4 of 1280 x 5000 (400) x 4096 298 / 267;
-// 2 of 8192 x 1024 (512) x 1024 54 / 67.
+// Products the one launch takes and serves better than a launch each: at least 32 x 32 (bf16), fewer 128 x 128 tiles than the chip has CUs; contractions that need no
+// parts.  Layers of one pass, a launch each / one launch, us: 12 of 1024 x 1024 over 4096 tokens 307 / 164, 6 of 1024 x 3096 (200 tiles) x 1024 115 / 97, x 4096 306 / 283,
+// 4 of 1536 x 1024 x 8192 175 / 145.  Beyond: 3 of 1024 x 4096 (256 tiles) x 4096 137 / 159, 4 of 1000 x 4000 (256) x 4000 211 / 225, 4 of 1280 x 5000 (400) x 4096
+// 307 / 367, x 1024 106 / 121.
 bool Graph::left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out) {
     if (backward_root_ == (size_t)-1 || rows == 0 || rows > 16384) return false;
     if (dtype == EISEN_BF16 ? in % 8 || out % 8 || in < 32 || out < 32 : in % 4 || out % 4) return false;
-    if (((in + 127) / 128) * ((out + 127) / 128) >= (in % 256 || out % 256 ? 512u : 256u)) return false;
+    if (((in + 127) / 128) * ((out + 127) / 128) >= 256u) return false;
     if ((uintptr_t)x % 16 || (uintptr_t)dy % 16) return false;
     const Tensor& tw = at(weight);
     return tw.is_param && tw.grad.dtype == EISEN_F32 && tw.size() == in * out;

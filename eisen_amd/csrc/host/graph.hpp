@@ -230,7 +230,7 @@ class Graph {
     // The products of a narrow model's layers are each too small for the chip, and nothing in the pass reads them: they are left until
     // the pass ends, or until something else writes, reads or clears the gradient of one of the weights, and then run together
     // (eisen_hip_gemm_weight_gradients).  Operands are kept as for the window.  The bits of a product do not depend on when its turn comes or on what
-    // runs with it.  The step of the ~14 M model: see leave_dw.
+    // runs with it.  Which products: left_fits.
     void flush_left_dw();
 
    private:
