@@ -440,6 +440,7 @@ bool Graph::leave_dw(size_t weight, const void* x, const void* dy, int dtype, si
 void Graph::settle_dw(size_t weight) {
     for (const LeftDW& e : left_dw_)
         if (e.weight == weight) {
+            if (in_beside_) throw Error("a weight's products were not settled before its side work began");
             flush_left_dw();
             return;
         }
@@ -500,6 +501,9 @@ void Graph::run_beside(bool beside, const std::vector<const void*>& reads, const
         check(launch(), what);
         return;
     }
+    // What the pass has left of these weights runs now, on the main stream: left_dw_ holds other weights' products too, and inside the section all of them would
+    // run on the side stream, where nothing later waits for the others.
+    for (size_t w : weights) settle_dw(w);
     int forked = 0;
     check(eisen_hip_side_begin_if_behind(ctx_, &forked), "side stream");
     if (!forked) {  // the main stream's like any other work: outside the section, where a write to what the side stream still writes can wait for it

@@ -2,12 +2,13 @@
 // work runs at once, the side stream's as late as it may (when something waits for it).  What eisen_hip_side_begin_if_behind answers is
 // given on the command line, one digit per call: 1 forked, 0 caught up.
 //
-// Backward of two products with one weight, Y = (X W) W, in two passes that add up; exit status 0 if the gradients of W and X are
-// those of the same graph with the weight gradients on the main stream, bit for bit.
+// One argument: backward of two products with one weight, Y = (X W) W, in two passes that add up; exit status 0 if the gradients of W and X are
+// those of the same graph with the weight gradients on the main stream, bit for bit.  Two arguments: the graph that the first one names.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <string>
 #include <vector>
 
 #include "../eisen_amd/csrc/host/graph.hpp"
@@ -57,13 +58,23 @@ int eisen_hip_cast(eisen_ctx* ctx, const void* s, int from, void* d, int to, siz
 }
 int eisen_hip_gemm(eisen_ctx* ctx, const void* A, const void* B, void* C, int dtype_ab, int dtype_c, int ta, int tb, size_t M, size_t N, size_t K, int accumulate) {
     return give(ctx, [=] {
-        for (size_t m = 0; m < M; m++)
-            for (size_t n = 0; n < N; n++) {
-                float sum = accumulate ? get(C, m * N + n, dtype_c) : 0.f;
-                for (size_t k = 0; k < K; k++) sum += get(A, ta ? k * M + m : m * K + k, dtype_ab) * get(B, tb ? n * K + k : k * N + n, dtype_ab);
-                put(C, m * N + n, dtype_c, sum);
+        std::vector<float> b(K * N), sum(N);
+        for (size_t k = 0; k < K; k++)
+            for (size_t n = 0; n < N; n++) b[k * N + n] = get(B, tb ? n * K + k : k * N + n, dtype_ab);
+        for (size_t m = 0; m < M; m++) {
+            for (size_t n = 0; n < N; n++) sum[n] = accumulate ? get(C, m * N + n, dtype_c) : 0.f;
+            for (size_t k = 0; k < K; k++) {
+                const float a = get(A, ta ? k * M + m : m * K + k, dtype_ab);
+                for (size_t n = 0; n < N; n++) sum[n] += a * b[k * N + n];
             }
+            for (size_t n = 0; n < N; n++) put(C, m * N + n, dtype_c, sum[n]);
+        }
     });
+}
+int eisen_hip_gemm_weight_gradients(eisen_ctx* ctx, size_t n, const void* const* A, const void* const* B, void* const* C, const size_t* M, const size_t* N, const int* accumulate,
+                                    int dtype, size_t K) {
+    for (size_t p = 0; p < n; p++) eisen_hip_gemm(ctx, A[p], B[p], C[p], dtype, EISEN_F32, 1, 0, M[p], N[p], K, accumulate[p]);
+    return 0;
 }
 // sections of side work, as runtime.hip has them
 int eisen_hip_side_begin(eisen_ctx* ctx) {
@@ -114,18 +125,49 @@ static std::vector<float> gradients(const char* answers, bool beside) {
     return seen;
 }
 
+static std::vector<float> ramp(size_t n, size_t step, size_t of, float scale) {
+    std::vector<float> v(n);
+    for (size_t i = 0; i < n; i++) v[i] = ((float)(i * step % of) - (float)(of / 2)) * scale;
+    return v;
+}
+
+// Two weights, each used over few rows (left for the end of the pass) and W1 over many as well (beside the chain): P = S W2, Q = P W1, R = Q W2, Y = (X W1) R^T.
+static std::vector<float> rows_of_two_lengths(const char* answers, bool beside) {
+    constexpr size_t kFew = 8, kMany = 16392, kHidden = 32;
+    eisen_ctx ctx;
+    ctx.answers = answers;
+    std::vector<float> seen;
+    eisen::Graph g(&ctx, eisen::PrecisionMode::Bf16Mixed);
+    g.set_weight_gradients_beside(beside);
+    const size_t w1 = g.alloc({kHidden, kHidden}, ramp(kHidden * kHidden, 7, 11, 0.125f)), w2 = g.alloc({kHidden, kHidden}, ramp(kHidden * kHidden, 5, 17, 0.0625f));
+    g.mark_params();
+    for (size_t w : {w1, w2}) g.request_zero_grad(w);
+    const size_t s = g.alloc({kFew, kHidden}, ramp(kFew * kHidden, 5, 13, 0.25f)), x = g.alloc({kMany, kHidden}, ramp(kMany * kHidden, 3, 7, 0.5f));
+    const size_t p = g.matmul(s, w2), many = g.matmul(x, w1), q = g.matmul(p, w1), r = g.matmul(q, w2);
+    g.backward(g.matmul_trans_b(many, r));
+    for (size_t id : {w1, w2, s})
+        for (size_t i = 0; i < g.at(id).size(); i++) seen.push_back(get(g.at(id).grad.ptr, i, g.at(id).grad.dtype));
+    g.clear_activations();
+    if (beside && (ctx.forks + ctx.inlines == 0 || !ctx.late.empty())) throw eisen::Error("no section was meant to be left open, and one to be there");
+    return seen;
+}
+
 int main(int argc, char** argv) {
-    if (argc != 2) return 2;
+    if (argc < 2 || argc > 3) return 2;
+    const char* answers = argv[argc - 1];
+    const std::string graph = argc == 3 ? argv[1] : "weight_used_twice";
     try {
-        const std::vector<float> plain = gradients("", false), beside = gradients(argv[1], true);
+        const auto run = graph == "weight_used_twice" ? gradients : graph == "rows_of_two_lengths" ? rows_of_two_lengths : nullptr;
+        if (!run) return 2;
+        const std::vector<float> plain = run("", false), beside = run(answers, true);
         bool some = false;
         for (float v : plain) some |= v != 0.f;
         if (!some || plain.size() != beside.size() || std::memcmp(plain.data(), beside.data(), plain.size() * sizeof(float))) {
-            std::fprintf(stderr, "%s: gradients differ\n", argv[1]);
+            std::fprintf(stderr, "%s %s: gradients differ\n", graph.c_str(), answers);
             return 1;
         }
     } catch (const std::exception& e) {
-        std::fprintf(stderr, "%s: %s\n", argv[1], e.what());
+        std::fprintf(stderr, "%s %s: %s\n", graph.c_str(), answers, e.what());
         return 1;
     }
     return 0;

@@ -12,7 +12,7 @@ from tests.conftest import ROOT
 def stub(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("stub") / "stub_device")
     # the entry points that the stub leaves out belong to operators that it does not run
-    subprocess.check_call(["g++", "-O1", "-std=c++17", "-no-pie", "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "stub_device.cpp"),
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-no-pie", "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "stub_device.cpp"),
                            os.path.join(ROOT, "eisen_amd", "csrc", "host", "graph.cpp"), "-Wl,--unresolved-symbols=ignore-all", "-Wl,-z,lazy", "-o", exe])
     return exe
 
@@ -20,4 +20,11 @@ def stub(tmp_path_factory):
 @pytest.mark.parametrize("answers", ["".join(a) for a in itertools.product("10", repeat=4)])
 def test_weight_used_twice_has_the_same_gradient_whenever_the_device_catches_up(stub, answers):
     done = subprocess.run([stub, answers], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stderr
+
+
+@pytest.mark.parametrize("answers", ["".join(a) for a in itertools.product("10", repeat=2)])
+def test_products_left_for_the_pass_stay_off_the_side_stream(stub, answers):
+    # a weight whose second product runs beside the chain must not take the other weights' products there with it
+    done = subprocess.run([stub, "rows_of_two_lengths", answers], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stderr
