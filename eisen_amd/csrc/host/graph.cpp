@@ -523,10 +523,13 @@ void Graph::run_beside(bool beside, const std::vector<const void*>& reads, const
     in_beside_ = false;
     const int rc_end = eisen_hip_side_end(ctx_);  // back on the main stream whatever the launch returned
     for (const void* p : reads) retained_.emplace(p, false);
-    for (size_t w : weights)
-        if (std::find(side_written_.begin(), side_written_.end(), w) == side_written_.end()) side_written_.push_back(w);
+    for (size_t w : weights) side_writes(w);
     check(rc, what);
     check(rc_end, "side stream");
+}
+
+void Graph::side_writes(size_t weight) {
+    if (std::find(side_written_.begin(), side_written_.end(), weight) == side_written_.end()) side_written_.push_back(weight);
 }
 
 const Storage& Graph::grad_for_read(size_t id) {
@@ -819,6 +822,7 @@ size_t Graph::swiglu_matmul_residual(size_t gate, size_t up, size_t b, size_t r,
             const int rc = eisen_hip_gemm(g.ctx(), g.at(h).data.ptr, go.ptr, gb.ptr, go.dtype, gb.dtype, 1, 0, K, N, M, acc);
             const int rc_end = eisen_hip_side_end(g.ctx());  // back on the main stream whatever the GEMM returned
             g.side_guards.push_back(go.ptr);
+            g.side_writes(b);  // ... and whoever touches b's gradient next on the main stream waits as well
             g.check(rc, "swiglu_matmul_residual backward dB");
             g.check(rc_end, "side stream");
         }

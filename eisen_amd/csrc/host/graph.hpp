@@ -252,6 +252,7 @@ class Graph {
     size_t window_ = 0, window_passes_ = 0;
     bool beside_ = true, in_beside_ = false;
     std::vector<size_t> side_written_;  // parameters whose gradients the side stream is writing: the main stream waits before it touches them
+    void side_writes(size_t weight);
     // Runs `launch` (weight-gradient GEMMs reading `reads`, writing the gradients of `weights`) on the side stream when
     // the products are small and no window is set, on the current stream otherwise.
     bool beside_fits(size_t in, size_t out) const;

@@ -16,7 +16,7 @@
 struct eisen_ctx {
     const char* answers = "";
     bool side = false, section = false;
-    int forks = 0, inlines = 0;
+    int forks = 0, inlines = 0, sides = 0;
     std::vector<std::function<void()>> late;  // the side stream
 };
 
@@ -76,10 +76,30 @@ int eisen_hip_gemm_weight_gradients(eisen_ctx* ctx, size_t n, const void* const*
     for (size_t p = 0; p < n; p++) eisen_hip_gemm(ctx, A[p], B[p], C[p], dtype, EISEN_F32, 1, 0, M[p], N[p], K, accumulate[p]);
     return 0;
 }
+int eisen_hip_gemm_residual(eisen_ctx* ctx, const void* A, const void* B, const void* R, void* C, int dtype_ab, int dtype_c, int ta, int tb, size_t M, size_t N, size_t K) {
+    eisen_hip_dtod(ctx, C, R, M * N * (dtype_c == EISEN_BF16 ? 2 : 4));
+    return eisen_hip_gemm(ctx, A, B, C, dtype_ab, dtype_c, ta, tb, M, N, K, 1);
+}
+// (h = gate * up: which function of them it is does not matter here)
+int eisen_hip_swiglu(eisen_ctx* ctx, const void* gate, const void* up, void* h, int dtype, size_t n) {
+    return give(ctx, [=] { for (size_t i = 0; i < n; i++) put(h, i, dtype, get(gate, i, dtype) * get(up, i, dtype)); });
+}
+int eisen_hip_gemm_swiglu_backward(eisen_ctx* ctx, const void* A, const void* B, const void* gate, const void* up, void* dgate, void* dup, int dtype, int ta, int tb, size_t M,
+                                   size_t N, size_t K) {
+    eisen_hip_gemm(ctx, A, B, dup, dtype, dtype, ta, tb, M, N, K, 0);
+    return give(ctx, [=] {
+        for (size_t i = 0; i < M * N; i++) {
+            const float dh = get(dup, i, dtype);
+            put(dgate, i, dtype, dh * get(up, i, dtype));
+            put(dup, i, dtype, dh * get(gate, i, dtype));
+        }
+    });
+}
 // sections of side work, as runtime.hip has them
 int eisen_hip_side_begin(eisen_ctx* ctx) {
     if (ctx->section) return -1;
     ctx->section = ctx->side = true;
+    ctx->sides++;
     return 0;
 }
 int eisen_hip_side_begin_if_behind(eisen_ctx* ctx, int* forked) {
@@ -152,12 +172,47 @@ static std::vector<float> rows_of_two_lengths(const char* answers, bool beside) 
     return seen;
 }
 
+// A weight large enough that the feed-forward tail forms its gradient on the side stream, used once more by the node behind it: R = X W, Y = R + (gate * up) W.
+static std::vector<float> tail_and_its_residual(const char* answers, bool beside) {
+    constexpr size_t kRows = 64, kIn = 256, kOut = 16384;
+    eisen_ctx ctx;
+    ctx.answers = answers;
+    std::vector<float> seen;
+    eisen::Graph g(&ctx, eisen::PrecisionMode::Bf16Mixed);
+    g.set_weight_gradients_beside(beside);
+    const size_t w = g.alloc({kIn, kOut}, ramp(kIn * kOut, 7, 11, 0.125f));
+    g.mark_params();
+    g.request_zero_grad(w);
+    std::vector<size_t> in;
+    for (size_t i = 0; i < 3; i++) {
+        in.push_back(g.alloc_pooled({kRows, kIn}));
+        g.load_tensor_data(in.back(), ramp(kRows * kIn, 3 + 2 * i, 13, 0.25f).data(), kRows * kIn);
+    }
+    const size_t r = g.matmul(in[0], w), y = g.swiglu_matmul_residual(in[1], in[2], w, r);
+    g.backward(y);
+    if (ctx.sides == 0) throw eisen::Error("no work went to the side stream");
+    // what both products add up to, whichever stream they ran on
+    std::vector<float> got(kIn * kOut);
+    for (size_t i = 0; i < got.size(); i++) got[i] = get(g.at(w).grad.ptr, i, EISEN_F32);
+    for (size_t k = 0; k < kIn; k++) {
+        float want = 0.f;
+        for (size_t m = 0; m < kRows; m++)
+            want += get(g.at(in[0]).data.ptr, m * kIn + k, EISEN_BF16) +
+                    widen(narrow(get(g.at(in[1]).data.ptr, m * kIn + k, EISEN_BF16) * get(g.at(in[2]).data.ptr, m * kIn + k, EISEN_BF16)));
+        for (size_t n = 0; n < kOut; n++)  // (dY is one everywhere, and every term a multiple of 1/16)
+            if (got[k * kOut + n] != want) throw eisen::Error("the gradient is not the sum of both products");
+    }
+    seen = {1.f};
+    g.clear_activations();
+    return seen;
+}
+
 int main(int argc, char** argv) {
     if (argc < 2 || argc > 3) return 2;
     const char* answers = argv[argc - 1];
     const std::string graph = argc == 3 ? argv[1] : "weight_used_twice";
     try {
-        const auto run = graph == "weight_used_twice" ? gradients : graph == "rows_of_two_lengths" ? rows_of_two_lengths : nullptr;
+        const auto run = graph == "weight_used_twice" ? gradients : graph == "rows_of_two_lengths" ? rows_of_two_lengths : graph == "tail_and_its_residual" ? tail_and_its_residual : nullptr;
         if (!run) return 2;
         const std::vector<float> plain = run("", false), beside = run(answers, true);
         bool some = false;

@@ -28,3 +28,8 @@ def test_products_left_for_the_pass_stay_off_the_side_stream(stub, answers):
     # a weight whose second product runs beside the chain must not take the other weights' products there with it
     done = subprocess.run([stub, "rows_of_two_lengths", answers], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stderr
+
+
+def test_weight_of_the_feed_forward_tail_used_again_waits_for_the_side_stream(stub):
+    done = subprocess.run([stub, "tail_and_its_residual", ""], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stderr
