@@ -60,7 +60,7 @@ Graph::~Graph() {
     (void)eisen_hip_side_wait(ctx_);
     for (auto& t : tensors) release(t);
     for (auto& kv : retained_)
-        if (kv.second) eisen_hip_free(ctx_, const_cast<void*>(kv.first));
+        if (kv.second.released) eisen_hip_free(ctx_, const_cast<void*>(kv.first));
 }
 
 void Graph::check(int rc, const char* what) const {
@@ -84,8 +84,8 @@ void Graph::free_buffer(void* ptr) {
     if (!ptr) return;
     if (!retained_.empty()) {
         auto it = retained_.find(ptr);
-        if (it != retained_.end()) {  // a windowed weight-gradient GEMM still has to read it: flush_weight_gradients frees it
-            it->second = true;
+        if (it != retained_.end()) {  // a weight-gradient GEMM still has to read it: release_retained frees it
+            it->second.released = true;
             return;
         }
     }
@@ -256,7 +256,7 @@ Storage& Graph::grad_for_write(size_t id, int* accumulate, const void** add_from
         if (*accumulate && !add_from)
             check(eisen_hip_dtod(ctx_, t.grad.ptr, old.ptr, old.numel * (old.dtype == EISEN_BF16 ? 2 : 4)), "gradient copy");
         if (t.grad_borrowed) t.grad_borrowed = false;  // the fresh buffer is this tensor's own
-        else retained_[old.ptr] = true;                // the tensor owned the old one: the flush frees it
+        else retained_[old.ptr].released = true;       // the tensor owned the old one: the last hold frees it
     }
     return t.grad;
 }
@@ -321,8 +321,8 @@ bool Graph::window_take(size_t weight, const void* x, const void* dy, int dtype,
     }
     e->x.push_back(x);
     e->dy.push_back(dy);
-    retained_.emplace(x, false);
-    retained_.emplace(dy, false);
+    hold(x, kForWindow);
+    hold(dy, kForWindow);
     return true;
 }
 
@@ -409,7 +409,7 @@ void Graph::flush_weight_gradients(size_t only_weight) {
         if (rc) break;
     }
     // the operands go back to the pool (stream order keeps them intact until the launches above have read them)
-    if (all) release_retained();
+    if (all) release_retained(kForWindow);
     check(rc, "weight gradients of the window");
 }
 
@@ -432,8 +432,8 @@ bool Graph::leave_dw(size_t weight, const void* x, const void* dy, int dtype, si
     if (!left_fits(weight, x, dy, dtype, rows, in, out)) return false;
     settle_dw(weight);  // a weight used twice: its products one after the other
     left_dw_.push_back(LeftDW{weight, x, dy, rows, in, out, dtype});
-    retained_.emplace(x, false);
-    retained_.emplace(dy, false);
+    hold(x, kForPass);
+    hold(dy, kForPass);
     return true;
 }
 
@@ -449,7 +449,8 @@ void Graph::settle_dw(size_t weight) {
 void Graph::flush_left_dw() {
     std::vector<LeftDW> list;
     list.swap(left_dw_);
-    while (!list.empty()) {  // one launch per contraction length and element type: one for a pass
+    int rc = 0;
+    while (!list.empty() && !rc) {  // one launch per contraction length and element type: one for a pass
         const LeftDW first = list.front();
         std::vector<const void*> As, Bs;
         std::vector<void*> Cs;
@@ -470,24 +471,29 @@ void Graph::flush_left_dw() {
             accs.push_back(acc);
         }
         list.swap(rest);
-        check(eisen_hip_gemm_weight_gradients(ctx_, Cs.size(), As.data(), Bs.data(), Cs.data(), Ms.data(), Ns.data(), accs.data(), first.dtype, first.rows),
-              "weight gradients of the pass");
+        rc = eisen_hip_gemm_weight_gradients(ctx_, Cs.size(), As.data(), Bs.data(), Cs.data(), Ms.data(), Ns.data(), accs.data(), first.dtype, first.rows);
     }
+    release_retained(kForPass);  // (stream order keeps the operands intact until the launches above have read them)
+    check(rc, "weight gradients of the pass");
 }
 
 void Graph::side_join() {
     check(eisen_hip_side_wait(ctx_), "side stream join");
     side_guards.clear();
     side_written_.clear();
-    if (window_dw.empty()) release_retained();  // operands of side-stream GEMMs: what the main stream does next is ordered after them
+    release_retained(kForSide);  // what the main stream does next is ordered after the side stream's GEMMs
 }
 
-void Graph::release_retained() {
-    if (retained_.empty() || !left_dw_.empty()) return;  // (what is left for the pass's launch still has to be read)
-    std::unordered_map<const void*, bool> held;
-    held.swap(retained_);
-    for (auto& kv : held)
-        if (kv.second) (void)eisen_hip_free(ctx_, const_cast<void*>(kv.first));
+void Graph::release_retained(HeldBy who) {
+    for (auto it = retained_.begin(); it != retained_.end();) {
+        it->second.by &= ~(unsigned)who;
+        if (it->second.by) {
+            ++it;
+            continue;
+        }
+        if (it->second.released) (void)eisen_hip_free(ctx_, const_cast<void*>(it->first));
+        it = retained_.erase(it);
+    }
 }
 
 // a weight gradient of fewer 128 x 128 tiles than the chip has CUs, formed by its own backward pass (no window)
@@ -522,7 +528,7 @@ void Graph::run_beside(bool beside, const std::vector<const void*>& reads, const
     }
     in_beside_ = false;
     const int rc_end = eisen_hip_side_end(ctx_);  // back on the main stream whatever the launch returned
-    for (const void* p : reads) retained_.emplace(p, false);
+    for (const void* p : reads) hold(p, kForSide);
     for (size_t w : weights) side_writes(w);
     check(rc, what);
     check(rc_end, "side stream");

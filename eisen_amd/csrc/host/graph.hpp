@@ -229,7 +229,7 @@ class Graph {
     // ---- weight gradients of a pass as one launch ------------------------------------------------------------------
     // The products of a narrow model's layers are each too small for the chip, and nothing in the pass reads them: they are left until
     // the pass ends, or until something else writes, reads or clears the gradient of one of the weights, and then run together
-    // (eisen_hip_gemm_weight_gradients).  Operands are kept as for the window.  The bits of a product do not depend on when its turn comes or on what
+    // (eisen_hip_gemm_weight_gradients).  Operands are kept as for the window, until that launch.  The bits of a product do not depend on when its turn comes or on what
     // runs with it.  Which products: left_fits.
     void flush_left_dw();
 
@@ -257,13 +257,19 @@ class Graph {
     // the products are small and no window is set, on the current stream otherwise.
     bool beside_fits(size_t in, size_t out) const;
     void run_beside(bool beside, const std::vector<const void*>& reads, const std::vector<size_t>& weights, const std::function<int()>& launch, const char* what);
-    void release_retained();
-    // buffers a windowed weight-gradient GEMM will read -> whether their owner has released them (then the flush frees them)
-    std::unordered_map<const void*, bool> retained_;
+    // Buffers that weight-gradient GEMMs still have to read: for whom, and whether their owner has released them (then they are freed with the last hold).
+    enum HeldBy : unsigned { kForWindow = 1, kForPass = 2, kForSide = 4 };
+    struct Hold {
+        unsigned by = 0;
+        bool released = false;
+    };
+    std::unordered_map<const void*, Hold> retained_;
+    void hold(const void* p, HeldBy who) { retained_[p].by |= who; }
+    void release_retained(HeldBy who);
     // the product x^T dy joins the window when it can; false: the caller forms it now
     bool window_take(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out);
     bool window_fits(size_t weight, int dtype, size_t rows, size_t in, size_t out);
-    void free_buffer(void* ptr);  // eisen_hip_free unless the buffer is retained
+    void free_buffer(void* ptr);  // eisen_hip_free unless the buffer is held
     size_t push_tensor(const std::vector<size_t>& shape, int dtype, bool pooled);
     Storage device_alloc(size_t numel, int dtype, bool zero);
     void download(const Storage& s, float* out);

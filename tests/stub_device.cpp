@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -18,6 +19,12 @@ struct eisen_ctx {
     bool side = false, section = false;
     int forks = 0, inlines = 0, sides = 0;
     std::vector<std::function<void()>> late;  // the side stream
+    std::map<void*, size_t> live;            // bytes of every buffer
+    size_t bytes() const {
+        size_t n = 0;
+        for (const auto& b : live) n += b.second;
+        return n;
+    }
 };
 
 static float widen(uint16_t h) {
@@ -44,9 +51,16 @@ static int give(eisen_ctx* ctx, std::function<void()> work) {
 
 extern "C" {
 const char* eisen_hip_last_error(eisen_ctx*) { return "refused by the stub"; }
-int eisen_hip_malloc(eisen_ctx*, size_t bytes, void** out) { return (*out = std::malloc(bytes + 16)) ? 0 : -1; }
-int eisen_hip_malloc_zeroed(eisen_ctx*, size_t bytes, void** out) { return (*out = std::calloc(bytes + 16, 1)) ? 0 : -1; }
-int eisen_hip_free(eisen_ctx* ctx, void* p) { return give(ctx, [=] { std::free(p); }); }
+int eisen_hip_malloc_zeroed(eisen_ctx* ctx, size_t bytes, void** out) {
+    if (!(*out = std::calloc(bytes + 16, 1))) return -1;
+    ctx->live[*out] = bytes;
+    return 0;
+}
+int eisen_hip_malloc(eisen_ctx* ctx, size_t bytes, void** out) { return eisen_hip_malloc_zeroed(ctx, bytes, out); }
+int eisen_hip_free(eisen_ctx* ctx, void* p) {
+    if (ctx->live.erase(p) != 1) return -1;
+    return give(ctx, [=] { std::free(p); });
+}
 int eisen_hip_memset_zero(eisen_ctx* ctx, void* p, size_t bytes) { return give(ctx, [=] { std::memset(p, 0, bytes); }); }
 int eisen_hip_htod(eisen_ctx*, void* d, const void* s, size_t bytes) { return std::memcpy(d, s, bytes), 0; }
 int eisen_hip_dtod(eisen_ctx* ctx, void* d, const void* s, size_t bytes) { return give(ctx, [=] { std::memmove(d, s, bytes); }); }
@@ -94,6 +108,13 @@ int eisen_hip_gemm_swiglu_backward(eisen_ctx* ctx, const void* A, const void* B,
             put(dup, i, dtype, dh * get(gate, i, dtype));
         }
     });
+}
+int eisen_hip_gemm_weight_gradients_window(eisen_ctx* ctx, size_t n, size_t pieces, const void* const* A, const void* const* B, void* const* C, const size_t* M, const size_t* N, size_t K,
+                                           const int* accumulate) {
+    for (size_t p = 0; p < n; p++)
+        for (size_t s = 0; s < pieces; s++)
+            eisen_hip_gemm(ctx, A[p * pieces + s], B[p * pieces + s], C[p], EISEN_BF16, EISEN_F32, 1, 0, M[p], N[p], K, s > 0 || accumulate[p]);
+    return 0;
 }
 // sections of side work, as runtime.hip has them
 int eisen_hip_side_begin(eisen_ctx* ctx) {
@@ -207,12 +228,38 @@ static std::vector<float> tail_and_its_residual(const char* answers, bool beside
     return seen;
 }
 
+// A window of three passes over a layer that it holds and one too narrow for it, Y = (X W) V: what stays allocated behind a pass are the operands of W alone.
+static std::vector<float> window_with_a_narrow_layer(const char* answers, bool beside) {
+    constexpr size_t kRows = 128, kHidden = 1024, kNarrow = 32;
+    eisen_ctx ctx;
+    ctx.answers = answers;
+    eisen::Graph g(&ctx, eisen::PrecisionMode::Bf16Mixed);
+    g.set_weight_gradients_beside(beside);
+    const size_t w = g.alloc({kHidden, kHidden}, ramp(kHidden * kHidden, 7, 11, 0.125f)), v = g.alloc({kHidden, kNarrow}, ramp(kHidden * kNarrow, 5, 17, 0.0625f));
+    g.mark_params();
+    g.set_weight_gradient_window(3);
+    for (size_t id : {w, v}) g.request_zero_grad(id);
+    const size_t base = ctx.bytes();
+    for (size_t pass = 1; pass <= 3; pass++) {
+        const size_t x = g.alloc_pooled({kRows, kHidden});
+        g.load_tensor_data(x, ramp(kRows * kHidden, 2 + pass, 13, 0.25f).data(), kRows * kHidden);
+        g.backward(g.matmul(g.matmul(x, w), v));
+        g.clear_activations();
+        if (ctx.bytes() != base + (pass < 3 ? pass * 2 * kRows * kHidden * 2 : 0)) throw eisen::Error("pass " + std::to_string(pass) + ": not W's operands alone are kept");
+    }
+    std::vector<float> seen;
+    for (size_t id : {w, v})
+        for (size_t i = 0; i < g.at(id).size(); i++) seen.push_back(get(g.at(id).grad.ptr, i, EISEN_F32));
+    return seen;
+}
+
 int main(int argc, char** argv) {
     if (argc < 2 || argc > 3) return 2;
     const char* answers = argv[argc - 1];
     const std::string graph = argc == 3 ? argv[1] : "weight_used_twice";
     try {
-        const auto run = graph == "weight_used_twice" ? gradients : graph == "rows_of_two_lengths" ? rows_of_two_lengths : graph == "tail_and_its_residual" ? tail_and_its_residual : nullptr;
+        const auto run = graph == "weight_used_twice" ? gradients : graph == "rows_of_two_lengths" ? rows_of_two_lengths : graph == "tail_and_its_residual" ? tail_and_its_residual
+                         : graph == "window_with_a_narrow_layer" ? window_with_a_narrow_layer : nullptr;
         if (!run) return 2;
         const std::vector<float> plain = run("", false), beside = run(answers, true);
         bool some = false;

@@ -33,3 +33,9 @@ def test_products_left_for_the_pass_stay_off_the_side_stream(stub, answers):
 def test_weight_of_the_feed_forward_tail_used_again_waits_for_the_side_stream(stub):
     done = subprocess.run([stub, "tail_and_its_residual", ""], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stderr
+
+
+def test_a_window_keeps_the_operands_of_its_own_products_only(stub):
+    # those that the pass's launch has read go back with the pass
+    done = subprocess.run([stub, "window_with_a_narrow_layer", ""], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stderr
