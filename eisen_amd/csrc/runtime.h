@@ -160,6 +160,10 @@ int eisen_staging(eisen_ctx* ctx, size_t bytes, eisen_ctx::StageSlot** out);
     } while (0)
 
 static inline bool eisen_aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
+static inline bool eisen_ranges_meet(const void* p, size_t p_bytes, const void* q, size_t q_bytes) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+    return a < b + q_bytes && b < a + p_bytes;
+}
 static inline size_t eisen_dtype_size(int dtype) { return dtype == EISEN_BF16 ? 2 : 4; }
 static inline bool eisen_dtype_ok(int dtype) { return dtype == EISEN_F32 || dtype == EISEN_BF16; }
 static inline size_t eisen_ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }

@@ -373,7 +373,7 @@ int eisen_hip_gemm_ksegments(eisen_ctx* ctx, size_t n_segments, const void* cons
  * q_strides / kv_strides: optional {batch, seq, head} element strides (NULL = the contiguous
  * layouts above; {Hq*S*hd, hd, S*hd} addresses the reference's [B,H,S,hd] tensors).
  * Query head h attends KV head h / (Hq/Hkv); dk, dv are summed over the heads of each group.
- * dq, dk, dv are overwritten.  bf16: hd a multiple of 16 up to 128, sequence strides of 0 to 2^25 elements (K and V) and up
+ * dq, dk, dv are overwritten.  bf16: dq may lie where out is, dk and dv where k, v or out are, in the same layout; hd a multiple of 16 up to 128, sequence strides of 0 to 2^25 elements (K and V) and up
  * to 2^26 (Q in the backward pass; not negative for hd <= 64).  f32: hd <= 256; above 128 S <= 16384 forward and 8192 backward.
  * Causal, f32: what rows hold that a query does not see reaches nothing, Inf and NaN included.  bf16: K, V, Q and dO must be
  * finite in the 64 rows around a visible one (masked pairs of a tile are multiplied with weight zero). */
