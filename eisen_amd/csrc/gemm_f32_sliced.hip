@@ -316,27 +316,26 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g, 
     int left = 0;
     if (n_mine > 0) left = issue(0);
     clear();
-    // kLayers: four waves take whole contractions, where other launches give eight waves a part each.  The sums of two slices are added up apart, so that no
-    // accumulator rounds a longer one: error against float64, two slices / all of a wave's / eight waves and parts, 256 x 1024 x 448 1.0e-7 / 1.5e-7 / 1.05e-7,
-    // x 4096 1.3e-7 / 4.9e-7 / 1.7e-7, positive 5.0e-8 / 1.7e-7 / 5.0e-8, x 16384 1.8e-7 / 9.8e-7 / 3.4e-7, 96 x 256 x 1351 1.1e-7 / 2.7e-7 / 0.9e-7; us, the products of
-    // the ~14 M model's layers over 4096 tokens 535 / 498 / 832 in launches of their own.
-    constexpr int kRun = 2;
-    f32x16 total[KIND == Kind::kLayers ? TM : 1][KIND == Kind::kLayers ? TM : 1];
-    auto add_to_total = [&](bool first) __attribute__((always_inline)) {
+    // kLayers: four waves take whole contractions, where other launches give eight waves a part each.  The sums of two slices are added to a total, so that no accumulator
+    // rounds a longer one; where those launches leave a wave a slice or few (contractions of at most eight slices, products of fewer than 64 tiles of 64 x 64, which
+    // they split), every slice by itself, and what the addition to the total rounds away opens the next slice's sum.  Error against float64, each slice / two slices /
+    // a launch of its own: 64 x 64 x 256 6.0e-8 / 1.0e-7 / 6.6e-8, 96 x 256 x 1351 6.3e-8 / 1.1e-7 / 9.0e-8, 256 x 256 x 4096 6.3e-8 / 1.3e-7 / 1.7e-7, 64 x 64 x 16384
+    // 6.3e-8 / 1.8e-7 / 1.5e-7, 256 x 1024 x 4096 6.2e-8 / 1.3e-7 / 1.7e-7 (all of a wave's slices in one accumulator 4.9e-7).  us, the products of the ~14 M model's layers
+    // over 4096 tokens, each slice everywhere / this / two slices everywhere 492 / 455 / 438, in launches of their own 832.
+    f32x16 total[KIND == Kind::kLayers ? TM : 1][KIND == Kind::kLayers ? TM : 1] = {};
+    auto add_to_total = [&](auto carry_c) __attribute__((always_inline)) {
 #pragma unroll
         for (int p = 0; p < TM; p++)
 #pragma unroll
             for (int q = 0; q < TM; q++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) total[p][q][v] = first ? acc[p][q][v] : total[p][q][v] + acc[p][q][v];
+                for (int v = 0; v < 16; v++) {
+                    const float sum = total[p][q][v] + acc[p][q][v];
+                    acc[p][q][v] = decltype(carry_c)::value ? acc[p][q][v] - (sum - total[p][q][v]) : 0.f;
+                    total[p][q][v] = sum;
+                }
     };
-    if constexpr (KIND == Kind::kLayers) add_to_total(true);
-    for (int i = 0; i < n_mine; i++) {
-        if constexpr (KIND == Kind::kLayers)
-            if (i > 0 && i % kRun == 0) {
-                add_to_total(false);
-                clear();
-            }
+    auto slice = [&](int i) __attribute__((always_inline)) {
         wait_loads_but<0>();
         float a[2][TM][8], b[2][TM][8];
         read(0, a[0], b[0]);
@@ -397,13 +396,26 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g, 
             block(I0{}, I0{}, I0{}, Yes{});
             block(I1{}, I0{}, I0{}, No{});
         }
-    }
+    };
     if constexpr (KIND == Kind::kLayers) {
-        add_to_total(false);
+        if (g.K <= 8 * FK || ((g.M + 63) / 64) * ((g.N + 63) / 64) < 64) {
+            for (int i = 0; i < n_mine; i++) {
+                if (i > 0) add_to_total(std::true_type{});
+                slice(i);
+            }
+        } else {
+            for (int i = 0; i < n_mine; i++) {
+                if (i > 0 && i % 2 == 0) add_to_total(std::false_type{});
+                slice(i);
+            }
+        }
+        add_to_total(std::false_type{});
 #pragma unroll
         for (int p = 0; p < TM; p++)
 #pragma unroll
             for (int q = 0; q < TM; q++) acc[p][q] = total[p][q];
+    } else {
+        for (int i = 0; i < n_mine; i++) slice(i);
     }
     const int bad = meet(-1.f, kUnscale);
     if (__syncthreads_or(bad)) {  // something that is not finite: once more in f32
