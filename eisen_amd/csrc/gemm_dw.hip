@@ -6,16 +6,19 @@
 // for every fourth 16-deep slice, through a private ring of four with no barrier, and the four sums meet in LDS once, added in wave order.  A tile of 128 x 64 reads 6
 // operands per 8 MFMAs, one of 64 x 64 8; but the former leaves one workgroup on a CU, whose start and end nothing hides.  Both give the same bits: the slices of a wave do not
 // depend on the tile.
-// The sums of a few slices are added up apart, so that no accumulator rounds a long one, nor the total many short ones (`run`).  Error against float64, these / all of a wave's
-// slices in one accumulator / a launch of its own before: 256 x 1024 x 2048 8.1e-8 / 1.3e-7 / 8.6e-8, x 4096 9.2e-8 / 1.9e-7 / 9.2e-8, x 8192 1.1e-7 / 2.7e-7 / 1.1e-7, x 16384
-// 1.2e-7 / 4.0e-7 / 1.4e-7; 8192 x 256 x 8192 1.1e-7 / 2.7e-7 / 4.0e-7; 1024 x 1024 x 4096 9.2e-8 / 1.9e-7 / 2.7e-7; 288 x 768 x 1351 7.7e-8 / 1.1e-7 / 9.1e-8;
-// of positive operands 256 x 1024 x 8192 4.7e-8 / 1.3e-7 / 4.7e-8.  At most a tenth more than before where there are a few tiles only (64 x 64 x 16384 1.2e-7, before 1.1e-7).
+// The sums of a few slices are added up apart, so that no accumulator rounds a long one, nor the total many short ones (`run`).  Products of fewer than 64 tiles of 64 x 64 over
+// more than 2048 tokens, which a launch of their own splits, come in parts of 4096 tokens, each added to C before the next, and add the waves' sums two and two (`dw_exact`).
+// Error against float64, these / all of a wave's slices in one accumulator / a launch of its own: 256 x 1024 x 2048 8.1e-8 / 1.3e-7 / 8.6e-8, x 4096 9.2e-8 / 1.9e-7 / 9.2e-8, x
+// 8192 1.1e-7 / 2.7e-7 / 1.1e-7, x 16384 1.2e-7 / 4.0e-7 / 1.4e-7; 8192 x 256 x 8192 1.1e-7 / 2.7e-7 / 4.0e-7; 1024 x 1024 x 4096 9.2e-8 / 1.9e-7 / 2.7e-7; 288 x 768 x
+// 1351 7.7e-8 / 1.1e-7 / 9.1e-8; of positive operands 256 x 1024 x 8192 4.7e-8 / 1.3e-7 / 4.7e-8.  Few tiles, these / in one part / a launch of its own: 256 x 256 x 4096 9.1e-8 / 9.3e-8 /
+// 9.2e-8, x 8192 9.5e-8 / 1.10e-7 / 1.00e-7, x 16384 1.00e-7 / 1.22e-7 / 1.12e-7, 64 x 64 x 8192 9.5e-8 / 1.10e-7 / 9.9e-8.
 // Rates: 4 x 1536 x 1024 over 8192 tokens 710 TFLOP/s, 12 x 1024 x 1024 over 4096 630.  A pass's layers, a launch each / this, us:
-// hidden 256, ffn 1024, 6 layers and a head of 8192 over 8192 tokens 636 / 292; 288, 768, 4 layers over 1351 187 / 33; 512, 1536, 4 layers over 4096 460 / 226;
+// hidden 256, ffn 1024, 6 layers and a head of 8192 over 8192 tokens 636 / 268 (254 without the parts); 288, 768, 4 layers over 1351 187 / 33; 512, 1536, 4 layers over 4096 460 / 226;
 // 720, 2120, 6 layers over 896 456 / 241.
 // (Tried: wave tiles of 128 x 128, which leave no registers for sums apart, 209 us for the first of these sets and the error in the middle above; with them a persistent grid that
 // requests the next tile's slices before the meeting, 258 -> 285 us at 8192 x 8192 x 1024, and a meeting in which a wave receives only the quarter that it stores, 258 -> 289.
-// Compensated sums instead of plain ones: 180 registers in scratch, or 5 to 20 % longer with 64 x 64.)
+// Compensated sums instead of plain ones: 180 registers in scratch, or 5 to 20 % longer with 64 x 64; a carry from each run into the next for the few tiles' products alone, a loop of its
+// own, 276 instead of 268 for the first of these sets.)
 //
 // Operand rows start on 16-byte boundaries and sides are multiples of 8.  Columns past the end re-read the last chunk and reach only outputs that are not
 // stored; contraction indices past the end re-read the last one, and both operands are zeroed there.
@@ -23,30 +26,25 @@
 
 namespace {
 
-constexpr int kCols = 64, kSlice = 16, kRing = 4, kWaves = 4;
+constexpr int kCols = 64, kSlice = 16, kRing = 4, kWaves = 4, kPart = 4096;
+
+__host__ __device__ constexpr bool dw_exact(int M, int N, int K) { return K > 2048 && ((M + 63) / 64) * ((N + 63) / 64) < 64; }
 
 template <int ROWS>
-__global__ __launch_bounds__(64 * kWaves, ROWS == 64 ? 2 : 1) void gemm_dw_kernel(DwArgs g) {
+using DwStages = bf16_t[kWaves][kRing][DirectOperandTile<ROWS, false, kSlice, 1>::ELEMS + DirectOperandTile<kCols, false, kSlice, 1>::ELEMS];
+
+// A tile's sum over the K tokens from k0 on, by the whole workgroup; added to C where add_old.  pairs: the waves' sums are added two and two.
+template <int ROWS>
+__device__ __forceinline__ void dw_tile(const DwProduct& pr, DwStages<ROWS>& lds, int m0, int n0, int k0, int K, bool add_old, bool pairs) {
     using TA = DirectOperandTile<ROWS, false, kSlice, 1>;
     using TB = DirectOperandTile<kCols, false, kSlice, 1>;
     constexpr int TM = ROWS / 32, TN = kCols / 32, LOADS = TA::LOADS + TB::LOADS, STAGE = TA::ELEMS + TB::ELEMS;
-    __shared__ __attribute__((aligned(1024))) bf16_t lds[kWaves][kRing][STAGE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    // which product this tile belongs to: every lane looks at one
-    int t = xcd_contiguous_id(blockIdx.x, g.tiles);
-    const int p = __popcll(__ballot(lane < g.n && t >= g.tile_end[lane]));
-    const DwProduct& pr = g.p[p];
-    if (p > 0) t -= g.tile_end[p - 1];
-    const int M = pr.M, N = pr.N, K = g.K;
-    int mt, nt;
-    block_tile<4, 8>(t, (M + ROWS - 1) / ROWS, (N + kCols - 1) / kCols, mt, nt);
-    const int m0 = __builtin_amdgcn_readfirstlane(mt * ROWS), n0 = __builtin_amdgcn_readfirstlane(nt * kCols);
-
+    const int M = pr.M, N = pr.N;
     const int slices = (K + kSlice - 1) / kSlice, n_mine = slices > wave ? (slices - wave + kWaves - 1) / kWaves : 0, n_parts = min(kWaves, slices);
-    const char* A = static_cast<const char*>(pr.A) + ((long long)wave * kSlice * M + m0) * 2;
-    const char* B = static_cast<const char*>(pr.B) + ((long long)wave * kSlice * N + n0) * 2;
+    const char* A = static_cast<const char*>(pr.A) + ((long long)(k0 + wave * kSlice) * M + m0) * 2;
+    const char* B = static_cast<const char*>(pr.B) + ((long long)(k0 + wave * kSlice) * N + n0) * 2;
     const int a_last = (M - 1 - m0) / 8, b_last = (N - 1 - n0) / 8;
     unsigned a_off[TA::LOADS], b_off[TB::LOADS];  // a lane's bytes in a slice
 #pragma unroll
@@ -173,13 +171,25 @@ __global__ __launch_bounds__(64 * kWaves, ROWS == 64 ? 2 : 1) void gemm_dw_kerne
             float* dst = static_cast<float*>(pr.C) + (long long)m * N + n;
             float val[8] = {};
             const float* src = reinterpret_cast<const float*>(&lds[0][0][0]) + place(r, cg * 8);
+            float held[8] = {};
             for (int w = 0; w < n_parts; w++) {
+                if (pairs && w == 2) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        held[e] = val[e];
+                        val[e] = 0.f;
+                    }
+                }
                 const float4 lo = *reinterpret_cast<const float4*>(src + w * (kRing * STAGE / 2)), hi = *reinterpret_cast<const float4*>(src + w * (kRing * STAGE / 2) + 4);
                 val[0] += lo.x; val[1] += lo.y; val[2] += lo.z; val[3] += lo.w;
                 val[4] += hi.x; val[5] += hi.y; val[6] += hi.z; val[7] += hi.w;
             }
+            if (pairs) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) val[e] += held[e];
+            }
             float4 lo = make_float4(val[0], val[1], val[2], val[3]), hi = make_float4(val[4], val[5], val[6], val[7]);
-            if (pr.accumulate) {
+            if (add_old) {
                 const float4 o0 = reinterpret_cast<const float4*>(dst)[0], o1 = reinterpret_cast<const float4*>(dst)[1];
                 lo.x += o0.x; lo.y += o0.y; lo.z += o0.z; lo.w += o0.w;
                 hi.x += o1.x; hi.y += o1.y; hi.z += o1.z; hi.w += o1.w;
@@ -190,9 +200,43 @@ __global__ __launch_bounds__(64 * kWaves, ROWS == 64 ? 2 : 1) void gemm_dw_kerne
     }
 }
 
+template <int ROWS, bool EXACT>
+__global__ __launch_bounds__(64 * kWaves, ROWS == 64 ? 2 : 1) void gemm_dw_kernel(DwArgs g) {
+    __shared__ __attribute__((aligned(1024))) DwStages<ROWS> lds;
+    const int lane = threadIdx.x & 63;
+
+    // which product this tile belongs to: every lane looks at one
+    int t = xcd_contiguous_id(blockIdx.x, g.tiles);
+    const int p = __popcll(__ballot(lane < g.n && t >= g.tile_end[lane]));
+    const DwProduct& pr = g.p[p];
+    if (p > 0) t -= g.tile_end[p - 1];
+    const int M = pr.M, N = pr.N, K = g.K;
+    int mt, nt;
+    block_tile<4, 8>(t, (M + ROWS - 1) / ROWS, (N + kCols - 1) / kCols, mt, nt);
+    const int m0 = __builtin_amdgcn_readfirstlane(mt * ROWS), n0 = __builtin_amdgcn_readfirstlane(nt * kCols);
+
+    if constexpr (EXACT) {
+        const bool exact = dw_exact(M, N, K);
+        const int part = exact ? min(K, kPart) : K;
+        for (int k0 = 0; k0 < K; k0 += part) {
+            if (k0 > 0) __syncthreads();  // the last part's sums have been read
+            dw_tile<ROWS>(pr, lds, m0, n0, k0, min(part, K - k0), k0 > 0 || pr.accumulate, exact);
+        }
+    } else {
+        dw_tile<ROWS>(pr, lds, m0, n0, 0, K, pr.accumulate, false);
+    }
+}
+
 }  // namespace
 
 void eisen_gemm_launch_dw(eisen_ctx* ctx, const DwArgs& g, int rows) {
-    if (rows == 128) gemm_dw_kernel<128><<<(unsigned)g.tiles, 64 * kWaves, 0, ctx->stream>>>(g);
-    else gemm_dw_kernel<64><<<(unsigned)g.tiles, 64 * kWaves, 0, ctx->stream>>>(g);
+    bool exact = false;
+    for (int p = 0; p < g.n; p++) exact = exact || dw_exact(g.p[p].M, g.p[p].N, g.K);
+    auto launch = [&](auto rows_c) {
+        constexpr int ROWS = decltype(rows_c)::value;
+        if (exact) gemm_dw_kernel<ROWS, true><<<(unsigned)g.tiles, 64 * kWaves, 0, ctx->stream>>>(g);
+        else gemm_dw_kernel<ROWS, false><<<(unsigned)g.tiles, 64 * kWaves, 0, ctx->stream>>>(g);
+    };
+    if (rows == 128) launch(std::integral_constant<int, 128>{});
+    else launch(std::integral_constant<int, 64>{});
 }
