@@ -1,6 +1,8 @@
 // Graph / Tensor / Tape for Device::Gpu over the eisen_hip C-ABI.  See graph.hpp.
 #include "graph.hpp"
 
+#include "../gemm_dw_rule.h"
+
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -415,8 +417,8 @@ void Graph::flush_weight_gradients(size_t only_weight) {
 
 // ---- weight gradients of a pass as one launch (see graph.hpp) -----------------------------------------------------
 
-// Products the one launch takes and serves better than a launch each: at least 32 x 32 (bf16), fewer 128 x 128 tiles than the chip has CUs; contractions that need no
-// parts.  Layers of one pass, a launch each / one launch, us: 12 of 1024 x 1024 over 4096 tokens 307 / 164, 6 of 1024 x 3096 (200 tiles) x 1024 115 / 97, x 4096 306 / 283,
+// Products the one launch takes and, enough of them (gemm_dw_rule.h), serves better than a launch each: at least 32 x 32 (bf16), fewer 128 x 128 tiles than the chip has CUs;
+// contractions that need no parts.  Layers of one pass, a launch each / one launch, us: 12 of 1024 x 1024 over 4096 tokens 307 / 164, 6 of 1024 x 3096 (200 tiles) x 1024 115 / 97, x 4096 306 / 283,
 // 4 of 1536 x 1024 x 8192 175 / 145.  Beyond: 3 of 1024 x 4096 (256 tiles) x 4096 137 / 159, 4 of 1000 x 4000 (256) x 4000 211 / 225, 4 of 1280 x 5000 (400) x 4096
 // 307 / 367, x 1024 106 / 121.
 bool Graph::left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out) {
@@ -450,7 +452,7 @@ void Graph::flush_left_dw() {
     std::vector<LeftDW> list;
     list.swap(left_dw_);
     int rc = 0;
-    while (!list.empty() && !rc) {  // one launch per contraction length and element type: one for a pass
+    while (!list.empty() && !rc) {  // one launch per contraction length and element type, one for a pass, or a launch each
         const LeftDW first = list.front();
         std::vector<const void*> As, Bs;
         std::vector<void*> Cs;
@@ -471,7 +473,11 @@ void Graph::flush_left_dw() {
             accs.push_back(acc);
         }
         list.swap(rest);
-        rc = eisen_hip_gemm_weight_gradients(ctx_, Cs.size(), As.data(), Bs.data(), Cs.data(), Ms.data(), Ns.data(), accs.data(), first.dtype, first.rows);
+        if (eisen_dw_together(first.dtype == EISEN_BF16, Cs.size(), Ms.data(), Ns.data(), first.rows)) {
+            rc = eisen_hip_gemm_weight_gradients(ctx_, Cs.size(), As.data(), Bs.data(), Cs.data(), Ms.data(), Ns.data(), accs.data(), first.dtype, first.rows);
+        } else {
+            for (size_t p = 0; p < Cs.size() && !rc; p++) rc = eisen_hip_gemm(ctx_, As[p], Bs[p], Cs[p], first.dtype, EISEN_F32, 1, 0, Ms[p], Ns[p], first.rows, accs[p]);
+        }
     }
     release_retained(kForPass);  // (stream order keeps the operands intact until the launches above have read them)
     check(rc, "weight gradients of the pass");

@@ -229,8 +229,8 @@ class Graph {
     // ---- weight gradients of a pass as one launch ------------------------------------------------------------------
     // The products of a narrow model's layers are each too small for the chip, and nothing in the pass reads them: they are left until
     // the pass ends, or until something else writes, reads or clears the gradient of one of the weights, and then run together
-    // (eisen_hip_gemm_weight_gradients).  Operands are kept as for the window, until that launch.  The bits of a product do not depend on when its turn comes or on what
-    // runs with it.  Which products: left_fits.
+    // (eisen_hip_gemm_weight_gradients).  Operands are kept as for the window, until that launch.  Which products: left_fits;
+    // few of them over many tokens are formed by a launch each at that time (gemm_dw_rule.h).
     void flush_left_dw();
 
    private:

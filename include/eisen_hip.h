@@ -318,7 +318,7 @@ int eisen_hip_gemm_grouped_ksegments(eisen_ctx* ctx, size_t n_products, size_t n
                                      void* const* C, const size_t* M, const size_t* N, size_t seg_k, int accumulate);
 
 /* The same with an accumulate state per product.  What the one launch does not take and has fewer 128 x 128 tiles than the chip has CUs runs as one launch per
- * piece (eisen_hip_gemm_weight_gradients). */
+ * piece of up to 16384 rows (eisen_hip_gemm_weight_gradients) where that is faster than a launch each. */
 int eisen_hip_gemm_weight_gradients_window(eisen_ctx* ctx, size_t n_products, size_t n_segments, const void* const* A, const void* const* B,
                                            void* const* C, const size_t* M, const size_t* N, size_t seg_k, const int* accumulate);
 

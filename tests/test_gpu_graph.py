@@ -367,6 +367,35 @@ def test_weight_used_twice_per_pass_outgrows_its_window_entry_alone(ctx):
         assert_close(b, a, 1e-4, f"weight gradient of {name}")
 
 
+@pytest.mark.parametrize("precision,rows,layers,together", [(G.BF16_MIXED, 1024, 1, True), (G.BF16_MIXED, 8192, 1, False), (G.BF16_MIXED, 8192, 2, False), (G.BF16_MIXED, 8192, 3, True),
+                                                            (G.FP32, 512, 1, False), (G.FP32, 512, 3, True), (G.FP32, 4096, 2, False)])
+def test_weight_gradients_of_few_layers_over_many_tokens_are_launches_of_their_own(ctx, precision, rows, layers, together):
+    # layers of 256 x 256: one workgroup to a tile would walk all tokens.  Against float64 from the same activations; 2^-8 where they and their gradients are bf16.
+    hidden = 256
+    g = G.Graph(ctx, precision)
+    ws = [g.alloc((hidden, hidden), gen.normal(990 + i, (hidden, hidden), hidden ** -0.5)) for i in range(layers)]
+    g.mark_params()
+    x, t = gen.normal(995, (rows, hidden)), gen.uniform_ids(996, (rows,), hidden)
+    h = g.input(x)
+    for w in ws:
+        h = g.matmul(h, w)
+    loss = g.cross_entropy(h, t)
+    ctx.profile_start()
+    g.backward(loss)
+    names = list(ctx.profile_stop())
+    assert any(n.endswith("_layers") for n in names) == together, names
+    weights = [g.sync_to_cpu(w).astype(np.float64) for w in ws]
+    acts = [x.astype(np.float64)]
+    for w in weights:
+        acts.append(acts[-1] @ w)
+    p = np.exp(acts[-1] - acts[-1].max(1, keepdims=True))
+    dy = (p / p.sum(1, keepdims=True) - np.eye(hidden)[t]) / rows
+    for i in reversed(range(layers)):
+        assert_close(g.sync_grad_to_cpu(ws[i]), acts[i].T @ dy, 1e-4 if precision == G.FP32 else 2e-2, f"gradient {i}")
+        dy = dy @ weights[i].T
+    g.close()
+
+
 @pytest.mark.parametrize("tie,checkpointing", [(True, False), (False, False), (True, True)], ids=["tied", "untied", "tied-recompute"])
 def test_weight_gradients_beside_the_chain_give_the_same_bits(ctx, tie, checkpointing):
     # Graph::set_weight_gradients_beside (the default): the weight-gradient GEMMs of narrow layers run on the side stream
