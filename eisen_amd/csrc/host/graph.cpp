@@ -430,12 +430,16 @@ bool Graph::left_fits(size_t weight, const void* x, const void* dy, int dtype, s
     return tw.is_param && tw.grad.dtype == EISEN_F32 && tw.size() == in * out;
 }
 
-bool Graph::leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out) {
+bool Graph::leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out, bool more) {
     if (!left_fits(weight, x, dy, dtype, rows, in, out)) return false;
     settle_dw(weight);  // a weight used twice: its products one after the other
     left_dw_.push_back(LeftDW{weight, x, dy, rows, in, out, dtype});
-    hold(x, kForPass);
-    hold(dy, kForPass);
+    if (beside_) {
+        hold(x, kForPass);
+        hold(dy, kForPass);
+    } else if (!more) {  // products in the order of the tape: those of this node now
+        flush_left_dw();
+    }
     return true;
 }
 
@@ -931,8 +935,8 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
             for (size_t i = 0; i < n; i++)
                 if (g.has_grad(outs[i])) left = left && g.left_fits(ws[i], xa, g.grad_for_read(outs[i]).ptr, EISEN_F32, M, K, N[i]);
             if (left) {
-                for (size_t i = 0; i < n; i++)
-                    if (g.has_grad(outs[i])) g.leave_dw(ws[i], xa, g.grad_for_read(outs[i]).ptr, EISEN_F32, M, K, N[i]);
+                for (size_t i = 0, left_of = m; i < n; i++)
+                    if (g.has_grad(outs[i])) g.leave_dw(ws[i], xa, g.grad_for_read(outs[i]).ptr, EISEN_F32, M, K, N[i], --left_of > 0);
                 return;
             }
             int accs[3];
@@ -1028,7 +1032,7 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
                 for (size_t i = 0; i < n; i++) {
                     const void* dy = g.grad_for_read(outs[i]).ptr;
                     if (fits) g.window_take(ws[i], xa.ptr, dy, EISEN_BF16, M, K, N[i]);
-                    else g.leave_dw(ws[i], xa.ptr, dy, EISEN_BF16, M, K, N[i]);
+                    else g.leave_dw(ws[i], xa.ptr, dy, EISEN_BF16, M, K, N[i], i + 1 < n);
                 }
                 for (size_t e = 0; e < g.pending_dw.size();) {  // gradients this group was to collect (none in a model whose layers all join the window)
                     const PendingDW p = g.pending_dw[e];

@@ -212,10 +212,10 @@ class Graph {
     // the n-th pass ends, and before anything reads, clears or scales a parameter's gradient; what a caller can observe
     // is the reference's sum in a different rounding order (one f32 accumulation over all tokens of the window).
     // The price is memory: the operands of every windowed product of every pass in the window stay allocated.
-    // Without a window, the weight-gradient GEMMs of narrow layers (each too small to fill the chip) run on the context's
+    // Without a window, the weight gradients of narrow layers wait for the end of the pass (below), and those that are not left for it run on the context's
     // side stream beside the chain of input gradients, which never waits for them: their operands are kept as above
     // (a gradient buffer that a later node adds to in place is replaced by a fresh one) until the backward pass ends
-    // and the main stream has waited for the side stream.  Same kernels, same bits.  On by default.
+    // and the main stream has waited for the side stream.  Off: every product at its node, on the one stream, nothing kept.  On by default.
     void set_weight_gradients_beside(bool on) { beside_ = on; }
     void set_weight_gradient_window(size_t backward_passes);
     size_t weight_gradient_window() const { return window_; }
@@ -242,8 +242,8 @@ class Graph {
     };
     std::vector<LeftDW> left_dw_;
     bool left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out);
-    // left until later when left_fits; false: the caller forms the product now
-    bool leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out);
+    // left until later when left_fits (until the node's last product, after which no more come, when weight gradients keep to the tape); false: the caller forms the product now
+    bool leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out, bool more = false);
     // before anything else touches the gradient of a weight
     void settle_dw(size_t weight);
     eisen_ctx* ctx_;

@@ -18,6 +18,7 @@ struct eisen_ctx {
     const char* answers = "";
     bool side = false, section = false;
     int forks = 0, inlines = 0, sides = 0;
+    std::string order;  // of the products: d(ense), w(eight gradients), each with their number
     std::vector<std::function<void()>> late;  // the side stream
     std::map<void*, size_t> live;            // bytes of every buffer
     size_t bytes() const {
@@ -71,6 +72,7 @@ int eisen_hip_cast(eisen_ctx* ctx, const void* s, int from, void* d, int to, siz
     return give(ctx, [=] { for (size_t i = 0; i < n; i++) put(d, i, to, get(s, i, from)); });
 }
 int eisen_hip_gemm(eisen_ctx* ctx, const void* A, const void* B, void* C, int dtype_ab, int dtype_c, int ta, int tb, size_t M, size_t N, size_t K, int accumulate) {
+    ctx->order += 'd';
     return give(ctx, [=] {
         std::vector<float> b(K * N), sum(N);
         for (size_t k = 0; k < K; k++)
@@ -87,7 +89,9 @@ int eisen_hip_gemm(eisen_ctx* ctx, const void* A, const void* B, void* C, int dt
 }
 int eisen_hip_gemm_weight_gradients(eisen_ctx* ctx, size_t n, const void* const* A, const void* const* B, void* const* C, const size_t* M, const size_t* N, const int* accumulate,
                                     int dtype, size_t K) {
+    const std::string before = ctx->order;
     for (size_t p = 0; p < n; p++) eisen_hip_gemm(ctx, A[p], B[p], C[p], dtype, EISEN_F32, 1, 0, M[p], N[p], K, accumulate[p]);
+    ctx->order = before + 'w' + std::to_string(n);
     return 0;
 }
 int eisen_hip_gemm_residual(eisen_ctx* ctx, const void* A, const void* B, const void* R, void* C, int dtype_ab, int dtype_c, int ta, int tb, size_t M, size_t N, size_t K) {
@@ -115,6 +119,23 @@ int eisen_hip_gemm_weight_gradients_window(eisen_ctx* ctx, size_t n, size_t piec
         for (size_t s = 0; s < pieces; s++)
             eisen_hip_gemm(ctx, A[p * pieces + s], B[p * pieces + s], C[p], EISEN_BF16, EISEN_F32, 1, 0, M[p], N[p], K, s > 0 || accumulate[p]);
     return 0;
+}
+int eisen_hip_gemm_forward_group(eisen_ctx* ctx, size_t n, const void* A, const void* const* B, void* const* C, const size_t* N, int dtype, size_t M, size_t K, size_t, size_t, size_t) {
+    for (size_t p = 0; p < n; p++) eisen_hip_gemm(ctx, A, B[p], C[p], dtype, dtype, 0, 0, M, N[p], K, 0);
+    return 0;
+}
+int eisen_hip_gemm_ksegments(eisen_ctx* ctx, size_t n, const void* const* A, const void* const* B, const size_t* K, void* C, int dtype_ab, int dtype_c, int ta, int tb, size_t M, size_t N,
+                             int accumulate) {
+    const std::string before = ctx->order;
+    for (size_t p = 0; p < n; p++) eisen_hip_gemm(ctx, A[p], B[p], C, dtype_ab, dtype_c, ta, tb, M, N, K[p], p > 0 || accumulate);
+    ctx->order = before + 's';
+    return 0;
+}
+int eisen_hip_add(eisen_ctx* ctx, const void* a, const void* b, void* c, int dtype, size_t n) {
+    return give(ctx, [=] { for (size_t i = 0; i < n; i++) put(c, i, dtype, get(a, i, dtype) + get(b, i, dtype)); });
+}
+int eisen_hip_accumulate(eisen_ctx* ctx, void* a, const void* b, int dtype, size_t n, int accumulate) {
+    return give(ctx, [=] { for (size_t i = 0; i < n; i++) put(a, i, dtype, (accumulate ? get(a, i, dtype) : 0.f) + get(b, i, dtype)); });
 }
 // sections of side work, as runtime.hip has them
 int eisen_hip_side_begin(eisen_ctx* ctx) {
@@ -253,13 +274,38 @@ static std::vector<float> window_with_a_narrow_layer(const char* answers, bool b
     return seen;
 }
 
+// When the products run: Y = ((X V) U) + ((X V) W), V alone, U and W as one node.  Kept to the tape, a node's products follow its input gradient and nothing is kept.
+static std::vector<float> order_of_products(const char* answers, bool beside) {
+    constexpr size_t kRows = 16, kHidden = 32;
+    eisen_ctx ctx;
+    ctx.answers = answers;
+    eisen::Graph g(&ctx, eisen::PrecisionMode::Bf16Mixed);
+    g.set_weight_gradients_beside(beside);
+    std::vector<size_t> w;
+    for (size_t i = 0; i < 3; i++) w.push_back(g.alloc({kHidden, kHidden}, ramp(kHidden * kHidden, 3 + 2 * i, 11, 0.125f)));
+    g.mark_params();
+    const size_t x = g.alloc({kRows, kHidden}, ramp(kRows * kHidden, 3, 13, 0.25f));
+    const size_t h = g.matmul(x, w[0]);
+    const std::vector<size_t> both = g.matmul_group(h, {w[1], w[2]});
+    const size_t y = g.add(both[0], both[1]);
+    ctx.order.clear();
+    g.backward(y);
+    // (the group's input gradient is one call, s; V's product with X comes behind the input gradient of X)
+    if (ctx.order != (beside ? "sdw3" : "sw2dw1")) throw eisen::Error("products ran in the order " + ctx.order);
+    std::vector<float> seen;
+    for (size_t id : w)
+        for (size_t i = 0; i < g.at(id).size(); i++) seen.push_back(get(g.at(id).grad.ptr, i, EISEN_F32));
+    return seen;
+}
+
 int main(int argc, char** argv) {
     if (argc < 2 || argc > 3) return 2;
     const char* answers = argv[argc - 1];
     const std::string graph = argc == 3 ? argv[1] : "weight_used_twice";
     try {
         const auto run = graph == "weight_used_twice" ? gradients : graph == "rows_of_two_lengths" ? rows_of_two_lengths : graph == "tail_and_its_residual" ? tail_and_its_residual
-                         : graph == "window_with_a_narrow_layer" ? window_with_a_narrow_layer : nullptr;
+                         : graph == "window_with_a_narrow_layer" ? window_with_a_narrow_layer
+                         : graph == "order_of_products" ? order_of_products : nullptr;
         if (!run) return 2;
         const std::vector<float> plain = run("", false), beside = run(answers, true);
         bool some = false;

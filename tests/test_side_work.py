@@ -39,3 +39,9 @@ def test_a_window_keeps_the_operands_of_its_own_products_only(stub):
     # those that the pass's launch has read go back with the pass
     done = subprocess.run([stub, "window_with_a_narrow_layer", ""], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stderr
+
+
+def test_products_kept_to_the_tape_run_at_their_nodes(stub):
+    # and have the bits of those that the pass leaves
+    done = subprocess.run([stub, "order_of_products", ""], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stderr
