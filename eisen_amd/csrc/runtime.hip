@@ -74,6 +74,9 @@ int wait_word(eisen_ctx* ctx, const unsigned* word, unsigned number, hipStream_t
             std::this_thread::yield();
             continue;
         }
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;  // a stream under capture cannot be asked; the word comes from before the capture
+        EISEN_HIP_TRY(ctx, hipStreamIsCapturing(stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) continue;
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (asking a stream ends a capture in another mode)
         EISEN_HIP_TRY(ctx, hipThreadExchangeStreamCaptureMode(&mode));
         const hipError_t q = hipStreamQuery(stream);
