@@ -8,7 +8,7 @@ step of the config-4 architecture (rtol 2e-2 on gradients).
 import numpy as np
 import pytest
 
-from eisen_amd import graph as G
+from eisen_amd import graph as G, hip
 from eisen_amd.lib import EisenHipError
 from oracle import cpu_ref as R
 from tests import gen
@@ -431,6 +431,79 @@ def test_weight_gradients_beside_the_chain_give_the_same_bits(ctx, tie, checkpoi
     assert l0 == l1
     for i, (a, b) in enumerate(zip(g0, g1)):
         assert a.any() and np.array_equal(a, b), f"gradient of parameter {i} differs when the weight gradients run beside the chain"
+
+
+@pytest.mark.parametrize("hidden,rows", [(100, 600), (30, 200), (64, 16640)])  # sides that are no multiples of 8, one below 32, more than 16384 rows
+def test_products_on_the_side_stream_give_the_bits_of_the_tape(ctx, hidden, rows):
+    # What the launch at the end of the pass does not take runs beside the chain, here with a queue ahead of every pass so that it forks.  One weight is used twice, two
+    # passes add up, and nothing stays allocated.
+    big, out = ctx.malloc(4096 * 4096 * 2, zero=True), ctx.malloc(4096 * 4096 * 2)
+    w0 = [gen.normal(940 + i, (hidden, hidden), hidden ** -0.5) for i in range(3)]
+    x0, t0 = gen.normal(950, (rows, hidden)), gen.uniform_ids(951, (rows,), hidden)
+    results = []
+    for beside in (False, True):
+        g = G.Graph(ctx, G.BF16_MIXED)
+        g.set_weight_gradients_beside(beside)
+        ws = [g.alloc(w.shape, w) for w in w0]
+        g.mark_params()
+        ctx.sync()
+        base = ctx.pool_stats()[0]
+        ctx.profile_start()
+        for _ in range(2):
+            h = g.input(x0)
+            for w in ws + [ws[0]]:
+                h = g.matmul(h, w)
+            loss = g.cross_entropy(h, t0)
+            for _ in range(4):
+                ctx.gemm(big, big, out, hip.BF16, hip.BF16, 0, 0, 4096, 4096, 4096)
+            g.backward(loss)
+            g.clear_activations()
+        assert not any(n.endswith("_layers") for n in ctx.profile_stop())
+        ctx.sync()
+        assert ctx.pool_stats()[0] == base
+        results.append([g.sync_grad_to_cpu(w) for w in ws])
+        g.close()
+    for a, b in zip(*results):
+        assert a.any() and np.array_equal(a, b)
+    big.free()
+    out.free()
+
+
+def test_products_left_for_the_pass_stay_off_the_side_stream(ctx):
+    # Two weights, each used over 8 rows (left) and W1 over 16640 as well (beside the chain): P = S W2, Q = P W1, R = Q W2, Y = (X W1) R^T.  The bits of the tape; 2^-8 of float64,
+    # where every activation is bf16.
+    hidden, few, many = 64, 8, 16640
+    w1_0, w2_0 = gen.normal(960, (hidden, hidden), hidden ** -0.5), gen.normal(961, (hidden, hidden), hidden ** -0.5)
+    s0, x0 = gen.normal(962, (few, hidden)), gen.normal(963, (many, hidden))
+    big, out = ctx.malloc(4096 * 4096 * 2, zero=True), ctx.malloc(4096 * 4096 * 2)
+    results = []
+    for beside in (False, True):
+        g = G.Graph(ctx, G.BF16_MIXED)
+        g.set_weight_gradients_beside(beside)
+        w1, w2 = g.alloc(w1_0.shape, w1_0), g.alloc(w2_0.shape, w2_0)
+        g.mark_params()
+        opt = G.AdamW(g, [w1, w2], 1e-3)
+        opt.zero_grad()
+        y1 = g.matmul(g.input(x0), w1)
+        r = g.matmul(g.matmul(g.matmul(g.input(s0), w2), w1), w2)
+        y = g.matmul_trans_b(y1, r)
+        for _ in range(4):
+            ctx.gemm(big, big, out, hip.BF16, hip.BF16, 0, 0, 4096, 4096, 4096)
+        g.backward(y)
+        results.append([g.sync_grad_to_cpu(w) for w in (w1, w2)])
+        g.close()
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
+    w1, w2, s, x = (v.astype(np.float64) for v in (w1_0, w2_0, s0, x0))
+    p = s @ w2
+    q = p @ w1
+    dy1 = np.ones((many, few)) @ (q @ w2)
+    dr = np.ones((few, many)) @ (x @ w1)
+    dq = dr @ w2.T
+    assert_close(results[1][0], x.T @ dy1 + p.T @ dq, 2e-2, "W1")
+    assert_close(results[1][1], q.T @ dr + s.T @ (dq @ w1.T), 2e-2, "W2")
+    big.free()
+    out.free()
 
 
 # ---- composed training step against the oracle ---------------------------------------------------
