@@ -298,6 +298,52 @@ static std::vector<float> order_of_products(const char* answers, bool beside) {
     return seen;
 }
 
+// Passes that throw when all their products are left: a gradient read behind one has them, one cleared behind one loses them, and the next pass is whole.  W is used over two
+// numbers of rows: Y = (X W) ((S W) V)^T.
+static std::vector<float> pass_that_threw(const char* answers, bool beside) {
+    constexpr size_t kHidden = 32;
+    eisen_ctx ctx;
+    ctx.answers = answers;
+    eisen::Graph g(&ctx, eisen::PrecisionMode::Bf16Mixed);
+    g.set_weight_gradients_beside(beside);
+    const size_t w = g.alloc({kHidden, kHidden}, ramp(kHidden * kHidden, 7, 11, 0.125f)), v = g.alloc({kHidden, kHidden}, ramp(kHidden * kHidden, 5, 17, 0.0625f));
+    g.mark_params();
+    for (size_t id : {w, v}) g.request_zero_grad(id);
+    const size_t base = ctx.bytes();
+    std::vector<float> seen;
+    auto read = [&](size_t id) {
+        g.materialize_grad(id);
+        for (size_t i = 0; i < g.at(id).size(); i++) seen.push_back(get(g.at(id).grad.ptr, i, EISEN_F32));
+    };
+    auto pass = [&](bool throws) {
+        const size_t s = g.alloc({8, kHidden}, ramp(8 * kHidden, 5, 13, 0.25f)), x = g.alloc({16, kHidden}, ramp(16 * kHidden, 3, 7, 0.5f));
+        if (throws) g.tape.nodes.push_back(eisen::TapeNode{{}, x, [](eisen::Graph&) { throw eisen::Error("meant"); }});
+        const size_t y = g.matmul_trans_b(g.matmul(x, w), g.matmul(g.matmul(s, w), v));
+        try {
+            g.backward(y);
+        } catch (const eisen::Error& e) {
+            if (std::string(e.what()) != "meant") throw;
+        }
+    };
+    pass(true);
+    read(v);
+    read(w);
+    g.clear_activations();
+    pass(true);
+    for (size_t id : {w, v}) g.request_zero_grad(id);
+    g.clear_activations();
+    pass(false);
+    read(w);
+    read(v);
+    g.clear_activations();
+    pass(true);
+    g.clear_activations();  // (nobody has asked for a gradient: the products are added before their operands go)
+    read(v);
+    read(w);
+    if (ctx.bytes() != base) throw eisen::Error("operands are still allocated");
+    return seen;
+}
+
 int main(int argc, char** argv) {
     if (argc < 2 || argc > 3) return 2;
     const char* answers = argv[argc - 1];
@@ -305,7 +351,8 @@ int main(int argc, char** argv) {
     try {
         const auto run = graph == "weight_used_twice" ? gradients : graph == "rows_of_two_lengths" ? rows_of_two_lengths : graph == "tail_and_its_residual" ? tail_and_its_residual
                          : graph == "window_with_a_narrow_layer" ? window_with_a_narrow_layer
-                         : graph == "order_of_products" ? order_of_products : nullptr;
+                         : graph == "order_of_products" ? order_of_products
+                         : graph == "pass_that_threw" ? pass_that_threw : nullptr;
         if (!run) return 2;
         const std::vector<float> plain = run("", false), beside = run(answers, true);
         bool some = false;

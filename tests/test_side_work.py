@@ -45,3 +45,9 @@ def test_products_kept_to_the_tape_run_at_their_nodes(stub):
     # and have the bits of those that the pass leaves
     done = subprocess.run([stub, "order_of_products", ""], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stderr
+
+
+def test_products_left_by_a_pass_that_threw(stub):
+    # a gradient read, cleared or left alone behind it is that of products formed at their nodes
+    done = subprocess.run([stub, "pass_that_threw", ""], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stderr
