@@ -22,10 +22,12 @@ namespace {
 // ---- copies between device memory and pinned host memory as kernels --------------------------------------------
 // The runtime's own copies of 32 KB and more go through a copy engine, which a chain of kernels waits for: a kernel, such a copy and a kernel take 19.5 us where the
 // copy as a kernel of one workgroup makes it 9; and an event behind a copy, recorded to know when its staging memory is free, is 3 us of
-// the stream.  So an upload of up to kCopyKernelBytes is one workgroup here, and says itself that it is done.  (Not the tickets of eisen_hip_dtoh_begin: a
+// the stream.  So an upload of up to kCopyKernelBytes is one workgroup here, and says itself that it is done.  The runtime's copy / this, in us, a kernel, the upload and a kernel in
+// a row | uploads alone in a row: 32 KB 27 / 14 | 15 / 6, 64 KB 28 / 16 | 15 / 9, 96 KB 29 / 20 | 16 / 13; beyond the line 128 KB 30 / 23 | 17 / 16 but one upload, a kernel and the wait
+// for them 29 / 32, 192 KB 31 / 30 | 18 / 22, 256 KB 32 / 36 | 20 / 29: one workgroup reads 9 GB/s from the host.  (Not the tickets of eisen_hip_dtoh_begin: a
 // few bytes, where making them visible to the host writes the caches back: 1 us more than the event.)
 constexpr int kCopyThreads = 1024;
-constexpr size_t kCopyKernelBytes = size_t(256) << 10;
+constexpr size_t kCopyKernelBytes = size_t(96) << 10;
 
 template <typename T>
 __device__ __forceinline__ void copy_by_workgroup(const T* __restrict__ src, T* __restrict__ dst, unsigned n) {
