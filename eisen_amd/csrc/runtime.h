@@ -70,6 +70,7 @@ struct eisen_ctx {
     void* back = nullptr;       // pinned ring of a read-back
     size_t back_bytes = 0;
     unsigned back_number = 0;
+    bool waited = false;        // the host has waited for all work of the main stream and launched no kernel since (a stream asked for this while kernels run delays them by 20 us)
     // grow-only device workspace for two-stage reductions and tables
     void* ws = nullptr;
     size_t ws_bytes = 0;
@@ -157,6 +158,7 @@ int eisen_staging(eisen_ctx* ctx, size_t bytes, eisen_ctx::StageSlot** out);
         if (_e != hipSuccess)                                                                 \
             return eisen_set_error((ctx), (int)_e, "launch of %s failed: %s", (name),         \
                                    hipGetErrorString(_e));                                    \
+        (ctx)->waited = false;                                                                \
     } while (0)
 
 static inline bool eisen_aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }

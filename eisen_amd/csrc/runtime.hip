@@ -283,6 +283,7 @@ extern "C" int eisen_hip_stream_sync(eisen_ctx* ctx) {
     EISEN_CHECK_CTX(ctx);
     if (ctx->side_pending || ctx->side_active) EISEN_HIP_TRY(ctx, hipStreamSynchronize(ctx->side_stream));
     EISEN_HIP_TRY(ctx, hipStreamSynchronize(ctx->main_stream));
+    ctx->waited = true;
     return 0;
 }
 
@@ -488,9 +489,18 @@ extern "C" int eisen_hip_htod(eisen_ctx* ctx, void* dst, const void* src, size_t
     return 0;
 }
 
+// Memory that the device writes itself (pinned).
+static bool known_to_device(const void* p) {
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
 // Device memory into the caller's, as it is or (widen) bf16 as f32.  Through pinned memory in pieces (read_back_kernel); what is small, not aligned or under capture
-// goes by the runtime's copy.  That copy and this, in us: 4 KB 24 and 25 (the line is at 16 KB, where they part), 64 KB 37 and 19, 256 KB 118 and 25, 1 MB 67 and
-// 50, 8 MB 512 and 240, 512 MB 32100 and 24900.  A forward pass with its 201 x 8192 bf16 logits read back 579 and 369.
+// goes by the runtime's copy.  That copy and this behind a kernel, in us: 4 KB 24 and 25 (the line is at 16 KB, where they part), 64 KB 28 and 24, 256 KB 37 and 30, 1 MB 78
+// and 54, 4 MB 264 and 129; 512 MB 32100 and 24900.  A forward pass with its 201 x 8192 bf16 logits read back 579 and 369.
+// The runtime's copy also where it is ahead: into pinned memory (64 KB 10 and 19, 1 MB 27 and 48, 64 MB 1185 and 2370), and from 32 KB to 1 MB where its copy engine has no kernel to
+// wait for (64 KB 12 and 19, 256 KB 20 and 25, 512 KB 31 and 36, 1 MB 60 and 49); to be widened, there, into the ring (128 KB of bf16 19 and 28, 256 KB 28 and 35, 512 KB 44 and 46).
 static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, bool widen) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     EISEN_HIP_TRY(ctx, hipStreamIsCapturing(ctx->stream, &capture));
@@ -507,7 +517,10 @@ static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, b
         out += widen ? 2 * n : n;
     };
     size_t done = 0;
-    if (whole >= (size_t(16) << 10) && eisen_aligned(src, 16) && capture == hipStreamCaptureStatusNone) {
+    bool ring = whole >= (size_t(16) << 10) && eisen_aligned(src, 16) && capture == hipStreamCaptureStatusNone;
+    const bool on_main = ctx->stream == ctx->main_stream, idle = ctx->waited && on_main;
+    if (ring && !widen) ring = !known_to_device(dst) && !(idle && whole >= (size_t(32) << 10) && whole < (size_t(1) << 20));
+    if (ring) {
         const int rc = eisen_words(ctx);
         if (rc) return rc;
         const size_t want = (std::min(whole, kBackRing) + kBackPiece - 1) / kBackPiece * kBackPiece;
@@ -518,6 +531,12 @@ static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, b
             ctx->driver_allocs++;
             EISEN_HIP_TRY(ctx, hipHostMalloc(&ctx->back, want, hipHostMallocDefault));
             ctx->back_bytes = want;
+        }
+        if (widen && idle && whole >= (size_t(96) << 10) && whole < (size_t(512) << 10)) {
+            EISEN_HIP_TRY(ctx, hipMemcpyAsync(ctx->back, src, whole, hipMemcpyDeviceToHost, ctx->stream));
+            EISEN_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+            take(ctx->back, whole);
+            done = whole;
         }
         unsigned* words = ctx->words + 16 * eisen_ctx::kStageSlots;
         while (done < whole) {
@@ -536,6 +555,7 @@ static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, b
             done += n;
         }
     }
+    if (on_main) ctx->waited = true;
     if (done == bytes) return 0;
     const size_t left = bytes - done;
     char* raw = widen ? out + left : out;  // (in the upper half of what is to hold it as f32: element i is read before any write reaches it)
@@ -602,6 +622,7 @@ extern "C" int eisen_hip_dtod(eisen_ctx* ctx, void* dst, const void* src, size_t
     EISEN_REQUIRE(ctx, dst && src, EISEN_E_ARG, "eisen_hip_dtod: null pointer");
     if (bytes == 0) return 0;
     EISEN_HIP_TRY(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+    ctx->waited = false;
     return 0;
 }
 
@@ -657,6 +678,7 @@ extern "C" int eisen_hip_launch(eisen_ctx* ctx, eisen_function* fn, const unsign
                   "eisen_hip_launch: more than 1024 threads per block");
     EISEN_HIP_TRY(ctx, hipModuleLaunchKernel(fn->fn, grid[0], grid[1], grid[2], block[0], block[1], block[2],
                                              shared_bytes, ctx->stream, args, nullptr));
+    ctx->waited = false;
     return 0;
 }
 
