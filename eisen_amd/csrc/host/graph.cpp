@@ -477,7 +477,9 @@ void Graph::flush_left_dw() {
             accs.push_back(acc);
         }
         list.swap(rest);
-        if (eisen_dw_together(first.dtype == EISEN_BF16, Cs.size(), Ms.data(), Ns.data(), first.rows)) {
+        // (kept to the tape, a node's product takes the kernel that it would take among a pass's)
+        const bool bf16 = first.dtype == EISEN_BF16, alone = beside_ && Cs.size() == 1;
+        if (alone ? eisen_dw_alone(bf16, Ms[0], Ns[0], first.rows) : eisen_dw_together(bf16, Cs.size(), Ms.data(), Ns.data(), first.rows)) {
             rc = eisen_hip_gemm_weight_gradients(ctx_, Cs.size(), As.data(), Bs.data(), Cs.data(), Ms.data(), Ns.data(), accs.data(), first.dtype, first.rows);
         } else {
             for (size_t p = 0; p < Cs.size() && !rc; p++) rc = eisen_hip_gemm(ctx_, As[p], Bs[p], Cs[p], first.dtype, EISEN_F32, 1, 0, Ms[p], Ns[p], first.rows, accs[p]);

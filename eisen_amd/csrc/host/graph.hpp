@@ -230,7 +230,7 @@ class Graph {
     // The products of a narrow model's layers are each too small for the chip, and nothing in the pass reads them: they are left until
     // the pass ends, or until something else writes, reads or clears the gradient of one of the weights, and then run together
     // (eisen_hip_gemm_weight_gradients).  Operands are kept as for the window, until that launch.  Which products: left_fits;
-    // few of them over many tokens are formed by a launch each at that time (gemm_dw_rule.h).
+    // one alone, or few over many tokens, are formed by a launch each at that time (gemm_dw_rule.h).
     void flush_left_dw();
 
    private:
