@@ -312,7 +312,7 @@ int eisen_hip_gemm_grouped(eisen_ctx* ctx, size_t n, const void* const* A, const
  * micro-batch at a time, in f32; here the pieces of a product are summed in the MFMA accumulators of one launch (any
  * number of products of up to 8 pieces, every M_p and N_p a multiple of 256, seg_k of 128, at least 176 tiles of
  * 256 x 256 in all), which reads and writes each gradient once per window instead of once per micro-batch.  Other
- * shapes are added piece by piece, in piece order. */
+ * shapes are added piece by piece, in piece order; where a result meets another or an operand, one product after the other. */
 #define EISEN_GEMM_MAX_KSEGMENTS 8
 int eisen_hip_gemm_grouped_ksegments(eisen_ctx* ctx, size_t n_products, size_t n_segments, const void* const* A, const void* const* B,
                                      void* const* C, const size_t* M, const size_t* N, size_t seg_k, int accumulate);
@@ -325,7 +325,7 @@ int eisen_hip_gemm_weight_gradients_window(eisen_ctx* ctx, size_t n_products, si
 /* C_p (+)= A_p^T B_p for any number of products over one contraction: the dB += A^T dC of the matmul backward
  * (src/graph/ops/linear.rs:279-287) for the layers of a backward pass at once, whose products are each too small to fill the
  * chip.  A[p] is [K, M_p], B[p] [K, N_p] (both `dtype`), C[p] f32 [M_p, N_p], added to where accumulate[p].  The bits of a
- * product do not depend on the others of the call. */
+ * product do not depend on the others of the call.  Results lie apart from the operands. */
 int eisen_hip_gemm_weight_gradients(eisen_ctx* ctx, size_t n, const void* const* A, const void* const* B, void* const* C, const size_t* M, const size_t* N,
                                     const int* accumulate, int dtype, size_t K);
 
