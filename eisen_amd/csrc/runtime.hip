@@ -499,8 +499,9 @@ static bool known_to_device(const void* p) {
 // Device memory into the caller's, as it is or (widen) bf16 as f32.  Through pinned memory in pieces (read_back_kernel); what is small, not aligned or under capture
 // goes by the runtime's copy.  That copy and this behind a kernel, in us: 4 KB 24 and 25 (the line is at 16 KB, where they part), 64 KB 28 and 24, 256 KB 37 and 30, 1 MB 78
 // and 54, 4 MB 264 and 129; 512 MB 32100 and 24900.  A forward pass with its 201 x 8192 bf16 logits read back 579 and 369.
-// The runtime's copy also where it is ahead: into pinned memory (64 KB 10 and 19, 1 MB 27 and 48, 64 MB 1185 and 2370), and from 32 KB to 1 MB where its copy engine has no kernel to
-// wait for (64 KB 12 and 19, 256 KB 20 and 25, 512 KB 31 and 36, 1 MB 60 and 49); to be widened, there, into the ring (128 KB of bf16 19 and 28, 256 KB 28 and 35, 512 KB 44 and 46).
+// The runtime's copy also where it is ahead: into pinned memory (64 KB 10 and 19, 1 MB 27 and 48, 64 MB 1185 and 2370), and above 16 KB (up to which it is 24 and this 19) to 1 MB where its
+// copy engine has no kernel to wait for (20 KB 11 and 18, 64 KB 12 and 19, 256 KB 20 and 25, 512 KB 31 and 36, 1 MB 60 and 49); to be widened, there, into the ring (20 KB of bf16 11 and
+// 19, 64 KB 15 and 21, 128 KB 19 and 28, 256 KB 28 and 35, 512 KB 44 and 46).
 static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, bool widen) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     EISEN_HIP_TRY(ctx, hipStreamIsCapturing(ctx->stream, &capture));
@@ -519,7 +520,7 @@ static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, b
     size_t done = 0;
     bool ring = whole >= (size_t(16) << 10) && eisen_aligned(src, 16) && capture == hipStreamCaptureStatusNone;
     const bool on_main = ctx->stream == ctx->main_stream, idle = ctx->waited && on_main;
-    if (ring && !widen) ring = !known_to_device(dst) && !(idle && whole >= (size_t(32) << 10) && whole < (size_t(1) << 20));
+    if (ring && !widen) ring = !known_to_device(dst) && !(idle && whole > (size_t(16) << 10) && whole < (size_t(1) << 20));
     if (ring) {
         const int rc = eisen_words(ctx);
         if (rc) return rc;
@@ -532,7 +533,7 @@ static int read_back(eisen_ctx* ctx, void* dst, const void* src, size_t bytes, b
             EISEN_HIP_TRY(ctx, hipHostMalloc(&ctx->back, want, hipHostMallocDefault));
             ctx->back_bytes = want;
         }
-        if (widen && idle && whole >= (size_t(96) << 10) && whole < (size_t(512) << 10)) {
+        if (widen && idle && whole > (size_t(16) << 10) && whole < (size_t(512) << 10)) {
             EISEN_HIP_TRY(ctx, hipMemcpyAsync(ctx->back, src, whole, hipMemcpyDeviceToHost, ctx->stream));
             EISEN_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
             take(ctx->back, whole);
