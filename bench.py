@@ -44,7 +44,7 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 TRAFFIC_SOURCE = {"c5": "profiles/c5_step_hbm_traffic_pmc.md", "c4": "profiles/c4_step_hbm_traffic_pmc.md", "c3": "profiles/c2_c3_hbm_traffic_pmc.md", "c2": "profiles/c2_c3_hbm_traffic_pmc.md"}
 MEASURED_TRAFFIC = {
     "c5": {"gemm_tn_bf16_f32out_256x256x32_window": 18263.6e6, "gemm_tn_bf16_f32out_256x256x32": 902.8e6, "gemm_nt_bf16_bf16out_256x128x64": 213.4e6},
-    "c4": {"gemm_tn_bf16_f32out_128x64x16_layers": 955.5e6, "gemm_tn_bf16_f32out_64x64x32_sliced_splitk": 46.8e6, "gemm_nt_bf16_bf16out_128x128x64": 35.6e6, "gemm_nt_bf16_bf16out_256x128x64_swiglu_bwd": 101.3e6,
+    "c4": {"gemm_tn_bf16_f32out_128x64x16_layers": 998.4e6, "gemm_tn_bf16_f32out_64x64x32_sliced_splitk": 46.8e6, "gemm_nt_bf16_bf16out_128x128x64": 35.6e6, "gemm_nt_bf16_bf16out_256x128x64_swiglu_bwd": 101.3e6,
            "gemm_nn_bf16_bf16out_128x128x64_splitk": 167.9e6, "gemm_tn_bf16_f32out_128x128x64_splitk": 167.7e6, "gemm_nn_bf16_swiglu_256x128x32": 85.0e6},
     "c3": {"attn_bwd": 78.7e6 + 52.4e6},
     "c2": {"ce_fused_bf16": 1048.9e6},
