@@ -25,3 +25,14 @@ inline bool eisen_dw_alone(bool bf16, size_t M, size_t N, size_t K) {
     const size_t tiles = M / 64 * (N / 64);
     return bf16 && K >= 2048 && M % 64 == 0 && N % 64 == 0 && (tiles == 256 || tiles == 512);
 }
+
+// The same for the bf16 products of one node (a weight, or the weights that share an input), whose launch each is one launch too, and which are not left for others: where weight
+// gradients keep to the tape.  (By this, the bits of narrow layers over few tokens are those of a pass's launch.)
+// Steps kept to the tape with bf16 nodes by this and f32 ones by their own launches / all nodes by eisen_dw_together, a launch per product where it says no, us: the ~14 M model 1606 / 1875, in
+// f32 2737 / 2954; hidden 1536, 3 layers, 4096 tokens 3723 / 3773; hidden 1024, 4 layers, 1024 tokens 1409 / 1425; hidden 128 in f32, 4 layers, 512 tokens 625 / 682.
+inline bool eisen_dw_node(size_t n, const size_t* M, const size_t* N, size_t K) {
+    double tiles = 0.0;
+    for (size_t p = 0; p < n; p++) tiles += (double)((M[p] + 63) / 64) * (double)((N[p] + 63) / 64);
+    if (n == 1 && tiles >= 256.0) return eisen_dw_alone(true, M[0], N[0], K);
+    return 4.2 + (double)K / 360.0 * std::max(1.0, tiles / 256.0) <= 7.0 + tiles * (double)K / 65536.0;
+}

@@ -430,15 +430,24 @@ bool Graph::left_fits(size_t weight, const void* x, const void* dy, int dtype, s
     return tw.is_param && tw.grad.dtype == EISEN_F32 && tw.size() == in * out;
 }
 
-bool Graph::leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out, bool more) {
-    if (!left_fits(weight, x, dy, dtype, rows, in, out)) return false;
-    settle_dw(weight);  // a weight used twice: its products one after the other
-    left_dw_.push_back(LeftDW{weight, x, dy, rows, in, out, dtype});
-    if (beside_) {
-        hold(x, kForPass);
-        hold(dy, kForPass);
-    } else if (!more) {  // products in the order of the tape: those of this node now
-        flush_left_dw();
+// The products of a node: all of them are left until later, or run here, or the caller forms them now (false).
+bool Graph::leave_dw(const std::vector<LeftDW>& node) {
+    std::vector<size_t> Ms, Ns;
+    for (const LeftDW& e : node) {
+        if (!left_fits(e.weight, e.x, e.dy, e.dtype, e.rows, e.in, e.out)) return false;
+        Ms.push_back(e.in);
+        Ns.push_back(e.out);
+    }
+    if (!beside_) {  // in the order of the tape
+        if (node.empty() || node[0].dtype != EISEN_BF16 || !eisen_dw_node(Ms.size(), Ms.data(), Ns.data(), node[0].rows)) return false;
+        form_dw(node);
+        return true;
+    }
+    for (const LeftDW& e : node) {
+        settle_dw(e.weight);  // a weight used twice: its products one after the other
+        left_dw_.push_back(e);
+        hold(e.x, kForPass);
+        hold(e.dy, kForPass);
     }
     return true;
 }
@@ -455,6 +464,10 @@ void Graph::settle_dw(size_t weight) {
 void Graph::flush_left_dw() {
     std::vector<LeftDW> list;
     list.swap(left_dw_);
+    form_dw(std::move(list));
+}
+
+void Graph::form_dw(std::vector<LeftDW> list) {
     int rc = 0;
     while (!list.empty() && !rc) {  // one launch per contraction length and element type, one for a pass, or a launch each
         const LeftDW first = list.front();
@@ -477,9 +490,8 @@ void Graph::flush_left_dw() {
             accs.push_back(acc);
         }
         list.swap(rest);
-        // (kept to the tape, a node's product takes the kernel that it would take among a pass's)
-        const bool bf16 = first.dtype == EISEN_BF16, alone = beside_ && Cs.size() == 1;
-        if (alone ? eisen_dw_alone(bf16, Ms[0], Ns[0], first.rows) : eisen_dw_together(bf16, Cs.size(), Ms.data(), Ns.data(), first.rows)) {
+        const bool bf16 = first.dtype == EISEN_BF16;
+        if (!beside_ || (Cs.size() == 1 ? eisen_dw_alone(bf16, Ms[0], Ns[0], first.rows) : eisen_dw_together(bf16, Cs.size(), Ms.data(), Ns.data(), first.rows))) {
             rc = eisen_hip_gemm_weight_gradients(ctx_, Cs.size(), As.data(), Bs.data(), Cs.data(), Ms.data(), Ns.data(), accs.data(), first.dtype, first.rows);
         } else {
             for (size_t p = 0; p < Cs.size() && !rc; p++) rc = eisen_hip_gemm(ctx_, As[p], Bs[p], Cs[p], first.dtype, EISEN_F32, 1, 0, Ms[p], Ns[p], first.rows, accs[p]);
@@ -734,7 +746,7 @@ size_t Graph::matmul(size_t a, size_t b) {
         Storage& ga = g.grad_for_write(a, &acc);
         g.check(eisen_hip_gemm(g.ctx(), go.ptr, g.compute_data(b).ptr, ga.ptr, go.dtype, ga.dtype, 0, 1, M, K, N, acc), "matmul backward dA");
         if (g.window_take(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N)) return;
-        if (g.leave_dw(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N)) return;
+        if (g.leave_dw({{b, g.compute_data(a).ptr, go.ptr, M, K, N, go.dtype}})) return;
         const void* xa = g.compute_data(a).ptr;
         g.run_beside(g.at(b).is_param && g.beside_fits(K, N), {xa, go.ptr}, {b}, [&]() {
             int accb = 0;
@@ -777,7 +789,7 @@ size_t Graph::matmul_residual(size_t a, size_t b, size_t r, bool defer_dw) {
         }
         Storage& ga = g.grad_for_write(a, &acc);
         g.check(eisen_hip_gemm(g.ctx(), go.ptr, g.compute_data(b).ptr, ga.ptr, go.dtype, ga.dtype, 0, 1, M, K, N, acc), "matmul_residual backward dA");
-        if (g.window_take(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N) || g.leave_dw(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N)) {
+        if (g.window_take(b, g.compute_data(a).ptr, go.ptr, go.dtype, M, K, N) || g.leave_dw({{b, g.compute_data(a).ptr, go.ptr, M, K, N, go.dtype}})) {
             // left for the window's or the pass's launch; whoever adds to dOut's buffer (now dR's) next gets a fresh one
         } else if (defer_dw && go.dtype == EISEN_BF16 && g.at(b).is_param) {
             // dOut's buffer (now also dR's) is only added to by nodes that run after the collecting group
@@ -830,7 +842,7 @@ size_t Graph::swiglu_matmul_residual(size_t gate, size_t up, size_t b, size_t r,
             g.check(eisen_hip_accumulate(g.ctx(), gr.ptr, go.ptr, go.dtype, M * N, acc), "swiglu_matmul_residual backward dR");
         }
         // large products only: a small one gains nothing from running beside the chain
-        const bool windowed = g.window_take(b, g.at(h).data.ptr, go.ptr, go.dtype, M, K, N) || g.leave_dw(b, g.at(h).data.ptr, go.ptr, go.dtype, M, K, N);
+        const bool windowed = g.window_take(b, g.at(h).data.ptr, go.ptr, go.dtype, M, K, N) || g.leave_dw({{b, g.at(h).data.ptr, go.ptr, M, K, N, go.dtype}});
         const bool side = !windowed && go.dtype == EISEN_BF16 && g.at(b).is_param && K % 256 == 0 && N % 128 == 0 && M % 64 == 0 && (K / 256) * (N / 128) >= 128;
         if (side) {
             // dB beside the input-gradient chain: it reads h and dOut; dOut's buffer (now dR's) is next written by whoever
@@ -933,14 +945,10 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
             Storage& ga = g.grad_for_write(a, &acc);
             g.check(eisen_hip_gemm_ksegments(g.ctx(), m, As, Bs, Ks, ga.ptr, EISEN_F32, ga.dtype, 0, 1, M, K, acc), "matmul_group backward dA");
             const void* xa = g.compute_data(a).ptr;
-            bool left = true;
+            std::vector<LeftDW> node;
             for (size_t i = 0; i < n; i++)
-                if (g.has_grad(outs[i])) left = left && g.left_fits(ws[i], xa, g.grad_for_read(outs[i]).ptr, EISEN_F32, M, K, N[i]);
-            if (left) {
-                for (size_t i = 0, left_of = m; i < n; i++)
-                    if (g.has_grad(outs[i])) g.leave_dw(ws[i], xa, g.grad_for_read(outs[i]).ptr, EISEN_F32, M, K, N[i], --left_of > 0);
-                return;
-            }
+                if (g.has_grad(outs[i])) node.push_back({ws[i], xa, g.grad_for_read(outs[i]).ptr, M, K, N[i], EISEN_F32});
+            if (g.leave_dw(node)) return;
             int accs[3];
             size_t Ns[3];
             m = 0;
@@ -1024,18 +1032,16 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
         const Storage xa = g.compute_data(a);
         if (all) {
             // every member joins the window (or is left for the pass's launch) or none: a group split between them and this node gains nothing
-            bool fits = true, left = true;
-            for (const PendingDW& p : g.pending_dw) left = left && std::find(collect_dw.begin(), collect_dw.end(), p.weight) == collect_dw.end();  // these wait for this node's launch
+            bool fits = true, waiting = false;
+            for (const PendingDW& p : g.pending_dw) waiting = waiting || std::find(collect_dw.begin(), collect_dw.end(), p.weight) != collect_dw.end();  // for this node's launch
+            std::vector<LeftDW> node;
             for (size_t i = 0; i < n; i++) {
                 fits = fits && g.window_fits(ws[i], EISEN_BF16, M, K, N[i]);
-                left = left && g.left_fits(ws[i], xa.ptr, g.grad_for_read(outs[i]).ptr, EISEN_BF16, M, K, N[i]);
+                node.push_back({ws[i], xa.ptr, g.grad_for_read(outs[i]).ptr, M, K, N[i], EISEN_BF16});
             }
-            if (fits || left) {
-                for (size_t i = 0; i < n; i++) {
-                    const void* dy = g.grad_for_read(outs[i]).ptr;
-                    if (fits) g.window_take(ws[i], xa.ptr, dy, EISEN_BF16, M, K, N[i]);
-                    else g.leave_dw(ws[i], xa.ptr, dy, EISEN_BF16, M, K, N[i], i + 1 < n);
-                }
+            if (fits || (!waiting && g.leave_dw(node))) {
+                for (const LeftDW& e : node)
+                    if (fits) g.window_take(e.weight, e.x, e.dy, EISEN_BF16, M, K, e.out);
                 for (size_t e = 0; e < g.pending_dw.size();) {  // gradients this group was to collect (none in a model whose layers all join the window)
                     const PendingDW p = g.pending_dw[e];
                     if (std::find(collect_dw.begin(), collect_dw.end(), p.weight) == collect_dw.end()) {
@@ -1179,7 +1185,7 @@ size_t Graph::matmul_trans_b(size_t a, size_t b) {
         Storage& ga = g.grad_for_write(a, &acc);
         g.check(eisen_hip_gemm(g.ctx(), go.ptr, g.compute_data(b).ptr, ga.ptr, go.dtype, ga.dtype, 0, 0, M, K, N, acc), "matmul_trans_b backward dA");
         const void* xa = g.compute_data(a).ptr;
-        if (g.window_take(b, go.ptr, xa, go.dtype, M, N, K) || g.leave_dw(b, go.ptr, xa, go.dtype, M, N, K)) return;
+        if (g.window_take(b, go.ptr, xa, go.dtype, M, N, K) || g.leave_dw({{b, go.ptr, xa, M, N, K, go.dtype}})) return;
         g.run_beside(g.at(b).is_param && g.beside_fits(N, K), {go.ptr, xa}, {b}, [&]() {
             int accb = 0;
             Storage& gb = g.grad_for_write(b, &accb);

@@ -242,8 +242,9 @@ class Graph {
     };
     std::vector<LeftDW> left_dw_;
     bool left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out);
-    // left until later when left_fits (until the node's last product, after which no more come, when weight gradients keep to the tape); false: the caller forms the product now
-    bool leave_dw(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out, bool more = false);
+    // the products of a node, left until later (formed here, when weight gradients keep to the tape); false: the caller forms them now
+    bool leave_dw(const std::vector<LeftDW>& node);
+    void form_dw(std::vector<LeftDW> list);
     // before anything else touches the gradient of a weight
     void settle_dw(size_t weight);
     eisen_ctx* ctx_;

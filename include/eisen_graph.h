@@ -61,8 +61,8 @@ int eisen_graph_set_weight_gradient_window(eisen_graph* g, size_t backward_passe
  * alone or few over many tokens, as a launch each; their operands are kept that long.  What that launch does not take in bf16 (sides that are no multiples of 8 or below 32, more than
  * 16384 rows) runs on the context's side stream beside the chain of input gradients, the operands kept until the pass has ended and the main stream has waited
  * for the side stream.
- * 0: in tape order on the one stream, as in the reference (src/graph/mod.rs:670-796); no operands are kept.  The kernels and bits are those of 1 but where one
- * product alone, or few over many tokens, run as a launch each and more of them would share one. */
+ * 0: in tape order on the one stream, as in the reference (src/graph/mod.rs:670-796), a launch for each node's; no operands are kept past their block.  Over few tokens the bits
+ * of bf16 layers are those of 1; over many, and in f32, a node's launch may add up in another order. */
 int eisen_graph_set_weight_gradients_beside(eisen_graph* g, int on);
 int eisen_graph_flush_weight_gradients(eisen_graph* g);
 int eisen_graph_restore_save_point_keep(eisen_graph* g, size_t save_point, size_t keep, size_t* new_id_out);

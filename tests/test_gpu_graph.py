@@ -396,6 +396,30 @@ def test_weight_gradients_of_few_layers_over_many_tokens_are_launches_of_their_o
     g.close()
 
 
+@pytest.mark.parametrize("precision,rows,launch_of_the_pass", [(G.BF16_MIXED, 512, True), (G.BF16_MIXED, 8192, False), (G.FP32, 512, False)])
+def test_weight_gradients_kept_to_the_tape_take_the_faster_launch(ctx, precision, rows, launch_of_the_pass):
+    # over many tokens, and in f32, the nodes' own launches; the bound is that of f32 sums in another order
+    cfg = dict(vocab=512, hidden=256, heads=4, kv_heads=2, ffn=512, layers=1, tie=False)
+    x, y = gen.lm_batch(975, rows // 128, 128, cfg["vocab"], "zipf")
+    results = []
+    for beside in (False, True):
+        g = G.Graph(ctx, precision)
+        lm = G.TransformerLM(g, **cfg)
+        for pid, (_, w) in enumerate(gen.lm_weights(36, **cfg)):
+            g.load_tensor_data(pid, w)
+        g.mark_params()
+        g.set_weight_gradients_beside(beside)
+        ctx.profile_start()
+        lm.micro_step(x, y)
+        names = list(ctx.profile_stop())
+        assert any(n.endswith("_layers") for n in names) == (beside or launch_of_the_pass), names
+        results.append([g.sync_grad_to_cpu(p).astype(np.float64) for p in lm.params()])
+        g.close()
+    for a, b in zip(*results):
+        assert a.any() and np.linalg.norm(a - b) <= 1e-6 * np.linalg.norm(a)
+        assert np.array_equal(a, b) or not launch_of_the_pass
+
+
 @pytest.mark.parametrize("tie,checkpointing", [(True, False), (False, False), (True, True)], ids=["tied", "untied", "tied-recompute"])
 def test_weight_gradients_beside_the_chain_give_the_same_bits(ctx, tie, checkpointing):
     # Graph::set_weight_gradients_beside (the default): the weight-gradient GEMMs of narrow layers run on the side stream
