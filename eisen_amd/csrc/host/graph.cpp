@@ -421,10 +421,15 @@ void Graph::flush_weight_gradients(size_t only_weight) {
 // contractions that need no parts.  Layers of one pass, a launch each / one launch, us: 12 of 1024 x 1024 over 4096 tokens 307 / 164, 6 of 1024 x 3096 (200 tiles) x 1024 115 / 97, x 4096 306 / 283,
 // 4 of 1536 x 1024 x 8192 175 / 145.  Beyond: 3 of 1024 x 4096 (256 tiles) x 4096 137 / 159, 4 of 1000 x 4000 (256) x 4000 211 / 225, 4 of 1280 x 5000 (400) x 4096
 // 307 / 367, x 1024 106 / 121.
+// Where they could run beside the chain of input gradients instead, large ones do: the launches of the chain leave CUs idle that one launch at the end does not get back.  Steps of three layers, all left / the
+// large ones beside / all beside, us: hidden 960, ffn 3656 (232 tiles), 8192 tokens 4197 / 3903 / 3967, 2048 tokens 1600 / 1541 / 1587; 1024, 3096 (200) over 2470 1846 / 1726 / 1805; 640, 2560 (100) over 4096
+// 1501 / 1446 / 1452; 768, 2048 (96) over 8192 2560 / 2413 / 2491; but 896, 3584 (196) over 1024 946 / 948 / 1073.  64 tiles and less are behind beside the chain for longer: 1024, 4096, 8192 tokens,
+// projections of 64 tiles left / beside 3842 / 4023; and so is a side below 384: the ~14 M model's head of 8192 x 256 over 8192 1556 / 1566.
 bool Graph::left_fits(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out) {
     if (backward_root_ == (size_t)-1 || rows == 0 || rows > 16384) return false;
     if (dtype == EISEN_BF16 ? in % 8 || out % 8 || in < 32 || out < 32 : in % 4 || out % 4) return false;
-    if (((in + 127) / 128) * ((out + 127) / 128) >= 256u) return false;
+    const size_t tiles = ((in + 127) / 128) * ((out + 127) / 128);
+    if (tiles >= 256u || (beside_fits(in, out) && std::min(in, out) >= 384 && tiles * rows > (tiles <= 64 ? 600000u : 350000u))) return false;
     if ((uintptr_t)x % 16 || (uintptr_t)dy % 16) return false;
     const Tensor& tw = at(weight);
     return tw.is_param && tw.grad.dtype == EISEN_F32 && tw.size() == in * out;

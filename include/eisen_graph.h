@@ -59,7 +59,7 @@ int eisen_graph_set_weight_gradient_window(eisen_graph* g, size_t backward_passe
 /* When the weight gradients of layers of fewer 128 x 128 tiles than the chip has CUs are formed, without a window.
  * 1 (the default): when the backward pass ends, or something else touches the gradient of one of their weights, as one launch (eisen_hip_gemm_weight_gradients), or, one
  * alone or few over many tokens, as a launch each; their operands are kept that long.  What that launch does not take in bf16 (sides that are no multiples of 8 or below 32, more than
- * 16384 rows) runs on the context's side stream beside the chain of input gradients, the operands kept until the pass has ended and the main stream has waited
+ * 16384 rows), or would take without filling the CUs that the chain leaves idle (many tiles over many rows), runs on the context's side stream beside the chain of input gradients, the operands kept until the pass has ended and the main stream has waited
  * for the side stream.
  * 0: in tape order on the one stream, as in the reference (src/graph/mod.rs:670-796), a launch for each node's; no operands are kept past their block.  Over few tokens the bits
  * of bf16 layers are those of 1; over many, and in f32, a node's launch may add up in another order. */

@@ -420,6 +420,28 @@ def test_weight_gradients_kept_to_the_tape_take_the_faster_launch(ctx, precision
         assert np.array_equal(a, b) or not launch_of_the_pass
 
 
+@pytest.mark.parametrize("rows,left", [(4608, True), (5120, False)])
+def test_large_weight_gradients_run_beside_the_chain(ctx, rows, left):
+    # two weights of 72 tiles of 128 x 128: left for the pass's launch up to 350,000 tiles x rows.  Against those of the tape: f32 sums of the same operands in another order
+    w0 = [gen.normal(1010, (1024, 1152), 2.0 ** -5), gen.normal(1011, (1152, 1024), 2.0 ** -5)]
+    x0, t0 = gen.normal(1012, (rows, 1024)), gen.uniform_ids(1013, (rows,), 1024)
+    results = []
+    for beside in (False, True):
+        g = G.Graph(ctx, G.BF16_MIXED)
+        g.set_weight_gradients_beside(beside)
+        ws = [g.alloc(w.shape, w) for w in w0]
+        g.mark_params()
+        loss = g.cross_entropy(g.matmul(g.matmul(g.input(x0), ws[0]), ws[1]), t0)
+        ctx.profile_start()
+        g.backward(loss)
+        names = list(ctx.profile_stop())
+        assert not beside or any(n.endswith("_layers") for n in names) == left, names
+        results.append([g.sync_grad_to_cpu(w).astype(np.float64) for w in ws])
+        g.close()
+    for a, b in zip(*results):
+        assert a.any() and np.linalg.norm(a - b) <= 1e-6 * np.linalg.norm(a)
+
+
 @pytest.mark.parametrize("tie,checkpointing", [(True, False), (False, False), (True, True)], ids=["tied", "untied", "tied-recompute"])
 def test_weight_gradients_beside_the_chain_give_the_same_bits(ctx, tie, checkpointing):
     # Graph::set_weight_gradients_beside (the default): the weight-gradient GEMMs of narrow layers run on the side stream
