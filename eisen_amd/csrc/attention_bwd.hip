@@ -371,18 +371,18 @@ bool eisen_attention_dkv32_supports(const AttnArgs& a) {
 
 // Whether a result lies over an operand, or dQ is where dK or dV is.  In two launches dQ may take the place of O, and dK and dV that of K, V or O, which nobody reads any more by
 // then; in one they are still being read.
-static bool writes_over_operand(const AttnArgs& a) {
+bool eisen_attention_writes_over_operand(const AttnArgs& a, size_t element) {
     struct Range {
         const void* from;
         size_t bytes;
     };
-    auto range = [&](const void* p, size_t element, int heads, long long sb, long long ss, long long sh) {
+    auto range = [&](const void* p, int heads, long long sb, long long ss, long long sh) {
         long long lowest = 0, end = a.hd;
         for (const long long reach : {(a.B - 1) * sb, (a.S - 1) * ss, (heads - 1) * sh}) (reach < 0 ? lowest : end) += reach;
         return Range{static_cast<const char*>(p) + lowest * (long long)element, (size_t)(end - lowest) * element};
     };
-    auto q = [&](const void* p) { return range(p, 2, a.Hq, a.q_sb, a.q_ss, a.q_sh); };
-    auto k = [&](const void* p) { return range(p, 2, a.Hkv, a.k_sb, a.k_ss, a.k_sh); };
+    auto q = [&](const void* p) { return range(p, a.Hq, a.q_sb, a.q_ss, a.q_sh); };
+    auto k = [&](const void* p) { return range(p, a.Hkv, a.k_sb, a.k_ss, a.k_sh); };
     for (const Range& out : {q(a.dQ), k(a.dK), k(a.dV)})
         for (const Range& in : {q(a.Q), k(a.K), k(a.V), q(a.O), q(a.dO), Range{a.LSE, sizeof(float) * a.B * a.Hq * a.S}})
             if (eisen_ranges_meet(out.from, out.bytes, in.from, in.bytes)) return true;
@@ -400,7 +400,7 @@ bool eisen_attention_bwd_short_supports(const AttnArgs& a, int dq_blocks) {
     const int n_qt = (a.S + 31) / 32;
     const int most = a.G <= 2 ? kOwnTiles : a.G <= 4 && a.hd != 64 ? 32 : 16;
     const long long blocks = dq_blocks + (long long)(n_qt + 1) / 2 * a.Hkv * a.B;
-    return a.G * n_qt <= most && blocks <= (a.hd <= 64 ? 512 : 256) && a.ablation == kAblNone && eisen_attention_dkv32_supports(a) && !writes_over_operand(a);
+    return a.G * n_qt <= most && blocks <= (a.hd <= 64 ? 512 : 256) && a.ablation == kAblNone && eisen_attention_dkv32_supports(a) && !eisen_attention_writes_over_operand(a, 2);
 }
 
 void eisen_attention_launch_bwd_short(eisen_ctx* ctx, AttnArgs a, int gw, int dq_blocks) {

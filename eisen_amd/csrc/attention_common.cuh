@@ -55,6 +55,9 @@ void eisen_attention_launch_dkv32(eisen_ctx* ctx, AttnArgs a);
 bool eisen_attention_bwd_short_supports(const AttnArgs& a, int dq_blocks);
 void eisen_attention_launch_bwd_short(eisen_ctx* ctx, AttnArgs a, int gw, int dq_blocks);
 
+// whether a result of the backward lies over one of its operands, of `element` bytes each (attention_bwd.hip)
+bool eisen_attention_writes_over_operand(const AttnArgs& a, size_t element);
+
 // attention_f32.hip: f32 operands, head_dim up to 128
 bool eisen_attention_f32_mfma_supports(const AttnArgs& a);
 void eisen_attention_launch_f32(eisen_ctx* ctx, const AttnArgs& a, bool backward);

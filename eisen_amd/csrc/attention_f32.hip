@@ -21,39 +21,54 @@ namespace {
 
 struct __attribute__((packed, aligned(4))) Quad { float v[4]; };
 
-// This lane's share of one row: d = 8 kk + 4 h + 0..3.  FULL: head_dim is 8 * K8.
+// Rows `stride` apart (|stride| < 2^24).  A load takes the tile's origin in scalar registers and an unsigned 32-bit byte offset per
+// lane, so that the loops spend few vector instructions on addresses (64-bit sums per lane and load had been a third of those of a
+// dK/dV item).  A negative stride moves the origin to the lowest of 32 rows.
+struct RowStride {
+    long long stride;
+    int low;  // elements
+    __device__ __forceinline__ explicit RowStride(long long s) : stride(s), low(min(0, 31 * (int)s)) {}
+};
+template <class T>
+__device__ __forceinline__ const T& at_bytes(const float* origin, unsigned bytes) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(origin) + bytes);
+}
+// This lane's share of row first_row + c (the last row, past the end): d = 8 kk + 4 h + 0..3.  FULL: head_dim is 8 * K8.
 template <int K8, bool FULL>
-__device__ __forceinline__ void load_row(const float* row, int hd, int h, float (&f)[K8][4]) {
+__device__ __forceinline__ void load_row(const float* base, const RowStride& rs, int first_row, int rows, int hd, int c, int h, float (&f)[K8][4]) {
+    const float* origin = base + first_row * rs.stride + rs.low;
+    const unsigned off = (unsigned)(min(c, rows - 1 - first_row) * (int)rs.stride - rs.low) * 4u + 16u * h;
 #pragma unroll
     for (int kk = 0; kk < K8; kk++) {
         const int d = 8 * kk + 4 * h;
         if (FULL || d + 4 <= hd) {
-            const Quad q = *reinterpret_cast<const Quad*>(row + d);
+            const Quad q = at_bytes<Quad>(origin + 8 * kk, off);
 #pragma unroll
             for (int j = 0; j < 4; j++) f[kk][j] = q.v[j];
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) f[kk][j] = d + j < hd ? row[d + j] : 0.f;
+            for (int j = 0; j < 4; j++) f[kk][j] = d + j < hd ? at_bytes<float>(origin + 8 * kk + j, off) : 0.f;
         }
     }
 }
-// Column d = 32 dt + lane % 32 of the 32 rows at first_row, in the order of a score tile's registers.  Rows past the end
+// Columns d = 32 dt + lane % 32 of the 32 rows at first_row, in the order of a score tile's registers.  Rows past the end
 // repeat the last one (their weight is zero).
 template <int K8, bool FULL>
-__device__ __forceinline__ void load_column(const float* base, long long stride, int first_row, int rows, int hd, int c, int h, int dt, float (&f)[16]) {
-    const bool whole = first_row + 32 <= rows;
-    const int d = 32 * dt + c;
+__device__ __forceinline__ void load_column(const float* base, const RowStride& rs, int first_row, int rows, int hd, int c, int h, int dt, float (&f)[16]) {
+    const float* origin = base + first_row * rs.stride + rs.low + 32 * dt;
+    const int d = 32 * dt + c, last = rows - 1 - first_row, stride = (int)rs.stride;
     const bool in = FULL ? (32 * dt + 32 <= 8 * K8 || d < 8 * K8) : d < hd;
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const int r = first_row + acc_row(v, h);
-        f[v] = in ? base[(long long)(whole ? r : min(r, rows - 1)) * stride + d] : 0.f;
+    for (int v = 0; v < 16; v++) {  // the products are scalar
+        const int r0 = min(acc_row(v, 0), last) * stride, r1 = min(acc_row(v, 1), last) * stride;
+        const unsigned off = (unsigned)((h ? r1 : r0) - rs.low + c) * 4u;
+        f[v] = in ? at_bytes<float>(origin, off) : 0.f;
     }
 }
 template <int K8, int DT, bool FULL>
-__device__ __forceinline__ void load_columns(const float* base, long long stride, int first_row, int rows, int hd, int c, int h, float (&f)[DT][16]) {
+__device__ __forceinline__ void load_columns(const float* base, const RowStride& rs, int first_row, int rows, int hd, int c, int h, float (&f)[DT][16]) {
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++) load_column<K8, FULL>(base, stride, first_row, rows, hd, c, h, dt, f[dt]);
+    for (int dt = 0; dt < DT; dt++) load_column<K8, FULL>(base, rs, first_row, rows, hd, c, h, dt, f[dt]);
 }
 // registers of a transposed result tile -> row `row` (d = 32 dt + 8 vg + 4 h + 0..3)
 template <int K8, bool FULL>
@@ -90,7 +105,7 @@ __device__ __forceinline__ f32x16 row_product(const float (&a)[K8][4], const flo
 // operand, and behind the loop, where the registers are free, put_back_nonfinite() gives them to the lanes that do see their
 // row.  The look is one instruction per value: of V itself in the forward pass, of the first products' 16 results in the
 // backward pass (a row of Q, K or dO that is not finite makes them not finite).  16 x 83, one head of 64, forward and
-// backward: 8.6 + 27.2 us without the look, 8.7 + 27.9 with it, 9.0 + 30.1 with every operand of such tiles cleaned.
+// backward in three launches: 8.6 + 27.2 us without the look, 8.7 + 27.9 with it, 9.0 + 30.1 with every operand of such tiles cleaned.
 __device__ __forceinline__ float look(float x, float seen) { return fmaf(x, 0.f, seen); }  // stays 0, or becomes NaN for good
 __device__ __forceinline__ bool any_nan(float seen) { return __builtin_amdgcn_ballot_w64(seen != seen) != 0; }
 template <int DT>
@@ -108,7 +123,7 @@ __device__ __forceinline__ bool take_out_nonfinite(float (&col)[DT][16]) {  // w
 }
 // +-Inf for the weights P of V and dO, which are not negative (POSITIVE), NaN for the others and for NaN.
 template <bool POSITIVE, int K8, int DT, bool FULL, class Visible>
-__device__ __forceinline__ void put_back_nonfinite(const float* base, long long stride, int first_row, int rows, int hd, int c, int h, f32x16 (&acc)[DT],
+__device__ __forceinline__ void put_back_nonfinite(const float* base, const RowStride& stride, int first_row, int rows, int hd, int c, int h, f32x16 (&acc)[DT],
                                                    Visible visible) {
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) {
@@ -130,40 +145,43 @@ __device__ __forceinline__ void put_back_nonfinite(const float* base, long long 
 
 // workgroup -> (query block or key block, head, batch): heads and batches fastest, the longest causal blocks first
 struct RowBlock { int blk, head, b; };
-__device__ __forceinline__ RowBlock decode_block(int heads, int B, int n_blk, bool descending) {
-    const int per = heads * B, id = blockIdx.x;
+__device__ __forceinline__ RowBlock decode_block(int id, int heads, int B, int n_blk, bool descending) {
+    const int per = heads * B;
     const int i = id / per, r = id % per;
     return RowBlock{descending ? n_blk - 1 - i : i, r % heads, r / heads};
 }
 
-constexpr int kMaxKeyWaves = 4;
+// Waves of a workgroup, at most: two to a SIMD where their registers allow it.
+template <int K8>
+constexpr int kMaxWaves = K8 <= 4 ? 8 : 4;
 
 template <int K8, bool FULL>
-__global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_fwd_kernel(AttnArgs a) {
+__global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_fwd_kernel(AttnArgs a) {
     constexpr int DT = (K8 + 3) / 4;
-    __shared__ float meet[kMaxKeyWaves - 1][DT * 16 * 64 + 128];
+    __shared__ float meet[kMaxWaves<K8> - 1][DT * 16 * 64 + 128];
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    const RowBlock rb = decode_block(a.Hq, a.B, (a.S + 31) / 32, a.causal);
+    const RowBlock rb = decode_block(blockIdx.x, a.Hq, a.B, (a.S + 31) / 32, a.causal);
     const int q0 = rb.blk * 32, q = min(q0 + c, a.S - 1);
     const long long qoff = rb.b * a.q_sb + rb.head * a.q_sh + (long long)q * a.q_ss;
     const long long kvoff = rb.b * a.k_sb + (rb.head / a.G) * a.k_sh;
     const float* Kp = static_cast<const float*>(a.K) + kvoff;
     const float* Vp = static_cast<const float*>(a.V) + kvoff;
+    const RowStride qs(a.q_ss), ks(a.k_ss);
     float qf[K8][4], kf[K8][4];
-    load_row<K8, FULL>(static_cast<const float*>(a.Q) + qoff, a.hd, h, qf);
+    load_row<K8, FULL>(static_cast<const float*>(a.Q) + rb.b * a.q_sb + rb.head * a.q_sh, qs, q0, a.S, a.hd, c, h, qf);
     f32x16 o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) o[dt] = zero16();
     float m = -INFINITY, l = 0.f;  // m in units of log2
     int odd_at = -1;               // first row of the tile with masked pairs, if it holds a value that is not finite
     const int n_kt = a.causal ? min(rb.blk + 1, (a.S + 31) / 32) : (a.S + 31) / 32;
-    if (wave < n_kt) load_row<K8, FULL>(Kp + (long long)min(wave * 32 + c, a.S - 1) * a.k_ss, a.hd, h, kf);
+    if (wave < n_kt) load_row<K8, FULL>(Kp, ks, wave * 32, a.S, a.hd, c, h, kf);
     for (int kt = wave; kt < n_kt; kt += nw) {
         float vc[DT][16];
-        load_columns<K8, DT, FULL>(Vp, a.k_ss, kt * 32, a.S, a.hd, c, h, vc);
+        load_columns<K8, DT, FULL>(Vp, ks, kt * 32, a.S, a.hd, c, h, vc);
         f32x16 s = row_product<K8>(kf, qf, zero16());
-        if (kt + nw < n_kt) load_row<K8, FULL>(Kp + (long long)min((kt + nw) * 32 + c, a.S - 1) * a.k_ss, a.hd, h, kf);
+        if (kt + nw < n_kt) load_row<K8, FULL>(Kp, ks, (kt + nw) * 32, a.S, a.hd, c, h, kf);
         const int k0 = kt * 32, lim = (a.causal ? q : a.S - 1) - k0;  // tile rows above lim are masked
         if (k0 + 32 > a.S || (a.causal && k0 + 31 > q0)) {
 #pragma unroll
@@ -205,7 +223,7 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_fwd_kernel(AttnArg
     }
     if (odd_at >= 0) {
         const int lim = (a.causal ? q : a.S - 1) - odd_at;
-        put_back_nonfinite<true, K8, DT, FULL>(Vp, a.k_ss, odd_at, a.S, a.hd, c, h, o, [&](int v) { return acc_row(v, h) <= lim; });
+        put_back_nonfinite<true, K8, DT, FULL>(Vp, ks, odd_at, a.S, a.hd, c, h, o, [&](int v) { return acc_row(v, h) <= lim; });
     }
     l += __shfl_xor(l, 32, 64);
     if (nw > 1) {  // the waves' keys are disjoint: (m, l, O) of each, added in wave order against the common maximum
@@ -253,46 +271,53 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_fwd_kernel(AttnArg
     if (h == 0) a.LSE[((long long)rb.b * a.Hq + rb.head) * a.S + q] = (m + log2f(l)) * kLn2;
 }
 
-// dQ^T = scale K^T dS^T; also writes D = rowsum(dO o O) for the dK/dV kernel
-template <int K8, bool FULL>
-__global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_bwd_dq_kernel(AttnArgs a) {
+// D = rowsum(dO o O) of this lane's row, from its two lanes' shares
+template <int K8>
+__device__ __forceinline__ float row_dot(const float (&x)[K8][4], const float (&y)[K8][4]) {
+    float d = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < K8; kk++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) d += x[kk][j] * y[kk][j];
+    return d + __shfl_xor(d, 32, 64);
+}
+
+// dQ^T = scale K^T dS^T of query block `id` (none, past the last: the wave only meets the others at the barrier), by nw waves of
+// which this is the `wave`-th; WRITE_D: also leaves D = rowsum(dO o O) for a dK/dV launch that follows.
+template <int K8, bool FULL, bool WRITE_D>
+__device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int nw, float* meet) {
     constexpr int DT = (K8 + 3) / 4;
-    __shared__ float meet[kMaxKeyWaves - 1][DT * 16 * 64];
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    const RowBlock rb = decode_block(a.Hq, a.B, (a.S + 31) / 32, a.causal);
+    const int n_t = (a.S + 31) / 32;
+    const bool exists = id < n_t * a.Hq * a.B;
+    const RowBlock rb = decode_block(exists ? id : 0, a.Hq, a.B, n_t, a.causal);
     const int q0 = rb.blk * 32, q = min(q0 + c, a.S - 1);
-    const long long qoff = rb.b * a.q_sb + rb.head * a.q_sh + (long long)q * a.q_ss;
+    const long long qoff = rb.b * a.q_sb + rb.head * a.q_sh;
     const long long kvoff = rb.b * a.k_sb + (rb.head / a.G) * a.k_sh;
     const long long stat = ((long long)rb.b * a.Hq + rb.head) * a.S + q;
     const float* Kp = static_cast<const float*>(a.K) + kvoff;
     const float* Vp = static_cast<const float*>(a.V) + kvoff;
+    const RowStride qs(a.q_ss), ks(a.k_ss);
     float qf[K8][4], dof[K8][4], kf[K8][4], vf[K8][4];
-    load_row<K8, FULL>(static_cast<const float*>(a.dO) + qoff, a.hd, h, dof);
-    load_row<K8, FULL>(static_cast<const float*>(a.O) + qoff, a.hd, h, qf);
-    float Dq = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < K8; kk++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) Dq += dof[kk][j] * qf[kk][j];
-    Dq += __shfl_xor(Dq, 32, 64);
-    load_row<K8, FULL>(static_cast<const float*>(a.Q) + qoff, a.hd, h, qf);
+    load_row<K8, FULL>(static_cast<const float*>(a.dO) + qoff, qs, q0, a.S, a.hd, c, h, dof);
+    load_row<K8, FULL>(static_cast<const float*>(a.O) + qoff, qs, q0, a.S, a.hd, c, h, qf);
+    const float Dq = row_dot<K8>(dof, qf);
+    load_row<K8, FULL>(static_cast<const float*>(a.Q) + qoff, qs, q0, a.S, a.hd, c, h, qf);
     const float lse2 = a.LSE[stat] * kLog2e;
-    if (wave == 0 && h == 0 && q0 + c < a.S) a.D[stat] = Dq;
+    if (WRITE_D && exists && wave == 0 && h == 0 && q0 + c < a.S) a.D[stat] = Dq;
     f32x16 dq[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) dq[dt] = zero16();
     int odd_at = -1;  // see the forward kernel
-    const int n_kt = a.causal ? min(rb.blk + 1, (a.S + 31) / 32) : (a.S + 31) / 32;
+    const int n_kt = !exists ? 0 : a.causal ? min(rb.blk + 1, n_t) : n_t;
     auto fetch = [&](int kt) {
-        const long long at = (long long)min(kt * 32 + c, a.S - 1) * a.k_ss;
-        load_row<K8, FULL>(Kp + at, a.hd, h, kf);
-        load_row<K8, FULL>(Vp + at, a.hd, h, vf);
+        load_row<K8, FULL>(Kp, ks, kt * 32, a.S, a.hd, c, h, kf);
+        load_row<K8, FULL>(Vp, ks, kt * 32, a.S, a.hd, c, h, vf);
     };
     if (wave < n_kt) fetch(wave);
     for (int kt = wave; kt < n_kt; kt += nw) {
         float kc[DT][16];
-        load_columns<K8, DT, FULL>(Kp, a.k_ss, kt * 32, a.S, a.hd, c, h, kc);
+        load_columns<K8, DT, FULL>(Kp, ks, kt * 32, a.S, a.hd, c, h, kc);
         f32x16 s = row_product<K8>(kf, qf, zero16());
         const f32x16 dp = row_product<K8>(vf, dof, zero16());
         if (kt + nw < n_kt) fetch(kt + nw);
@@ -321,14 +346,14 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_bwd_dq_kernel(Attn
     }
     if (odd_at >= 0) {
         const int lim = (a.causal ? q : a.S - 1) - odd_at;
-        put_back_nonfinite<false, K8, DT, FULL>(Kp, a.k_ss, odd_at, a.S, a.hd, c, h, dq, [&](int v) { return acc_row(v, h) <= lim; });
+        put_back_nonfinite<false, K8, DT, FULL>(Kp, ks, odd_at, a.S, a.hd, c, h, dq, [&](int v) { return acc_row(v, h) <= lim; });
     }
     if (nw > 1) {
         if (wave > 0) {
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) meet[wave - 1][(dt * 16 + v) * 64 + lane] = dq[dt][v];
+                for (int v = 0; v < 16; v++) meet[(((wave - 1) * DT + dt) * 16 + v) * 64 + lane] = dq[dt][v];
         }
         __syncthreads();
         if (wave > 0) return;
@@ -336,10 +361,10 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_bwd_dq_kernel(Attn
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) dq[dt][v] += meet[w][(dt * 16 + v) * 64 + lane];
+                for (int v = 0; v < 16; v++) dq[dt][v] += meet[((w * DT + dt) * 16 + v) * 64 + lane];
     }
-    if (q0 + c >= a.S) return;
-    float* dQp = static_cast<float*>(a.dQ) + qoff;
+    if (!exists || q0 + c >= a.S) return;
+    float* dQp = static_cast<float*>(a.dQ) + qoff + (long long)q * a.q_ss;
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -357,20 +382,23 @@ __global__ __launch_bounds__(64 * kMaxKeyWaves) void attn_f32_bwd_dq_kernel(Attn
         }
 }
 
-// dK^T = scale Q^T dS, dV^T = dO^T P, summed over the query heads of the group (ascending within a wave, then over the waves)
-template <int K8, bool FULL>
-__global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(AttnArgs a) {
-    constexpr int DT = (K8 + 3) / 4, MAXW = K8 <= 4 ? 8 : 4;
-    __shared__ float meet[2][MAXW][16 * 64];
+// dK^T = scale Q^T dS, dV^T = dO^T P of key block `id`, summed over the query heads of the group (ascending within a wave, then
+// over the waves).  OWN_D: D is formed from the rows of O here, as the dQ pass forms it, and not read.  The rows and statistics
+// of an item are requested under the products of the one before, its columns under its own first products: a lane loads the
+// statistics of the row it holds, and the lanes that need them ask it.
+template <int K8, bool FULL, bool OWN_D>
+__device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int nw, float* meet) {
+    constexpr int DT = (K8 + 3) / 4;
+    constexpr bool AHEAD = K8 <= 8;  // (above, the registers are all taken)
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int n_t = (a.S + 31) / 32;
-    const RowBlock rb = decode_block(a.Hkv, a.B, n_t, false);  // ascending: the first keys see the most queries
+    const RowBlock rb = decode_block(id, a.Hkv, a.B, n_t, false);  // ascending: the first keys see the most queries
     const int k0 = rb.blk * 32, key = min(k0 + c, a.S - 1);
-    const long long koff = rb.b * a.k_sb + rb.head * a.k_sh + (long long)key * a.k_ss;
+    const long long kvoff = rb.b * a.k_sb + rb.head * a.k_sh;
+    const RowStride qs(a.q_ss), ks(a.k_ss);
     float kf[K8][4], vf[K8][4];
-    load_row<K8, FULL>(static_cast<const float*>(a.K) + koff, a.hd, h, kf);
-    load_row<K8, FULL>(static_cast<const float*>(a.V) + koff, a.hd, h, vf);
+    load_row<K8, FULL>(static_cast<const float*>(a.K) + kvoff, ks, k0, a.S, a.hd, c, h, kf);
+    load_row<K8, FULL>(static_cast<const float*>(a.V) + kvoff, ks, k0, a.S, a.hd, c, h, vf);
     f32x16 dk[DT], dv[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) dk[dt] = dv[dt] = zero16();
@@ -380,27 +408,44 @@ __global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(A
         const int r = q0 + acc_row(v, h);
         return r < a.S && !(a.causal && k0 + c > r);
     };
+    float qr[K8][4], dor[K8][4], orow[K8][4], lse_row = 0.f, d_row = 0.f;
+    auto fetch = [&](int item) {
+        const int hq = rb.head * a.G + item / per_head, q0 = (qt_start + item % per_head) * 32;
+        const long long base = rb.b * a.q_sb + hq * a.q_sh, stat = ((long long)rb.b * a.Hq + hq) * a.S + q0;
+        load_row<K8, FULL>(static_cast<const float*>(a.dO) + base, qs, q0, a.S, a.hd, c, h, dor);
+        if (OWN_D) load_row<K8, FULL>(static_cast<const float*>(a.O) + base, qs, q0, a.S, a.hd, c, h, orow);
+        if (OWN_D && !AHEAD) {
+            d_row = row_dot<K8>(dor, orow);
+            asm volatile("" : "+v"(d_row)::"memory");  // the rows of O are done with before the other operands arrive
+        }
+        load_row<K8, FULL>(static_cast<const float*>(a.Q) + base, qs, q0, a.S, a.hd, c, h, qr);
+        const int r = min(c, a.S - 1 - q0);
+        lse_row = a.LSE[stat + r];
+        if (!OWN_D) d_row = a.D[stat + r];
+    };
     bool odd = false;
+    if (AHEAD && wave < n_items) fetch(wave);
     for (int item = wave; item < n_items; item += nw) {
         const int hq = rb.head * a.G + item / per_head, q0 = (qt_start + item % per_head) * 32;
         const long long base = rb.b * a.q_sb + hq * a.q_sh;
-        const float* Qp = static_cast<const float*>(a.Q) + base;
-        const float* dOp = static_cast<const float*>(a.dO) + base;
-        const long long stat = ((long long)rb.b * a.Hq + hq) * a.S;
-        float qr[K8][4], dor[K8][4], qc[DT][16], doc[DT][16], lse2[16], D[16];
-        const long long at = (long long)min(q0 + c, a.S - 1) * a.q_ss;
-        load_row<K8, FULL>(Qp + at, a.hd, h, qr);
-        load_row<K8, FULL>(dOp + at, a.hd, h, dor);
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = q0 + acc_row(v, h);
-            lse2[v] = r < a.S ? a.LSE[stat + r] : INFINITY;  // a query past the end has no weight
-            D[v] = r < a.S ? a.D[stat + r] : 0.f;
-        }
-        load_columns<K8, DT, FULL>(dOp, a.q_ss, q0, a.S, a.hd, c, h, doc);
-        load_columns<K8, DT, FULL>(Qp, a.q_ss, q0, a.S, a.hd, c, h, qc);
+        if (!AHEAD) fetch(item);
+        float qc[DT][16], doc[DT][16];
+        auto columns_of_do = [&] { load_columns<K8, DT, FULL>(static_cast<const float*>(a.dO) + base, qs, q0, a.S, a.hd, c, h, doc); };
+        auto columns_of_q = [&] { load_columns<K8, DT, FULL>(static_cast<const float*>(a.Q) + base, qs, q0, a.S, a.hd, c, h, qc); };
+        columns_of_do();
+        if (AHEAD) columns_of_q();
         f32x16 s = row_product<K8>(qr, kf, zero16());
+        if (!AHEAD) {  // the columns of Q take the registers of its rows, which the products above have read
+            asm volatile("" : "+v"(s)::"memory");
+            columns_of_q();
+        }
         f32x16 dp = row_product<K8>(dor, vf, zero16());
+        const bool in = q0 + c < a.S;  // a query past the end has no weight
+        const float d_here = OWN_D && AHEAD ? row_dot<K8>(dor, orow) : d_row, l_here = lse_row * kLog2e;
+        const float l_own = in ? l_here : INFINITY, d_own = in ? d_here : 0.f;
+        auto lse2 = [&](int v) { return __shfl(l_own, acc_row(v, h), 64); };
+        auto D = [&](int v) { return __shfl(d_own, acc_row(v, h), 64); };
+        if (AHEAD && item + nw < n_items) fetch(item + nw);
         // Up to head size 96 the tile is looked at before its operands are touched; above, where the look's registers would go to
         // scratch (1 x 800, 8 heads of 128: backward 411 -> 421 us), every such tile is cleaned.
         constexpr bool kLook = K8 <= 12;
@@ -408,18 +453,18 @@ __global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(A
         if (kLook && masked_tile(q0)) {
             float seen = 0.f;
 #pragma unroll
-            for (int v = 0; v < 16; v++) seen = look(dp[v] - D[v], look(s[v], seen));
+            for (int v = 0; v < 16; v++) seen = look(dp[v] - D(v), look(s[v], seen));
             odd_here = any_nan(seen);
         }
 #pragma unroll
-        for (int v = 0; v < 16; v++) s[v] = fast_exp2(fmaf(s[v], a.scale_log2e, -lse2[v] * kLog2e));
+        for (int v = 0; v < 16; v++) s[v] = fast_exp2(fmaf(s[v], a.scale_log2e, -lse2(v)));
         if (kLook && a.causal && q0 < k0 + 31) {
 #pragma unroll
             for (int v = 0; v < 16; v++)
                 if (k0 + c > q0 + acc_row(v, h)) s[v] = 0.f;
         }
 #pragma unroll
-        for (int v = 0; v < 16; v++) dp[v] = s[v] * (dp[v] - D[v]) * a.scale;
+        for (int v = 0; v < 16; v++) dp[v] = s[v] * (dp[v] - D(v)) * a.scale;
         if (kLook ? odd_here : masked_tile(q0)) {
 #pragma unroll
             for (int v = 0; v < 16; v++)
@@ -440,25 +485,26 @@ __global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(A
             const int hq = rb.head * a.G + item / per_head, q0 = (qt_start + item % per_head) * 32;
             const long long base = rb.b * a.q_sb + hq * a.q_sh;
             if (!masked_tile(q0)) continue;
-            put_back_nonfinite<true, K8, DT, FULL>(static_cast<const float*>(a.dO) + base, a.q_ss, q0, a.S, a.hd, c, h, dv, [&](int v) { return visible(q0, v); });
-            put_back_nonfinite<false, K8, DT, FULL>(static_cast<const float*>(a.Q) + base, a.q_ss, q0, a.S, a.hd, c, h, dk, [&](int v) { return visible(q0, v); });
+            put_back_nonfinite<true, K8, DT, FULL>(static_cast<const float*>(a.dO) + base, qs, q0, a.S, a.hd, c, h, dv, [&](int v) { return visible(q0, v); });
+            put_back_nonfinite<false, K8, DT, FULL>(static_cast<const float*>(a.Q) + base, qs, q0, a.S, a.hd, c, h, dk, [&](int v) { return visible(q0, v); });
         }
     }
+    const long long koff = kvoff + (long long)key * a.k_ss;
     float* outs[2] = {static_cast<float*>(a.dK) + koff, static_cast<float*>(a.dV) + koff};
 #pragma unroll
     for (int i = 0; i < 2 * DT; i++) {  // one 32-column tile of dK or dV at a time; the waves take turns in adding up
         const int dt = i >> 1;
         f32x16 r = (i & 1) ? dv[dt] : dk[dt];
         if (nw > 1) {
-            float(*p)[16 * 64] = meet[i & 1];
+            float* p = meet + (i & 1) * kMaxWaves<K8> * 16 * 64;
 #pragma unroll
-            for (int v = 0; v < 16; v++) p[wave][v * 64 + lane] = r[v];
+            for (int v = 0; v < 16; v++) p[(wave * 16 + v) * 64 + lane] = r[v];
             __syncthreads();  // (the buffer of tile i was last read before the barrier of tile i - 1)
             if (i % nw != wave) continue;
             r = zero16();
             for (int w = 0; w < nw; w++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) r[v] += p[w][v * 64 + lane];
+                for (int v = 0; v < 16; v++) r[v] += p[(w * 16 + v) * 64 + lane];
         }
         if (k0 + c >= a.S) continue;
 #pragma unroll
@@ -477,6 +523,35 @@ __global__ __launch_bounds__(K8 <= 4 ? 512 : 256) void attn_f32_bwd_dkv_kernel(A
     }
 }
 
+// Both passes in one launch: the first kblocks workgroups form dK and dV of a key block each, the others dQ of as many query blocks
+// as they have wq waves for.  The two do not wait for one another (the dK/dV pass forms D itself), so a grid that does not fill the
+// chip takes the time of the longer pass, and one that does fills the gaps that the uneven causal key blocks leave.  Two launches with
+// an address of its own per load, and a dK/dV item's rows requested only when it began / this, us, causal, batch x sequence, query
+// heads on KV heads, head size: 2 x 32 4 on 4 16 12.2 / 5.5; 1 x 448 3 on 3 32 32.5 / 17.2; 16 x 256 8 on 2 32 56.7 / 34.5; 7 x 448
+// 4 on 4 64 66.4 / 57.4; 8 x 300 4 on 4 96 66.6 / 56.5; 1 x 800 8 on 8 128 163 / 92; 16 x 200 8 on 8 128 178 / 167 (one wave per
+// SIMD, registers full: its items still wait for their rows).
+template <int K8>
+constexpr int kMeetFloats = kMaxWaves<K8> * 16 * 64 * (2 > (K8 + 3) / 4 ? 2 : (K8 + 3) / 4);
+template <int K8, bool FULL>
+__global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_kernel(AttnArgs a, int kblocks, int wq) {
+    __shared__ float meet[kMeetFloats<K8>];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    if ((int)blockIdx.x < kblocks) return bwd_dkv<K8, FULL, true>(a, blockIdx.x, wave, nw, meet);
+    const int sub = wave / wq;
+    bwd_dq<K8, FULL, false>(a, ((int)blockIdx.x - kblocks) * (nw / wq) + sub, wave % wq, wq, meet + sub * wq * ((K8 + 3) / 4) * 16 * 64);
+}
+// One after the other, where a result lies over an operand.
+template <int K8, bool FULL>
+__global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dq_kernel(AttnArgs a) {
+    __shared__ float meet[kMeetFloats<K8>];
+    bwd_dq<K8, FULL, true>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);
+}
+template <int K8, bool FULL>
+__global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dkv_kernel(AttnArgs a) {
+    __shared__ float meet[kMeetFloats<K8>];
+    bwd_dkv<K8, FULL, false>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);
+}
+
 // waves per workgroup: enough for two waves per SIMD of the chip, but none without at least one tile of the longest row
 int waves_for(long long blocks, int tiles, int most) {
     int w = 1;
@@ -488,20 +563,26 @@ template <int K8, bool FULL>
 void launch_f32(eisen_ctx* ctx, const AttnArgs& a, bool backward) {
     const int n_t = (a.S + 31) / 32;
     const long long qblocks = (long long)n_t * a.Hq * a.B, kblocks = (long long)n_t * a.Hkv * a.B;
-    const int wq = waves_for(qblocks, n_t, kMaxKeyWaves), wk = waves_for(kblocks, n_t * a.G, K8 <= 4 ? 8 : 4);
+    const int wq = waves_for(qblocks, n_t, kMaxWaves<K8>), wk = waves_for(kblocks, n_t * a.G, kMaxWaves<K8>);
     if (!backward) {
         attn_f32_fwd_kernel<K8, FULL><<<dim3((unsigned)qblocks), 64 * wq, 0, ctx->stream>>>(a);
         return;
     }
-    attn_f32_bwd_dq_kernel<K8, FULL><<<dim3((unsigned)qblocks), 64 * wq, 0, ctx->stream>>>(a);
-    attn_f32_bwd_dkv_kernel<K8, FULL><<<dim3((unsigned)kblocks), 64 * wk, 0, ctx->stream>>>(a);
+    if (eisen_attention_writes_over_operand(a, sizeof(float))) {
+        attn_f32_bwd_dq_kernel<K8, FULL><<<dim3((unsigned)qblocks), 64 * wq, 0, ctx->stream>>>(a);
+        attn_f32_bwd_dkv_kernel<K8, FULL><<<dim3((unsigned)kblocks), 64 * wk, 0, ctx->stream>>>(a);
+        return;
+    }
+    const long long dq_groups = eisen_ceil_div(qblocks, (long long)(wk / wq));  // (wq <= wk: there are no fewer query blocks than key blocks)
+    attn_f32_bwd_kernel<K8, FULL><<<dim3((unsigned)(kblocks + dq_groups)), 64 * wk, 0, ctx->stream>>>(a, (int)kblocks, wq);
 }
 
 }  // namespace
 
 bool eisen_attention_f32_mfma_supports(const AttnArgs& a) {
     const long long n_t = (a.S + 31) / 32;
-    return a.hd <= 128 && n_t * a.Hq * a.B < (1ll << 31);
+    // (32 rows in an unsigned 32-bit byte offset)
+    return a.hd <= 128 && n_t * (a.Hq + a.Hkv) * a.B < (1ll << 31) && std::abs(a.q_ss) < (1ll << 24) && std::abs(a.k_ss) < (1ll << 24);
 }
 
 void eisen_attention_launch_f32(eisen_ctx* ctx, const AttnArgs& a, bool backward) {
