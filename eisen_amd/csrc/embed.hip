@@ -90,28 +90,174 @@ __global__ __launch_bounds__(kThreads) void scatter_rows_scalar_kernel(const T* 
 }
 
 // ---- position index built on the device ---------------------------------------------------------
-// index = [sorted ids | positions in sorted order | runs], n ints each.  The third part lists where the runs of equal ids
-// begin, in order, so that run r is [runs[r], runs[r + 1]); after the last run it is filled with the number of valid ids, and
-// from its end backwards it holds the number of long runs and their numbers, complemented: ~count, ~r0, ~r1, ...  (A run
-// of kLongRun occurrences frees kLongRun - 1 entries, so the two lists never meet; with n runs there is neither filling nor a
-// long run.)  Ids outside [0, vocab) sort behind all others as kNoId and belong to no run.
+// index = [ids | positions], n ints each: the positions of every id stand together, in ascending order, beside the id (in which order
+// the ids follow one another is each builder's own).  Ids outside [0, vocab) stand behind all others as kNoId and belong to no run.
 constexpr int kNoId = 0x7fffffff;
-constexpr int kLongRun = 128;
 
+// One launch: 256 workgroups, each with the ids of one residue.  All of them read the whole batch (128 KB from the L2s for 32768 ids),
+// count what lies before their part and, per id and wave, their own, and place their positions; a wave's ids are consecutive, so the
+// places of an id ascend.  What bounds it is the dozen instructions per id and workgroup.  Chunks sorted by a bitonic network, merged and
+// listed in three launches had taken 30 us for 32768 ids, one chunk of up to 1024 and 2048 7.0 and 12.6; this takes 14.1, 4.7 and 5.1.
+constexpr int kBucketBits = 8, kBuckets = 1 << kBucketBits, kBucketThreads = 1024, kBucketWaves = kBucketThreads / kWave, kBucketIds = 960;  // (60 KB of LDS)
+constexpr size_t kBucketMax = 65536, kBucketVocab = (size_t)kBuckets * kBucketIds;
+__global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const int32_t* __restrict__ ids, int n, int vocab, int32_t* __restrict__ out_ids,
+                                                                       int32_t* __restrict__ order, int32_t* __restrict__ first_bad) {
+    extern __shared__ int places[];  // [wave][id >> kBucketBits]: how many the wave has of it, then where its next one goes
+    __shared__ int sums[kBucketWaves][2];
+    constexpr int LIST = 512;
+    __shared__ int list[kBucketWaves][LIST];  // a wave's own ids, id >> kBucketBits | index << 10, in order
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), bucket = blockIdx.x;
+    const int here = (vocab + kBuckets - 1) >> kBucketBits;  // ids of this residue, at most
+    // (an odd number of 256-byte lines: the waves, and with them all workgroups, would otherwise ask one channel of the L2 at a time)
+    const int share = ((n + kBucketWaves * kWave - 1) / (kBucketWaves * kWave) | 1) * kWave;
+    const int from = wave * share, to = min(n, from + share);
+    int* const mine = places + wave * here;
+    for (int i = tid; i < kBucketWaves * here; i += kBucketThreads) places[i] = 0;
+    __syncthreads();
+    constexpr int U = 8;
+    int before = 0, bad = kNoId, own = 0;  // before: of smaller residues, per lane
+    for (int i0 = from; i0 < to; i0 += U * kWave) {
+        int id[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) id[u] = ids[min(i0 + u * kWave + lane, n - 1)];
+        if (i0 + U * kWave > to)
+#pragma unroll
+            for (int u = 0; u < U; u++) id[u] = i0 + u * kWave + lane < to ? id[u] : -1;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int b = (unsigned)id[u] < (unsigned)vocab ? id[u] & (kBuckets - 1) : kBuckets;
+            before += b < bucket;
+            const unsigned long long hits = __ballot(b == bucket);
+            if (hits) {
+                if (b == bucket) {
+                    atomicAdd(&mine[id[u] >> kBucketBits], 1);
+                    const int k = own + __popcll(hits & ((1ull << lane) - 1));
+                    if (k < LIST) list[wave][k] = id[u] >> kBucketBits | (i0 + u * kWave + lane) << 10;
+                }
+                own += __popcll(hits);
+            }
+        }
+        if (bucket == 0 && bad == kNoId) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = i0 + u * kWave + lane;
+                const unsigned long long wrong = __ballot(i < to && (unsigned)id[u] >= (unsigned)vocab);
+                if (wrong) bad = min(bad, i0 + u * kWave + __ffsll(wrong) - 1);
+            }
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    if (lane == 0) { sums[wave][0] = before; sums[wave][1] = bucket == 0 ? bad : own; }
+    __syncthreads();
+    before = 0;
+#pragma unroll
+    for (int w = 0; w < kBucketWaves; w++) before += sums[w][0];
+    if (bucket == 0 && tid == 0 && first_bad) {
+        for (int w = 0; w < kBucketWaves; w++) bad = min(bad, sums[w][1]);
+        *first_bad = bad;
+    }
+    if (bucket == kBuckets - 1) {
+        int valid = before;
+        for (int w = 0; w < kBucketWaves; w++) valid += sums[w][1];
+        for (int i = valid + tid; i < n; i += kBucketThreads) {
+            out_ids[i] = kNoId;
+            order[i] = 0;
+        }
+    }
+    // where the first position of each id goes: thread t takes id t
+    int count[kBucketWaves], total = 0;
+#pragma unroll
+    for (int w = 0; w < kBucketWaves; w++) {
+        count[w] = tid < here ? places[w * here + tid] : 0;
+        total += count[w];
+    }
+    int upto = total;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int other = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += other;
+    }
+    __syncthreads();  // the sums above have been read
+    if (lane == 63) sums[wave][0] = upto;
+    __syncthreads();
+    int at = before + upto - total;
+#pragma unroll
+    for (int w = 0; w < kBucketWaves; w++) at += w < wave ? sums[w][0] : 0;
+    if (tid < here) {
+#pragma unroll
+        for (int w = 0; w < kBucketWaves; w++) {
+            places[w * here + tid] = at;
+            at += count[w];
+        }
+    }
+    __syncthreads();
+    if (own <= LIST) {
+        for (int k0 = 0; k0 < own; k0 += kWave) {
+            const int these = min(kWave, own - k0), entry = list[wave][min(k0 + lane, own - 1)], slot = entry & 1023;
+            int rank = 0, all = 0;  // among the lanes with this id: those before this one, and all
+            unsigned long long left = these == kWave ? ~0ull : (1ull << these) - 1;
+            while (left) {
+                const unsigned long long same = __ballot(slot == __builtin_amdgcn_readlane(slot, __ffsll(left) - 1)) & left;
+                if (same >> lane & 1) {
+                    rank = __popcll(same & ((1ull << lane) - 1));
+                    all = __popcll(same);
+                }
+                left &= ~same;
+            }
+            if (lane < these) {
+                const int place = mine[slot] + rank;
+                out_ids[place] = slot << kBucketBits | bucket;
+                order[place] = (int)((unsigned)entry >> 10);
+                if (rank == all - 1) mine[slot] = place + 1;  // (a wave's reads of the step above are done)
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        return;
+    }
+    for (int i0 = from; i0 < to; i0 += U * kWave) {  // hot ids: once more through the batch
+        int id[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) id[u] = ids[min(i0 + u * kWave + lane, n - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = i0 + u * kWave + lane;
+            unsigned long long left = __ballot(i < to && id[u] >= 0 && id[u] < vocab && (id[u] & (kBuckets - 1)) == bucket);
+            while (left) {  // the lanes with the id of the first one that is left: places in a row
+                const int this_id = __builtin_amdgcn_readlane(id[u], __ffsll(left) - 1);
+                const unsigned long long same = __ballot(id[u] == this_id) & left;
+                const int next = mine[this_id >> kBucketBits];
+                if (same >> lane & 1) {
+                    const int place = next + __popcll(same & ((1ull << lane) - 1));
+                    out_ids[place] = this_id;
+                    order[place] = i;
+                }
+                if (lane == 0) mine[this_id >> kBucketBits] = next + __popcll(same);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                left &= ~same;
+            }
+        }
+    }
+}
+
+// Batches and vocabularies beyond that.
 // Keys id * 2^shift + position in the chunk are unique, so sorting them is the stable sort of the positions by id.  One
 // workgroup of 1024 threads sorts 1024 * R of them (R = 1..16) with a bitonic network whose keys stay in registers: thread t
 // holds elements t, t + 1024, ...; a compare-exchange at distance j >= 1024 pairs two registers of one thread, j < 64 two
 // lanes of one wave (a shuffle), and only the distances 64..512 go through LDS (18 to 26 of the 55 to 105 steps).  Workgroup c
 // takes the ids of chunk c and writes them and their positions in key order; first_bad (may be null) receives per chunk the
-// position of its first id outside [0, vocab), or kNoId.  A batch of one chunk is complete with this kernel: it also lists the runs.
+// position of its first id outside [0, vocab), or kNoId.  A batch of one chunk is complete with this kernel.
 constexpr int kSortThreads = 1024, kSortMax = 16384;
 template <int R>
 __global__ __launch_bounds__(kSortThreads) void scatter_sort_kernel(const int32_t* __restrict__ ids_all, int n_all, int shift, int vocab,
                                                                    int32_t* __restrict__ sorted_ids, int32_t* __restrict__ order,
-                                                                   int32_t* __restrict__ runs, int32_t* __restrict__ first_bad) {
+                                                                   int32_t* __restrict__ first_bad) {
     constexpr int NP = kSortThreads * R;
     __shared__ unsigned keys[NP];
-    __shared__ int totals[kSortThreads / kWave][2];
     __shared__ int bad;
     const int tid = threadIdx.x;
     const int first = blockIdx.x * NP, n = min(NP, n_all - first);
@@ -174,55 +320,6 @@ __global__ __launch_bounds__(kSortThreads) void scatter_sort_kernel(const int32_
         // the padding keys' positions do not matter: they lie in no run
         order[first + i] = k == 0xffffffffu ? 0 : first + (int32_t)(k & mask);
     }
-    if (!runs) return;
-    // one chunk: thread t lists the runs that begin in elements [t R, t R + R)
-    int begins = 0, longs = 0;
-    unsigned begin_bits = 0, long_bits = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int i = tid * R + r;
-        if (i >= n || keys[i] == 0xffffffffu) continue;
-        const unsigned id = keys[i] >> shift;
-        if (i > 0 && (keys[i - 1] >> shift) == id) continue;
-        begins++;
-        begin_bits |= 1u << r;
-        const int last = i + kLongRun - 1;
-        if (last < n && keys[last] != 0xffffffffu && (keys[last] >> shift) == id) {
-            longs++;
-            long_bits |= 1u << r;
-        }
-    }
-    const int lane = tid & 63, wid = tid >> 6;
-    int b = begins, l = longs;  // inclusive sums over the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int bo = __shfl_up(b, o, 64), lo = __shfl_up(l, o, 64);
-        if (lane >= o) { b += bo; l += lo; }
-    }
-    if (lane == 63) { totals[wid][0] = b; totals[wid][1] = l; }
-    __syncthreads();
-    int b_all = 0, l_all = 0, b_before = 0, l_before = 0;
-#pragma unroll
-    for (int w = 0; w < kSortThreads / kWave; w++) {
-        if (w == wid) { b_before = b_all; l_before = l_all; }
-        b_all += totals[w][0];
-        l_all += totals[w][1];
-    }
-    int at_b = b_before + b - begins, at_l = l_before + l - longs;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        if (long_bits >> r & 1) runs[n - 2 - at_l++] = ~at_b;
-        if (begin_bits >> r & 1) runs[at_b++] = tid * R + r;
-    }
-    // the number of valid ids: where the padding keys begin
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (keys[mid] != 0xffffffffu) lo = mid + 1;
-        else hi = mid;
-    }
-    for (int i = b_all + tid; i < n - (l_all ? l_all + 1 : 0); i += kSortThreads) runs[i] = lo;
-    if (tid == 0 && l_all) runs[n - 1] = ~l_all;
 }
 
 // The sorted chunks become one sorted batch.  An element's place is its place in its own chunk plus, for every earlier chunk,
@@ -296,195 +393,275 @@ __global__ __launch_bounds__(kThreads) void scatter_merge_kernel(const int32_t* 
     order[rank] = chunk_order[e];
 }
 
-// Lists the runs of a merged batch.  A workgroup takes 1024 sorted ids and counts by itself what begins before them (each of
-// its threads looks at every 1024th id): a handful of reads per thread instead of a scan over workgroups.
-__global__ __launch_bounds__(kSortThreads) void scatter_runs_list_kernel(const int32_t* __restrict__ sorted_ids, int n, int32_t* __restrict__ runs) {
-    __shared__ int before[kSortThreads / kWave][3], own[kSortThreads / kWave][2];  // per wave: what it counted before this workgroup's ids, and among them
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int first = blockIdx.x * kSortThreads;
-    int b = 0, l = 0, valid = 0;
-    for (int i0 = 0; i0 < first; i0 += 8 * kSortThreads) {  // 24 loads in flight: the loop is a chain of load latencies
-        int id[8], prev[8], far[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int i = min(i0 + u * kSortThreads + tid, n - 1);
-            id[u] = sorted_ids[i];
-            prev[u] = sorted_ids[max(i - 1, 0)];
-            far[u] = sorted_ids[min(i + kLongRun - 1, n - 1)];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int i = i0 + u * kSortThreads + tid;
-            if (i >= first || id[u] == kNoId) continue;
-            valid++;
-            if (i > 0 && prev[u] == id[u]) continue;
-            b++;
-            l += i + kLongRun <= n && far[u] == id[u];
-        }
-    }
-    const int i = first + tid, own_id = i < n ? sorted_ids[i] : kNoId;
-    const bool begins = own_id != kNoId && (i == 0 || sorted_ids[i - 1] != own_id);
-    const bool is_long = begins && i + kLongRun <= n && sorted_ids[i + kLongRun - 1] == own_id;
-    valid += own_id != kNoId;
-    const unsigned long long bm = __ballot(begins), lm = __ballot(is_long), below = (1ull << lane) - 1;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        b += __shfl_xor(b, o, 64);
-        l += __shfl_xor(l, o, 64);
-        valid += __shfl_xor(valid, o, 64);
-    }
-    if (lane == 0) {
-        before[wid][0] = b; before[wid][1] = l; before[wid][2] = valid;
-        own[wid][0] = __popcll(bm); own[wid][1] = __popcll(lm);
-    }
-    __syncthreads();
-    int b_at = 0, l_at = 0, b_all = 0, l_all = 0, v_all = 0;
-#pragma unroll
-    for (int w = 0; w < kSortThreads / kWave; w++) {
-        b_at += before[w][0] + (w < wid ? own[w][0] : 0);
-        l_at += before[w][1] + (w < wid ? own[w][1] : 0);
-        b_all += before[w][0] + own[w][0];
-        l_all += before[w][1] + own[w][1];
-        v_all += before[w][2];
-    }
-    b_at += __popcll(bm & below);
-    l_at += __popcll(lm & below);
-    if (begins) runs[b_at] = i;
-    if (is_long) runs[n - 2 - l_at] = ~b_at;
-    if (blockIdx.x == gridDim.x - 1) {  // the last workgroup has counted everything
-        for (int k = b_all + tid; k < n - (l_all ? l_all + 1 : 0); k += kSortThreads) runs[k] = v_all;
-        if (tid == 0 && l_all) runs[n - 1] = ~l_all;
-    }
-}
-
 // ---- the scatter along the index ----------------------------------------------------------------
 // gw[row] = ((gw[row] + go[i1]) + go[i2]) + ... with i1 < i2 < ... (the CPU arm's order, src/graph/ops/transform.rs:309-314):
 // a run is one chain of dependent adds per column, whatever the schedule.  What bounds it is how many rows of dOut are in
 // flight, and for the hot rows of text (thousands of occurrences) the length of the chain:
-//  * a long run (>= kLongRun) is a workgroup's per 64 columns: all four waves fetch the next 32 KB of its rows into registers
-//    while one wave adds the rows that stand in LDS;
-//  * a short run is a wave's per 64 * C columns, up to 16 rows in flight.
-// The first workgroups take the long runs, the others the short ones.
-// lane l's column of 32 rows of 64 values in LDS.  bf16: the transposing read hands every lane four rows of its column at once
-// (one 2-byte read per row and lane made the adds of a long run cost 24 cycles each).
-__device__ __forceinline__ void read_columns(const float* rows, float* x) {
+//  * a long run, one that holds two multiples of 64 among its places in the index, is a workgroup's per 64 columns: four waves fetch its
+//    rows, four rows of four columns to a thread and several stages ahead, and leave them in LDS as f32, the rows of a column side by
+//    side; the first wave, a lane to a column, adds: a quarter of an LDS read and one add per row.  With the adding wave among those
+//    that fetch, rows in bf16 and read by columns, a run of 16384 took 8.2 ns per row; now 5.8, of which 2 are the chain of adds.
+//  * the short runs that begin in 2 or 8 places in a row are a wave's per 256 columns, all their rows in flight: waves with equal
+//    work, and no list of runs.  (A wave to a run, its rows 16 at a time: 1396 ids, rows of 448 bf16, lookup and scatter 25.5 us, now 14.4.)
+// 32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 -> 91 us, of which lookup 15, index 14, scatter 40 (the 4649 occurrences of the first id).
+// The first workgroups take the long runs, the others the short ones.  first_bad, if given, points at kNoId or nothing is added.
+constexpr int kRunThreads = 320, kRunStage = 64, kRunWindow = 8;
+template <typename T> struct Four { typedef T type __attribute__((ext_vector_type(4))); };
+template <typename T> struct Two { typedef T type __attribute__((ext_vector_type(2))); };
+// four columns from col on of a row of `hidden`; WIDE: rows are whole packets, else they are whole pairs.  Columns past the end repeat
+// the last ones: without a branch around a load the compiler knows how many are in flight.
+template <bool WIDE, typename T>
+__device__ __forceinline__ typename Four<T>::type load_four(const T* row, int col, int hidden) {
+    typename Four<T>::type x;
+    if (WIDE) {
+        x = *reinterpret_cast<const typename Four<T>::type*>(row + min(col, hidden - 4));
+    } else {
 #pragma unroll
-    for (int u = 0; u < 32; u++) x[u] = rows[u * 64 + (threadIdx.x & 63)];
+        for (int j = 0; j < 4; j += 2) {
+            const typename Two<T>::type y = *reinterpret_cast<const typename Two<T>::type*>(row + min(col + j, hidden - 2));
+            x[j] = y[0];
+            x[j + 1] = y[1];
+        }
+    }
+    return x;
 }
-__device__ __forceinline__ void read_columns(const bf16_t* rows, float* x) {
-    typedef bf16x4 __attribute__((address_space(3))) * lds_ptr;
-    const int lane = threadIdx.x & 63, L = lane & 15;
-    const bf16_t* p = rows + (L >> 2) * 64 + (lane & 48) + 4 * (L & 3);
+template <bool WIDE>
+__device__ __forceinline__ void store_four(float* row, int col, int hidden, const Four<float>::type& x) {
+    if (WIDE) {
+        if (col < hidden) *reinterpret_cast<Four<float>::type*>(row + col) = x;
+    } else {
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        const bf16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_ptr)(p + u * 256));
-#pragma unroll
-        for (int j = 0; j < 4; j++) x[4 * u + j] = (float)v[j];
+        for (int j = 0; j < 4; j += 2)
+            if (col + j < hidden) *reinterpret_cast<float2*>(row + col + j) = make_float2(x[j], x[j + 1]);
     }
 }
-template <typename T, int N> struct Cols { typedef T type __attribute__((ext_vector_type(N))); };
+// The number-th long run of the index, [begin, end), and its id; false if there are not as many.  All threads of the workgroup.  Every
+// thread looks at 4 of the multiples of 64 at once; what the marks leave open of begin and end are 64 places each.
+constexpr int kRunMarks = 4, kRunWaves = kRunThreads / kWave;
+struct RunLds {
+    unsigned long long starts[kRunMarks * kRunWaves], goes_on[kRunMarks * kRunWaves];  // bit l of [i]: multiple 64 * i + l of this turn
+};
+__device__ __forceinline__ bool find_long_run(const int32_t* __restrict__ ids, int n, int number, RunLds& lds, int& begin, int& end, int& id) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int marks = (n + 63) / 64;
+    int first = -1, last = -1;  // the run's first and last multiple
+    for (int k0 = 0; k0 < marks && last < 0; k0 += kRunMarks * kRunThreads) {
+        int x[kRunMarks][3];
+#pragma unroll
+        for (int u = 0; u < kRunMarks; u++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) x[u][j] = ids[min(max((k0 + u * kRunThreads + (int)threadIdx.x + j - 1) * 64, 0), n - 1)];
+        __syncthreads();  // the marks of the turn or the search before have been read
+#pragma unroll
+        for (int u = 0; u < kRunMarks; u++) {
+            const int k = k0 + u * kRunThreads + threadIdx.x;
+            const bool behind = (k + 1) * 64 < n && x[u][1] != kNoId && x[u][2] == x[u][1], ahead = k > 0 && x[u][0] == x[u][1];
+            const unsigned long long starts = __ballot(behind && !ahead), goes_on = __ballot(behind);
+            if (lane == 0) {
+                lds.starts[u * kRunWaves + wave] = starts;
+                lds.goes_on[u * kRunWaves + wave] = goes_on;
+            }
+        }
+        __syncthreads();
+        constexpr int WORDS = kRunMarks * kRunWaves;  // lane i takes word i
+        static_assert(WORDS <= 32, "a wave's prefix sums");
+        const unsigned long long starts = lane < WORDS ? lds.starts[lane] : 0, on = lane < WORDS ? lds.goes_on[lane] : ~0ull;
+        unsigned long long stops = ~on;
+        if (first < 0) {
+            const int count = __popcll(starts);
+            int upto = count;
+#pragma unroll
+            for (int o = 1; o < 32; o <<= 1) {
+                const int other = __shfl_up(upto, o, 64);
+                if (lane >= o) upto += other;
+            }
+            const unsigned long long hit = __ballot(number >= upto - count && number < upto);
+            if (!hit) {
+                number -= __builtin_amdgcn_readlane(upto, WORDS - 1);
+                continue;
+            }
+            const int word = __ffsll(hit) - 1;
+            unsigned long long left = __shfl(starts, word, 64);
+            for (int skip = number - __builtin_amdgcn_readlane(upto - count, word); skip > 0; skip--) left &= left - 1;
+            const int bit = __ffsll(left) - 1;
+            first = k0 + word * 64 + bit;
+            stops = lane < word ? 0 : lane == word ? stops & ~((1ull << bit) - 1) : stops;
+        }
+        const unsigned long long ends = __ballot(stops != 0);
+        if (ends) last = k0 + (__ffsll(ends) - 1) * 64 + __ffsll((unsigned long long)__shfl(stops, __ffsll(ends) - 1, 64)) - 1;
+    }
+    if (first < 0) return false;
+    if (last < 0) last = marks - 1;
+    first = __builtin_amdgcn_readfirstlane(first);
+    last = __builtin_amdgcn_readfirstlane(last);
+    id = __builtin_amdgcn_readfirstlane(ids[first * 64]);
+    const int before = first * 64 - 63 + lane, after = last * 64 + 1 + lane;
+    begin = first * 64 - 63 + __ffsll(__ballot(before >= 0 && ids[max(before, 0)] == id)) - 1;
+    end = last * 64 + 1 + __popcll(__ballot(after < n && ids[min(after, n - 1)] == id));
+    return true;
+}
+// Where four rows of a column stand in a stage: turned so that 16 lanes in a row meet all banks, be they neighbouring columns (the adding
+// wave's) or every fourth (those of the waves that fetch).
+__device__ __forceinline__ int stage_at(int column, int quad) { return column * kRunStage + 4 * ((quad + (column >> 2) + 4 * (column & 3)) & 15); }
 template <typename T, bool WIDE>
-__global__ __launch_bounds__(kThreads) void scatter_runs_kernel(const T* __restrict__ go, float* __restrict__ gw, const int32_t* __restrict__ sorted_ids,
-                                                               const int32_t* __restrict__ order, const int32_t* __restrict__ runs, int n, int hidden) {
-    constexpr int E = WIDE ? 16 / (int)sizeof(T) : 2;  // columns per load of a long run
-    constexpr int LPR = 64 / E;                        // lanes per row of 64 columns
-    constexpr int RPI = kThreads / LPR;                // rows per load of the workgroup
-    constexpr int U = sizeof(T) * E == 16 ? 8 : 16;    // loads in flight per thread
-    constexpr int ST = RPI * U;                        // rows per stage
-    typedef typename Cols<T, E>::type VE;
-    __shared__ __attribute__((aligned(16))) T stage[ST * 64];
+__device__ __forceinline__ void scatter_long_run(const T* __restrict__ go, float* __restrict__ gw, const int32_t* __restrict__ order,
+                                                 int hidden, int id, int begin, int end, int col0, float* stage) {
+    constexpr int D = sizeof(T) == 2 ? 4 : 3;  // stages of rows on their way, per thread
+    constexpr int BUF = 64 * kRunStage;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int n_long = runs[n - 1] < 0 ? ~runs[n - 1] : 0;
-    const int long_slabs = (hidden + 63) / 64;
-    const long long long_items = (long long)n_long * long_slabs;
-    const int long_blocks = (int)min(long_items, (long long)(gridDim.x / 2));
-    if ((int)blockIdx.x < long_blocks) {
-        for (long long item = blockIdx.x; item < long_items; item += long_blocks) {
-            const int r = ~runs[n - 2 - (int)(item / long_slabs)];
-            const int begin = runs[r], end = r + 1 < n ? runs[r + 1] : n;
-            const int col0 = (int)(item % long_slabs) * 64;
-            const int col = col0 + (tid % LPR) * E, sub = tid / LPR;
-            const bool in = col < hidden;  // hidden is a multiple of E
-            const T* src = go + (in ? col : 0);
-            float* dst = gw + (size_t)sorted_ids[begin] * hidden + col0 + lane;
-            float acc = tid < 64 && col0 + lane < hidden ? *dst : 0.f;
-            VE v[U];
-            int at[U];  // positions of the rows to be fetched next, a stage ahead of the rows
-            auto look_up = [&](int k0) {
+    // whole turns of D stages: with an exit in between the compiler loses count of the loads in flight and waits for all of them
+    const int turns = ((end - begin + kRunStage - 1) / kRunStage + D - 1) / D * D;
+    if (tid < kWave) {
+        float* dst = gw + (size_t)id * hidden + col0 + lane;
+        const bool in = col0 + lane < hidden;
+        float acc = in ? *dst : 0.f;
+        __builtin_amdgcn_s_setprio(3);  // this wave's adds are what the workgroup takes, and the longest run what the launch takes
+        for (int s = 0; s < turns; s++) {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // stage s is there
+            const int rows = end - begin - s * kRunStage;
+            if (rows <= 0) continue;
+            const float* from = stage + (s & 1) * BUF;
+            float4 x[kRunStage / 4];
 #pragma unroll
-                for (int u = 0; u < U; u++) at[u] = order[min(k0 + u * RPI + sub, end - 1)];
-            };
-            auto fetch = [&] {
+            for (int r = 0; r < kRunStage / 4; r++) x[r] = *reinterpret_cast<const float4*>(from + stage_at(lane, r));
+            __builtin_amdgcn_sched_barrier(0);  // all of them on their way before the first add: a read takes as long as 30 adds
+            if (rows >= kRunStage) {
 #pragma unroll
-                for (int u = 0; u < U; u++) v[u] = *reinterpret_cast<const VE*>(src + (size_t)at[u] * hidden);
-            };
-            look_up(begin);
-            fetch();
-            look_up(begin + ST);
-            for (int k0 = begin; k0 < end; k0 += ST) {
-                __syncthreads();  // the previous stage has been added up
-#pragma unroll
-                for (int u = 0; u < U; u++) *reinterpret_cast<VE*>(&stage[(u * RPI + sub) * 64 + (tid % LPR) * E]) = v[u];
-                __syncthreads();
-                if (k0 + ST < end) {
-                    fetch();
-                    look_up(k0 + 2 * ST);
+                for (int r = 0; r < kRunStage / 4; r++) {
+                    acc += x[r].x;
+                    acc += x[r].y;
+                    acc += x[r].z;
+                    acc += x[r].w;
                 }
-                if (tid < 64) {
-                    const int rows = min(ST, end - k0);
-                    int k = 0;
-                    for (; k + 32 <= rows; k += 32) {
-                        float x[32];
-                        read_columns(&stage[k * 64], x);
+            } else {
 #pragma unroll
-                        for (int u = 0; u < 32; u++) acc += x[u];
-                    }
-                    for (; k < rows; k++) acc += to_f32(stage[k * 64 + lane]);
+                for (int r = 0; r < kRunStage; r++) {
+                    const float sum = acc + (r % 4 == 0 ? x[r / 4].x : r % 4 == 1 ? x[r / 4].y : r % 4 == 2 ? x[r / 4].z : x[r / 4].w);
+                    acc = r < rows ? sum : acc;
                 }
             }
-            if (tid < 64 && col0 + lane < hidden) *dst = acc;
         }
-        return;
-    }
-    constexpr int C = WIDE ? 4 : 2, F = 16;  // columns per lane, rows in flight
-    typedef typename Cols<T, C>::type VC;
-    typedef typename Cols<float, C>::type VF;
-    const int slabs = (hidden + 64 * C - 1) / (64 * C);
-    const int waves = (int)(gridDim.x - long_blocks) * (kThreads / kWave);
-    const int item = __builtin_amdgcn_readfirstlane((blockIdx.x - long_blocks) * (kThreads / kWave) + (tid >> 6));
-    int r = item / slabs, slab = item % slabs;
-    for (; r < n; r += waves / slabs + (slab + waves % slabs >= slabs), slab = (slab + waves % slabs) % slabs) {
-        const int begin = runs[r];
-        if (begin < 0 || begin >= n) return;
-        const int end = r + 1 < n ? runs[r + 1] : n, row = sorted_ids[begin];
-        if (end <= begin || row == kNoId) return;  // behind the last run
-        if (end - begin >= kLongRun) continue;
-        const int col = (slab * 64 + lane) * C;
-        if (col >= hidden) continue;  // hidden is a multiple of C
-        VF acc = *reinterpret_cast<const VF*>(gw + (size_t)row * hidden + col);
-        const T* src = go + col;
-        for (int k = begin; k < end; k += F) {
-            VC p[F];
+        __builtin_amdgcn_s_setprio(0);
+        if (in) *dst = acc;
+    } else {
+        const int quad = (tid - kWave) / 16, group = tid % 16, col = col0 + 4 * group;
+        typename Four<T>::type v[D][4];
+        int at[D][4];  // positions, D stages ahead of the rows: the wait for them is then no wait for rows that are needed later
+        auto look_up = [&](int s, int (&to)[4]) {
 #pragma unroll
-            for (int u = 0; u < F; u++)
-                if (k + u < end) p[u] = *reinterpret_cast<const VC*>(src + (size_t)order[k + u] * hidden);
+            for (int j = 0; j < 4; j++) to[j] = order[min(begin + s * kRunStage + 4 * quad + j, end - 1)];
+        };
+        auto fetch = [&](const int (&from)[4], typename Four<T>::type (&rows)[4]) {
 #pragma unroll
-            for (int u = 0; u < F; u++)
-                if (k + u < end)
+            for (int j = 0; j < 4; j++) rows[j] = load_four<WIDE>(go + (size_t)from[j] * hidden, col, hidden);
+        };
 #pragma unroll
-                    for (int j = 0; j < C; j++) acc[j] += (float)p[u][j];
+        for (int d = 0; d < D; d++) look_up(d, at[d]);
+#pragma unroll
+        for (int d = 0; d < D; d++) {  // (in the loop's order: the compiler's counts of loads in flight hold for both)
+            fetch(at[d], v[d]);
+            look_up(D + d, at[d]);
         }
-        *reinterpret_cast<VF*>(gw + (size_t)row * hidden + col) = acc;
+        for (int s0 = 0; s0 < turns; s0 += D) {
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                const int s = s0 + d;
+                float* to = stage + (s & 1) * BUF;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    *reinterpret_cast<float4*>(to + stage_at(4 * group + j, quad)) = make_float4((float)v[d][0][j], (float)v[d][1][j], (float)v[d][2][j], (float)v[d][3][j]);
+                fetch(at[d], v[d]);  // (past the end: its last row again)
+                look_up(s + 2 * D, at[d]);
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the adding wave is done with stage s - 1)
+            }
+        }
     }
+    __syncthreads();  // both stages may be written again
+}
+template <typename T, bool WIDE>
+__global__ __launch_bounds__(kRunThreads, 3) void scatter_runs_kernel(const T* __restrict__ go, float* __restrict__ gw, const int32_t* __restrict__ ids,
+                                                                  const int32_t* __restrict__ order, const int32_t* __restrict__ first_bad, int n, int hidden,
+                                                                  int long_blocks, int window) {
+    __shared__ __attribute__((aligned(16))) float stage[2 * 64 * kRunStage];
+    __shared__ RunLds marks;
+    if (first_bad && *first_bad != kNoId) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    if ((int)blockIdx.x < long_blocks) {
+        const int slabs = (hidden + 63) / 64;
+        for (int item = blockIdx.x;; item += long_blocks) {
+            int begin, end, id;
+            if (!find_long_run(ids, n, item / slabs, marks, begin, end, id)) return;
+            scatter_long_run<T, WIDE>(go, gw, order, hidden, id, begin, end, item % slabs * 64, stage);
+        }
+    }
+    typedef Four<float>::type F4;
+    const int slabs = (hidden + 255) / 256;
+    const int item = __builtin_amdgcn_readfirstlane(((int)blockIdx.x - long_blocks) * (kRunThreads / kWave) + (tid >> 6));
+    const int col = (item % slabs * 64 + lane) * 4;
+    F4 acc = {};
+    int row = -1;  // of the run that is being added up
+    auto row_of = [&](int pos, int u) { return load_four<WIDE>(go + (size_t)__builtin_amdgcn_readlane(pos, u) * hidden, col, hidden); };
+    for (int p = item / slabs * window, first = p; p < n; p += kWave) {
+        const int i = p + lane, far = ((i + 63) & ~63) + 64;
+        const int id = i < n ? ids[i] : kNoId, ahead = i > 0 && i < n ? ids[i - 1] : -1, behind = far < n ? ids[far] : -1, pos = i < n ? order[i] : 0;
+        const unsigned long long in_window = (1ull << window) - 1;
+        const unsigned long long past = __ballot(id == kNoId), begins = __ballot(id != kNoId && id != ahead), is_long = __ballot(id != kNoId && id != ahead && id == behind);
+        // from the first run that begins in the window on, up to a long one, or to where the last run ends
+        unsigned long long stop = begins | past;
+        int done = 0;
+        if (p == first) {
+            if (!(begins & in_window)) return;
+            stop = (is_long & in_window) | (begins & ~in_window) | past;
+            const int from = __ffsll(begins) - 1, to = stop ? min(__ffsll(stop) - 1, window) : window;
+            typename Four<T>::type x[kRunWindow];
+            F4 g[kRunWindow];
+#pragma unroll
+            for (int u = 0; u < kRunWindow; u++)
+                if (u >= from && u < to) {
+                    x[u] = row_of(pos, u);
+                    if (begins >> u & 1) g[u] = load_four<WIDE>(gw + (size_t)__builtin_amdgcn_readlane(id, u) * hidden, col, hidden);
+                }
+            // all of them have arrived: behind the branches the compiler would wait for everything at each use, the stores in between included
+#pragma unroll
+            for (int u = 0; u < kRunWindow; u++) asm volatile("" : "+v"(x[u]), "+v"(g[u]));
+#pragma unroll
+            for (int u = 0; u < kRunWindow; u++)
+                if (u >= from && u < to) {
+                    if (begins >> u & 1) {
+                        if (row >= 0) store_four<WIDE>(gw + (size_t)row * hidden, col, hidden, acc);
+                        acc = g[u];
+                        row = __builtin_amdgcn_readlane(id, u);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[j] += (float)x[u][j];
+                }
+            if (row < 0) return;
+            done = window;
+        }
+        const int to = stop ? __ffsll(stop) - 1 : kWave;
+        for (; done < to; done += 2 * kRunWindow) {  // what is left of the last run
+            typename Four<T>::type x[2 * kRunWindow];
+#pragma unroll
+            for (int u = 0; u < 2 * kRunWindow; u++)
+                if (done + u < to) x[u] = row_of(pos, done + u);
+#pragma unroll
+            for (int u = 0; u < 2 * kRunWindow; u++) asm volatile("" : "+v"(x[u]));
+#pragma unroll
+            for (int u = 0; u < 2 * kRunWindow; u++)
+                if (done + u < to)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[j] += (float)x[u][j];
+        }
+        if (to < kWave) break;
+    }
+    if (row >= 0) store_four<WIDE>(gw + (size_t)row * hidden, col, hidden, acc);
 }
 
-// How a batch is sorted: chunks of 1024 << k ids, one workgroup each, whose keys (id, position in the chunk) fit 32 bits.  A
-// batch of up to 2048 ids is one chunk, complete with one launch (2048 ids: 11.8 us for the index, 15.6 in two chunks).  Beyond that
+// How a batch beyond scatter_bucket_kernel's is sorted: chunks of 1024 << k ids, one workgroup each, whose keys (id, position in the chunk)
+// fit 32 bits, and a merge.  A batch of up to 2048 ids is one chunk (2048 ids: 11.8 us for the index, 15.6 in two chunks).  Beyond that
 // short chunks and a merge beat one long bitonic network, the shorter ones up to where the merge's searches, which grow with the
-// number of chunks, outweigh the sort (chunks of 1024 / 2048 / 4096 / all in one, us for the index): 2049 ids 15.7 / 19.7 / 19.5,
-// 4096 16.6 / 20.8 / 20.2, 8192 17.7 / 21.9 / 29.8 / 39.6, 16384 20.3 / 24.4 / 32.6 / 85; with the scatter, 24000 ids 62.6 / 62.0, 32768 74.4 / 73.3,
-// 65536 141 / 130.  Beyond 65536 ids chunks of 16384.  32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 us, of which sort 10,
-// merge 11, list of runs 10, scatter 48; with the host's stable_sort and four rows of a run in flight 2790 us.
+// number of chunks, outweigh the sort (chunks of 1024 / 2048 / 4096 / all in one, us for the index when it ended with a list of the runs): 2049 ids
+// 15.7 / 19.7 / 19.5, 4096 16.6 / 20.8 / 20.2, 8192 17.7 / 21.9 / 29.8 / 39.6, 16384 20.3 / 24.4 / 32.6 / 85.  Beyond 65536 ids chunks of 16384.
 struct ScatterPlan {
     int per_thread, shift;
     size_t chunk, chunks;
@@ -511,9 +688,24 @@ bool scatter_rows_ok(const void* go, const float* gw, size_t hidden) {
     return hidden % 2 == 0 && eisen_aligned(go, 8) && eisen_aligned(gw, 8);
 }
 
-// Builds the index (3 * n_ids ints).  first_bad, if asked for, points at plan.chunks ints that the first kernel has written.
+// Whether the index is one launch of scatter_bucket_kernel; first_bad is one position then, else one per chunk.
+bool scatter_by_bucket(size_t n_ids, size_t vocab) { return n_ids <= kBucketMax && vocab <= kBucketVocab; }
+
+// Builds the index (the first 2 * n_ids ints of it).  first_bad, if asked for, points at what the first kernel has written.
 int scatter_launch_index(eisen_ctx* ctx, const int32_t* ids_dev, size_t n_ids, size_t vocab, const ScatterPlan& plan, int32_t* index, int32_t** first_bad) {
-    int32_t *sorted_ids = index, *order = index + n_ids, *runs = index + 2 * n_ids, *bad = nullptr;
+    int32_t *sorted_ids = index, *order = index + n_ids, *bad = nullptr;
+    if (scatter_by_bucket(n_ids, vocab)) {
+        if (first_bad) {
+            void* ws = nullptr;
+            const int rc = eisen_workspace(ctx, sizeof(int32_t), &ws);
+            if (rc) return rc;
+            *first_bad = (int32_t*)ws;
+        }
+        const size_t lds = kBucketWaves * eisen_ceil_div(vocab, (size_t)kBuckets) * sizeof(int);
+        scatter_bucket_kernel<<<kBuckets, kBucketThreads, lds, ctx->stream>>>(ids_dev, (int)n_ids, (int)vocab, sorted_ids, order, first_bad ? *first_bad : nullptr);
+        EISEN_LAUNCH_CHECK(ctx, "scatter_bucket_kernel");
+        return 0;
+    }
     int32_t *chunk_ids = sorted_ids, *chunk_order = order;
     if (plan.chunks > 1 || first_bad) {
         void* ws = nullptr;
@@ -526,78 +718,83 @@ int scatter_launch_index(eisen_ctx* ctx, const int32_t* ids_dev, size_t n_ids, s
         }
     }
     if (first_bad) *first_bad = bad;
-    int32_t* runs_now = plan.chunks == 1 ? runs : nullptr;
     const unsigned wgs = (unsigned)plan.chunks;
     if (plan.per_thread == 1)
-        scatter_sort_kernel<1><<<wgs, kSortThreads, 0, ctx->stream>>>(ids_dev, (int)n_ids, plan.shift, (int)vocab, chunk_ids, chunk_order, runs_now, bad);
+        scatter_sort_kernel<1><<<wgs, kSortThreads, 0, ctx->stream>>>(ids_dev, (int)n_ids, plan.shift, (int)vocab, chunk_ids, chunk_order, bad);
     else if (plan.per_thread == 2)
-        scatter_sort_kernel<2><<<wgs, kSortThreads, 0, ctx->stream>>>(ids_dev, (int)n_ids, plan.shift, (int)vocab, chunk_ids, chunk_order, runs_now, bad);
+        scatter_sort_kernel<2><<<wgs, kSortThreads, 0, ctx->stream>>>(ids_dev, (int)n_ids, plan.shift, (int)vocab, chunk_ids, chunk_order, bad);
     else
-        scatter_sort_kernel<16><<<wgs, kSortThreads, 0, ctx->stream>>>(ids_dev, (int)n_ids, plan.shift, (int)vocab, chunk_ids, chunk_order, runs_now, bad);
+        scatter_sort_kernel<16><<<wgs, kSortThreads, 0, ctx->stream>>>(ids_dev, (int)n_ids, plan.shift, (int)vocab, chunk_ids, chunk_order, bad);
     EISEN_LAUNCH_CHECK(ctx, "scatter_sort_kernel");
     return 0;
 }
-int scatter_launch_merge(eisen_ctx* ctx, size_t n_ids, const ScatterPlan& plan, int32_t* index) {
-    if (plan.chunks == 1) return 0;
+int scatter_launch_merge(eisen_ctx* ctx, size_t n_ids, size_t vocab, const ScatterPlan& plan, int32_t* index) {
+    if (plan.chunks == 1 || scatter_by_bucket(n_ids, vocab)) return 0;
     void* ws = nullptr;  // what scatter_launch_index filled: the same block, nothing has asked for a larger one since
     const int rc = eisen_workspace(ctx, (2 * n_ids + plan.chunks) * sizeof(int32_t), &ws);
     if (rc) return rc;
-    int32_t *sorted_ids = index, *order = index + n_ids, *runs = index + 2 * n_ids;
+    int32_t *sorted_ids = index, *order = index + n_ids;
     scatter_merge_kernel<<<(unsigned)eisen_ceil_div(n_ids, (size_t)kWave), kThreads, 0, ctx->stream>>>((const int32_t*)ws, (const int32_t*)ws + n_ids, (int)n_ids,
                                                                                                      (int)plan.chunk, sorted_ids, order);
-    scatter_runs_list_kernel<<<(unsigned)eisen_ceil_div(n_ids, (size_t)kSortThreads), kSortThreads, 0, ctx->stream>>>(sorted_ids, (int)n_ids, runs);
     EISEN_LAUNCH_CHECK(ctx, "scatter_merge_kernel");
     return 0;
 }
 
 template <typename T, bool WIDE>
-void scatter_launch_runs_as(eisen_ctx* ctx, const int32_t* index, const void* go, float* gw, size_t n_ids, size_t hidden) {
-    const size_t slabs = eisen_ceil_div(hidden, (size_t)kWave * (WIDE ? 4 : 2));
-    // at most 8 workgroups per CU for the short runs (they stride over the list), and what the long runs can use
-    const size_t blocks = std::max<size_t>(2, std::min<size_t>(256 * 8, eisen_ceil_div(n_ids * slabs, (size_t)(kThreads / kWave))) +
-                                                  std::min<size_t>(256 * 4, n_ids / kLongRun * eisen_ceil_div(hidden, (size_t)kWave)));
-    scatter_runs_kernel<T, WIDE><<<(unsigned)blocks, kThreads, 0, ctx->stream>>>((const T*)go, gw, index, index + n_ids, index + 2 * n_ids, (int)n_ids, (int)hidden);
+void scatter_launch_runs_as(eisen_ctx* ctx, const int32_t* index, const int32_t* first_bad, const void* go, float* gw, size_t n_ids, size_t hidden) {
+    // a workgroup for every long run (of more than 64 occurrences) and 64 columns that there can be, up to four per CU; a wave per window and 256 columns
+    // for the others
+    const size_t long_blocks = std::min<size_t>(1024, (n_ids - 1) / 64 * eisen_ceil_div(hidden, (size_t)64));
+    // (small batches: windows of 2 places, the waves are there)
+    const size_t slabs = eisen_ceil_div(hidden, (size_t)256), window = eisen_ceil_div(n_ids, (size_t)2) * slabs <= 4096 ? 2 : kRunWindow;
+    const size_t waves = eisen_ceil_div(n_ids, window) * slabs;
+    const size_t blocks = long_blocks + eisen_ceil_div(waves, (size_t)(kRunThreads / kWave));
+    scatter_runs_kernel<T, WIDE><<<(unsigned)blocks, kRunThreads, 0, ctx->stream>>>((const T*)go, gw, index, index + n_ids, first_bad, (int)n_ids, (int)hidden,
+                                                                                   (int)long_blocks, (int)window);
 }
-void scatter_launch_runs(eisen_ctx* ctx, const int32_t* index, const void* go, float* gw, int dtype, size_t n_ids, size_t hidden) {
+void scatter_launch_runs(eisen_ctx* ctx, const int32_t* index, const int32_t* first_bad, const void* go, float* gw, int dtype, size_t n_ids, size_t hidden) {
     // whole 16-byte packets of a row where the sizes and addresses give them, pairs of columns otherwise
     const bool wide = hidden % (dtype == EISEN_F32 ? 4 : 8) == 0 && eisen_aligned(go, 16) && eisen_aligned(gw, 16);
     if (dtype == EISEN_F32) {
-        if (wide) scatter_launch_runs_as<float, true>(ctx, index, go, gw, n_ids, hidden);
-        else scatter_launch_runs_as<float, false>(ctx, index, go, gw, n_ids, hidden);
+        if (wide) scatter_launch_runs_as<float, true>(ctx, index, first_bad, go, gw, n_ids, hidden);
+        else scatter_launch_runs_as<float, false>(ctx, index, first_bad, go, gw, n_ids, hidden);
     } else {
-        if (wide) scatter_launch_runs_as<bf16_t, true>(ctx, index, go, gw, n_ids, hidden);
-        else scatter_launch_runs_as<bf16_t, false>(ctx, index, go, gw, n_ids, hidden);
+        if (wide) scatter_launch_runs_as<bf16_t, true>(ctx, index, first_bad, go, gw, n_ids, hidden);
+        else scatter_launch_runs_as<bf16_t, false>(ctx, index, first_bad, go, gw, n_ids, hidden);
     }
 }
 
-// ids_dev -> index -> scatter.  With `check` the ids are checked first: the positions of the bad ones come back beside the
-// merge, the host waits for that copy alone, and *bad tells that nothing was added.
+// ids_dev -> index -> scatter.  With `check` the ids are checked first: the positions of the bad ones come back beside what
+// follows, the host waits for that copy alone, and *bad tells that nothing was added.  One position: the scatter itself looks at it
+// and is launched before the host knows.
 int scatter_device_route(eisen_ctx* ctx, const int32_t* ids_dev, const void* go, float* gw, int dtype, size_t n_ids, size_t vocab, size_t hidden,
                          const ScatterPlan& plan, bool check, bool* bad) {
     *bad = false;
     void* dev = nullptr;
-    int rc = eisen_hip_malloc(ctx, 3 * n_ids * sizeof(int32_t), &dev);
+    int rc = eisen_hip_malloc(ctx, 2 * n_ids * sizeof(int32_t), &dev);
     if (rc) return rc;
     {
         // algorithmic bytes: every row of dOut read once, every touched row of the f32 gradient read and written once; the
         // touched rows are not known on the host here, so the entry counts dOut and the index only (a lower bound)
         EisenProfScope prof(ctx, dtype == EISEN_BF16 ? "scatter_rows_bf16" : "scatter_rows_f32",
                             (double)n_ids * (double)hidden * eisen_dtype_size(dtype) + 16.0 * (double)n_ids);
+        const bool one = scatter_by_bucket(n_ids, vocab);
         int32_t* first_bad = nullptr;
         rc = scatter_launch_index(ctx, ids_dev, n_ids, vocab, plan, (int32_t*)dev, check ? &first_bad : nullptr);
         int32_t found[kIndexMax / 2048];
         int ticket = -1;
-        const size_t found_bytes = plan.chunks * sizeof(int32_t);
+        const size_t chunks = one ? 1 : plan.chunks, found_bytes = chunks * sizeof(int32_t);
         if (!rc && check && eisen_hip_dtoh_begin(ctx, first_bad, found_bytes, &ticket)) {
             ticket = -1;  // every staging slot is taken: a plain copy
             rc = eisen_hip_dtoh(ctx, found, first_bad, found_bytes);
         }
-        const int rc_merge = rc ? rc : scatter_launch_merge(ctx, n_ids, plan, (int32_t*)dev);
+        const int rc_merge = rc ? rc : scatter_launch_merge(ctx, n_ids, vocab, plan, (int32_t*)dev);
+        if (!rc_merge && one) scatter_launch_runs(ctx, (const int32_t*)dev, first_bad, go, gw, dtype, n_ids, hidden);
         if (ticket >= 0) rc = eisen_hip_dtoh_finish(ctx, ticket, found, found_bytes);
         if (!rc) rc = rc_merge;
         if (!rc && check)
-            for (size_t c = 0; c < plan.chunks; c++) *bad = *bad || found[c] != kNoId;
-        if (!rc && !*bad) scatter_launch_runs(ctx, (const int32_t*)dev, go, gw, dtype, n_ids, hidden);
+            for (size_t c = 0; c < chunks; c++) *bad = *bad || found[c] != kNoId;
+        if (!rc && !*bad && !one) scatter_launch_runs(ctx, (const int32_t*)dev, nullptr, go, gw, dtype, n_ids, hidden);
     }
     hipError_t e = hipGetLastError();
     const int rc_free = eisen_hip_free(ctx, dev);  // stream-ordered: the block is reused only by later work
@@ -738,7 +935,7 @@ extern "C" int eisen_hip_gather_index_dev(eisen_ctx* ctx, const int32_t* ids_dev
                   "gather_index_dev: %zu ids of a vocabulary of %zu are more than the device-side index takes", n_ids, vocab);
     EisenProfScope prof(ctx, "scatter_index", 16.0 * (double)n_ids);
     const int rc = scatter_launch_index(ctx, ids_dev, n_ids, vocab, plan, index, nullptr);
-    return rc ? rc : scatter_launch_merge(ctx, n_ids, plan, index);
+    return rc ? rc : scatter_launch_merge(ctx, n_ids, vocab, plan, index);
 }
 
 extern "C" int eisen_hip_gather_backward_indexed(eisen_ctx* ctx, const int32_t* index, const void* go, float* gw, int dtype, size_t n_ids,
@@ -752,7 +949,7 @@ extern "C" int eisen_hip_gather_backward_indexed(eisen_ctx* ctx, const int32_t* 
     EISEN_REQUIRE(ctx, scatter_rows_ok(go, gw, hidden) && scatter_index_ahead(n_ids, vocab), EISEN_E_SHAPE,
                   "gather_backward_indexed: rows of %zu values at these addresses need eisen_hip_gather_backward_dev", hidden);
     EisenProfScope prof(ctx, dtype == EISEN_BF16 ? "scatter_rows_bf16" : "scatter_rows_f32", (double)n_ids * (double)hidden * eisen_dtype_size(dtype) + 16.0 * (double)n_ids);
-    scatter_launch_runs(ctx, index, go, gw, dtype, n_ids, hidden);
+    scatter_launch_runs(ctx, index, nullptr, go, gw, dtype, n_ids, hidden);
     EISEN_LAUNCH_CHECK(ctx, "scatter_runs_kernel");
     return 0;
 }

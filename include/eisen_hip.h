@@ -459,7 +459,7 @@ int eisen_hip_gather_backward(eisen_ctx* ctx, const int32_t* ids_host, const voi
                               size_t n_ids, size_t vocab, size_t hidden);
 /* The same scatter with the ids already on the device (the int32 buffer eisen_hip_gather read): nothing is sorted or
  * uploaded by the host.  Up to 2^20 ids whose keys fit 32 bits (vocab * 2048, or * 16384 beyond 65536 ids) are indexed on
- * the device (stable sorts of chunks by id in LDS, merged) and scattered run by run; other shapes read the ids back (which
+ * the device (counted and placed by residue, or stable sorts of chunks by id in LDS, merged) and scattered run by run; other shapes read the ids back (which
  * synchronises) and take eisen_hip_gather_backward.  The ids must lie in [0, vocab), as they did for the gather.  An id outside
  * is skipped in the batches that eisen_hip_gather_index_dev takes; in others it is an error and nothing is added (the call
  * waits for that check, which runs beside the indexing). */
