@@ -62,7 +62,8 @@ struct DqLds {
     __attribute__((aligned(1024))) bf16_t v[kDqTiles<HD>];
     __attribute__((aligned(1024))) bf16_t rows[kDqRows<HD, kAblNone>];
 };
-template <int HD, int ABL, int GW = 0>
+// ONE: a workgroup takes one key block, not a pair (key_blocks_paired; head sizes above 64 have a.kb_paired in launches of their own).
+template <int HD, int ABL, int GW = 0, bool ONE = false>
 __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(AttnArgs a) {
     constexpr bool OWN = GW > 0;
     constexpr int KSTEPS = HD / 16, DT = (HD + 31) / 32, NST = 2;
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void fa_bwd_dkv32_kernel(Att
     // grid: x = key-block pair, fastest; then KV head, then batch.  Blocks of one (batch, KV head) read the same
     // Q / dO tiles, so they are kept on one XCD.
     // Without pairs: the key block slowest, longest (causal) first.
-    const bool paired = HD <= 64 || OWN || a.paired;
+    const bool paired = !ONE && (HD <= 64 || OWN || a.kb_paired);
     const int bid = paired ? xcd_contiguous_id(block, blocks) : block;
     const int pair = paired ? bid % n_pairs : bid / (a.Hkv * a.B), of = paired ? bid / n_pairs : bid % (a.Hkv * a.B);
     const int kvh = of % a.Hkv, b = of / a.Hkv;
@@ -389,6 +390,13 @@ bool eisen_attention_writes_over_operand(const AttnArgs& a, size_t element) {
     return a.dQ == a.dK || a.dQ == a.dV;
 }
 
+// Whether a dK / dV workgroup takes two key blocks, a long one and its short mirror image (for equal work), or one: where there are places for all of
+// them at once (two workgroups to a CU; one for head sizes above 64), beside those of the dQ pass that share the launch, the pair would only be done one after the
+// other.  The results are the same to the bit.  Backward with pairs / without, us, batch x sequence, query heads on KV heads, head size: 10 x 44 8 on 8 64 7.9 / 6.2; 1 x
+// 130 3 on 3 64 9.2 / 7.2; 7 x 193 6 on 6 48 8.9 / 8.1; 1 x 506 4 on 2 64 20.6 / 18.2; 3 x 512 8 on 8 64 16.2 / 14.2; 2 x 1000 6 on 6 64 24.7 / 21.3; 1 x 512 8 on 4
+// 96 30.1 / 26.3; 1 x 2048 2 on 2 128 61.8 / 57.2; in two launches 2 x 448 9 on 3 80 34.2 / 29.2; 7 x 668 6 on 3 64 30.0 / 30.0.
+static bool key_blocks_paired(const AttnArgs& a, int dq_blocks) { return dq_blocks + (long long)((a.S + 31) / 32) * a.Hkv * a.B > (a.hd <= 64 ? 512 : 256); }
+
 // Where one launch (fa_bwd_dkv32_kernel with GW > 0) takes less time than two: where every workgroup is on the chip at once, two to a CU (head sizes above 64: one), and a
 // workgroup of the dK / dV role has few enough statistics to compute before it starts.  With larger query groups there are fewer of these
 // workgroups, each with more tiles, and the statistics come on top of what was the longer pass already.  Two launches / one, us, causal, batch x sequence,
@@ -396,21 +404,30 @@ bool eisen_attention_writes_over_operand(const AttnArgs& a, size_t element) {
 // 38.3; 4 x 256 8 on 8 128 30.6 / 19.4.  Beyond the lines: 8 x 256 16 on 16 64 (768 workgroups) 20.2 / 20.6, 16 x 256 33.0 / 37.9; 4 x 256 24 on 8 64 19.3 / 19.8;
 // 1 x 512 32 on 8 64 28.6 / 33.4; 1 x 512 16 on 4 128 53.5 / 61.2; 2 x 256 32 on 4 64 26.2 / 34.2.  At them: 8 x 128 8 on 2 64 15.3 / 13.9; 21 x 256 8 on 2 32 17.6 / 16.2;
 // 8 x 256 8 on 2 48 19.0 / 18.1; 4 x 64 16 on 2 64 15.2 / 14.6; 1 x 1024 16 on 8 64 35.3 / 34.1.
+// Three query heads on a KV head, no pairs of key blocks: 2 x 448 9 on 3 80 29.0 / 24.6; 3 x 500 6 on 2 48 22.2 / 17.7; 1 x 400 24 on 8 32 16.4 / 14.6; 2 x 200 9 on 3 64 15.6 / 14.1, but 1 x
+// 600 9 on 3 64 26.3 / 28.2 and 1 x 640 9 on 3 128 48.0 / 54.6.
 bool eisen_attention_bwd_short_supports(const AttnArgs& a, int dq_blocks) {
     const int n_qt = (a.S + 31) / 32;
-    const int most = a.G <= 2 ? kOwnTiles : a.G <= 4 && a.hd != 64 ? 32 : 16;
+    const bool three = a.G == 3 && !key_blocks_paired(a, dq_blocks);
+    const int most = a.G <= 2 || (three && (a.hd < 64 || a.hd == 80)) ? kOwnTiles : three || (a.G <= 4 && a.hd != 64) ? 32 : 16;
     const long long blocks = dq_blocks + (long long)(n_qt + 1) / 2 * a.Hkv * a.B;
     return a.G * n_qt <= most && blocks <= (a.hd <= 64 ? 512 : 256) && a.ablation == kAblNone && eisen_attention_dkv32_supports(a) && !eisen_attention_writes_over_operand(a, 2);
 }
 
 void eisen_attention_launch_bwd_short(eisen_ctx* ctx, AttnArgs a, int gw, int dq_blocks) {
     a.dq_blocks = dq_blocks;
-    const int blocks = dq_blocks + ((a.S + 31) / 32 + 1) / 2 * a.Hkv * a.B;
+    a.kb_paired = key_blocks_paired(a, dq_blocks);
+    const int blocks = dq_blocks + (a.kb_paired ? ((a.S + 31) / 32 + 1) / 2 : (a.S + 31) / 32) * a.Hkv * a.B;
     auto launch = [&](auto hd) {
         constexpr int HD = decltype(hd)::value;
-        if (gw == 4) fa_bwd_dkv32_kernel<HD, kAblNone, 4><<<blocks, 256, 0, ctx->stream>>>(a);
-        else if (gw == 2) fa_bwd_dkv32_kernel<HD, kAblNone, 2><<<blocks, 256, 0, ctx->stream>>>(a);
-        else fa_bwd_dkv32_kernel<HD, kAblNone, 1><<<blocks, 256, 0, ctx->stream>>>(a);
+        auto as = [&](auto one_c) {
+            constexpr bool ONE = decltype(one_c)::value;
+            if (gw == 4) fa_bwd_dkv32_kernel<HD, kAblNone, 4, ONE><<<blocks, 256, 0, ctx->stream>>>(a);
+            else if (gw == 2) fa_bwd_dkv32_kernel<HD, kAblNone, 2, ONE><<<blocks, 256, 0, ctx->stream>>>(a);
+            else fa_bwd_dkv32_kernel<HD, kAblNone, 1, ONE><<<blocks, 256, 0, ctx->stream>>>(a);
+        };
+        if (a.kb_paired) as(std::false_type{});
+        else as(std::true_type{});
     };
     switch (a.hd) {
         case 16: return launch(std::integral_constant<int, 16>{});
@@ -428,9 +445,9 @@ void eisen_attention_launch_bwd_short(eisen_ctx* ctx, AttnArgs a, int gw, int dq
 void eisen_attention_launch_dkv32(eisen_ctx* ctx, AttnArgs a) {
     const int n_kb = (a.S + 31) / 32;  // 32-key blocks, handled in heavy / light pairs or one by one
     const long long pairs = (long long)(n_kb + 1) / 2 * a.Hkv * a.B;
-    a.paired = a.hd <= 64 || pairs <= 256;
-    dim3 grid((unsigned)(a.paired ? pairs : (long long)n_kb * a.Hkv * a.B));
-    if (a.hd == 64) {
+    a.kb_paired = (a.hd <= 64 || pairs <= 256) && (a.ablation != kAblNone || key_blocks_paired(a, 0));
+    dim3 grid((unsigned)(a.kb_paired ? pairs : (long long)n_kb * a.Hkv * a.B));
+    if (a.hd == 64 && (a.kb_paired || a.ablation != kAblNone)) {
         switch (a.ablation) {  // hd 64 only: the head size the measurements are quoted for
             case kAblTransposedReads: fa_bwd_dkv32_kernel<64, kAblTransposedReads><<<grid, 256, 0, ctx->stream>>>(a); break;
             case kAblOperandReads: fa_bwd_dkv32_kernel<64, kAblOperandReads><<<grid, 256, 0, ctx->stream>>>(a); break;
@@ -446,7 +463,11 @@ void eisen_attention_launch_dkv32(eisen_ctx* ctx, AttnArgs a) {
     else if (a.hd == 112) fa_bwd_dkv32_kernel<112, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
     else if (a.hd == 96) fa_bwd_dkv32_kernel<96, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
     else if (a.hd == 80) fa_bwd_dkv32_kernel<80, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
-    else if (a.hd == 48) fa_bwd_dkv32_kernel<48, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
-    else if (a.hd == 32) fa_bwd_dkv32_kernel<32, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
-    else fa_bwd_dkv32_kernel<16, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
+    else if (a.hd == 64) fa_bwd_dkv32_kernel<64, kAblNone, 0, true><<<grid, 256, 0, ctx->stream>>>(a);
+    else if (a.hd == 48 && a.kb_paired) fa_bwd_dkv32_kernel<48, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
+    else if (a.hd == 48) fa_bwd_dkv32_kernel<48, kAblNone, 0, true><<<grid, 256, 0, ctx->stream>>>(a);
+    else if (a.hd == 32 && a.kb_paired) fa_bwd_dkv32_kernel<32, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
+    else if (a.hd == 32) fa_bwd_dkv32_kernel<32, kAblNone, 0, true><<<grid, 256, 0, ctx->stream>>>(a);
+    else if (a.kb_paired) fa_bwd_dkv32_kernel<16, kAblNone><<<grid, 256, 0, ctx->stream>>>(a);
+    else fa_bwd_dkv32_kernel<16, kAblNone, 0, true><<<grid, 256, 0, ctx->stream>>>(a);
 }

@@ -16,7 +16,8 @@ struct AttnArgs {
     long long k_sb, k_ss, k_sh;
     float scale, scale_log2e;
     int causal;
-    int paired;  // a block runs a long query (dK / dV kernel: key) block and its short mirror image
+    int paired;  // a block runs a long query block and its short mirror image
+    int kb_paired;  // the same for the key blocks of the dK / dV kernel
     int dq_blocks;  // both passes of the backward in one launch: the workgroups of the dQ pass
     // backward only: when set ([S][hd/2] cos/sin), Q and K are rotary-embedded projections and dQ, dK are the
     // gradients of the projections before the rotation (the inverse rotation is applied as the gradients are stored)
