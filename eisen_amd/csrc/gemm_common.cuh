@@ -45,7 +45,7 @@ struct GemmArgs {
     const void* B_seg[2];
     int lda_seg[2], ldb_seg[2];
     int seg_end[2];
-    // Rotary-embedding epilogue (rope != nullptr; bf16 C, no accumulation or residual; of a split product in the reduction): the batch members
+    // Rotary-embedding epilogue (rope != nullptr; bf16 C, or f32 C of a group; no accumulation or residual; of a split product in the reduction): the batch members
     // below rope_members leave as rope(A*B), row m at position m % rope_seq, heads of rope_head_dim columns (a multiple of 8)
     const float2* rope;                // cos/sin table [>= rope_seq][rope_head_dim / 2]
     int rope_seq, rope_head_dim, rope_members;
@@ -203,7 +203,7 @@ __device__ __forceinline__ void store_eight(TC* p, typename Eight<TC>::V v) { *r
 // Row m, columns n..n+7 of the product, stored with whatever epilogue the launch asks for; columns from g.N on are left out.
 // P: the partial result goes there instead.  first: the old C or the residual (add_old), or gate, and second: up, for the
 // columns of a whole packet (a cut one reads its own).
-template <typename TC>
+template <typename TC, bool ROPE = sizeof(TC) == 2>
 __device__ __forceinline__ void gemm_store_eight(const GemmArgs& g, float (&val)[8], int m, int n, int bz, TC* C, const TC* Rsrc, bool add_old, float* P,
                                                  typename Eight<TC>::V first, typename Eight<TC>::V second) {
     const long long at = (long long)m * g.ldc + n;
@@ -256,8 +256,8 @@ __device__ __forceinline__ void gemm_store_eight(const GemmArgs& g, float (&val)
         }
         return;
     }
-    if constexpr (sizeof(TC) == 2) {
-        if (g.rope && bz < g.rope_members) {  // the product rounded to bf16 and then rotated, as the separate rotary kernel would find it (N is whole heads)
+    if constexpr (ROPE) {
+        if (g.rope && bz < g.rope_members) {  // the product rounded to C's type and then rotated, as the separate rotary kernel would find it (N is whole heads)
             const float4* t = reinterpret_cast<const float4*>(g.rope + (long long)(m % g.rope_seq) * (g.rope_head_dim >> 1) + ((n % g.rope_head_dim) >> 1));
 #pragma unroll
             for (int q = 0; q < 2; q++) {

@@ -147,7 +147,8 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g, 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int split = g.split > 1 ? g.split : 1;
-    int nt, mt = 0, zz;
+    constexpr bool kRope = KIND == Kind::kGroup && A_KC && !B_KC;  // (the rotary epilogue: of X W)
+    int nt, mt = 0, zz, member = 0;
     if constexpr (KIND == Kind::kGroup) {  // which product this tile belongs to (uniform); static indices keep the tables in scalar registers
         const int tiles = g.grp_tile_end[kMaxGroup - 1];
         const int lin = xcd_contiguous_id(blockIdx.x, tiles * split);
@@ -159,6 +160,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g, 
 #pragma unroll
         for (int q = 1; q < kMaxGroup; q++)
             if (t >= g.grp_tile_end[q - 1]) {
+                if constexpr (kRope) member = q;
                 first = g.grp_tile_end[q - 1];
                 partial_off = g.grp_partial_off[q];
                 g.A = g.grp_A[q]; g.B = g.grp_B[q]; g.C = g.grp_C[q]; g.N = g.grp_N[q];
@@ -469,7 +471,8 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_f32_sliced_kernel(GemmArgs g, 
                 second = load_eight(static_cast<const float*>(g.up) + (long long)bz * g.sC + at);
             }
         }
-        gemm_store_eight<float>(g, val[ps], m, n, bz, C, Rsrc, add_old, P, first, second);
+        // (part 0 of a split contraction stands in C as it is: the reduction rotates)
+        gemm_store_eight<float, kRope>(g, val[ps], m, n, !kRope ? bz : split > 1 ? g.rope_members : member, C, Rsrc, add_old, P, first, second);
     });
 }
 

@@ -929,7 +929,14 @@ std::vector<size_t> Graph::matmul_group(size_t a, const std::vector<size_t>& ws,
         const bool with_h = swiglu_h && n == 2 && N[0] == N[1];
         if (swiglu_h) *swiglu_h = with_h ? push_tensor({M, N[0]}, da.dtype, true) : (size_t)-1;
         if (with_h) check(eisen_hip_gemm_swiglu_forward(ctx_, da.ptr, Bs[0], Bs[1], Cs[0], Cs[1], at(*swiglu_h).data.ptr, EISEN_F32, M, N[0], K), "matmul_group");
-        else check(eisen_hip_gemm_grouped(ctx_, n, As, Bs, Cs, N.data(), EISEN_F32, EISEN_F32, 0, 0, M, K, 0), "matmul_group");
+        else {
+            // rotary embedding of the first outputs by the launch that forms them, where it can (see eisen_hip_gemm_grouped_rope)
+            size_t rope_n = rotated && !swiglu_h && sa.size() == 3 && sa[1] > 0 && K % 4 == 0 && rope_head_dim >= 8 && rope_head_dim % 8 == 0 ? std::min(rope_members, n) : 0;
+            for (size_t i = 0; i < n; i++)
+                if (N[i] % 4 || (i < rope_n && N[i] % rope_head_dim)) rope_n = 0;
+            if (rope_n > 0) *rotated = true;
+            check(eisen_hip_gemm_grouped_rope(ctx_, n, da.ptr, Bs, Cs, N.data(), M, K, rope_n, rope_n ? sa[1] : 0, rope_head_dim), "matmul_group");
+        }
         auto epoch = std::make_shared<size_t>((size_t)-1);
         auto fn = [=](Graph& g) {
             if (*epoch == g.backward_epoch()) return;  // the node is on the tape once per output; it runs once per backward

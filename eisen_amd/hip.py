@@ -300,6 +300,11 @@ class Context:
         self._call("eisen_hip_gemm_forward_group", _sz(n), _ptr(A), (_vp * n)(*[_ptr(b) for b in Bs]), (_vp * n)(*[_ptr(c) for c in Cs]), (_sz * n)(*Ns),
                    _i(dtype), _sz(M), _sz(K), _sz(rope_members), _sz(seq), _sz(head_dim))
 
+    def gemm_grouped_rope(self, A, Bs, Cs, Ns, M, K, rope_members=0, seq=0, head_dim=0):
+        n = len(Bs)
+        self._call("eisen_hip_gemm_grouped_rope", _sz(n), _ptr(A), (_vp * n)(*[_ptr(b) for b in Bs]), (_vp * n)(*[_ptr(c) for c in Cs]), (_sz * n)(*Ns),
+                   _sz(M), _sz(K), _sz(rope_members), _sz(seq), _sz(head_dim))
+
     def rope_backward(self, go, gx, dtype, batch, seq, hidden, head_dim, accumulate=0):
         self._call("eisen_hip_rope_backward", _ptr(go), _ptr(gx), _i(dtype), _sz(batch), _sz(seq), _sz(hidden), _sz(head_dim), _i(accumulate))
 

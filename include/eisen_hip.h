@@ -246,6 +246,11 @@ int eisen_hip_gemm_rope(eisen_ctx* ctx, const void* A, const void* B, void* C, i
 int eisen_hip_gemm_forward_group(eisen_ctx* ctx, size_t n, const void* A, const void* const* B, void* const* C, const size_t* N, int dtype, size_t M,
                                  size_t K, size_t rope_members, size_t seq, size_t head_dim);
 
+/* The same for f32: eisen_hip_gemm_grouped over products that share A, the first `rope_members` of them rotated.  The rotation is part of that launch
+ * where the operands' rows start on 16-byte boundaries and head_dim is a multiple of 8, else launches behind it; the same bits either way. */
+int eisen_hip_gemm_grouped_rope(eisen_ctx* ctx, size_t n, const void* A, const void* const* B, void* const* C, const size_t* N, size_t M, size_t K,
+                                size_t rope_members, size_t seq, size_t head_dim);
+
 /* eisen_hip_rope of two tensors that share batch, seq and head_dim in one launch: the q and k projections of
  * GroupedQueryAttention::forward_with_mask (src/nn/attention.rs:304-305, two `g.rope` calls). */
 int eisen_hip_rope_pair(eisen_ctx* ctx, const void* q, void* q_out, size_t hidden_q, const void* k, void* k_out, size_t hidden_k, int dtype,
