@@ -24,6 +24,17 @@ std::string shape_str(const std::vector<size_t>& s) {
     return r + "]";
 }
 constexpr size_t kHostCopyLimit = size_t(1) << 22;  // elements; token-id tensors are far below
+constexpr size_t kIdsLimit = size_t(24) << 10;      // elements that eisen_hip_htod_values takes in one launch
+
+// Whether all values are whole numbers from 0 below 2^23 (in blocks: what is no ids says so in its first one).
+bool whole_numbers(const float* v, size_t n) {
+    for (size_t b = 0; b < n; b += 64) {
+        bool whole = true;
+        for (size_t i = b; i < std::min(n, b + 64); i++) whole &= (v[i] >= 0.0f) & (v[i] < 8388608.0f) & ((v[i] + 8388608.0f) - 8388608.0f == v[i]);
+        if (!whole) return false;
+    }
+    return true;
+}
 }  // namespace
 
 std::vector<size_t> compute_strides(const std::vector<size_t>& shape) {
@@ -98,18 +109,18 @@ void Graph::device_free(Storage& s) {
     s = Storage();
 }
 void Graph::release(Tensor& t) {
-    void* const bufs[3] = {t.data.ptr, t.grad_borrowed ? nullptr : t.grad.ptr, t.shadow.ptr};
-    t.data = t.grad = t.shadow = Storage();
+    void* const bufs[4] = {t.data.ptr, t.grad_borrowed ? nullptr : t.grad.ptr, t.shadow.ptr, t.ids.ptr};
+    t.data = t.grad = t.shadow = t.ids = Storage();
     for (void* p : bufs) free_buffer(p);
 }
 
-size_t Graph::push_tensor(const std::vector<size_t>& shape, int dtype, bool pooled) {
+size_t Graph::push_tensor(const std::vector<size_t>& shape, int dtype, bool pooled, bool with_data) {
     Tensor t;
     t.id = tensors.size();
     t.shape = shape;
     t.strides = compute_strides(shape);
     t.is_pooled = pooled;
-    t.data = device_alloc(numel_of(shape), dtype, false);
+    if (with_data) t.data = device_alloc(numel_of(shape), dtype, false);
     tensors.push_back(std::move(t));
     return tensors.size() - 1;
 }
@@ -155,15 +166,15 @@ void Graph::load_tensor_data(size_t id, const float* host, size_t n) {
     if (n != t.size()) throw Error("Shape mismatch: Tensor " + std::to_string(id) + " expects " + std::to_string(t.size()) + " elements, but got " + std::to_string(n) + ".");
     if (n <= kHostCopyLimit) t.host_copy.assign(host, host + n);
     else t.host_copy.clear();
-    if (t.data.dtype == EISEN_F32) {
-        check(eisen_hip_htod(ctx_, t.data.ptr, host, n * sizeof(float)), "load_tensor_data");
-        refresh_shadow(id);
-    } else {
-        Storage tmp = device_alloc(n, EISEN_F32, false);
-        check(eisen_hip_htod(ctx_, tmp.ptr, host, n * sizeof(float)), "load_tensor_data");
-        check(eisen_hip_cast(ctx_, tmp.ptr, EISEN_F32, t.data.ptr, EISEN_BF16, n), "load_tensor_data cast");
-        device_free(tmp);
+    // what may be token ids goes to the device as int32 too, for a gather (as one launch, so for small tensors only)
+    const bool ids = t.is_pooled && n > 0 && n <= kIdsLimit && whole_numbers(host, n);
+    if (!ids) device_free(t.ids);
+    else if (t.ids.numel != n) {
+        device_free(t.ids);
+        t.ids = device_alloc(n, EISEN_F32, false);
     }
+    check(eisen_hip_htod_values(ctx_, t.data.ptr, t.data.dtype, (int32_t*)t.ids.ptr, host, n), "load_tensor_data");
+    if (t.data.dtype == EISEN_F32) refresh_shadow(id);
 }
 
 // A storage's values as f32, straight into the caller's memory (of what a large read-back costs, fresh host memory touched for the first time is a good part).
@@ -1361,21 +1372,23 @@ size_t Graph::gather(size_t weights, size_t indices) {
         std::vector<float> host = sync_to_cpu(indices);  // ids that never came from the host: read them back
         at(indices).host_copy = host;
     }
-    std::vector<int32_t> ids(n);
+    const bool loaded = n > 0 && at(indices).ids.numel == n;  // (the int32 of host_copy)
+    std::vector<int32_t> ids(loaded ? 0 : n);
     const std::vector<float>& hc = at(indices).host_copy;
     for (size_t i = 0; i < n; i++) {
         const float f = hc[i];
         if (!(f >= 0.0f) || (size_t)f >= vocab) throw Error("gather: index " + std::to_string(f) + " at position " + std::to_string(i) + " outside [0, " + std::to_string(vocab) + ")");
-        ids[i] = (int32_t)f;
+        if (!loaded) ids[i] = (int32_t)f;
     }
     const Storage dw = compute_data(weights);
     std::vector<size_t> os = at(indices).shape;
     os.push_back(hidden);
     // the ids as int32 on the device: a pooled tensor, so that the backward pass finds them there and they leave with
     // the activations
-    const size_t dids = push_tensor({n}, EISEN_F32, true);  // int32 payload
+    const size_t dids = push_tensor({n}, EISEN_F32, true, !loaded);  // int32 payload
+    if (loaded) std::swap(at(dids).data, at(indices).ids);  // what load_tensor_data has brought (a second gather from it uploads its own)
     const size_t out = push_tensor(os, dw.dtype, true);
-    check(eisen_hip_htod(ctx_, at(dids).data.ptr, ids.data(), n * sizeof(int32_t)), "gather ids");
+    if (!loaded) check(eisen_hip_htod(ctx_, at(dids).data.ptr, ids.data(), n * sizeof(int32_t)), "gather ids");
     check(eisen_hip_gather(ctx_, dw.ptr, (const int32_t*)at(dids).data.ptr, at(out).data.ptr, dw.dtype, n, vocab, hidden), "gather");
     // The position index of the backward scatter depends on the ids alone: it is built now, on the side stream beside the
     // forward pass (10 to 20 us for up to 16384 ids), instead of in front of the last kernel of the backward pass.

@@ -41,6 +41,7 @@ struct Tensor {
     Storage data;            // activations: f32 or bf16; parameters: f32 master
     Storage grad;            // parameters: f32, allocated with the tensor; activations: lazily, activation dtype
     Storage shadow;          // parameters in Bf16Mixed: bf16 copy of `data` the kernels read
+    Storage ids;             // host_copy as int32 on the device (the payload of an f32 storage), until a gather takes it over
     std::string name;
     bool is_pooled = false;
     bool is_param = false;        // allocated through alloc()/alloc_param_bf16(): owns an f32 grad
@@ -271,7 +272,7 @@ class Graph {
     bool window_take(size_t weight, const void* x, const void* dy, int dtype, size_t rows, size_t in, size_t out);
     bool window_fits(size_t weight, int dtype, size_t rows, size_t in, size_t out);
     void free_buffer(void* ptr);  // eisen_hip_free unless the buffer is held
-    size_t push_tensor(const std::vector<size_t>& shape, int dtype, bool pooled);
+    size_t push_tensor(const std::vector<size_t>& shape, int dtype, bool pooled, bool with_data = true);
     Storage device_alloc(size_t numel, int dtype, bool zero);
     void download(const Storage& s, float* out);
     void device_free(Storage& s);

@@ -3,6 +3,8 @@
 // (src/graph/mod.rs:152-307, src/graph/memory.rs:189-266, src/tensor.rs:145-223).
 #include "runtime.h"
 
+#include "device_utils.cuh"
+
 #include <algorithm>
 #include <atomic>
 #include <thread>
@@ -46,6 +48,39 @@ __device__ __forceinline__ void copy_by_workgroup(const T* __restrict__ src, T* 
 template <typename T>
 __global__ __launch_bounds__(kCopyThreads) void copy_in_kernel(const T* __restrict__ src, T* __restrict__ dst, unsigned n, unsigned* word, unsigned number) {
     copy_by_workgroup(src, dst, n);
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// f32 values to a tensor of T and, if asked for, as int32 beside it (token ids: what the lookup reads).  dst and ids begin 16 bytes aligned.
+// What bounds it is the latency of the host's memory, so one launch instead of three (the values, their rounding, the ids: 5 + 3 + 5 us): training steps of 8 micro-batches of
+// 1024 tokens 10427 -> 10338 us, of one of 1351 593 -> 584, of 64 (f32, where nothing is rounded) 272 -> 262.
+template <typename T>
+__global__ __launch_bounds__(kCopyThreads) void copy_in_values_kernel(const float* __restrict__ src, T* __restrict__ dst, int* __restrict__ ids, unsigned n, unsigned* word,
+                                                                      unsigned number) {
+    constexpr int U = 4;
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const unsigned quads = n / 4;
+    for (unsigned i = threadIdx.x; i < quads; i += U * kCopyThreads) {
+        float4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i + u * kCopyThreads < quads) v[u] = reinterpret_cast<const float4*>(src)[i + u * kCopyThreads];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const unsigned at = i + u * kCopyThreads;
+            if (at >= quads) continue;
+            T4 o;
+            o[0] = from_f32<T>(v[u].x); o[1] = from_f32<T>(v[u].y); o[2] = from_f32<T>(v[u].z); o[3] = from_f32<T>(v[u].w);
+            reinterpret_cast<T4*>(dst)[at] = o;
+            if (ids) reinterpret_cast<int4*>(ids)[at] = make_int4((int)v[u].x, (int)v[u].y, (int)v[u].z, (int)v[u].w);
+        }
+    }
+    if (threadIdx.x < n % 4) {
+        const unsigned at = quads * 4 + threadIdx.x;
+        const float v = src[at];
+        dst[at] = from_f32<T>(v);
+        if (ids) ids[at] = (int)v;
+    }
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -96,11 +131,14 @@ int wait_slot(eisen_ctx* ctx, eisen_ctx::StageSlot& s) {
     EISEN_HIP_TRY(ctx, hipEventSynchronize(s.done));
     return 0;
 }
-// The slot's memory to the device by a kernel, where size and alignment let it and nothing is being captured (a replay would set the word again); false: not.
-bool upload_by_kernel(eisen_ctx* ctx, eisen_ctx::StageSlot& s, void* dst, size_t bytes) {
-    if (bytes > kCopyKernelBytes || bytes % 4 != 0 || !eisen_aligned(dst, 4)) return false;
+// Under capture no kernel uploads: a replay would set the word again.
+bool stream_captures(eisen_ctx* ctx) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+    return hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+}
+// The slot's memory to the device by a kernel, where size and alignment let it; false: not.
+bool upload_by_kernel(eisen_ctx* ctx, eisen_ctx::StageSlot& s, void* dst, size_t bytes) {
+    if (bytes > kCopyKernelBytes || bytes % 4 != 0 || !eisen_aligned(dst, 4) || stream_captures(ctx)) return false;
     s.number++;
     if (bytes % 16 == 0 && eisen_aligned(dst, 16))
         copy_in_kernel<<<1, kCopyThreads, 0, ctx->stream>>>(static_cast<const uint4*>(s.ptr), static_cast<uint4*>(dst), (unsigned)(bytes / 16), s.word, s.number);
@@ -487,6 +525,44 @@ extern "C" int eisen_hip_htod(eisen_ctx* ctx, void* dst, const void* src, size_t
     EISEN_HIP_TRY(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     EISEN_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return 0;
+}
+
+extern "C" int eisen_hip_htod_values(eisen_ctx* ctx, void* dst, int dtype, int32_t* ids, const float* src, size_t n) {
+    EISEN_CHECK_CTX(ctx);
+    EISEN_REQUIRE(ctx, dst && src, EISEN_E_ARG, "eisen_hip_htod_values: null pointer");
+    EISEN_REQUIRE(ctx, eisen_dtype_ok(dtype), EISEN_E_ARG, "eisen_hip_htod_values: unknown dtype %d", dtype);
+    if (n == 0) return 0;
+    if (n <= kCopyKernelBytes / sizeof(float) && eisen_aligned(dst, 16) && eisen_aligned(ids, 16) && !stream_captures(ctx)) {
+        eisen_ctx::StageSlot* st = nullptr;
+        const int rc = eisen_staging(ctx, n * sizeof(float), &st);
+        if (rc) return rc;
+        memcpy(st->ptr, src, n * sizeof(float));
+        st->number++;
+        const float* from = static_cast<const float*>(st->ptr);
+        if (dtype == EISEN_F32) copy_in_values_kernel<float><<<1, kCopyThreads, 0, ctx->stream>>>(from, static_cast<float*>(dst), ids, (unsigned)n, st->word, st->number);
+        else copy_in_values_kernel<bf16_t><<<1, kCopyThreads, 0, ctx->stream>>>(from, static_cast<bf16_t*>(dst), ids, (unsigned)n, st->word, st->number);
+        st->stream = ctx->stream;
+        st->by_word = true;
+        EISEN_LAUNCH_CHECK(ctx, "eisen_hip_htod_values");
+        st->in_flight = true;
+        return 0;
+    }
+    int rc = 0;
+    if (dtype == EISEN_F32) {
+        rc = eisen_hip_htod(ctx, dst, src, n * sizeof(float));
+    } else {
+        void* tmp = nullptr;
+        rc = eisen_hip_malloc(ctx, n * sizeof(float), &tmp);
+        if (rc) return rc;
+        rc = eisen_hip_htod(ctx, tmp, src, n * sizeof(float));
+        if (!rc) rc = eisen_hip_cast(ctx, tmp, EISEN_F32, dst, EISEN_BF16, n);
+        const int rc_free = eisen_hip_free(ctx, tmp);
+        if (!rc) rc = rc_free;
+    }
+    if (rc || !ids) return rc;
+    std::vector<int32_t> whole(n);
+    for (size_t i = 0; i < n; i++) whole[i] = src[i] >= -2147483648.0f && src[i] < 2147483648.0f ? (int32_t)src[i] : 0;
+    return eisen_hip_htod(ctx, ids, whole.data(), n * sizeof(int32_t));
 }
 
 // Memory that the device writes itself (pinned).

@@ -112,6 +112,11 @@ class Context:
             self._call("eisen_hip_htod", _vp(buf.ptr), arr.ctypes.data_as(_vp), _sz(arr.nbytes))
         return buf
 
+    def htod_values(self, dst, dtype, ids, values):
+        """f32 host values into a tensor of `dtype` and, unless ids is None, as int32 beside it."""
+        v = np.ascontiguousarray(values, dtype=np.float32).reshape(-1)
+        self._call("eisen_hip_htod_values", _ptr(dst), _i(dtype), _ptr(ids) if ids is not None else None, v.ctypes.data_as(_vp), _sz(v.size))
+
     def download(self, buf, shape, dtype=F32):
         """device -> numpy float32 (dtype F32/BF16) or the given numpy dtype."""
         shape = tuple(int(s) for s in np.atleast_1d(shape)) if not isinstance(shape, tuple) else shape

@@ -92,6 +92,9 @@ int eisen_hip_pool_peak(eisen_ctx* ctx, size_t* peak_in_use_bytes, int reset);
  * asynchronous on the stream; the host buffer is copied to a staging area first, so it may
  * be reused as soon as the call returns. */
 int eisen_hip_htod(eisen_ctx* ctx, void* dst_device, const void* src_host, size_t bytes);
+/* n f32 host values into a tensor of `dtype` (bf16: rounded to the nearest, as eisen_hip_cast does) and, if ids is not null, truncated to int32 there as well
+ * (values outside of int32 leave anything): one launch up to 96 KB of 16-byte aligned tensors outside of a capture. */
+int eisen_hip_htod_values(eisen_ctx* ctx, void* dst, int dtype, int32_t* ids, const float* src_host, size_t n);
 /* stream.clone_dtoh (src/tensor.rs:177-223): synchronises the stream before returning. */
 int eisen_hip_dtoh(eisen_ctx* ctx, void* dst_host, const void* src_device, size_t bytes);
 /* n bf16 values as f32. */

@@ -56,6 +56,32 @@ def test_broadcast_add_reference(g):
     assert g.sync_grad_to_cpu(b).reshape(-1).tolist() == [2.0] * 3
 
 
+@pytest.mark.parametrize("beside", [True, False])
+def test_gather_from_a_loaded_tensor_again_and_after_another_load(g, beside):
+    # the ids of a load serve the first lookup, a second one uploads its own; the backward passes use the ids of their forward pass, whatever was loaded since
+    g.set_weight_gradients_beside(beside)
+    w = g.alloc((5, 2), np.arange(10, dtype=np.float32))
+    x = g.alloc_pooled((2, 3))
+    first, second, cut = [4, 0, 4, 1, 1, 4], [2, 3, 3, 2, 0, 0], [1.5, 0.0, 2.25, 3.0, 4.75, 1.0]  # (ids that are not whole are truncated)
+    rows = np.arange(10, dtype=np.float32).reshape(5, 2)
+    outs, used = [], []
+    for load in (first, first, None, second, cut):
+        if load is not None:
+            g.load_tensor_data(x, np.array(load, np.float32))
+            ids = np.array(load, np.float32).astype(np.int64)
+        outs.append(g.gather(w, x))
+        used.append(ids)
+    with pytest.raises(EisenHipError):
+        g.load_tensor_data(x, np.array([0, 1, 2, 3, 4, 5], np.float32))
+        g.gather(w, x)
+    for o, ids in zip(outs, used):
+        assert np.array_equal(g.sync_to_cpu(o).reshape(6, 2), rows[ids])
+    total = g.add(g.add(g.add(outs[0], outs[1]), g.add(outs[2], outs[3])), outs[4])
+    g.backward(total)
+    counts = np.bincount(np.concatenate(used), minlength=5).astype(np.float32)
+    assert np.array_equal(g.sync_grad_to_cpu(w), np.stack([counts, counts], 1))
+
+
 def test_silu_gather_rmsnorm_ce_rope_reference(g):
     # SiLU closed form, tests/gpu_kernels.rs:114-152
     x = np.array([-2.0, -1.0, 0.0, 1.0, 2.0], np.float32)
