@@ -166,14 +166,20 @@ void Graph::load_tensor_data(size_t id, const float* host, size_t n) {
     if (n != t.size()) throw Error("Shape mismatch: Tensor " + std::to_string(id) + " expects " + std::to_string(t.size()) + " elements, but got " + std::to_string(n) + ".");
     if (n <= kHostCopyLimit) t.host_copy.assign(host, host + n);
     else t.host_copy.clear();
-    // what may be token ids goes to the device as int32 too, for a gather (as one launch, so for small tensors only)
     const bool ids = t.is_pooled && n > 0 && n <= kIdsLimit && whole_numbers(host, n);
-    if (!ids) device_free(t.ids);
-    else if (t.ids.numel != n) {
-        device_free(t.ids);
-        t.ids = device_alloc(n, EISEN_F32, false);
+    if (t.ids.numel != (ids ? n : 0)) device_free(t.ids);
+    if (ids) {
+        // what may be token ids goes to the device as int32 too, for a gather, in the launch that brings the values (small tensors: others take the copy engine)
+        if (!t.ids.valid()) t.ids = device_alloc(n, EISEN_F32, false);
+        check(eisen_hip_htod_values(ctx_, t.data.ptr, t.data.dtype, (int32_t*)t.ids.ptr, host, n), "load_tensor_data");
+    } else if (t.data.dtype == EISEN_F32) {
+        check(eisen_hip_htod(ctx_, t.data.ptr, host, n * sizeof(float)), "load_tensor_data");
+    } else {
+        Storage tmp = device_alloc(n, EISEN_F32, false);
+        check(eisen_hip_htod(ctx_, tmp.ptr, host, n * sizeof(float)), "load_tensor_data");
+        check(eisen_hip_cast(ctx_, tmp.ptr, EISEN_F32, t.data.ptr, EISEN_BF16, n), "load_tensor_data cast");
+        device_free(tmp);
     }
-    check(eisen_hip_htod_values(ctx_, t.data.ptr, t.data.dtype, (int32_t*)t.ids.ptr, host, n), "load_tensor_data");
     if (t.data.dtype == EISEN_F32) refresh_shadow(id);
 }
 
