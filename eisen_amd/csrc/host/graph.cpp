@@ -167,11 +167,17 @@ void Graph::load_tensor_data(size_t id, const float* host, size_t n) {
     if (n <= kHostCopyLimit) t.host_copy.assign(host, host + n);
     else t.host_copy.clear();
     const bool ids = t.is_pooled && n > 0 && n <= kIdsLimit && whole_numbers(host, n);
-    if (t.ids.numel != (ids ? n : 0)) device_free(t.ids);
+    const bool same_size = ids && t.ids.numel == n;
+    t.ids.numel = 0;  // until the new ones are there: behind a load that failed a gather uploads its own
+    if (!same_size) device_free(t.ids);
     if (ids) {
         // what may be token ids goes to the device as int32 too, for a gather, in the launch that brings the values (small tensors: others take the copy engine)
-        if (!t.ids.valid()) t.ids = device_alloc(n, EISEN_F32, false);
+        if (!same_size) {
+            t.ids = device_alloc(n, EISEN_F32, false);
+            t.ids.numel = 0;
+        }
         check(eisen_hip_htod_values(ctx_, t.data.ptr, t.data.dtype, (int32_t*)t.ids.ptr, host, n), "load_tensor_data");
+        t.ids.numel = n;
     } else if (t.data.dtype == EISEN_F32) {
         check(eisen_hip_htod(ctx_, t.data.ptr, host, n * sizeof(float)), "load_tensor_data");
     } else {
