@@ -16,6 +16,7 @@
 #include <cmath>
 
 #include "attention_common.cuh"
+#include "attention_f32_plan.h"
 
 namespace {
 
@@ -151,14 +152,13 @@ __device__ __forceinline__ RowBlock decode_block(int id, int heads, int B, int n
     return RowBlock{descending ? n_blk - 1 - i : i, r % heads, r / heads};
 }
 
-// Waves of a workgroup, at most: two to a SIMD where their registers allow it.
 template <int K8>
-constexpr int kMaxWaves = K8 <= 4 ? 8 : 4;
+constexpr int kMaxWaves = f32_attn_max_waves(K8);
+extern __shared__ float meet[];  // where the waves of a workgroup meet: as much as the launch's waves need (attention_f32_plan.h)
 
 template <int K8, bool FULL>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_fwd_kernel(AttnArgs a) {
     constexpr int DT = (K8 + 3) / 4;
-    __shared__ float meet[kMaxWaves<K8> - 1][DT * 16 * 64 + 128];
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const RowBlock rb = decode_block(blockIdx.x, a.Hq, a.B, (a.S + 31) / 32, a.causal);
@@ -227,8 +227,9 @@ __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_fwd_kernel(AttnAr
     }
     l += __shfl_xor(l, 32, 64);
     if (nw > 1) {  // the waves' keys are disjoint: (m, l, O) of each, added in wave order against the common maximum
+        auto share = [&](int w) { return meet + f32_attn_fwd_meet(DT, w); };  // of wave w > 0
         if (wave > 0) {
-            float* p = meet[wave - 1];
+            float* p = share(wave);
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -239,20 +240,21 @@ __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_fwd_kernel(AttnAr
         __syncthreads();
         if (wave > 0) return;
         float mn = m;
-        for (int w = 0; w < nw - 1; w++) mn = fmaxf(mn, meet[w][DT * 16 * 64 + lane]);
+        for (int w = 1; w < nw; w++) mn = fmaxf(mn, share(w)[DT * 16 * 64 + lane]);
         const float a0 = m == -INFINITY ? 0.f : fast_exp2(m - mn);
         l *= a0;
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
 #pragma unroll
             for (int v = 0; v < 16; v++) o[dt][v] *= a0;
-        for (int w = 0; w < nw - 1; w++) {
-            const float mw = meet[w][DT * 16 * 64 + lane], aw = mw == -INFINITY ? 0.f : fast_exp2(mw - mn);
-            l += meet[w][DT * 16 * 64 + 64 + lane] * aw;
+        for (int w = 1; w < nw; w++) {
+            const float* p = share(w);
+            const float mw = p[DT * 16 * 64 + lane], aw = mw == -INFINITY ? 0.f : fast_exp2(mw - mn);
+            l += p[DT * 16 * 64 + 64 + lane] * aw;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) o[dt][v] += meet[w][(dt * 16 + v) * 64 + lane] * aw;
+                for (int v = 0; v < 16; v++) o[dt][v] += p[(dt * 16 + v) * 64 + lane] * aw;
         }
         m = mn;
     }
@@ -285,7 +287,7 @@ __device__ __forceinline__ float row_dot(const float (&x)[K8][4], const float (&
 // dQ^T = scale K^T dS^T of query block `id` (none, past the last: the wave only meets the others at the barrier), by nw waves of
 // which this is the `wave`-th; WRITE_D: also leaves D = rowsum(dO o O) for a dK/dV launch that follows.
 template <int K8, bool FULL, bool WRITE_D>
-__device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int nw, float* meet) {
+__device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int nw, float* share) {
     constexpr int DT = (K8 + 3) / 4;
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
     const int n_t = (a.S + 31) / 32;
@@ -353,7 +355,7 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int 
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) meet[(((wave - 1) * DT + dt) * 16 + v) * 64 + lane] = dq[dt][v];
+                for (int v = 0; v < 16; v++) share[(((wave - 1) * DT + dt) * 16 + v) * 64 + lane] = dq[dt][v];
         }
         __syncthreads();
         if (wave > 0) return;
@@ -361,7 +363,7 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int 
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) dq[dt][v] += meet[((w * DT + dt) * 16 + v) * 64 + lane];
+                for (int v = 0; v < 16; v++) dq[dt][v] += share[((w * DT + dt) * 16 + v) * 64 + lane];
     }
     if (!exists || q0 + c >= a.S) return;
     float* dQp = static_cast<float*>(a.dQ) + qoff + (long long)q * a.q_ss;
@@ -387,7 +389,7 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int 
 // of an item are requested under the products of the one before, its columns under its own first products: a lane loads the
 // statistics of the row it holds, and the lanes that need them ask it.
 template <int K8, bool FULL, bool OWN_D>
-__device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int nw, float* meet) {
+__device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int nw) {
     constexpr int DT = (K8 + 3) / 4;
     constexpr bool AHEAD = K8 <= 8;  // (above, the registers are all taken)
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
@@ -496,7 +498,7 @@ __device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int
         const int dt = i >> 1;
         f32x16 r = (i & 1) ? dv[dt] : dk[dt];
         if (nw > 1) {
-            float* p = meet + (i & 1) * kMaxWaves<K8> * 16 * 64;
+            float* p = meet + (i & 1) * nw * kF32AttnTile;
 #pragma unroll
             for (int v = 0; v < 16; v++) p[(wave * 16 + v) * 64 + lane] = r[v];
             __syncthreads();  // (the buffer of tile i was last read before the barrier of tile i - 1)
@@ -530,51 +532,36 @@ __device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int
 // heads on KV heads, head size: 2 x 32 4 on 4 16 12.2 / 5.5; 1 x 448 3 on 3 32 32.5 / 17.2; 16 x 256 8 on 2 32 56.7 / 34.5; 7 x 448
 // 4 on 4 64 66.4 / 57.4; 8 x 300 4 on 4 96 66.6 / 56.5; 1 x 800 8 on 8 128 163 / 92; 16 x 200 8 on 8 128 178 / 167 (one wave per
 // SIMD, registers full: its items still wait for their rows).
-template <int K8>
-constexpr int kMeetFloats = kMaxWaves<K8> * 16 * 64 * (2 > (K8 + 3) / 4 ? 2 : (K8 + 3) / 4);
 template <int K8, bool FULL>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_kernel(AttnArgs a, int kblocks, int wq) {
-    __shared__ float meet[kMeetFloats<K8>];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    if ((int)blockIdx.x < kblocks) return bwd_dkv<K8, FULL, true>(a, blockIdx.x, wave, nw, meet);
+    if ((int)blockIdx.x < kblocks) return bwd_dkv<K8, FULL, true>(a, blockIdx.x, wave, nw);
     const int sub = wave / wq;
-    bwd_dq<K8, FULL, false>(a, ((int)blockIdx.x - kblocks) * (nw / wq) + sub, wave % wq, wq, meet + sub * wq * ((K8 + 3) / 4) * 16 * 64);
+    bwd_dq<K8, FULL, false>(a, ((int)blockIdx.x - kblocks) * (nw / wq) + sub, wave % wq, wq, meet + sub * f32_attn_dq_meet((K8 + 3) / 4, wq));
 }
 // One after the other, where a result lies over an operand.
 template <int K8, bool FULL>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dq_kernel(AttnArgs a) {
-    __shared__ float meet[kMeetFloats<K8>];
     bwd_dq<K8, FULL, true>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);
 }
 template <int K8, bool FULL>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dkv_kernel(AttnArgs a) {
-    __shared__ float meet[kMeetFloats<K8>];
-    bwd_dkv<K8, FULL, false>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);
-}
-
-// waves per workgroup: enough for two waves per SIMD of the chip, but none without at least one tile of the longest row
-int waves_for(long long blocks, int tiles, int most) {
-    int w = 1;
-    while (w < most && blocks * w < 2048 && 2 * w <= tiles) w *= 2;
-    return w;
+    bwd_dkv<K8, FULL, false>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6);
 }
 
 template <int K8, bool FULL>
 void launch_f32(eisen_ctx* ctx, const AttnArgs& a, bool backward) {
-    const int n_t = (a.S + 31) / 32;
-    const long long qblocks = (long long)n_t * a.Hq * a.B, kblocks = (long long)n_t * a.Hkv * a.B;
-    const int wq = waves_for(qblocks, n_t, kMaxWaves<K8>), wk = waves_for(kblocks, n_t * a.G, kMaxWaves<K8>);
+    const F32AttnPlan p = f32_attn_plan(K8, a.B, a.S, a.Hq, a.Hkv);
     if (!backward) {
-        attn_f32_fwd_kernel<K8, FULL><<<dim3((unsigned)qblocks), 64 * wq, 0, ctx->stream>>>(a);
+        attn_f32_fwd_kernel<K8, FULL><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.fwd_lds, ctx->stream>>>(a);
         return;
     }
     if (eisen_attention_writes_over_operand(a, sizeof(float))) {
-        attn_f32_bwd_dq_kernel<K8, FULL><<<dim3((unsigned)qblocks), 64 * wq, 0, ctx->stream>>>(a);
-        attn_f32_bwd_dkv_kernel<K8, FULL><<<dim3((unsigned)kblocks), 64 * wk, 0, ctx->stream>>>(a);
+        attn_f32_bwd_dq_kernel<K8, FULL><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.dq_lds, ctx->stream>>>(a);
+        attn_f32_bwd_dkv_kernel<K8, FULL><<<dim3((unsigned)p.kblocks), 64 * p.wk, p.dkv_lds, ctx->stream>>>(a);
         return;
     }
-    const long long dq_groups = eisen_ceil_div(qblocks, (long long)(wk / wq));  // (wq <= wk: there are no fewer query blocks than key blocks)
-    attn_f32_bwd_kernel<K8, FULL><<<dim3((unsigned)(kblocks + dq_groups)), 64 * wk, 0, ctx->stream>>>(a, (int)kblocks, wq);
+    attn_f32_bwd_kernel<K8, FULL><<<dim3((unsigned)(p.kblocks + p.dq_groups)), 64 * p.wk, p.bwd_lds, ctx->stream>>>(a, (int)p.kblocks, p.wq);
 }
 
 }  // namespace
