@@ -22,13 +22,16 @@ namespace {
 
 struct __attribute__((packed, aligned(4))) Quad { float v[4]; };
 
-// Rows `stride` apart (|stride| < 2^24).  A load takes the tile's origin in scalar registers and an unsigned 32-bit byte offset per
+// Rows `stride` apart.  A load takes the tile's origin in scalar registers and an unsigned 32-bit byte offset per
 // lane, so that the loops spend few vector instructions on addresses (64-bit sums per lane and load had been a third of those of a
-// dK/dV item).  A negative stride moves the origin to the lowest of 32 rows.
+// dK/dV item).  A negative stride moves the origin to the lowest of 32 rows.  FAR: |stride| >= 2^24, which 32 rows of such an offset
+// do not reach; 64-bit sums, in kernels of their own (128 positions 2^24 apart, 8 heads of 128, forward and backward in us: 14 and 47; on the
+// plain kernels 237 and 979).
+template <bool FAR>
 struct RowStride {
     long long stride;
     int low;  // elements
-    __device__ __forceinline__ explicit RowStride(long long s) : stride(s), low(min(0, 31 * (int)s)) {}
+    __device__ __forceinline__ explicit RowStride(long long s) : stride(s), low(FAR ? 0 : min(0, 31 * (int)s)) {}
 };
 template <class T>
 __device__ __forceinline__ const T& at_bytes(const float* origin, unsigned bytes) {
@@ -38,9 +41,9 @@ __device__ __forceinline__ const T& at_bytes(const float* origin, unsigned bytes
 // not, a load may stand behind a branch of its lanes, and the row's own address in two registers does better than an offset that every
 // branch adds up again (offset / address, us: 8 x 512, 8 heads of 100 forward 88 / 77, backward 395 / 319; 1 x 800, 8 of 100 64 / 54 and
 // 159 / 133; 16 x 512, 8 of 40 backward 264 / 243; 16 x 512, 8 of 20 157 / 135).
-template <int K8, bool FULL>
-__device__ __forceinline__ void load_row(const float* base, const RowStride& rs, int first_row, int rows, int hd, int c, int h, float (&f)[K8][4]) {
-    if (FULL) {
+template <int K8, bool FULL, bool FAR>
+__device__ __forceinline__ void load_row(const float* base, const RowStride<FAR>& rs, int first_row, int rows, int hd, int c, int h, float (&f)[K8][4]) {
+    if (FULL && !FAR) {
         const float* origin = base + first_row * rs.stride + rs.low;
         const unsigned off = (unsigned)(min(c, rows - 1 - first_row) * (int)rs.stride - rs.low) * 4u + 16u * h;
 #pragma unroll
@@ -54,7 +57,7 @@ __device__ __forceinline__ void load_row(const float* base, const RowStride& rs,
 #pragma unroll
         for (int kk = 0; kk < K8; kk++) {
             const int d = 8 * kk + 4 * h;
-            if (d + 4 <= hd) {
+            if (FULL || d + 4 <= hd) {
                 const Quad q = *reinterpret_cast<const Quad*>(row + d);
 #pragma unroll
                 for (int j = 0; j < 4; j++) f[kk][j] = q.v[j];
@@ -67,11 +70,16 @@ __device__ __forceinline__ void load_row(const float* base, const RowStride& rs,
 }
 // Columns d = 32 dt + lane % 32 of the 32 rows at first_row, in the order of a score tile's registers.  Rows past the end
 // repeat the last one (their weight is zero).
-template <int K8, bool FULL>
-__device__ __forceinline__ void load_column(const float* base, const RowStride& rs, int first_row, int rows, int hd, int c, int h, int dt, float (&f)[16]) {
+template <int K8, bool FULL, bool FAR>
+__device__ __forceinline__ void load_column(const float* base, const RowStride<FAR>& rs, int first_row, int rows, int hd, int c, int h, int dt, float (&f)[16]) {
     const float* origin = base + first_row * rs.stride + rs.low + 32 * dt;
     const int d = 32 * dt + c, last = rows - 1 - first_row, stride = (int)rs.stride;
     const bool in = FULL ? (32 * dt + 32 <= 8 * K8 || d < 8 * K8) : d < hd;
+    if (FAR) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) f[v] = in ? base[min(first_row + acc_row(v, h), rows - 1) * rs.stride + d] : 0.f;
+        return;
+    }
 #pragma unroll
     for (int v = 0; v < 16; v++) {  // the products are scalar
         const int r0 = min(acc_row(v, 0), last) * stride, r1 = min(acc_row(v, 1), last) * stride;
@@ -79,8 +87,8 @@ __device__ __forceinline__ void load_column(const float* base, const RowStride& 
         f[v] = in ? at_bytes<float>(origin, off) : 0.f;
     }
 }
-template <int K8, int DT, bool FULL>
-__device__ __forceinline__ void load_columns(const float* base, const RowStride& rs, int first_row, int rows, int hd, int c, int h, float (&f)[DT][16]) {
+template <int K8, int DT, bool FULL, bool FAR>
+__device__ __forceinline__ void load_columns(const float* base, const RowStride<FAR>& rs, int first_row, int rows, int hd, int c, int h, float (&f)[DT][16]) {
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) load_column<K8, FULL>(base, rs, first_row, rows, hd, c, h, dt, f[dt]);
 }
@@ -136,8 +144,8 @@ __device__ __forceinline__ bool take_out_nonfinite(float (&col)[DT][16]) {  // w
     return __builtin_amdgcn_ballot_w64(found) != 0;
 }
 // +-Inf for the weights P of V and dO, which are not negative (POSITIVE), NaN for the others and for NaN.
-template <bool POSITIVE, int K8, int DT, bool FULL, class Visible>
-__device__ __forceinline__ void put_back_nonfinite(const float* base, const RowStride& stride, int first_row, int rows, int hd, int c, int h, f32x16 (&acc)[DT],
+template <bool POSITIVE, int K8, int DT, bool FULL, bool FAR, class Visible>
+__device__ __forceinline__ void put_back_nonfinite(const float* base, const RowStride<FAR>& stride, int first_row, int rows, int hd, int c, int h, f32x16 (&acc)[DT],
                                                    Visible visible) {
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) {
@@ -169,7 +177,7 @@ template <int K8>
 constexpr int kMaxWaves = f32_attn_max_waves(K8);
 extern __shared__ float meet[];  // where the waves of a workgroup meet: as much as the launch's waves need (attention_f32_plan.h)
 
-template <int K8, bool FULL>
+template <int K8, bool FULL, bool FAR>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_fwd_kernel(AttnArgs a) {
     constexpr int DT = (K8 + 3) / 4;
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
@@ -180,7 +188,7 @@ __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_fwd_kernel(AttnAr
     const long long kvoff = rb.b * a.k_sb + (rb.head / a.G) * a.k_sh;
     const float* Kp = static_cast<const float*>(a.K) + kvoff;
     const float* Vp = static_cast<const float*>(a.V) + kvoff;
-    const RowStride qs(a.q_ss), ks(a.k_ss);
+    const RowStride<FAR> qs(a.q_ss), ks(a.k_ss);
     float qf[K8][4], kf[K8][4];
     load_row<K8, FULL>(static_cast<const float*>(a.Q) + rb.b * a.q_sb + rb.head * a.q_sh, qs, q0, a.S, a.hd, c, h, qf);
     f32x16 o[DT];
@@ -299,7 +307,7 @@ __device__ __forceinline__ float row_dot(const float (&x)[K8][4], const float (&
 
 // dQ^T = scale K^T dS^T of query block `id` (none, past the last: the wave only meets the others at the barrier), by nw waves of
 // which this is the `wave`-th; WRITE_D: also leaves D = rowsum(dO o O) for a dK/dV launch that follows.
-template <int K8, bool FULL, bool WRITE_D>
+template <int K8, bool FULL, bool FAR, bool WRITE_D>
 __device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int nw, float* share) {
     constexpr int DT = (K8 + 3) / 4;
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
@@ -312,7 +320,7 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int 
     const long long stat = ((long long)rb.b * a.Hq + rb.head) * a.S + q;
     const float* Kp = static_cast<const float*>(a.K) + kvoff;
     const float* Vp = static_cast<const float*>(a.V) + kvoff;
-    const RowStride qs(a.q_ss), ks(a.k_ss);
+    const RowStride<FAR> qs(a.q_ss), ks(a.k_ss);
     float qf[K8][4], dof[K8][4], kf[K8][4], vf[K8][4];
     load_row<K8, FULL>(static_cast<const float*>(a.dO) + qoff, qs, q0, a.S, a.hd, c, h, dof);
     load_row<K8, FULL>(static_cast<const float*>(a.O) + qoff, qs, q0, a.S, a.hd, c, h, qf);
@@ -401,7 +409,7 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, int id, int wave, int 
 // over the waves).  OWN_D: D is formed from the rows of O here, as the dQ pass forms it, and not read.  The rows and statistics
 // of an item are requested under the products of the one before, its columns under its own first products: a lane loads the
 // statistics of the row it holds, and the lanes that need them ask it.
-template <int K8, bool FULL, bool OWN_D>
+template <int K8, bool FULL, bool FAR, bool OWN_D>
 __device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int nw) {
     constexpr int DT = (K8 + 3) / 4;
     constexpr bool AHEAD = K8 <= 8;  // (above, the registers are all taken)
@@ -410,7 +418,7 @@ __device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int
     const RowBlock rb = decode_block(id, a.Hkv, a.B, n_t, false);  // ascending: the first keys see the most queries
     const int k0 = rb.blk * 32, key = min(k0 + c, a.S - 1);
     const long long kvoff = rb.b * a.k_sb + rb.head * a.k_sh;
-    const RowStride qs(a.q_ss), ks(a.k_ss);
+    const RowStride<FAR> qs(a.q_ss), ks(a.k_ss);
     float kf[K8][4], vf[K8][4];
     load_row<K8, FULL>(static_cast<const float*>(a.K) + kvoff, ks, k0, a.S, a.hd, c, h, kf);
     load_row<K8, FULL>(static_cast<const float*>(a.V) + kvoff, ks, k0, a.S, a.hd, c, h, vf);
@@ -548,55 +556,60 @@ __device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int
 template <int K8, bool FULL>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_kernel(AttnArgs a, int kblocks, int wq) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    if ((int)blockIdx.x < kblocks) return bwd_dkv<K8, FULL, true>(a, blockIdx.x, wave, nw);
+    if ((int)blockIdx.x < kblocks) return bwd_dkv<K8, FULL, false, true>(a, blockIdx.x, wave, nw);
     const int sub = wave / wq;
-    bwd_dq<K8, FULL, false>(a, ((int)blockIdx.x - kblocks) * (nw / wq) + sub, wave % wq, wq, meet + sub * f32_attn_dq_meet((K8 + 3) / 4, wq));
+    bwd_dq<K8, FULL, false, false>(a, ((int)blockIdx.x - kblocks) * (nw / wq) + sub, wave % wq, wq, meet + sub * f32_attn_dq_meet((K8 + 3) / 4, wq));
 }
-// One after the other, where a result lies over an operand.
-template <int K8, bool FULL>
+// One after the other, where a result lies over an operand or rows are far apart.
+template <int K8, bool FULL, bool FAR>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dq_kernel(AttnArgs a) {
-    bwd_dq<K8, FULL, true>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);
+    bwd_dq<K8, FULL, FAR, true>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);
 }
-template <int K8, bool FULL>
+template <int K8, bool FULL, bool FAR>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dkv_kernel(AttnArgs a) {
-    bwd_dkv<K8, FULL, false>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6);
+    bwd_dkv<K8, FULL, FAR, false>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6);
 }
 
-template <int K8, bool FULL>
+template <int K8, bool FULL, bool FAR>
 void launch_f32(eisen_ctx* ctx, const AttnArgs& a, bool backward) {
     const F32AttnPlan p = f32_attn_plan(K8, a.B, a.S, a.Hq, a.Hkv);
     if (!backward) {
-        attn_f32_fwd_kernel<K8, FULL><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.fwd_lds, ctx->stream>>>(a);
+        attn_f32_fwd_kernel<K8, FULL, FAR><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.fwd_lds, ctx->stream>>>(a);
         return;
     }
-    if (eisen_attention_writes_over_operand(a, sizeof(float))) {
-        attn_f32_bwd_dq_kernel<K8, FULL><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.dq_lds, ctx->stream>>>(a);
-        attn_f32_bwd_dkv_kernel<K8, FULL><<<dim3((unsigned)p.kblocks), 64 * p.wk, p.dkv_lds, ctx->stream>>>(a);
+    if (FAR || eisen_attention_writes_over_operand(a, sizeof(float))) {
+        attn_f32_bwd_dq_kernel<K8, FULL, FAR><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.dq_lds, ctx->stream>>>(a);
+        attn_f32_bwd_dkv_kernel<K8, FULL, FAR><<<dim3((unsigned)p.kblocks), 64 * p.wk, p.dkv_lds, ctx->stream>>>(a);
         return;
     }
     attn_f32_bwd_kernel<K8, FULL><<<dim3((unsigned)(p.kblocks + p.dq_groups)), 64 * p.wk, p.bwd_lds, ctx->stream>>>(a, (int)p.kblocks, p.wq);
+}
+
+template <bool FAR>
+void launch_f32_by_head_dim(eisen_ctx* ctx, const AttnArgs& a, bool backward) {
+    switch (a.hd) {
+        case 16: return launch_f32<2, true, FAR>(ctx, a, backward);
+        case 32: return launch_f32<4, true, FAR>(ctx, a, backward);
+        case 48: return launch_f32<6, true, FAR>(ctx, a, backward);
+        case 64: return launch_f32<8, true, FAR>(ctx, a, backward);
+        case 80: return launch_f32<10, true, FAR>(ctx, a, backward);
+        case 96: return launch_f32<12, true, FAR>(ctx, a, backward);
+        case 128: return launch_f32<16, true, FAR>(ctx, a, backward);
+    }
+    if (a.hd < 16) launch_f32<2, false, FAR>(ctx, a, backward);
+    else if (a.hd < 32) launch_f32<4, false, FAR>(ctx, a, backward);
+    else if (a.hd < 64) launch_f32<8, false, FAR>(ctx, a, backward);
+    else launch_f32<16, false, FAR>(ctx, a, backward);
 }
 
 }  // namespace
 
 bool eisen_attention_f32_mfma_supports(const AttnArgs& a) {
     const long long n_t = (a.S + 31) / 32;
-    // (32 rows in an unsigned 32-bit byte offset)
-    return a.hd <= 128 && n_t * (a.Hq + a.Hkv) * a.B < (1ll << 31) && std::abs(a.q_ss) < (1ll << 24) && std::abs(a.k_ss) < (1ll << 24);
+    return a.hd <= 128 && n_t * a.Hq * a.B < (1ll << 31);
 }
 
 void eisen_attention_launch_f32(eisen_ctx* ctx, const AttnArgs& a, bool backward) {
-    switch (a.hd) {
-        case 16: return launch_f32<2, true>(ctx, a, backward);
-        case 32: return launch_f32<4, true>(ctx, a, backward);
-        case 48: return launch_f32<6, true>(ctx, a, backward);
-        case 64: return launch_f32<8, true>(ctx, a, backward);
-        case 80: return launch_f32<10, true>(ctx, a, backward);
-        case 96: return launch_f32<12, true>(ctx, a, backward);
-        case 128: return launch_f32<16, true>(ctx, a, backward);
-    }
-    if (a.hd < 16) launch_f32<2, false>(ctx, a, backward);
-    else if (a.hd < 32) launch_f32<4, false>(ctx, a, backward);
-    else if (a.hd < 64) launch_f32<8, false>(ctx, a, backward);
-    else launch_f32<16, false>(ctx, a, backward);
+    if (std::max(std::abs(a.q_ss), std::abs(a.k_ss)) < 1ll << 24) launch_f32_by_head_dim<false>(ctx, a, backward);
+    else launch_f32_by_head_dim<true>(ctx, a, backward);
 }
