@@ -723,7 +723,8 @@ static int attention_backward_common(eisen_ctx* ctx, const void* q, const void* 
         a.D = static_cast<float*>(ws);
     }
     a.L2 = a.D + B * Hq * S;
-    if (rope) {
+    const bool plain = dtype == EISEN_F32 && !eisen_attention_f32_mfma_supports(a);
+    if (rope && !plain) {
         rc = eisen_rope_table_get(ctx, S, hd, &a.rope);
         if (rc) return rc;
     }
@@ -735,7 +736,7 @@ static int attention_backward_common(eisen_ctx* ctx, const void* q, const void* 
                                eisen_aligned(dout, 16) && eisen_aligned(dq, 16) && eisen_aligned(dk, 16) && eisen_aligned(dv, 16),
                       EISEN_E_ALIGN, "attention_backward: bf16 buffers must be 16-byte aligned");
         with_head_dim((int)hd, [&](auto hd_c) { launch_bwd<decltype(hd_c)::value>(ctx, a); });
-    } else if (eisen_attention_f32_mfma_supports(a)) {
+    } else if (!plain) {
         EisenProfScope prof(ctx, "attn_bwd_f32", 4.0 * attn_pair_flops(a), true);
         eisen_attention_launch_f32(ctx, a, true);
     } else {
@@ -746,6 +747,11 @@ static int attention_backward_common(eisen_ctx* ctx, const void* q, const void* 
         attn_f32_wide_bwd_dkv_kernel<<<grid2, 64, 2 * S * sizeof(float), ctx->stream>>>(a);
     }
     EISEN_LAUNCH_CHECK(ctx, "attention backward");
+    if (rope && plain) {  // the plain kernels do not rotate dQ and dK back as they store them
+        rc = eisen_hip_rope_backward(ctx, dq, dq, dtype, B, S, Hq * hd, hd, 0);
+        if (!rc) rc = eisen_hip_rope_backward(ctx, dk, dk, dtype, B, S, Hkv * hd, hd, 0);
+        return rc;
+    }
     return 0;
 }
 
@@ -791,11 +797,5 @@ extern "C" int eisen_hip_attention_rope_backward(eisen_ctx* ctx, const void* q, 
                                                  const void* dout, const float* lse, void* dq, void* dk, void* dv, int dtype,
                                                  size_t B, size_t S, size_t Hq, size_t Hkv, size_t hd, float scale, int causal) {
     EISEN_CHECK_CTX(ctx);
-    if (dtype == EISEN_BF16 || hd <= 128)  // the MFMA kernels rotate dQ and dK back as they store them
-        return attention_backward_common(ctx, q, k, v, out, dout, lse, dq, dk, dv, dtype, B, S, Hq, Hkv, hd, nullptr, nullptr, scale, causal, true);
-    // f32, larger heads: the plain backward, then the rotary backward in place
-    int rc = attention_backward_common(ctx, q, k, v, out, dout, lse, dq, dk, dv, dtype, B, S, Hq, Hkv, hd, nullptr, nullptr, scale, causal, false);
-    if (!rc) rc = eisen_hip_rope_backward(ctx, dq, dq, dtype, B, S, Hq * hd, hd, 0);
-    if (!rc) rc = eisen_hip_rope_backward(ctx, dk, dk, dtype, B, S, Hkv * hd, hd, 0);
-    return rc;
+    return attention_backward_common(ctx, q, k, v, out, dout, lse, dq, dk, dv, dtype, B, S, Hq, Hkv, hd, nullptr, nullptr, scale, causal, true);
 }
