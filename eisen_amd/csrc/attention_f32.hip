@@ -560,7 +560,7 @@ __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_kernel(AttnAr
     const int sub = wave / wq;
     bwd_dq<K8, FULL, false, false>(a, ((int)blockIdx.x - kblocks) * (nw / wq) + sub, wave % wq, wq, meet + sub * f32_attn_dq_meet((K8 + 3) / 4, wq));
 }
-// One after the other, where a result lies over an operand or rows are far apart.
+// One after the other: where a result lies over an operand, rows are far apart or the workgroups are too many for one launch.
 template <int K8, bool FULL, bool FAR>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dq_kernel(AttnArgs a) {
     bwd_dq<K8, FULL, FAR, true>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);
@@ -577,12 +577,12 @@ void launch_f32(eisen_ctx* ctx, const AttnArgs& a, bool backward) {
         attn_f32_fwd_kernel<K8, FULL, FAR><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.fwd_lds, ctx->stream>>>(a);
         return;
     }
-    if (FAR || eisen_attention_writes_over_operand(a, sizeof(float))) {
+    if (FAR || !p.one || eisen_attention_writes_over_operand(a, sizeof(float))) {
         attn_f32_bwd_dq_kernel<K8, FULL, FAR><<<dim3((unsigned)p.qblocks), 64 * p.wq, p.dq_lds, ctx->stream>>>(a);
         attn_f32_bwd_dkv_kernel<K8, FULL, FAR><<<dim3((unsigned)p.kblocks), 64 * p.wk, p.dkv_lds, ctx->stream>>>(a);
         return;
     }
-    attn_f32_bwd_kernel<K8, FULL><<<dim3((unsigned)(p.kblocks + p.dq_groups)), 64 * p.wk, p.bwd_lds, ctx->stream>>>(a, (int)p.kblocks, p.wq);
+    if constexpr (!FAR) attn_f32_bwd_kernel<K8, FULL><<<dim3((unsigned)(p.kblocks + p.dq_groups)), 64 * p.wk, p.bwd_lds, ctx->stream>>>(a, (int)p.kblocks, p.wq);
 }
 
 template <bool FAR>

@@ -26,6 +26,7 @@ inline int f32_attn_waves(long long blocks, int tiles, int most) {
 struct F32AttnPlan {
     long long qblocks, kblocks, dq_groups;  // dq_groups: workgroups of the combined backward that form dQ, of wk / wq query blocks each
     int wq, wk;
+    bool one;  // the backward is one launch (its workgroups' threads are no more than a launch takes), not one for dQ and one for dK and dV
     size_t fwd_lds, dq_lds, dkv_lds, bwd_lds;  // bytes
 };
 inline F32AttnPlan f32_attn_plan(int k8, int B, int S, int Hq, int Hkv) {
@@ -41,5 +42,6 @@ inline F32AttnPlan f32_attn_plan(int k8, int B, int S, int Hq, int Hkv) {
     p.dq_lds = f32_attn_dq_meet(dt, p.wq) * sizeof(float);
     p.dkv_lds = f32_attn_dkv_meet(p.wk) * sizeof(float);
     p.bwd_lds = std::max(together * p.dq_lds, p.dkv_lds);
+    p.one = (p.kblocks + p.dq_groups) * 64 * p.wk < (1ll << 32);
     return p;
 }

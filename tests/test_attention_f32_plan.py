@@ -14,7 +14,7 @@ int main() {
     int k8, B, S, Hq, Hkv;
     while (std::scanf("%d %d %d %d %d", &k8, &B, &S, &Hq, &Hkv) == 5) {
         const F32AttnPlan p = f32_attn_plan(k8, B, S, Hq, Hkv);
-        std::printf("%lld %lld %lld %d %d %zu %zu %zu %zu\\n", p.qblocks, p.kblocks, p.dq_groups, p.wq, p.wk, p.fwd_lds, p.dq_lds, p.dkv_lds, p.bwd_lds);
+        std::printf("%lld %lld %lld %d %d %zu %zu %zu %zu %d\\n", p.qblocks, p.kblocks, p.dq_groups, p.wq, p.wk, p.fwd_lds, p.dq_lds, p.dkv_lds, p.bwd_lds, (int)p.one);
     }
 }
 """
@@ -30,7 +30,7 @@ def plans(tmp_path_factory):
 
     def run(sizes):
         out = subprocess.run([exe], input="\n".join(" ".join(map(str, s)) for s in sizes), capture_output=True, text=True, check=True).stdout
-        names = "qblocks kblocks dq_groups wq wk fwd_lds dq_lds dkv_lds bwd_lds".split()
+        names = "qblocks kblocks dq_groups wq wk fwd_lds dq_lds dkv_lds bwd_lds one".split()
         return [dict(zip(names, map(int, line.split()))) for line in out.splitlines()]
 
     return run
@@ -59,3 +59,16 @@ def test_lds_holds_what_the_waves_write_and_nothing_for_one_wave(plans):
         assert (p["dq_groups"] - 1) * together < p["qblocks"] <= p["dq_groups"] * together
         if p["kblocks"] >= 2048:
             assert p["wq"] == p["wk"] == 1 and p["fwd_lds"] == p["bwd_lds"] == 0
+
+
+def test_no_launch_of_more_threads_than_there_can_be(plans):
+    # 2^32 of them; either pass of its own may still fit where both together do not
+    sizes = [(2, 1 << 13, 32, 1 << 12, 1 << 12), (2, 1 << 13, 32, 1 << 11, 1 << 11), (16, 1 << 15, 64, 1000, 500), (4, 65535, 1, 1023, 1), (4, 65535, 33, 512, 512)] + some_sizes()
+    both = 0
+    for size, p in zip(sizes, plans(sizes)):
+        alone = max(p["qblocks"] * 64 * p["wq"], p["kblocks"] * 64 * p["wk"])
+        together = (p["kblocks"] + p["dq_groups"]) * 64 * p["wk"]
+        assert alone < 1 << 32, size
+        assert not p["one"] or together < 1 << 32, size
+        both += together >= 1 << 32
+    assert both >= 3
