@@ -548,7 +548,7 @@ __device__ __forceinline__ void bwd_dkv(const AttnArgs& a, int id, int wave, int
 
 // Both passes in one launch: the first kblocks workgroups form dK and dV of a key block each, the others dQ of as many query blocks
 // as they have wq waves for.  The two do not wait for one another (the dK/dV pass forms D itself), so a grid that does not fill the
-// chip takes the time of the longer pass, and one that does fills the gaps that the uneven causal key blocks leave.  Two launches with
+// chip takes the time of the longer pass, and in one that does either pass fills the gaps of the other (where that is not enough: F32AttnPlan).  Two launches with
 // an address of its own per load, and a dK/dV item's rows requested only when it began / this, us, causal, batch x sequence, query
 // heads on KV heads, head size: 2 x 32 4 on 4 16 12.2 / 5.5; 1 x 448 3 on 3 32 32.5 / 17.2; 16 x 256 8 on 2 32 56.7 / 34.5; 7 x 448
 // 4 on 4 64 66.4 / 57.4; 8 x 300 4 on 4 96 66.6 / 56.5; 1 x 800 8 on 8 128 163 / 92; 16 x 200 8 on 8 128 178 / 167 (one wave per
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_kernel(AttnAr
     const int sub = wave / wq;
     bwd_dq<K8, FULL, false, false>(a, ((int)blockIdx.x - kblocks) * (nw / wq) + sub, wave % wq, wq, meet + sub * f32_attn_dq_meet((K8 + 3) / 4, wq));
 }
-// One after the other: where a result lies over an operand, rows are far apart or the workgroups are too many for one launch.
+// One after the other: large grids of large heads (F32AttnPlan), and where a result lies over an operand or rows are far apart.
 template <int K8, bool FULL, bool FAR>
 __global__ __launch_bounds__(64 * kMaxWaves<K8>) void attn_f32_bwd_dq_kernel(AttnArgs a) {
     bwd_dq<K8, FULL, FAR, true>(a, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6, meet);

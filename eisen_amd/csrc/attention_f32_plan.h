@@ -23,10 +23,17 @@ inline int f32_attn_waves(long long blocks, int tiles, int most) {
     return w;
 }
 
+// One launch for the backward, or one for dQ and one for dK and dV.  One lets either pass fill the gaps of the other and has a dK/dV item read the rows of O as well;
+// for head sizes above 96, whose one wave per SIMD waits for all of an item's rows, that costs more than it gives once each pass fills the chip by itself.
+// Two / one, us, causal, batch x sequence, query heads on KV heads, head size: 16 x 256 8 on 8 128 128 / 140; 8 x 512 8 on 8 128 192 / 209; 16 x 512 8 on 8 128
+// 331 / 382; 16 x 512 16 on 4 128 663 / 747; 64 x 128 8 on 8 128 156 / 171; 128 x 32 8 on 8 128 49 / 53; 8 x 512 16 on 8 100 504 / 556; 512 x 32 8 on 8 100 297 / 307.
+// Below 1024 key blocks it depends on the shape: 4 x 512 8 on 8 128 131 / 137; 2 x 1500 8 on 4 128 407 / 423; but 4 x 512 16 on 4 128 247 / 215; 80 x 64 16 on 4 128
+// 153 / 145; 1 x 800 8 on 8 128 134 / 92.  Smaller heads: 32 x 256 8 on 8 32 64 / 51; 16 x 512 8 on 8 64 165 / 172; 8 x 512 8 on 2 64 131 / 103; 2 x 2000 8 on 2 96
+// 686 / 591; 16 x 512 8 on 8 96 254 / 273; 512 x 32 8 on 8 96 156 / 153.  And two where the workgroups of one have more threads than a launch takes.
 struct F32AttnPlan {
     long long qblocks, kblocks, dq_groups;  // dq_groups: workgroups of the combined backward that form dQ, of wk / wq query blocks each
     int wq, wk;
-    bool one;  // the backward is one launch (its workgroups' threads are no more than a launch takes), not one for dQ and one for dK and dV
+    bool one;  // the backward is one launch
     size_t fwd_lds, dq_lds, dkv_lds, bwd_lds;  // bytes
 };
 inline F32AttnPlan f32_attn_plan(int k8, int B, int S, int Hq, int Hkv) {
@@ -42,6 +49,6 @@ inline F32AttnPlan f32_attn_plan(int k8, int B, int S, int Hq, int Hkv) {
     p.dq_lds = f32_attn_dq_meet(dt, p.wq) * sizeof(float);
     p.dkv_lds = f32_attn_dkv_meet(p.wk) * sizeof(float);
     p.bwd_lds = std::max(together * p.dq_lds, p.dkv_lds);
-    p.one = (p.kblocks + p.dq_groups) * 64 * p.wk < (1ll << 32);
+    p.one = !(k8 > 12 && p.kblocks >= 1024) && (p.kblocks + p.dq_groups) * 64 * p.wk < (1ll << 32);
     return p;
 }

@@ -72,3 +72,11 @@ def test_no_launch_of_more_threads_than_there_can_be(plans):
         assert not p["one"] or together < 1 << 32, size
         both += together >= 1 << 32
     assert both >= 3
+
+
+def test_two_launches_for_large_grids_of_large_heads(plans):
+    def one(k8, B, S, Hq, Hkv):
+        return bool(plans([(k8, B, S, Hq, Hkv)])[0]["one"])
+
+    assert not one(16, 16, 512, 8, 8) and not one(16, 16, 256, 8, 8) and not one(16, 32, 1024, 8, 1)  # 1024 key blocks and more
+    assert one(16, 1, 800, 8, 8) and one(16, 1023, 32, 8, 1) and one(12, 16, 512, 8, 8) and one(4, 512, 32, 8, 8)
