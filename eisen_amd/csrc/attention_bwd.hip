@@ -404,12 +404,14 @@ static bool key_blocks_paired(const AttnArgs& a, int dq_blocks) { return dq_bloc
 // 38.3; 4 x 256 8 on 8 128 30.6 / 19.4.  Beyond the lines: 8 x 256 16 on 16 64 (768 workgroups) 20.2 / 20.6, 16 x 256 33.0 / 37.9; 4 x 256 24 on 8 64 19.3 / 19.8;
 // 1 x 512 32 on 8 64 28.6 / 33.4; 1 x 512 16 on 4 128 53.5 / 61.2; 2 x 256 32 on 4 64 26.2 / 34.2.  At them: 8 x 128 8 on 2 64 15.3 / 13.9; 21 x 256 8 on 2 32 17.6 / 16.2;
 // 8 x 256 8 on 2 48 19.0 / 18.1; 4 x 64 16 on 2 64 15.2 / 14.6; 1 x 1024 16 on 8 64 35.3 / 34.1.
-// Three query heads on a KV head, no pairs of key blocks: 2 x 448 9 on 3 80 29.0 / 24.6; 3 x 500 6 on 2 48 22.2 / 17.7; 1 x 400 24 on 8 32 16.4 / 14.6; 2 x 200 9 on 3 64 15.6 / 14.1, but 1 x
-// 600 9 on 3 64 26.3 / 28.2 and 1 x 640 9 on 3 128 48.0 / 54.6.
+// Three query heads on a KV head, no pairs of key blocks: up to 64 tiles where the head size is no multiple of 64 (1 x 672 3 on 1 16 20.1 / 14.0; 1 x 512 24 on 8 32 18.4 / 16.8; 3 x
+// 500 6 on 2 48 22.2 / 17.7; 2 x 448 9 on 3 80 29.1 / 23.7, 96 30.6 / 27.0, 112 36.4 / 31.4; 2 x 672 9 on 3 96 41.1 / 36.9, 112 48.2 / 43.2; 1 x 448 24 on 8 96 31.2 / 31.6; 1 x 672 24 on 8
+// 48 26.0 / 26.8), half as many where it is (2 x 250 9 on 3 64 16.4 / 14.8, 128 30.4 / 25.3; but 2 x 448 64 21.4 / 22.5, 128 38.4 / 40.5; 2 x 672 64 27.8 / 30.9, 128 50.7 / 56.6; why those
+// two sizes gain less is not known: their one launch takes about as long as that of the next larger size, 2 x 512 9 on 3 64 24.8 beside 26.4 for 80).
 bool eisen_attention_bwd_short_supports(const AttnArgs& a, int dq_blocks) {
     const int n_qt = (a.S + 31) / 32;
     const bool three = a.G == 3 && !key_blocks_paired(a, dq_blocks);
-    const int most = a.G <= 2 || (three && (a.hd < 64 || a.hd == 80)) ? kOwnTiles : three || (a.G <= 4 && a.hd != 64) ? 32 : 16;
+    const int most = a.G <= 2 || (three && a.hd % 64 != 0) ? kOwnTiles : three || (a.G <= 4 && a.hd != 64) ? 32 : 16;
     const long long blocks = dq_blocks + (long long)(n_qt + 1) / 2 * a.Hkv * a.B;
     return a.G * n_qt <= most && blocks <= (a.hd <= 64 ? 512 : 256) && a.ablation == kAblNone && eisen_attention_dkv32_supports(a) && !eisen_attention_writes_over_operand(a, 2);
 }
