@@ -3,6 +3,7 @@
 #include <numeric>
 
 #include "device_utils.cuh"
+#include "embed_plan.h"
 #include "runtime.h"
 
 namespace {
@@ -94,20 +95,20 @@ __global__ __launch_bounds__(kThreads) void scatter_rows_scalar_kernel(const T* 
 // the ids follow one another is each builder's own).  Ids outside [0, vocab) stand behind all others as kNoId and belong to no run.
 constexpr int kNoId = 0x7fffffff;
 
-// One launch: 256 workgroups, each with the ids of one residue.  All of them read the whole batch (128 KB from the L2s for 32768 ids),
-// count what lies before their part and, per id and wave, their own, and place their positions; a wave's ids are consecutive, so the
+// One launch: 256 workgroups, each with one id of every 256 in a row (scatter_bucket_of).  All of them read the whole batch (128 KB from the L2s for
+// 32768 ids), count what lies before their part and, per id and wave, their own, and place their positions; a wave's ids are consecutive, so the
 // places of an id ascend.  What bounds it is the dozen instructions per id and workgroup.  Chunks sorted by a bitonic network, merged and
 // listed in three launches had taken 30 us for 32768 ids, one chunk of up to 1024 and 2048 7.0 and 12.6; this takes 14.1, 4.7 and 5.1.
-constexpr int kBucketBits = 8, kBuckets = 1 << kBucketBits, kBucketThreads = 1024, kBucketWaves = kBucketThreads / kWave, kBucketIds = 960;  // (60 KB of LDS)
-constexpr size_t kBucketMax = 65536, kBucketVocab = (size_t)kBuckets * kBucketIds;
+constexpr int kBucketThreads = 1024, kBucketWaves = kBucketThreads / kWave;
+constexpr size_t kBucketMax = 65536, kBucketVocab = (size_t)kBuckets * kBucketSlots;
 __global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const int32_t* __restrict__ ids, int n, int vocab, int32_t* __restrict__ out_ids,
                                                                        int32_t* __restrict__ order, int32_t* __restrict__ first_bad) {
-    extern __shared__ int places[];  // [wave][id >> kBucketBits]: how many the wave has of it, then where its next one goes
+    extern __shared__ int places[];  // [wave][slot]: how many the wave has of it, then where its next one goes
     __shared__ int sums[kBucketWaves][2];
     constexpr int LIST = 512;
-    __shared__ int list[kBucketWaves][LIST];  // a wave's own ids, id >> kBucketBits | index << 10, in order
+    __shared__ int list[kBucketWaves][LIST];  // a wave's own ids, slot | index << 10, in order
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), bucket = blockIdx.x;
-    const int here = (vocab + kBuckets - 1) >> kBucketBits;  // ids of this residue, at most
+    const int here = (vocab + kBuckets - 1) >> kBucketBits;  // slots
     // (an odd number of 256-byte lines: the waves, and with them all workgroups, would otherwise ask one channel of the L2 at a time)
     const int share = ((n + kBucketWaves * kWave - 1) / (kBucketWaves * kWave) | 1) * kWave;
     const int from = wave * share, to = min(n, from + share);
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const in
     for (int i = tid; i < kBucketWaves * here; i += kBucketThreads) places[i] = 0;
     __syncthreads();
     constexpr int U = 8;
-    int before = 0, bad = kNoId, own = 0;  // before: of smaller residues, per lane
+    int before = 0, bad = kNoId, own = 0;  // before: of smaller buckets, per lane
     for (int i0 = from; i0 < to; i0 += U * kWave) {
         int id[U];
 #pragma unroll
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const in
             for (int u = 0; u < U; u++) id[u] = i0 + u * kWave + lane < to ? id[u] : -1;
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int b = (unsigned)id[u] < (unsigned)vocab ? id[u] & (kBuckets - 1) : kBuckets;
+            const int b = (unsigned)id[u] < (unsigned)vocab ? scatter_bucket_of(id[u]) : kBuckets;
             before += b < bucket;
             const unsigned long long hits = __ballot(b == bucket);
             if (hits) {
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const in
             }
             if (lane < these) {
                 const int place = mine[slot] + rank;
-                out_ids[place] = slot << kBucketBits | bucket;
+                out_ids[place] = scatter_bucket_id(slot, bucket);
                 order[place] = (int)((unsigned)entry >> 10);
                 if (rank == all - 1) mine[slot] = place + 1;  // (a wave's reads of the step above are done)
             }
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const in
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int i = i0 + u * kWave + lane;
-            unsigned long long left = __ballot(i < to && id[u] >= 0 && id[u] < vocab && (id[u] & (kBuckets - 1)) == bucket);
+            unsigned long long left = __ballot(i < to && id[u] >= 0 && id[u] < vocab && scatter_bucket_of(id[u]) == bucket);
             while (left) {  // the lanes with the id of the first one that is left: places in a row
                 const int this_id = __builtin_amdgcn_readlane(id[u], __ffsll(left) - 1);
                 const unsigned long long same = __ballot(id[u] == this_id) & left;
