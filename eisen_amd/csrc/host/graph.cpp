@@ -1406,7 +1406,7 @@ size_t Graph::gather(size_t weights, size_t indices) {
     // forward pass (5 to 14 us for up to 16384 ids), instead of in front of the last kernel of the backward pass.
     size_t didx = (size_t)-1;
     if (!no_grad && !tape_paused && beside_) {
-        didx = push_tensor({3 * n}, EISEN_F32, true);  // int32 payload
+        didx = push_tensor({2 * n}, EISEN_F32, true);  // int32 payload
         check(eisen_hip_side_begin(ctx_), "side stream");
         const int rc = eisen_hip_gather_index_dev(ctx_, (const int32_t*)at(dids).data.ptr, n, vocab, (int32_t*)at(didx).data.ptr);
         const int rc_end = eisen_hip_side_end(ctx_);  // back on the main stream whatever the call returned

@@ -466,7 +466,7 @@ class Context:
         self._call("eisen_hip_gather_backward_dev", _ptr(ids_dev), _ptr(go), _ptr(gw), _i(dtype), _sz(n_ids), _sz(vocab), _sz(hidden))
 
     def gather_index_dev(self, ids_dev, n_ids, vocab, index):
-        """The position index of the ordered scatter (3 * n_ids int32, device) from int32 ids on the device."""
+        """The position index of the ordered scatter (2 * n_ids int32, device) from int32 ids on the device."""
         self._call("eisen_hip_gather_index_dev", _ptr(ids_dev), _sz(n_ids), _sz(vocab), _ptr(index))
 
     def gather_backward_indexed(self, index, go, gw, dtype, n_ids, vocab, hidden):

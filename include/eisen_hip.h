@@ -467,7 +467,7 @@ int eisen_hip_gather_backward(eisen_ctx* ctx, const int32_t* ids_host, const voi
                               size_t n_ids, size_t vocab, size_t hidden);
 /* The same scatter with the ids already on the device (the int32 buffer eisen_hip_gather read): nothing is sorted or
  * uploaded by the host.  Up to 2^20 ids whose keys fit 32 bits (vocab * 2048, or * 16384 beyond 65536 ids) are indexed on
- * the device (counted and placed by residue, or stable sorts of chunks by id in LDS, merged) and scattered run by run; other shapes read the ids back (which
+ * the device (counted and placed by one launch, or stable sorts of chunks by id in LDS, merged) and scattered run by run; other shapes read the ids back (which
  * synchronises) and take eisen_hip_gather_backward.  The ids must lie in [0, vocab), as they did for the gather.  An id outside
  * is skipped in the batches that eisen_hip_gather_index_dev takes; in others it is an error and nothing is added (the call
  * waits for that check, which runs beside the indexing). */
@@ -475,7 +475,7 @@ int eisen_hip_gather_backward_dev(eisen_ctx* ctx, const int32_t* ids_dev, const 
                                   size_t n_ids, size_t vocab, size_t hidden);
 /* eisen_hip_gather_backward_dev in two halves, for a caller that knows the ids long before the gradient exists (the token
  * ids of a training step are known when its forward pass starts).  _index_dev builds the position index of the ordered
- * scatter from the ids alone: `index` receives 3 * n_ids int32 (device memory); EISEN_E_SHAPE when the batch is more
+ * scatter from the ids alone: `index` receives 2 * n_ids int32 (device memory); EISEN_E_SHAPE when the batch is more
  * than the device-side index takes (more than 16384 ids, or vocab * ids beyond 32 bits): then use _backward_dev.
  * _backward_indexed adds the rows of dOut into the f32 gradient in ascending position with that index, the result of
  * eisen_hip_gather_backward_dev bit for bit (src/graph/ops/transform.rs:306-315 is the order it keeps). */
