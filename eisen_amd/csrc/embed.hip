@@ -107,6 +107,7 @@ __global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const in
     __shared__ int sums[kBucketWaves][2];
     constexpr int LIST = 512;
     __shared__ int list[kBucketWaves][LIST];  // a wave's own ids, slot | index << 10, in order
+    static_assert(kBucketWaves * (kBucketSlots + LIST + 2) * sizeof(int) <= 160 << 10, "92 KB for the largest vocabulary, of a CU's 160 KB");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), bucket = blockIdx.x;
     const int here = (vocab + kBuckets - 1) >> kBucketBits;  // slots
     // (an odd number of 256-byte lines: the waves, and with them all workgroups, would otherwise ask one channel of the L2 at a time)
@@ -406,7 +407,7 @@ __global__ __launch_bounds__(kThreads) void scatter_merge_kernel(const int32_t* 
 //    work, and no list of runs.  (A wave to a run, its rows 16 at a time: 1396 ids, rows of 448 bf16, lookup and scatter 25.5 us, now 14.4.)
 // 32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 -> 91 us, of which lookup 15, index 14, scatter 40 (the 4649 occurrences of the first id).
 // The first workgroups take the long runs, the others the short ones.  first_bad, if given, points at kNoId or nothing is added.
-constexpr int kRunThreads = 320, kRunStage = 64, kRunWindow = 8;
+constexpr int kRunStage = 64;
 template <typename T> struct Four { typedef T type __attribute__((ext_vector_type(4))); };
 template <typename T> struct Two { typedef T type __attribute__((ext_vector_type(2))); };
 // four columns from col on of a row of `hidden`; WIDE: rows are whole packets, else they are whole pairs.  Columns past the end repeat
@@ -438,7 +439,7 @@ __device__ __forceinline__ void store_four(float* row, int col, int hidden, cons
 }
 // The number-th long run of the index, [begin, end), and its id; false if there are not as many.  All threads of the workgroup.  Every
 // thread looks at 4 of the multiples of 64 at once; what the marks leave open of begin and end are 64 places each.
-constexpr int kRunMarks = 4, kRunWaves = kRunThreads / kWave;
+constexpr int kRunMarks = 4;
 struct RunLds {
     unsigned long long starts[kRunMarks * kRunWaves], goes_on[kRunMarks * kRunWaves];  // bit l of [i]: multiple 64 * i + l of this turn
 };
@@ -582,7 +583,7 @@ __device__ __forceinline__ void scatter_long_run(const T* __restrict__ go, float
 template <typename T, bool WIDE>
 __global__ __launch_bounds__(kRunThreads, 3) void scatter_runs_kernel(const T* __restrict__ go, float* __restrict__ gw, const int32_t* __restrict__ ids,
                                                                   const int32_t* __restrict__ order, const int32_t* __restrict__ first_bad, int n, int hidden,
-                                                                  int long_blocks, int window) {
+                                                                  int long_blocks, int window, int first_block) {
     __shared__ __attribute__((aligned(16))) float stage[2 * 64 * kRunStage];
     __shared__ RunLds marks;
     if (first_bad && *first_bad != kNoId) return;
@@ -597,7 +598,7 @@ __global__ __launch_bounds__(kRunThreads, 3) void scatter_runs_kernel(const T* _
     }
     typedef Four<float>::type F4;
     const int slabs = (hidden + 255) / 256;
-    const int item = __builtin_amdgcn_readfirstlane(((int)blockIdx.x - long_blocks) * (kRunThreads / kWave) + (tid >> 6));
+    const int item = __builtin_amdgcn_readfirstlane(((int)blockIdx.x - long_blocks + first_block) * kRunWaves + (tid >> 6));
     const int col = (item % slabs * 64 + lane) * 4;
     F4 acc = {};
     int row = -1;  // of the run that is being added up
@@ -743,15 +744,12 @@ int scatter_launch_merge(eisen_ctx* ctx, size_t n_ids, size_t vocab, const Scatt
 
 template <typename T, bool WIDE>
 void scatter_launch_runs_as(eisen_ctx* ctx, const int32_t* index, const int32_t* first_bad, const void* go, float* gw, size_t n_ids, size_t hidden) {
-    // a workgroup for every long run (of more than 64 occurrences) and 64 columns that there can be, up to four per CU; a wave per window and 256 columns
-    // for the others
-    const size_t long_blocks = std::min<size_t>(1024, (n_ids - 1) / 64 * eisen_ceil_div(hidden, (size_t)64));
-    // (small batches: windows of 2 places, the waves are there)
-    const size_t slabs = eisen_ceil_div(hidden, (size_t)256), window = eisen_ceil_div(n_ids, (size_t)2) * slabs <= 4096 ? 2 : kRunWindow;
-    const size_t waves = eisen_ceil_div(n_ids, window) * slabs;
-    const size_t blocks = long_blocks + eisen_ceil_div(waves, (size_t)(kRunThreads / kWave));
-    scatter_runs_kernel<T, WIDE><<<(unsigned)blocks, kRunThreads, 0, ctx->stream>>>((const T*)go, gw, index, index + n_ids, first_bad, (int)n_ids, (int)hidden,
-                                                                                   (int)long_blocks, (int)window);
+    const ScatterRunsGrid g = scatter_runs_grid(n_ids, hidden);
+    for (size_t first = 0; first < g.short_blocks; first += kRunBlocksMax) {
+        const size_t longs = first == 0 ? g.long_blocks : 0, blocks = longs + std::min(kRunBlocksMax, g.short_blocks - first);
+        scatter_runs_kernel<T, WIDE><<<(unsigned)blocks, kRunThreads, 0, ctx->stream>>>((const T*)go, gw, index, index + n_ids, first_bad, (int)n_ids, (int)hidden,
+                                                                                       (int)longs, (int)g.window, (int)first);
+    }
 }
 void scatter_launch_runs(eisen_ctx* ctx, const int32_t* index, const int32_t* first_bad, const void* go, float* gw, int dtype, size_t n_ids, size_t hidden) {
     // whole 16-byte packets of a row where the sizes and addresses give them, pairs of columns otherwise

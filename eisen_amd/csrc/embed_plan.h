@@ -11,3 +11,15 @@ constexpr int kBucketBits = 8, kBuckets = 1 << kBucketBits, kBucketSlots = 960;
 constexpr int kBucketStep = 211;
 constexpr int scatter_bucket_of(int id) { return ((unsigned)id + ((unsigned)id >> kBucketBits) * kBucketStep) & (kBuckets - 1); }
 constexpr int scatter_bucket_id(int slot, int bucket) { return slot << kBucketBits | ((bucket - slot * kBucketStep) & (kBuckets - 1)); }
+
+// The scatter along the index: workgroups of five waves, the first long_blocks for the long runs, one for every long run and 64 columns that there can be, up to four per CU;
+// the others a wave per `window` places and 256 columns (small batches: windows of 2 places, the waves are there).
+constexpr int kRunThreads = 320, kRunWaves = kRunThreads / 64, kRunWindow = 8;
+constexpr size_t kRunBlocksMax = size_t(1) << 23;  // short_blocks of one launch, whose threads are fewer than 2^32; more of them are several launches
+struct ScatterRunsGrid {
+    size_t long_blocks, short_blocks, window;
+};
+inline ScatterRunsGrid scatter_runs_grid(size_t n_ids, size_t hidden) {
+    const size_t slabs = (hidden + 255) / 256, window = (n_ids + 1) / 2 * slabs <= 4096 ? 2 : kRunWindow, waves = (n_ids + window - 1) / window * slabs;
+    return {std::min<size_t>(1024, (n_ids - 1) / 64 * ((hidden + 63) / 64)), (waves + kRunWaves - 1) / kRunWaves, window};
+}

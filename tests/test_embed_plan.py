@@ -18,6 +18,17 @@ int main() {
     }
 }
 """
+GRID = """
+#include <cstdio>
+#include "embed_plan.h"
+int main() {
+    size_t n, hidden;
+    while (std::scanf("%zu %zu", &n, &hidden) == 2) {
+        const ScatterRunsGrid g = scatter_runs_grid(n, hidden);
+        std::printf("%zu %zu %zu %zu %d %d\\n", g.long_blocks, g.short_blocks, g.window, kRunBlocksMax, kRunThreads, kRunWaves);
+    }
+}
+"""
 
 
 @pytest.fixture(scope="module")
@@ -38,3 +49,16 @@ def test_ids_a_stride_apart_are_not_all_one_workgroups(bucket):
     for stride in range(1, 4097):
         ids = np.arange(0, bucket.size, stride)
         assert np.bincount(bucket[ids]).max() <= max(32, ids.size // 16), stride
+
+
+def test_the_scatters_launches_cover_all_rows_and_have_no_more_threads_than_a_launch_takes(tmp_path):
+    (tmp_path / "main.cpp").write_text(GRID)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "eisen_amd", "csrc"), str(tmp_path / "main.cpp"), "-o", str(tmp_path / "grid")])
+    # (rows of up to 2^30 - 1 columns, and as many of them as a card's memory holds: 121 of the widest, 2^20 of 131072)
+    sizes = [(1, 2), (64, 2), (65, 2), (8192, 256), (8193, 256), (32768, 1024), (1 << 20, 64), (121, (1 << 30) - 2), (1 << 20, 131072), (1, (1 << 30) - 2), (65536, 2_000_000)]
+    out = subprocess.run([str(tmp_path / "grid")], input="\n".join("%d %d" % s for s in sizes), capture_output=True, text=True, check=True).stdout
+    for (n, hidden), line in zip(sizes, out.splitlines()):
+        long_blocks, short_blocks, window, most, threads, waves = map(int, line.split())
+        assert (min(short_blocks, most) + long_blocks) * threads < 1 << 32
+        assert short_blocks * waves >= -(-n // window) * -(-hidden // 256) > (short_blocks - 1) * waves and short_blocks * waves < 1 << 31
+        assert (long_blocks > 0) == (n > 64) and window <= 8
