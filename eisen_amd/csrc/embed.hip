@@ -98,7 +98,10 @@ constexpr int kNoId = 0x7fffffff;
 // One launch: 256 workgroups, each with one id of every 256 in a row (scatter_bucket_of).  All of them read the whole batch (128 KB from the L2s for
 // 32768 ids), count what lies before their part and, per id and wave, their own, and place their positions; a wave's ids are consecutive, so the
 // places of an id ascend.  What bounds it is the dozen instructions per id and workgroup.  Chunks sorted by a bitonic network, merged and
-// listed in three launches had taken 30 us for 32768 ids, one chunk of up to 1024 and 2048 7.0 and 12.6; this takes 14.1, 4.7 and 5.1.
+// listed in three launches had taken 30 us for 32768 ids, 20.4 for 16384, one chunk of up to 1024 and 2048 7.2 and 11.9; this takes 14.6, 8.2, 5.1 and 5.0.
+// Built ahead beside a forward pass (Graph::gather) either hides: whole training steps with the index by sort and merge / by this, us (runs of one side differ by
+// 1 to 4 %): two layers of 64 in f32, 64 ids 254 / 253, 1024 273 / 271, 2048 286 / 286; two of 256 in bf16, 512 ids 308 / 309, 2048 372 / 371; two of 512, four
+// micro-batches of 1024 1704 / 1703; the ~14 M model, 8192 ids 1526 / 1527.
 constexpr int kBucketThreads = 1024, kBucketWaves = kBucketThreads / kWave;
 constexpr size_t kBucketMax = 65536, kBucketVocab = (size_t)kBuckets * kBucketSlots;
 __global__ __launch_bounds__(kBucketThreads) void scatter_bucket_kernel(const int32_t* __restrict__ ids, int n, int vocab, int32_t* __restrict__ out_ids,
@@ -659,11 +662,11 @@ __global__ __launch_bounds__(kRunThreads, 3) void scatter_runs_kernel(const T* _
     if (row >= 0) store_four<WIDE>(gw + (size_t)row * hidden, col, hidden, acc);
 }
 
-// How a batch beyond scatter_bucket_kernel's is sorted: chunks of 1024 << k ids, one workgroup each, whose keys (id, position in the chunk)
-// fit 32 bits, and a merge.  A batch of up to 2048 ids is one chunk (2048 ids: 11.8 us for the index, 15.6 in two chunks).  Beyond that
-// short chunks and a merge beat one long bitonic network, the shorter ones up to where the merge's searches, which grow with the
-// number of chunks, outweigh the sort (chunks of 1024 / 2048 / 4096 / all in one, us for the index when it ended with a list of the runs): 2049 ids
-// 15.7 / 19.7 / 19.5, 4096 16.6 / 20.8 / 20.2, 8192 17.7 / 21.9 / 29.8 / 39.6, 16384 20.3 / 24.4 / 32.6 / 85.  Beyond 65536 ids chunks of 16384.
+// How a batch beyond scatter_bucket_kernel's (a vocabulary above 245760, more than 65536 ids) is sorted: chunks of 1024 << k ids, one workgroup each, whose keys (id,
+// position in the chunk) fit 32 bits, and a merge.  A batch of up to 2048 ids is one chunk (index of 1500 and 2048 ids 9.2 us, in two chunks 10.8).  Beyond that short
+// chunks beat long ones up to where the merge's searches, which grow with their number, outweigh the sort (chunks of 1024 / 2048, us: index of 2049 ids 10.9 / 14.9,
+// 4096 11.6 / 15.7, 8192 12.3 / 16.6, 14000 12.9 / 17.3; index and scatter, rows of 64, of 16385 27.4 / 30.0, 24000 33.6 / 33.2, 32768 36.5 / 35.7, 65536 69 / 58).
+// Beyond 65536 ids chunks of 16384.
 struct ScatterPlan {
     int per_thread, shift;
     size_t chunk, chunks;
