@@ -2,6 +2,7 @@
 #include "graph.hpp"
 
 #include "../gemm_dw_rule.h"
+#include "../upload_rule.h"
 
 #include <algorithm>
 #include <cmath>
@@ -24,7 +25,7 @@ std::string shape_str(const std::vector<size_t>& s) {
     return r + "]";
 }
 constexpr size_t kHostCopyLimit = size_t(1) << 22;  // elements; token-id tensors are far below
-constexpr size_t kIdsLimit = size_t(24) << 10;      // elements that eisen_hip_htod_values takes in one launch
+constexpr size_t kIdsLimit = kCopyKernelBytes / sizeof(float);  // elements that eisen_hip_htod_values takes in one launch
 
 // Whether all values are whole numbers from 0 below 2^23 (in blocks: what is no ids says so in its first one).
 bool whole_numbers(const float* v, size_t n) {

@@ -4,6 +4,7 @@
 #include "runtime.h"
 
 #include "device_utils.cuh"
+#include "upload_rule.h"
 
 #include <algorithm>
 #include <atomic>
@@ -29,7 +30,6 @@ namespace {
 // for them 29 / 32, 192 KB 31 / 30 | 18 / 22, 256 KB 32 / 36 | 20 / 29: one workgroup reads 9 GB/s from the host.  (Not the tickets of eisen_hip_dtoh_begin: a
 // few bytes, where making them visible to the host writes the caches back: 1 us more than the event.)
 constexpr int kCopyThreads = 1024;
-constexpr size_t kCopyKernelBytes = size_t(96) << 10;
 
 template <typename T>
 __device__ __forceinline__ void copy_by_workgroup(const T* __restrict__ src, T* __restrict__ dst, unsigned n) {
@@ -539,6 +539,7 @@ extern "C" int eisen_hip_htod_values(eisen_ctx* ctx, void* dst, int dtype, int32
         memcpy(st->ptr, src, n * sizeof(float));
         st->number++;
         const float* from = static_cast<const float*>(st->ptr);
+        EisenProfScope prof(ctx, "htod_values", (double)n * (4.0 + eisen_dtype_size(dtype) + (ids ? 4.0 : 0.0)));
         if (dtype == EISEN_F32) copy_in_values_kernel<float><<<1, kCopyThreads, 0, ctx->stream>>>(from, static_cast<float*>(dst), ids, (unsigned)n, st->word, st->number);
         else copy_in_values_kernel<bf16_t><<<1, kCopyThreads, 0, ctx->stream>>>(from, static_cast<bf16_t*>(dst), ids, (unsigned)n, st->word, st->number);
         st->stream = ctx->stream;

@@ -82,6 +82,19 @@ def test_gather_from_a_loaded_tensor_again_and_after_another_load(g, beside):
     assert np.array_equal(g.sync_grad_to_cpu(w), np.stack([counts, counts], 1))
 
 
+@pytest.mark.parametrize("n,one", [(24576, True), (24577, False)])
+def test_token_ids_come_with_their_values_up_to_the_line_of_the_upload(ctx, n, one):
+    # the graph's line is the runtime's: no load takes the entry that brings both and finds it beyond what it takes in one launch
+    g = G.Graph(ctx, G.BF16_MIXED)
+    x = g.alloc_pooled((n,))
+    ids = np.arange(n, dtype=np.float32)
+    ctx.profile_start()
+    g.load_tensor_data(x, ids)
+    assert list(ctx.profile_stop()) == (["htod_values"] if one else [])
+    assert np.array_equal(g.sync_to_cpu(x), hip.round_bf16(ids))
+    g.close()
+
+
 def test_silu_gather_rmsnorm_ce_rope_reference(g):
     # SiLU closed form, tests/gpu_kernels.rs:114-152
     x = np.array([-2.0, -1.0, 0.0, 1.0, 2.0], np.float32)
