@@ -52,8 +52,9 @@ __global__ __launch_bounds__(kCopyThreads) void copy_in_kernel(const T* __restri
     if (threadIdx.x == 0) __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // f32 values to a tensor of T and, if asked for, as int32 beside it (token ids: what the lookup reads).  dst and ids begin 16 bytes aligned.
-// What bounds it is the latency of the host's memory, so one launch instead of three (the values, their rounding, the ids: 5 + 3 + 5 us): training steps of 8 micro-batches of
-// 1024 tokens 10427 -> 10338 us, of one of 1351 593 -> 584, of 64 (f32, where nothing is rounded) 272 -> 262.
+// What bounds it is the latency of the host's memory, so one launch instead of three (the values, their rounding, the ids: 5 + 3 + 5 us): training steps, three launches / one, six
+// processes each, us: 8 micro-batches of 1024 tokens, hidden 1024, 10444 / 10366 (a side's runs within 20), one of 2048, hidden 256, 384 / 376, one of 1351, hidden 288, 593 / 585, of 4096
+// in f32, where nothing is rounded, 2417 / 2411; of 64 in f32 261 / 258, within what runs differ by.
 template <typename T>
 __global__ __launch_bounds__(kCopyThreads) void copy_in_values_kernel(const float* __restrict__ src, T* __restrict__ dst, int* __restrict__ ids, unsigned n, unsigned* word,
                                                                       unsigned number) {
