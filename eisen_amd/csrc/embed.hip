@@ -94,6 +94,7 @@ __global__ __launch_bounds__(kThreads) void scatter_rows_scalar_kernel(const T* 
 // index = [ids | positions], n ints each: the positions of every id stand together, in ascending order, beside the id (in which order
 // the ids follow one another is each builder's own).  Ids outside [0, vocab) stand behind all others as kNoId and belong to no run.
 constexpr int kNoId = 0x7fffffff;
+constexpr size_t kIndexMax = size_t(1) << 20;  // ids of a batch that is indexed on the device
 
 // One launch: 256 workgroups, each with one id of every 256 in a row (scatter_bucket_of).  All of them read the whole batch (128 KB from the L2s for
 // 32768 ids), count what lies before their part and, per id and wave, their own, and place their positions; a wave's ids are consecutive, so the
@@ -402,13 +403,17 @@ __global__ __launch_bounds__(kThreads) void scatter_merge_kernel(const int32_t* 
 // gw[row] = ((gw[row] + go[i1]) + go[i2]) + ... with i1 < i2 < ... (the CPU arm's order, src/graph/ops/transform.rs:309-314):
 // a run is one chain of dependent adds per column, whatever the schedule.  What bounds it is how many rows of dOut are in
 // flight, and for the hot rows of text (thousands of occurrences) the length of the chain:
-//  * a long run, one that holds two multiples of 64 among its places in the index, is a workgroup's per 64 columns: four waves fetch its
-//    rows, four rows of four columns to a thread and several stages ahead, and leave them in LDS as f32, the rows of a column side by
-//    side; the first wave, a lane to a column, adds: a quarter of an LDS read and one add per row.  With the adding wave among those
-//    that fetch, rows in bf16 and read by columns, a run of 16384 took 8.2 ns per row; now 5.8, of which 2 are the chain of adds.
+//  * a long run, one that holds two or three multiples of 64 among its places in the index (ScatterRunsGrid), is a workgroup's per 64
+//    columns: four waves fetch its rows, four rows of four columns to a thread and several stages ahead, and leave them in LDS as f32,
+//    the rows of a column side by side; the first wave, a lane to a column, adds: a quarter of an LDS read and one add per row.  With
+//    the adding wave among those that fetch, rows in bf16 and read by columns, a run of 16384 took 8.2 ns per row; now 5.8, of which 2
+//    are the chain of adds.  What a run costs beside that is its start, three waits in a row: the workgroup marks the long runs of the
+//    whole index in LDS once, and finds the next one there.  (With a search of the index for every run, 32768 ids of 256, rows of 1024
+//    bf16, took 90 us with the index, and 57 with the runs listed in launches of their own; now 40.  The last turn of a run without
+//    requests for rows past its end: such batches 1 to 4 % shorter, but the hot runs of text 5 % longer.)
 //  * the short runs that begin in 2 or 8 places in a row are a wave's per 256 columns, all their rows in flight: waves with equal
 //    work, and no list of runs.  (A wave to a run, its rows 16 at a time: 1396 ids, rows of 448 bf16, lookup and scatter 25.5 us, now 14.4.)
-// 32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 -> 91 us, of which lookup 15, index 14, scatter 40 (the 4649 occurrences of the first id).
+// 32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 -> 91 us, of which lookup 15, index 14.5, scatter 39 (the 4649 occurrences of the first id).
 // The first workgroups take the long runs, the others the short ones.  first_bad, if given, points at kNoId or nothing is added.
 constexpr int kRunStage = 64;
 template <typename T> struct Four { typedef T type __attribute__((ext_vector_type(4))); };
@@ -440,70 +445,74 @@ __device__ __forceinline__ void store_four(float* row, int col, int hidden, cons
             if (col + j < hidden) *reinterpret_cast<float2*>(row + col + j) = make_float2(x[j], x[j + 1]);
     }
 }
-// The number-th long run of the index, [begin, end), and its id; false if there are not as many.  All threads of the workgroup.  Every
-// thread looks at 4 of the multiples of 64 at once; what the marks leave open of begin and end are 64 places each.
-constexpr int kRunMarks = 4;
+// The multiples of 64 among the places of the index, 64 to a word, and for each word the number of long runs whose first multiple lies up to its end.
+constexpr int kMarkWords = kIndexMax / 64 / 64;
 struct RunLds {
-    unsigned long long starts[kRunMarks * kRunWaves], goes_on[kRunMarks * kRunWaves];  // bit l of [i]: multiple 64 * i + l of this turn
+    unsigned long long starts[kMarkWords], goes_on[kMarkWords];  // bit l of word i, multiple 64 * i + l: the first of a long run; the next one is of the same run
+    int upto[kMarkWords];
 };
-__device__ __forceinline__ bool find_long_run(const int32_t* __restrict__ ids, int n, int number, RunLds& lds, int& begin, int& end, int& id) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int marks = (n + 63) / 64;
-    int first = -1, last = -1;  // the run's first and last multiple
-    for (int k0 = 0; k0 < marks && last < 0; k0 += kRunMarks * kRunThreads) {
-        int x[kRunMarks][3];
+// Marks them; how many long runs there are.  All threads of the workgroup.
+__device__ __forceinline__ int mark_long_runs(const int32_t* __restrict__ ids, int n, int long_marks, RunLds& lds) {
+    constexpr int U = 4;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, words = ((n + 63) / 64 + 63) / 64;
+    for (int w0 = wave; w0 < words; w0 += U * kRunWaves) {
+        int x[U][4];  // the multiple before, this one, the next, and the last one that a long run from here on holds at least
 #pragma unroll
-        for (int u = 0; u < kRunMarks; u++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int j = 0; j < 3; j++) x[u][j] = ids[min(max((k0 + u * kRunThreads + (int)threadIdx.x + j - 1) * 64, 0), n - 1)];
-        __syncthreads();  // the marks of the turn or the search before have been read
+            for (int j = 0; j < 4; j++) x[u][j] = ids[min(max(((w0 + u * kRunWaves) * 64 + lane + (j < 3 ? j - 1 : long_marks - 1)) * 64, 0), n - 1)];
 #pragma unroll
-        for (int u = 0; u < kRunMarks; u++) {
-            const int k = k0 + u * kRunThreads + threadIdx.x;
-            const bool behind = (k + 1) * 64 < n && x[u][1] != kNoId && x[u][2] == x[u][1], ahead = k > 0 && x[u][0] == x[u][1];
-            const unsigned long long starts = __ballot(behind && !ahead), goes_on = __ballot(behind);
-            if (lane == 0) {
-                lds.starts[u * kRunWaves + wave] = starts;
-                lds.goes_on[u * kRunWaves + wave] = goes_on;
+        for (int u = 0; u < U; u++) {
+            const int w = w0 + u * kRunWaves, k = w * 64 + lane;
+            const bool in = (k + 1) * 64 < n && x[u][1] != kNoId, ahead = k > 0 && x[u][0] == x[u][1];
+            const bool is_long = in && (k + long_marks - 1) * 64 < n && x[u][3] == x[u][1];
+            const unsigned long long starts = __ballot(is_long && !ahead), goes_on = __ballot(in && x[u][2] == x[u][1]);
+            if (lane == 0 && w < words) {
+                lds.starts[w] = starts;
+                lds.goes_on[w] = goes_on;
             }
         }
-        __syncthreads();
-        constexpr int WORDS = kRunMarks * kRunWaves;  // lane i takes word i
-        static_assert(WORDS <= 32, "a wave's prefix sums");
-        const unsigned long long starts = lane < WORDS ? lds.starts[lane] : 0, on = lane < WORDS ? lds.goes_on[lane] : ~0ull;
-        unsigned long long stops = ~on;
-        if (first < 0) {
-            const int count = __popcll(starts);
-            int upto = count;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        int before = 0;
+        for (int w0 = 0; w0 < words; w0 += kWave) {
+            int upto = w0 + lane < words ? __popcll(lds.starts[w0 + lane]) : 0;
 #pragma unroll
-            for (int o = 1; o < 32; o <<= 1) {
+            for (int o = 1; o < 64; o <<= 1) {
                 const int other = __shfl_up(upto, o, 64);
                 if (lane >= o) upto += other;
             }
-            const unsigned long long hit = __ballot(number >= upto - count && number < upto);
-            if (!hit) {
-                number -= __builtin_amdgcn_readlane(upto, WORDS - 1);
-                continue;
-            }
-            const int word = __ffsll(hit) - 1;
-            unsigned long long left = __shfl(starts, word, 64);
-            for (int skip = number - __builtin_amdgcn_readlane(upto - count, word); skip > 0; skip--) left &= left - 1;
-            const int bit = __ffsll(left) - 1;
-            first = k0 + word * 64 + bit;
-            stops = lane < word ? 0 : lane == word ? stops & ~((1ull << bit) - 1) : stops;
+            if (w0 + lane < words) lds.upto[w0 + lane] = before + upto;
+            before += __builtin_amdgcn_readlane(upto, 63);
         }
-        const unsigned long long ends = __ballot(stops != 0);
-        if (ends) last = k0 + (__ffsll(ends) - 1) * 64 + __ffsll((unsigned long long)__shfl(stops, __ffsll(ends) - 1, 64)) - 1;
     }
-    if (first < 0) return false;
-    if (last < 0) last = marks - 1;
-    first = __builtin_amdgcn_readfirstlane(first);
-    last = __builtin_amdgcn_readfirstlane(last);
-    id = __builtin_amdgcn_readfirstlane(ids[first * 64]);
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(lds.upto[words - 1]);
+}
+// The number-th of them, [begin, end), and its id.  What the marks leave open of begin and end are 64 places each.
+__device__ __forceinline__ void find_long_run(const int32_t* __restrict__ ids, int n, int number, const RunLds& lds, int& begin, int& end, int& id) {
+    const int lane = threadIdx.x & 63, words = ((n + 63) / 64 + 63) / 64;
+    int word = 0;
+    for (int w0 = 0; w0 < words; w0 += kWave) {  // the first word up to whose end there are more
+        const unsigned long long hit = __ballot(w0 + lane < words && lds.upto[w0 + lane] > number);
+        if (hit) {
+            word = w0 + __ffsll(hit) - 1;
+            break;
+        }
+    }
+    unsigned long long left = lds.starts[word];
+    for (int skip = number - (lds.upto[word] - __popcll(left)); skip > 0; skip--) left &= left - 1;
+    const int bit = __ffsll(left) - 1;
+    unsigned long long stops = ~lds.goes_on[word] & ~((1ull << bit) - 1);
+    int at = word;
+    while (!stops) stops = ~lds.goes_on[++at];  // (the last multiple goes on nowhere)
+    const int first = __builtin_amdgcn_readfirstlane(word * 64 + bit), last = __builtin_amdgcn_readfirstlane(at * 64 + __ffsll(stops) - 1);
     const int before = first * 64 - 63 + lane, after = last * 64 + 1 + lane;
-    begin = first * 64 - 63 + __ffsll(__ballot(before >= 0 && ids[max(before, 0)] == id)) - 1;
-    end = last * 64 + 1 + __popcll(__ballot(after < n && ids[min(after, n - 1)] == id));
-    return true;
+    const int at_first = ids[first * 64], at_before = ids[max(before, 0)], at_after = ids[min(after, n - 1)];  // (one wait for all three)
+    id = __builtin_amdgcn_readfirstlane(at_first);
+    begin = first * 64 - 63 + __ffsll(__ballot(before >= 0 && at_before == id)) - 1;
+    end = last * 64 + 1 + __popcll(__ballot(after < n && at_after == id));
 }
 // Where four rows of a column stand in a stage: turned so that 16 lanes in a row meet all banks, be they neighbouring columns (the adding
 // wave's) or every fourth (those of the waves that fetch).
@@ -586,80 +595,91 @@ __device__ __forceinline__ void scatter_long_run(const T* __restrict__ go, float
 template <typename T, bool WIDE>
 __global__ __launch_bounds__(kRunThreads, 3) void scatter_runs_kernel(const T* __restrict__ go, float* __restrict__ gw, const int32_t* __restrict__ ids,
                                                                   const int32_t* __restrict__ order, const int32_t* __restrict__ first_bad, int n, int hidden,
-                                                                  int long_blocks, int window, int first_block) {
+                                                                  int long_blocks, int long_marks, int window, int first_block) {
     __shared__ __attribute__((aligned(16))) float stage[2 * 64 * kRunStage];
     __shared__ RunLds marks;
     if (first_bad && *first_bad != kNoId) return;
     const int tid = threadIdx.x, lane = tid & 63;
     if ((int)blockIdx.x < long_blocks) {
-        const int slabs = (hidden + 63) / 64;
-        for (int item = blockIdx.x;; item += long_blocks) {
+        const int slabs = (hidden + 63) / 64, items = mark_long_runs(ids, n, long_marks, marks) * slabs;
+        for (int item = blockIdx.x; item < items; item += long_blocks) {
             int begin, end, id;
-            if (!find_long_run(ids, n, item / slabs, marks, begin, end, id)) return;
+            find_long_run(ids, n, item / slabs, marks, begin, end, id);
             scatter_long_run<T, WIDE>(go, gw, order, hidden, id, begin, end, item % slabs * 64, stage);
         }
+        return;
     }
     typedef Four<float>::type F4;
+    constexpr int ROWS = sizeof(T) == 2 ? 32 : 16;  // in flight behind the window (more in f32: fewer waves on a SIMD, also for the long runs)
     const int slabs = (hidden + 255) / 256;
     const int item = __builtin_amdgcn_readfirstlane(((int)blockIdx.x - long_blocks + first_block) * kRunWaves + (tid >> 6));
     const int col = (item % slabs * 64 + lane) * 4;
     F4 acc = {};
     int row = -1;  // of the run that is being added up
     auto row_of = [&](int pos, int u) { return load_four<WIDE>(go + (size_t)__builtin_amdgcn_readlane(pos, u) * hidden, col, hidden); };
-    for (int p = item / slabs * window, first = p; p < n; p += kWave) {
-        const int i = p + lane, far = ((i + 63) & ~63) + 64;
-        const int id = i < n ? ids[i] : kNoId, ahead = i > 0 && i < n ? ids[i - 1] : -1, behind = far < n ? ids[far] : -1, pos = i < n ? order[i] : 0;
-        const unsigned long long in_window = (1ull << window) - 1;
-        const unsigned long long past = __ballot(id == kNoId), begins = __ballot(id != kNoId && id != ahead), is_long = __ballot(id != kNoId && id != ahead && id == behind);
-        // from the first run that begins in the window on, up to a long one, or to where the last run ends
-        unsigned long long stop = begins | past;
-        int done = 0;
-        if (p == first) {
-            if (!(begins & in_window)) return;
-            stop = (is_long & in_window) | (begins & ~in_window) | past;
-            const int from = __ffsll(begins) - 1, to = stop ? min(__ffsll(stop) - 1, window) : window;
-            typename Four<T>::type x[kRunWindow];
-            F4 g[kRunWindow];
+    int p = item / slabs * window;
+    if (p >= n) return;
+    const int i = p + lane, far = ((i + 63) & ~63) + 64 * (long_marks - 1);
+    const int id = i < n ? ids[i] : kNoId, ahead = i > 0 && i < n ? ids[i - 1] : -1, behind = far < n ? ids[far] : -1;
+    int pos = i < n ? order[i] : 0;
+    const unsigned long long in_window = (1ull << window) - 1;
+    const unsigned long long past = __ballot(id == kNoId), begins = __ballot(id != kNoId && id != ahead), is_long = __ballot(id != kNoId && id != ahead && id == behind);
+    if (!(begins & in_window)) return;
+    // from the first run that begins in the window on, up to a long one, or to where the last run ends
+    const unsigned long long stop = (is_long & in_window) | (begins & ~in_window) | past;
+    const int end = stop ? __ffsll(stop) - 1 : kWave;
+    {
+        const int from = __ffsll(begins) - 1, to = min(end, window);
+        typename Four<T>::type x[kRunWindow];
+        F4 g[kRunWindow];
 #pragma unroll
-            for (int u = 0; u < kRunWindow; u++)
-                if (u >= from && u < to) {
-                    x[u] = row_of(pos, u);
-                    if (begins >> u & 1) g[u] = load_four<WIDE>(gw + (size_t)__builtin_amdgcn_readlane(id, u) * hidden, col, hidden);
+        for (int u = 0; u < kRunWindow; u++)
+            if (u >= from && u < to) {
+                x[u] = row_of(pos, u);
+                if (begins >> u & 1) g[u] = load_four<WIDE>(gw + (size_t)__builtin_amdgcn_readlane(id, u) * hidden, col, hidden);
+            }
+        // all of them have arrived: behind the branches the compiler would wait for everything at each use, the stores in between included
+#pragma unroll
+        for (int u = 0; u < kRunWindow; u++) asm volatile("" : "+v"(x[u]), "+v"(g[u]));
+#pragma unroll
+        for (int u = 0; u < kRunWindow; u++)
+            if (u >= from && u < to) {
+                if (begins >> u & 1) {
+                    if (row >= 0) store_four<WIDE>(gw + (size_t)row * hidden, col, hidden, acc);
+                    acc = g[u];
+                    row = __builtin_amdgcn_readlane(id, u);
                 }
-            // all of them have arrived: behind the branches the compiler would wait for everything at each use, the stores in between included
 #pragma unroll
-            for (int u = 0; u < kRunWindow; u++) asm volatile("" : "+v"(x[u]), "+v"(g[u]));
+                for (int j = 0; j < 4; j++) acc[j] += (float)x[u][j];
+            }
+        if (row < 0) return;
+    }
+    // what is left of the last run, here and in the next 64 places, whose ids and positions are requested before these rows
+    for (int done = window, to = end;;) {
+        const int next = p + kWave + lane;
+        const bool more = to == kWave && next < n;
+        const int next_id = more ? ids[next] : kNoId, next_pos = more ? order[next] : 0;
+        for (; done < to; done += ROWS) {
+            typename Four<T>::type x[ROWS];
 #pragma unroll
-            for (int u = 0; u < kRunWindow; u++)
-                if (u >= from && u < to) {
-                    if (begins >> u & 1) {
-                        if (row >= 0) store_four<WIDE>(gw + (size_t)row * hidden, col, hidden, acc);
-                        acc = g[u];
-                        row = __builtin_amdgcn_readlane(id, u);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; j++) acc[j] += (float)x[u][j];
-                }
-            if (row < 0) return;
-            done = window;
-        }
-        const int to = stop ? __ffsll(stop) - 1 : kWave;
-        for (; done < to; done += 2 * kRunWindow) {  // what is left of the last run
-            typename Four<T>::type x[2 * kRunWindow];
-#pragma unroll
-            for (int u = 0; u < 2 * kRunWindow; u++)
+            for (int u = 0; u < ROWS; u++)
                 if (done + u < to) x[u] = row_of(pos, done + u);
 #pragma unroll
-            for (int u = 0; u < 2 * kRunWindow; u++) asm volatile("" : "+v"(x[u]));
+            for (int u = 0; u < ROWS; u++) asm volatile("" : "+v"(x[u]));
 #pragma unroll
-            for (int u = 0; u < 2 * kRunWindow; u++)
+            for (int u = 0; u < ROWS; u++)
                 if (done + u < to)
 #pragma unroll
                     for (int j = 0; j < 4; j++) acc[j] += (float)x[u][j];
         }
         if (to < kWave) break;
+        p += kWave;
+        pos = next_pos;
+        done = 0;
+        const unsigned long long other = __ballot(next_id != row);
+        to = other ? __ffsll(other) - 1 : kWave;
     }
-    if (row >= 0) store_four<WIDE>(gw + (size_t)row * hidden, col, hidden, acc);
+    store_four<WIDE>(gw + (size_t)row * hidden, col, hidden, acc);
 }
 
 // How a batch beyond scatter_bucket_kernel's (a vocabulary above 245760, more than 65536 ids) is sorted: chunks of 1024 << k ids, one workgroup each, whose keys (id,
@@ -671,7 +691,6 @@ struct ScatterPlan {
     int per_thread, shift;
     size_t chunk, chunks;
 };
-constexpr size_t kIndexMax = size_t(1) << 20;
 bool scatter_plan(size_t n_ids, size_t vocab, ScatterPlan* plan) {
     if (n_ids == 0 || n_ids > kIndexMax) return false;
     const int per_thread = n_ids <= 1024 ? 1 : n_ids <= 2048 ? 2 : n_ids <= kSortMax ? 1 : n_ids <= 65536 ? 2 : 16;
@@ -751,7 +770,7 @@ void scatter_launch_runs_as(eisen_ctx* ctx, const int32_t* index, const int32_t*
     for (size_t first = 0; first < g.short_blocks; first += kRunBlocksMax) {
         const size_t longs = first == 0 ? g.long_blocks : 0, blocks = longs + std::min(kRunBlocksMax, g.short_blocks - first);
         scatter_runs_kernel<T, WIDE><<<(unsigned)blocks, kRunThreads, 0, ctx->stream>>>((const T*)go, gw, index, index + n_ids, first_bad, (int)n_ids, (int)hidden,
-                                                                                       (int)longs, (int)g.window, (int)first);
+                                                                                       (int)longs, g.long_marks, (int)g.window, (int)first);
     }
 }
 void scatter_launch_runs(eisen_ctx* ctx, const int32_t* index, const int32_t* first_bad, const void* go, float* gw, int dtype, size_t n_ids, size_t hidden) {

@@ -25,7 +25,7 @@ int main() {
     size_t n, hidden;
     while (std::scanf("%zu %zu", &n, &hidden) == 2) {
         const ScatterRunsGrid g = scatter_runs_grid(n, hidden);
-        std::printf("%zu %zu %zu %zu %d %d\\n", g.long_blocks, g.short_blocks, g.window, kRunBlocksMax, kRunThreads, kRunWaves);
+        std::printf("%zu %zu %zu %zu %d %d %d\\n", g.long_blocks, g.short_blocks, g.window, kRunBlocksMax, kRunThreads, kRunWaves, g.long_marks);
     }
 }
 """
@@ -58,7 +58,7 @@ def test_the_scatters_launches_cover_all_rows_and_have_no_more_threads_than_a_la
     sizes = [(1, 2), (64, 2), (65, 2), (8192, 256), (8193, 256), (32768, 1024), (1 << 20, 64), (121, (1 << 30) - 2), (1 << 20, 131072), (1, (1 << 30) - 2), (65536, 2_000_000)]
     out = subprocess.run([str(tmp_path / "grid")], input="\n".join("%d %d" % s for s in sizes), capture_output=True, text=True, check=True).stdout
     for (n, hidden), line in zip(sizes, out.splitlines()):
-        long_blocks, short_blocks, window, most, threads, waves = map(int, line.split())
+        long_blocks, short_blocks, window, most, threads, waves, long_marks = map(int, line.split())
         assert (min(short_blocks, most) + long_blocks) * threads < 1 << 32
         assert short_blocks * waves >= -(-n // window) * -(-hidden // 256) > (short_blocks - 1) * waves and short_blocks * waves < 1 << 31
-        assert (long_blocks > 0) == (n > 64) and window <= 8
+        assert (long_blocks > 0) == (-(-n // 64) >= long_marks) and long_marks in (2, 3) and window <= 8  # (a long run needs that many multiples of 64)
