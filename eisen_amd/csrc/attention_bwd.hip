@@ -394,7 +394,8 @@ bool eisen_attention_writes_over_operand(const AttnArgs& a, size_t element) {
 // them at once (two workgroups to a CU; one for head sizes above 64), beside those of the dQ pass that share the launch, the pair would only be done one after the
 // other.  The results are the same to the bit.  Backward with pairs / without, us, batch x sequence, query heads on KV heads, head size: 10 x 44 8 on 8 64 7.9 / 6.2; 1 x
 // 130 3 on 3 64 9.2 / 7.2; 7 x 193 6 on 6 48 8.9 / 8.1; 1 x 506 4 on 2 64 20.6 / 18.2; 3 x 512 8 on 8 64 16.2 / 14.2; 2 x 1000 6 on 6 64 24.7 / 21.3; 1 x 512 8 on 4
-// 96 30.1 / 26.3; 1 x 2048 2 on 2 128 61.8 / 57.2; in two launches 2 x 448 9 on 3 80 34.2 / 29.2; 7 x 668 6 on 3 64 30.0 / 30.0.
+// 96 30.1 / 26.3; 1 x 2048 2 on 2 128 61.8 / 57.2; in two launches 2 x 448 9 on 3 80 34.2 / 29.2; 7 x 668 6 on 3 64 30.0 / 30.0.  (Of 89 shapes at random that go one by one 7 lose by it, 2 % at most,
+// 1 x 3590 16 on 4 64 140.8 / 143.2; the median gains 13 %.)
 static bool key_blocks_paired(const AttnArgs& a, int dq_blocks) { return dq_blocks + (long long)((a.S + 31) / 32) * a.Hkv * a.B > (a.hd <= 64 ? 512 : 256); }
 
 // Where one launch (fa_bwd_dkv32_kernel with GW > 0) takes less time than two: where every workgroup is on the chip at once, two to a CU (head sizes above 64: one), and a
