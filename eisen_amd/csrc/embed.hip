@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kThreads) void scatter_merge_kernel(const int32_t* 
 //    requests for rows past its end: such batches 1 to 4 % shorter, but the hot runs of text 5 % longer.)
 //  * the short runs that begin in 2 or 8 places in a row are a wave's per 256 columns, all their rows in flight: waves with equal
 //    work, and no list of runs.  (A wave to a run, its rows 16 at a time: 1396 ids, rows of 448 bf16, lookup and scatter 25.5 us, now 14.4.)
-// 32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 -> 91 us, of which lookup 15, index 14.5, scatter 39 (the 4649 occurrences of the first id).
+// 32768 Zipf ids, rows of 1024 bf16, lookup and scatter: 114 -> 92 us, of which lookup 15, index 14.5, scatter 38 (the 4649 occurrences of the first id).
 // The first workgroups take the long runs, the others the short ones.  first_bad, if given, points at kNoId or nothing is added.
 // Four workgroups to a CU (96 registers in bf16).  With three the hot run of text has a little less beside it, everything else waits: 32768
 // Zipf ids x 1024 looked up and scattered from memory 90.9 / 92.2 us, but the scatter alone, three / four, of 32768 ids of 256 x 1024 49.7 / 46.8, of
